@@ -43,6 +43,11 @@ struct gz_packed_vec {
  * it each reads 16 words and sends a round of sources with more vectors than
  * one batch to the overflow queue. */
 #define GZ_SPARSE_PUSH_WIDE_VOTE 4096
+/* Wavefronts that push aims for before it widens a wavefront's share (two
+ * per SIMD).  CC over R-MAT s16 with trees 529 -> 387 us per run against 16
+ * words throughout; eight searches on R-MAT s17, s20, s24 with 512, 2048 and
+ * 8192: 2198 / 2260 / 2255, 2762 / 2696 / 2894, 8824 / 8804 / 8995 us. */
+#define GZ_SPARSE_PUSH_MIN_WAVES 2048
 /* Overflow queue: pieces of at most this many vectors (one batch of four
  * steps of 64), and room for this many pieces. */
 #define GZ_PUSH_PIECE_VECTORS 256

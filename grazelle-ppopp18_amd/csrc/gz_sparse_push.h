@@ -273,10 +273,22 @@ static inline bool gz_push_sparse_eligible(uint64_t hint)
 }
 
 /* Words of the bitmap one wavefront of the sparse push reads for a vote of
- * `hint`: a tiny frontier pays mostly for the grid; a larger one for the
- * wavefront that holds the most sources, so it gets fewer words each and the
- * overflow queue. */
-static inline uint64_t gz_push_sparse_words(uint64_t hint) { return hint <= GZ_SPARSE_PUSH_WIDE_VOTE ? 64 : 16; }
+ * `hint`.  A tiny frontier (up to GZ_SPARSE_PUSH_WIDE_VOTE) pays mostly for
+ * the grid, so a wavefront takes up to 64 words; a larger one for the
+ * wavefront that holds the most sources, so at most 16 and the overflow
+ * queue.  On a small graph those widths leave most SIMDs idle (64 wavefronts
+ * of 16 words at 2^16 vertices, each with a chain of several rounds), so the
+ * width shrinks by four until there are GZ_SPARSE_PUSH_MIN_WAVES wavefronts. */
+static inline uint64_t gz_push_sparse_words(uint64_t hint)
+{
+    const uint64_t nwords = (gz_graph.num_vertices + 63) >> 6;
+    uint64_t words = hint <= GZ_SPARSE_PUSH_WIDE_VOTE ? 64 : 16;
+    while (words > 1 && nwords < words * GZ_SPARSE_PUSH_MIN_WAVES) words /= 4;
+    return words;
+}
+
+/* Whether the push of a vote of `hint` sends long rounds to the queue. */
+static inline bool gz_push_sparse_queued(uint64_t hint) { return hint > GZ_SPARSE_PUSH_WIDE_VOTE; }
 
 /* Per-wave partials the sparse push writes for a vote of `hint`. */
 static inline uint64_t gz_push_sparse_waves(uint64_t hint)
@@ -284,7 +296,7 @@ static inline uint64_t gz_push_sparse_waves(uint64_t hint)
     const uint64_t words = gz_push_sparse_words(hint);
     const uint64_t waves = (((gz_graph.num_vertices + 63) >> 6) + words - 1) / words;
     const uint64_t blocks = (waves + GZ_WAVES_PER_BLOCK - 1) / GZ_WAVES_PER_BLOCK;
-    const uint64_t qblocks = (words == 64) ? 0 : GZ_PERSISTENT_BLOCKS / 4;
+    const uint64_t qblocks = gz_push_sparse_queued(hint) ? GZ_PERSISTENT_BLOCKS / 4 : 0;
     return (blocks + qblocks) * GZ_WAVES_PER_BLOCK;
 }
 
@@ -299,10 +311,10 @@ static void gz_launch_push_sparse(const Op& op, const gz_vec_t* edge_list, uint6
 {
     const uint64_t V = gz_graph.num_vertices;
     const uint64_t words = gz_push_sparse_words(hint);
-    const bool wide = words == 64;
+    const bool queued = gz_push_sparse_queued(hint);
     const uint64_t waves = (((V + 63) >> 6) + words - 1) / words;
     const uint64_t blocks = (waves + GZ_WAVES_PER_BLOCK - 1) / GZ_WAVES_PER_BLOCK;
-    const uint64_t qblocks = wide ? 0 : GZ_PERSISTENT_BLOCKS / 4;
+    const uint64_t qblocks = queued ? GZ_PERSISTENT_BLOCKS / 4 : 0;
     const uint64_t sw = blocks * GZ_WAVES_PER_BLOCK, all = sw + qblocks * GZ_WAVES_PER_BLOCK;
     gz_scratch_reserve(all, V);
     gz_scratch.partials_is_double = 0;
@@ -315,11 +327,23 @@ static void gz_launch_push_sparse(const Op& op, const gz_vec_t* edge_list, uint6
         gz_graph.frontier_has_info, V, gz_scratch.push_pieces, gz_scratch.push_queue + parity,                    \
         (uint64_t)gz_push_queue_cap, partials, gz_scratch.stats, gz_phase_config.collect_stats, stamp,             \
         gz_guard{nullptr, 0}
-    if (wide) {
-        hipLaunchKernelGGL((gz_k_push_sparse<Op, 64, false>), GZ_PUSH_SPARSE_ARGS);
+    if (!queued) {
+        if (words == 64)
+            hipLaunchKernelGGL((gz_k_push_sparse<Op, 64, false>), GZ_PUSH_SPARSE_ARGS);
+        else if (words == 16)
+            hipLaunchKernelGGL((gz_k_push_sparse<Op, 16, false>), GZ_PUSH_SPARSE_ARGS);
+        else if (words == 4)
+            hipLaunchKernelGGL((gz_k_push_sparse<Op, 4, false>), GZ_PUSH_SPARSE_ARGS);
+        else
+            hipLaunchKernelGGL((gz_k_push_sparse<Op, 1, false>), GZ_PUSH_SPARSE_ARGS);
         GZ_LAUNCH_CHECK();
     } else {
-        hipLaunchKernelGGL((gz_k_push_sparse<Op, 16, true>), GZ_PUSH_SPARSE_ARGS);
+        if (words == 16)
+            hipLaunchKernelGGL((gz_k_push_sparse<Op, 16, true>), GZ_PUSH_SPARSE_ARGS);
+        else if (words == 4)
+            hipLaunchKernelGGL((gz_k_push_sparse<Op, 4, true>), GZ_PUSH_SPARSE_ARGS);
+        else
+            hipLaunchKernelGGL((gz_k_push_sparse<Op, 1, true>), GZ_PUSH_SPARSE_ARGS);
         GZ_LAUNCH_CHECK();
         hipLaunchKernelGGL((gz_k_push_pieces<Op>), dim3((unsigned)qblocks), dim3(GZ_BLOCK), 0, gz_stream, op,
                            edge_list, gz_scratch.push_pieces, gz_scratch.push_queue, (uint64_t)gz_push_queue_cap,

@@ -1,0 +1,119 @@
+"""Work splits of the small-graph paths at the sizes where they change.
+
+The scheduler-aware PageRank pull gives a chunk a workgroup of four
+wavefronts on lists of at most 8192 chunks, and the sparse push gives a
+wavefront 1, 4, 16 or 64 bitmap words by vertex count.  Bars as for every
+other width: PageRank within 1e-12 of FP64 numpy (each sum is regrouped, and
+2^-53 times the at most 20 iterations and a few thousand terms of a sum
+stays below it; the oracle adds S over all edges in one chain, whose own
+rounding passes that on the lists of millions of equal terms here), CC labels
+and BFS words bit-exact with the oracle.
+"""
+import numpy as np
+import pytest
+
+import graphs
+
+pytestmark = pytest.mark.gpu
+
+PR_TOL = 1e-12
+
+
+def _rel(a, b):
+    return float(np.max(np.abs(a - b) / np.maximum(np.abs(b), 1e-300)))
+
+
+def _ranks(g, iterations, damping=0.875):
+    """PageRank in numpy: per-destination sums, S summed pairwise."""
+    src, dst = g.pull[:, 0].astype(np.int64), g.pull[:, 1].astype(np.int64)
+    nv = float(g.num_vertices)
+    deg = np.bincount(src, minlength=g.num_vertices).astype(np.float64)
+    deg[deg == 0] = nv
+    props = 1.0 / nv / deg
+    for _ in range(iterations):
+        acc = np.bincount(dst, weights=props[src], minlength=g.num_vertices)
+        props = ((acc + (1.0 - acc.sum()) / nv) * damping + (1.0 - damping) / nv) / deg
+    return props * deg
+
+
+def _line(gz, edges):
+    """One destination per vector: vertex i + 1 from i, `edges` of them."""
+    i = np.arange(edges, dtype=np.uint64)
+    return gz.make_graph(np.stack([i, i + 1], axis=1), edges + 1)
+
+
+def _fan(gz, width):
+    """Every vertex into vertex 0: one run over all the list."""
+    i = np.arange(1, width, dtype=np.uint64)
+    return gz.make_graph(np.stack([i, np.zeros_like(i)], axis=1), width)
+
+
+PULL_CASES = {
+    "one_vector": lambda gz: _line(gz, 1),
+    "quarter_and_one": lambda gz: _line(gz, 65),
+    "chunk_less_one": lambda gz: _line(gz, 255),
+    "chunk": lambda gz: _line(gz, 256),
+    "chunk_and_one": lambda gz: _line(gz, 257),
+    "one_run": lambda gz: _fan(gz, 9001),
+    "hub": lambda gz: graphs.hub_graph(gz),
+    "last_split_list": lambda gz: _line(gz, 256 * 8192),
+    "first_unsplit_list": lambda gz: _line(gz, 256 * 8192 + 1),
+}
+
+
+@pytest.mark.parametrize("case", sorted(PULL_CASES))
+@pytest.mark.parametrize("vpl", [1, 2])
+def test_split_pull(gz, device, case, vpl):
+    g = PULL_CASES[case](gz)
+    ref = _ranks(g, 5)
+    gz.set_chunk_vectors(256 * vpl)
+    gz.set_vectors_per_lane(vpl)
+    try:
+        gz.load(g)
+        gz.run(gz.options("pr", iterations=5))
+        got = gz.pr_ranks()
+        gz.run(gz.options("pr", iterations=1, collect_stats=True))
+        stats = gz.records()[0]
+    finally:
+        gz.set_chunk_vectors(512)
+        gz.set_vectors_per_lane(1)
+    assert _rel(got, ref) <= PR_TOL
+    assert stats.vectors == gz.pull_vector_count() and stats.edges == g.num_edges
+
+
+# bitmap words at which a wavefront's share changes: 2048 wavefronts of 4, 16 and 64
+@pytest.mark.parametrize("words", [1, 4 * 2048, 16 * 2048, 64 * 2048])
+@pytest.mark.parametrize("extra", [-1, 0, 1])
+def test_sparse_push_widths(gz, orc, device, words, extra):
+    n = 64 * words + extra
+    core = gz.rmat_edges(10, 8 << 10, seed=words + 2)
+    far = np.random.default_rng(words + extra).integers(0, n, size=(4000, 2), dtype=np.uint64)
+    tail = np.array([[0, n - 1], [n - 1, n - 2], [n - 2, n // 2]], dtype=np.uint64)
+    g = gz.make_graph(np.concatenate([core % np.uint64(n), far, tail]), n, symmetrize=True)
+    G = orc.Graph(g.num_vertices, g.pull, g.push)
+    gz.load(g)
+    gz.run(gz.options("bfs", root=0))
+    parents, depths = gz.bfs_result()
+    ref = orc.bfs(G, orc.options(root=0))
+    assert np.array_equal(parents, ref[0]) and np.array_equal(depths, ref[1])
+    gz.cc_push_tail(0)
+    try:
+        gz.run(gz.options("cc", engine="push"))
+        assert np.array_equal(gz.cc_labels(), orc.cc(G, orc.options())[0])
+    finally:
+        gz.cc_push_tail(4096)
+
+
+def test_iteration_end_past_one_workgroup_sum(gz, orc, device):
+    """More vote partials than one workgroup sums: the frontier words of the
+    iteration's end have a launch of their own."""
+    g = gz.rmat_graph(20, 16, seed=5)
+    gz.set_chunk_vectors(64)
+    try:
+        gz.load(g)
+        assert gz.pull_vector_count() > 64 * 65536
+        gz.run(gz.options("cc"))
+        got = gz.cc_labels()
+    finally:
+        gz.set_chunk_vectors(512)
+    assert np.array_equal(got, orc.cc(orc.Graph(g.num_vertices, g.pull, g.push), orc.options(threads=8))[0])
