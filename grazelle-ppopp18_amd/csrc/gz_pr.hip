@@ -70,6 +70,150 @@ __device__ __forceinline__ uint32_t gz_pr_pull_chunk(const gz_vec_t* __restrict_
     return edges;
 }
 
+/* A workgroup's pull over chunk `chunk`, its wavefronts taking consecutive
+ * quarters, for lists with too few chunks to fill the chip with a wavefront
+ * each (gz_pr_pull_splits): the chunk's chain of steps is a quarter as long
+ * and the merge records stay one per chunk.  Each quarter keeps its first
+ * run, when it completes, and its last one in LDS; thread 0 then joins them in
+ * quarter order, stores the runs that complete inside the chunk and leaves
+ * the chunk's last run and its share of S as gz_pr_pull_chunk does.  A run
+ * that spans quarters is summed quarter by quarter, so results differ from
+ * the one-wavefront walk by rounding only. */
+struct gz_pr_quarter {
+    uint64_t first_d, carry_d;
+    double first_v, carry_v, sum;
+    uint32_t first_done, edges;
+};
+
+/* gz_pr_pull_op whose first destination's run goes to the quarter's record. */
+struct gz_pr_quarter_op {
+    const double* __restrict__ props;
+    double* __restrict__ acc;
+    gz_pr_quarter* q;
+    uint64_t first_d;
+    double sum;
+    __device__ __forceinline__ double identity() const { return 0.0; }
+    __device__ __forceinline__ double combine(double a, double b) const { return a + b; }
+    __device__ __forceinline__ double gather(const gz_lanes& v, bool in_range, uint32_t& edges)
+    {
+        const double g = gz_pr_vector_sum<false>(v, props, edges, in_range);
+        sum += g;
+        return g;
+    }
+    __device__ __forceinline__ void store(uint64_t d, double s)
+    {
+        if (d == first_d) {
+            q->first_v = s;
+            q->first_done = 1u;
+        } else {
+            acc[d] = s;
+        }
+    }
+};
+
+/* Every thread of the workgroup calls it, with the same chunk < nchunks; the
+ * chunk's valid lanes go to *edges on thread 0. */
+template <int VPL>
+__device__ __forceinline__ void gz_pr_pull_chunk_split(const gz_vec_t* __restrict__ vecs, uint64_t nvec,
+                                                       uint64_t chunk_len, uint64_t chunk,
+                                                       const double* __restrict__ props, double* __restrict__ acc,
+                                                       mergeaccum_t* __restrict__ merge,
+                                                       double* __restrict__ partials, uint32_t* edges)
+{
+    __shared__ gz_pr_quarter quarters[GZ_WAVES_PER_BLOCK];
+    const uint64_t step = (uint64_t)GZ_WAVE * VPL;
+    const uint64_t share = (chunk_len / step + GZ_WAVES_PER_BLOCK - 1) / GZ_WAVES_PER_BLOCK * step;
+    const uint64_t b = chunk * chunk_len;
+    const uint64_t e = (b + chunk_len < nvec) ? b + chunk_len : nvec;
+    const uint32_t wave = threadIdx.x / GZ_WAVE;
+    const uint64_t wb = b + wave * share;
+    const uint64_t we = (wb + share < e) ? wb + share : e;
+    if (wb < e) {
+        gz_pr_quarter* q = &quarters[wave];
+        const uint64_t first = gz_shared_vertex(gz_load_vector(vecs, wb));
+        if (gz_lane() == 0) q->first_done = 0u;
+        gz_pr_quarter_op op{props, acc, q, first, 0.0};
+        uint64_t first_d, carry_d;
+        double carry_v;
+        uint32_t n = 0;
+        gz_walk_chunk<VPL, double>(vecs, wb, we, op, first_d, carry_d, carry_v, n);
+        const double S = gz_wave_sum(op.sum);
+        const uint64_t total = edges ? gz_wave_sum_u64(n) : 0;
+        if (gz_lane() == 0) {
+            q->first_d = first_d;
+            q->carry_d = carry_d;
+            q->carry_v = carry_v;
+            q->sum = S;
+            q->edges = (uint32_t)total;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const gz_pr_quarter& q0 = quarters[0];
+        uint64_t d = q0.carry_d;
+        double v = q0.carry_v, S = q0.sum;
+        uint32_t n = q0.edges;
+        if (q0.first_done) acc[q0.first_d] = q0.first_v;
+        for (uint32_t w = 1; w < GZ_WAVES_PER_BLOCK && b + w * share < e; ++w) {
+            const gz_pr_quarter& q = quarters[w];
+            S += q.sum;
+            n += q.edges;
+            if (q.first_d != d) {
+                acc[d] = v;
+                if (q.first_done) acc[q.first_d] = q.first_v;
+                v = q.carry_v;
+            } else if (q.first_done) {
+                acc[d] = v + q.first_v;
+                v = q.carry_v;
+            } else {
+                v = v + q.carry_v; /* the quarter is all one run */
+            }
+            d = q.carry_d;
+        }
+        mergeaccum_t r;
+        r.initial_vertex_id = q0.first_d;
+        r.final_vertex_id = d;
+        r.final_partial_value = v;
+        r.__padding__ = 0;
+        merge[chunk] = r;
+        partials[chunk] = S;
+        if (edges) *edges = n;
+    }
+}
+
+template <int VPL>
+__global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_pull_pr_split(const gz_vec_t* __restrict__ vecs, uint64_t nvec,
+                                                                    uint64_t chunk_len,
+                                                                    const double* __restrict__ props,
+                                                                    double* __restrict__ acc,
+                                                                    mergeaccum_t* __restrict__ merge,
+                                                                    double* __restrict__ partials,
+                                                                    uint64_t* __restrict__ stats, uint32_t collect)
+{
+    const uint64_t chunk = blockIdx.x;
+    uint32_t edges = 0;
+    gz_pr_pull_chunk_split<VPL>(vecs, nvec, chunk_len, chunk, props, acc, merge, partials, collect ? &edges : nullptr);
+    if (collect && threadIdx.x == 0) {
+        const uint64_t b = chunk * chunk_len;
+        stats[2 * chunk] = ((b + chunk_len < nvec) ? b + chunk_len : nvec) - b;
+        stats[2 * chunk + 1] = edges;
+    }
+}
+
+/* Whether the scheduler-aware pull gives each chunk a workgroup: while one
+ * wavefront per chunk leaves the SIMDs short of wavefronts and a chunk has
+ * a step for each of the four.  Bound by latency there, by memory above the
+ * line.  20 iterations over R-MAT with edge factor 16, chunks of 512, one
+ * wavefront per chunk / a workgroup per chunk: scale 12 334 / 235 us, 16
+ * (503 chunks) 407 / 291, 17 458 / 418, 18 792 / 761, 19 (4154) 1474 / 1409,
+ * 20 (8363) 2526 / 2504; with 14,300 chunks (24 M edges) 3502 / 3590. */
+#define GZ_PR_SPLIT_CHUNKS 8192u
+static bool gz_pr_pull_splits(uint64_t nchunks)
+{
+    return nchunks <= GZ_PR_SPLIT_CHUNKS &&
+           gz_chunk_len() >= (uint64_t)GZ_WAVE * gz_vectors_per_lane() * GZ_WAVES_PER_BLOCK;
+}
+
 template <bool kSchedAware, int VPL>
 __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_pull_pr(const gz_vec_t* __restrict__ vecs, uint64_t nvec,
                                                               uint64_t chunk_len, uint64_t nchunks,
@@ -94,11 +238,35 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_pull_pr(const gz_vec_t* __
     }
 }
 
+static void gz_launch_pr_pull_split(const gz_vec_t* vecs, uint64_t nvec, uint64_t chunk_len, uint64_t nchunks,
+                                    const double* props, double* acc, mergeaccum_t* merge, double* partials,
+                                    uint64_t* stats, uint32_t collect)
+{
+    const uint32_t vpl = gz_vectors_per_lane();
+#define GZ_PULL_PR_SPLIT_ARGS                                                                                  \
+    dim3((unsigned)nchunks), dim3(GZ_BLOCK), 0, gz_stream, vecs, nvec, chunk_len, props, acc, merge, partials,   \
+        stats, collect
+    if (vpl == 4)
+        hipLaunchKernelGGL(gz_k_edge_pull_pr_split<4>, GZ_PULL_PR_SPLIT_ARGS);
+    else if (vpl == 2)
+        hipLaunchKernelGGL(gz_k_edge_pull_pr_split<2>, GZ_PULL_PR_SPLIT_ARGS);
+    else
+        hipLaunchKernelGGL(gz_k_edge_pull_pr_split<1>, GZ_PULL_PR_SPLIT_ARGS);
+#undef GZ_PULL_PR_SPLIT_ARGS
+    GZ_LAUNCH_CHECK();
+}
+
 template <bool kSchedAware>
 static void gz_launch_pull_pr(uint64_t blocks, const gz_vec_t* edge_list, uint64_t count, uint64_t chunk_len,
                               uint64_t nchunks)
 {
     const uint32_t vpl = gz_vectors_per_lane();
+    if (kSchedAware && gz_pr_pull_splits(nchunks)) {
+        gz_launch_pr_pull_split(edge_list, count, chunk_len, nchunks, (const double*)gz_graph.vertex_props,
+                                (double*)gz_graph.vertex_accumulators, gz_merge_buffer, (double*)gz_scratch.partials,
+                                gz_scratch.stats, gz_phase_config.collect_stats);
+        return;
+    }
 #define GZ_PULL_PR_ARGS                                                                                        \
     dim3((unsigned)blocks), dim3(GZ_BLOCK), 0, gz_stream, edge_list, count, chunk_len, nchunks,                 \
         (const double*)gz_graph.vertex_props, (double*)gz_graph.vertex_accumulators, gz_merge_buffer,          \
@@ -157,6 +325,10 @@ void gz_launch_pr_pull_explicit(const gz_vec_t* vecs, uint64_t nvec, uint64_t ch
                                 const double* props, double* acc, mergeaccum_t* merge, double* partials)
 {
     if (nchunks == 0) return;
+    if (gz_pr_pull_splits(nchunks)) {
+        gz_launch_pr_pull_split(vecs, nvec, chunk_len, nchunks, props, acc, merge, partials, nullptr, 0u);
+        return;
+    }
     const uint64_t blocks = (nchunks + GZ_WAVES_PER_BLOCK - 1) / GZ_WAVES_PER_BLOCK;
     const uint32_t vpl = gz_vectors_per_lane();
 #define GZ_PULL_PR_EXPLICIT_ARGS                                                                               \
@@ -590,7 +762,7 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_pr_persistent(
     const gz_vec_t* __restrict__ vecs, uint64_t nvec, uint64_t chunk_len, uint64_t nchunks, double* props,
     double* acc, const double* __restrict__ outdeg, uint64_t num_vertices, mergeaccum_t* merge, double* partials,
     double* slots, uint32_t reduce_blocks, uint32_t* run_head, uint64_t* __restrict__ reduce_buffer,
-    double damping, uint64_t iterations, gz_grid_bar_t* bar, uint32_t spin_limit)
+    double damping, uint64_t iterations, gz_grid_bar_t* bar, uint32_t spin_limit, uint32_t split)
 {
     __shared__ double lds[GZ_WAVES_PER_BLOCK];
     __shared__ double slot_lds[2];
@@ -604,8 +776,15 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_pr_persistent(
     const bool local_sum = nchunks <= GZ_PR_ONE_LAUNCH_LOCAL_SUM_CHUNKS;
     const uint64_t per = (nchunks + reduce_blocks - 1) / reduce_blocks;
     for (uint64_t it = 0; it < iterations; ++it) {
-        for (uint64_t c = gw; c < nchunks; c += waves)
-            gz_pr_pull_chunk<true, VPL>(vecs, nvec, chunk_len, c, props, acc, merge, partials);
+        if (split) {
+            for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
+                gz_pr_pull_chunk_split<VPL>(vecs, nvec, chunk_len, c, props, acc, merge, partials, nullptr);
+                __syncthreads(); /* the next chunk rewrites the quarters */
+            }
+        } else {
+            for (uint64_t c = gw; c < nchunks; c += waves)
+                gz_pr_pull_chunk<true, VPL>(vecs, nvec, chunk_len, c, props, acc, merge, partials);
+        }
         if (!gz_grid_sync(bar, spin_limit)) return;
         if (it == 0) {
             /* run_head[final vertex of a run of records] = first record of
@@ -733,9 +912,10 @@ extern "C" int gz_pr_run_persistent(uint64_t iterations, uint64_t* reduce_buffer
     double damping = gz_phase_config.damping;
     gz_grid_bar_t* bar = gz_pr_bar;
     uint32_t spin = gz_pr_persistent_spin;
+    uint32_t split = gz_pr_pull_splits(nchunks) ? 1u : 0u;
     uint64_t n_vec = nvec, n_chunks = nchunks, n_v = V, iters = iterations;
     void* args[] = {&vecs, &n_vec, &chunk_len, &n_chunks, &props, &acc, &outdeg, &n_v, &merge, &partials,
-                    &slots, &reduce_blocks, &run_head, &reduce_buffer, &damping, &iters, &bar, &spin};
+                    &slots, &reduce_blocks, &run_head, &reduce_buffer, &damping, &iters, &bar, &spin, &split};
     /* A cooperative launch can be refused while another process holds the
      * device's cooperative resources; the per-phase launches then run, for
      * the rest of this process. */
