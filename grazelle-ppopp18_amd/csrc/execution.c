@@ -616,6 +616,10 @@ static void gz_run_hybrid(const gz_run_options_t* o, gz_run_result_t* r)
          * of the next frontier into their vote pass */
         if (bfs) gz_features_fold(1, indeg);
     }
+    /* the vote, BFS's retirement and the vertex phase's clear end an iteration
+     * in one launch (the host-decided learned BFS: in the launch that sums its
+     * features); the probe engine repeats its edge phases and keeps them apart */
+    if (bfs) gz_bfs_defer_retire(!features || host_decides);
     uint64_t ctr = 0;
     while (1) {
         ctr += 1;
@@ -655,6 +659,7 @@ static void gz_run_hybrid(const gz_run_options_t* o, gz_run_result_t* r)
                          (o->engine == GZ_ENGINE_PUSH || o->engine == GZ_ENGINE_HYBRID ||
                           o->engine == GZ_ENGINE_LEARNED) &&
                          gz_cc_push_tail_applies(vote);
+        const int fused_end = !features && !tail;
         if (probe) {
             /* the chosen engine runs last, so its result is what continues */
             gz_snapshot_take(&snap);
@@ -688,7 +693,10 @@ static void gz_run_hybrid(const gz_run_options_t* o, gz_run_result_t* r)
         /* with BFS statistics folded into the edge phase, the selector's
          * decision kernel also sums the vote */
         const int vote_in_step = features && bfs;
-        if (!vote_in_step && !tail) phase_op_write_global_accum_to_buf(gz_reduce_buffer);
+        if (fused_end)
+            gz_iteration_end(bfs, gz_reduce_buffer);
+        else if (!vote_in_step && !tail)
+            phase_op_write_global_accum_to_buf(gz_reduce_buffer);
         if (t && !probe) gz_timer_stop(t);
         if (host_decides) {
             gz_sel_dev_sums(gz_reduce_buffer, indeg);
@@ -715,12 +723,14 @@ static void gz_run_hybrid(const gz_run_options_t* o, gz_run_result_t* r)
         vote = next_vote;
         if (0 == vote) break;
         gz_swap_frontiers();
+        if (fused_end || host_decides) continue; /* HasInfo* is clear already */
         if (bfs)
             perform_vertex_phase_bfs(0, V, NULL);
         else
             perform_vertex_phase_cc(0, V, NULL);
     }
     r->iterations = ctr;
+    if (bfs) gz_bfs_defer_retire(0);
     gz_features_fold(0, NULL);
     if (t) gz_timer_destroy(t);
     if (probe) gz_snapshot_free(&snap);

@@ -483,8 +483,29 @@ static uint64_t gz_bfs_next_push_vote = ~0ull;
 
 extern "C" void gz_bfs_push_vote_hint(uint64_t vote) { gz_bfs_next_push_vote = vote; }
 
+/* The drivers' pushes leave the retirement to the iteration's end
+ * (gz_iteration_end), which saves its launch. */
+static int gz_bfs_retire_deferred = 0, gz_bfs_retire_due = 0;
+
+extern "C" void gz_bfs_defer_retire(int on)
+{
+    gz_bfs_retire_deferred = on ? 1 : 0;
+    gz_bfs_retire_due = 0;
+}
+
+extern "C" int gz_bfs_take_deferred_retire(void)
+{
+    const int due = gz_bfs_retire_due;
+    gz_bfs_retire_due = 0;
+    return due;
+}
+
 static void gz_bfs_retire(void)
 {
+    if (gz_bfs_retire_deferred) {
+        gz_bfs_retire_due = 1;
+        return;
+    }
     const uint64_t words = (gz_graph.num_vertices + 63) / 64;
     uint64_t rblocks = (words + GZ_BLOCK - 1) / GZ_BLOCK;
     if (rblocks > 4096) rblocks = 4096;

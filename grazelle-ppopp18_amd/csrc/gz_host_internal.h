@@ -114,6 +114,16 @@ void gz_scratch_reserve_public(uint64_t waves, uint64_t num_vertices);
 /* The same for the next BFS push (the vote of the level that built its
  * frontier). */
 void gz_bfs_push_vote_hint(uint64_t vote);
+/* The end of a CC or BFS iteration of the library's own drivers in one
+ * launch: the vote into reduce_buffer (phase_op_write_global_accum_to_buf), a
+ * BFS push's visited vertices out of WantsInfo, and the frontier just used
+ * cleared (the vertex phase after the swap).  gz_bfs_defer_retire(1) makes
+ * BFS pushes leave WantsInfo to it. */
+void gz_iteration_end(int bfs, uint64_t* reduce_buffer);
+void gz_bfs_defer_retire(int on);
+/* Whether the last BFS push left its visited vertices in WantsInfo; clears
+ * the mark. */
+int gz_bfs_take_deferred_retire(void);
 /* Drop the frontier compaction's per-vertex vector counts (graph release). */
 void gz_frontier_counts_release(void);
 /* Frees the BFS bottom-up step's pending-destination buffers. */
@@ -161,7 +171,7 @@ void gz_sel_dev_stamp(int by_compaction);
  * vote and frontier sums into the reduce words (0: vote; 2, 3, 4: activated
  * vertices, their out-edges, their in-edges; 5: the phase's device-clock ms
  * as a float). */
-void gz_sel_dev_sums(uint64_t* reduce_buffer, const uint32_t* indeg);
+void gz_sel_dev_sums(uint64_t* reduce_buffer, const uint32_t* indeg); /* and gz_iteration_end's words */
 void gz_sel_dev_step(const uint64_t* frontier, const uint32_t* indeg, uint64_t* reduce_buffer, int have_model,
                      int bfs, uint64_t iteration, uint32_t prev_engine, float prev_ms, int source, int with_vote);
 /* BFS edge phases fold the selector's features (vertices, out-edges and,

@@ -217,6 +217,9 @@ uint64_t gz_chunk_len(void);
 uint32_t gz_vectors_per_lane(void);
 /* Reduce gz_scratch.partials[0..count) into dst[0] (bit pattern). */
 void gz_reduce_partials(uint64_t* dst);
+/* The frontier words of the iteration that ends (gz_runtime.hip). */
+struct gz_end_words;
+gz_end_words gz_iteration_end_words(int bfs);
 /* Deterministic two-stage FP64 sum of in[count] into out[0] (as bits): up to
  * 1024 blocks write slots[], the last one sums them and clears *done, which
  * must be 0 when the launch starts. */
@@ -419,6 +422,38 @@ __device__ __forceinline__ void gz_mirror_words(uint64_t* __restrict__ mirror, c
     if (mirror == nullptr) return;
 #pragma unroll
     for (int i = 0; i < 8; ++i) mirror[i] = out[i];
+}
+
+/* The frontier words at the end of a CC or BFS iteration, done by the
+ * workgroups after the first of the kernel that sums its vote: the visited
+ * vertices leave WantsInfo (wants &= ~next, after a BFS push; wants is null
+ * otherwise) and the frontier just used is cleared (has = 0), since the swap
+ * makes it the next HasInfo*. */
+struct gz_end_words {
+    uint64_t* wants;
+    const uint64_t* next;
+    uint64_t* has;
+    uint64_t words; /* 0: no words to do, a grid of one workgroup */
+};
+
+#define GZ_END_THREADS 1024
+
+/* Workgroups of that kernel for w. */
+static inline unsigned gz_end_blocks(const gz_end_words& w)
+{
+    uint64_t blocks = (w.words + GZ_END_THREADS - 1) / GZ_END_THREADS;
+    if (blocks > 1024) blocks = 1024;
+    return (unsigned)(blocks + 1);
+}
+
+/* Workgroup b > 0 of a grid of gz_end_blocks(w) workgroups. */
+__device__ __forceinline__ void gz_end_words_do(const gz_end_words& w)
+{
+    const uint64_t stride = (uint64_t)(gridDim.x - 1) * blockDim.x;
+    for (uint64_t i = (uint64_t)(blockIdx.x - 1) * blockDim.x + threadIdx.x; i < w.words; i += stride) {
+        if (w.wants != nullptr) w.wants[i] &= ~w.next[i];
+        w.has[i] = 0;
+    }
 }
 
 /* One activated vertex: its frontier statistic (gz_frontier_stat) and, when

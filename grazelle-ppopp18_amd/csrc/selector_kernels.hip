@@ -358,8 +358,12 @@ __global__ __launch_bounds__(1024) void gz_k_sel_sums(const uint64_t* __restrict
                                                           uint64_t stride, const uint64_t* __restrict__ votes,
                                                           const gz_sel_dev_state* __restrict__ st, float clock_khz,
                                                           int out_from_vote, int with_in, uint64_t* __restrict__ out,
-                                                          uint64_t* __restrict__ mirror)
+                                                          uint64_t* __restrict__ mirror, gz_end_words end)
 {
+    if (blockIdx.x > 0) {
+        gz_end_words_do(end);
+        return;
+    }
     __shared__ uint64_t red[4][1024 / GZ_WAVE];
     const int j = threadIdx.x;
     const uint64_t t_end = (uint64_t)wall_clock64();
@@ -566,10 +570,11 @@ extern "C" void gz_sel_dev_sums(uint64_t* reduce_buffer, const uint32_t* indeg)
     if (gz_phase_config.stat_mode == GZ_STAT_COUNT_AND_OUTDEG) out_from_vote = 1;
     if (gz_phase_config.stat_mode == GZ_STAT_OUTDEG_ONLY) out_from_vote = 2;
     uint64_t* mirror = gz_reduce_mirror_target(reduce_buffer);
+    const gz_end_words end = gz_iteration_end_words(1);
     gz_ktimer_begin(GZ_K_REDUCE);
-    hipLaunchKernelGGL(gz_k_sel_sums, dim3(1), dim3(1024), 0, gz_stream, gz_scratch.features, gz_scratch.partials_count,
+    hipLaunchKernelGGL(gz_k_sel_sums, dim3(gz_end_blocks(end)), dim3(1024), 0, gz_stream, gz_scratch.features, gz_scratch.partials_count,
                        gz_scratch.partials_capacity, (const uint64_t*)gz_scratch.partials, gz_sel_dev_st, gz_sel_clock_khz, out_from_vote,
-                       indeg != nullptr ? 1 : 0, reduce_buffer, mirror);
+                       indeg != nullptr ? 1 : 0, reduce_buffer, mirror, end);
     GZ_LAUNCH_CHECK();
     gz_ktimer_end(GZ_K_REDUCE);
 }
