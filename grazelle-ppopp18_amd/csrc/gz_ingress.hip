@@ -8,24 +8,29 @@
  * as a device pipeline over 64-bit keys (group << b | neighbour), b = bits of
  * V-1:
  *   1. keys: drawn by the R-MAT kernel (the host generator's exact stream) or
- *      converted from uploaded (src, dst) pairs, optionally both directions;
+ *      converted from uploaded (src, dst) pairs, optionally both directions; a
+ *      self-loop becomes the all-ones key, itself a self-loop, which sorts last;
  *   2. LSD radix sort over the 2b key bits (pull: group = dst);
- *   3. drop self-loops and duplicates (a key equal to its predecessor);
- *   4. per-vertex edge offsets by binary search in the sorted keys, vector
- *      counts ceil(deg / 4) and their exclusive scan = the CSR vector offsets;
+ *   3. drop the all-ones keys and duplicates (a key equal to its predecessor)
+ *      and note each group's first and end position among the kept keys, in
+ *      two passes over the keys (tile counts, then the write);
+ *   4. vector counts ceil(deg / 4) and their exclusive scan = the CSR vector
+ *      offsets;
  *   5. pack: edge i of group g at rank r goes to lane r % 4 of vector
  *      offsets[g] + r / 4, which is the flush rule of graphdata.c:679-686 on a
  *      group-sorted list (a vector closes when the shared vertex changes or it
  *      holds four edges);
- *   6. the push layout: the kept keys with group and neighbour swapped,
- *      sorted again; FP64 outdegrees are its group sizes (graphdata.c:814
- *      counts sources of the pull file, which is the same number).
+ *   6. the push layout: the kept keys, in (dst, src) order, sorted again by
+ *      their b source bits alone (the sort is stable); FP64 outdegrees are its
+ *      group sizes (graphdata.c:814 counts sources of the pull file, which is
+ *      the same number).
  * The result equals gz_edges_sort(..., dedupe) + gz_pack_vectors on the host
  * bit for bit, invalid lanes included (shared-vertex piece, neighbour 0).
  */
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
-#include <rocprim/device/device_select.hpp>
+#include <rocprim/iterator/counting_iterator.hpp>
+#include <rocprim/iterator/transform_iterator.hpp>
 
 #include "grazelle_host.h"
 #include "gz_host_internal.h"
@@ -41,12 +46,22 @@ __device__ __forceinline__ uint64_t gz_splitmix64_dev(uint64_t x)
     return x ^ (x >> 31);
 }
 
+/* The key (group << b | neighbour) of an edge, all ones for a self-loop when
+ * `drop` (a renumbered graph counts self-loops first, gz_k_remap_keys then
+ * drops them). */
+__host__ __device__ __forceinline__ uint64_t gz_no_key(uint32_t b) { return b < 32 ? (1ull << (2 * b)) - 1ull : ~0ull; }
+
+__device__ __forceinline__ uint64_t gz_edge_key(uint64_t g, uint64_t nbr, uint32_t b, int drop)
+{
+    return (drop && g == nbr) ? gz_no_key(b) : ((g << b) | nbr);
+}
+
 /* The R-MAT draw of rmat.c for edges [0, n): key (dst << b | src), and with
  * `both` also (src << b | dst) at the odd slot.  Ids are shifted by id_base
  * (one graph of a disjoint union). */
 __global__ void gz_k_rmat_keys(uint64_t seed, uint64_t edge_offset, uint32_t scale, uint64_t nv, uint32_t ta,
-                               uint32_t tb, uint32_t tc, uint64_t n, uint32_t b, int both, uint64_t id_base,
-                               uint64_t* __restrict__ keys)
+                               uint32_t tb, uint32_t tc, uint64_t n, uint32_t b, int both, int drop,
+                               uint64_t id_base, uint64_t* __restrict__ keys)
 {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += stride) {
@@ -65,80 +80,184 @@ __global__ void gz_k_rmat_keys(uint64_t seed, uint64_t edge_offset, uint32_t sca
         s += id_base;
         d += id_base;
         if (both) {
-            keys[2 * e] = (d << b) | s;
-            keys[2 * e + 1] = (s << b) | d;
+            keys[2 * e] = gz_edge_key(d, s, b, drop);
+            keys[2 * e + 1] = gz_edge_key(s, d, b, drop);
         } else {
-            keys[e] = (d << b) | s;
+            keys[e] = gz_edge_key(d, s, b, drop);
         }
     }
 }
 
-__global__ void gz_k_pairs_keys(const uint64_t* __restrict__ pairs, uint64_t n, uint32_t b, int both,
+__global__ void gz_k_pairs_keys(const uint64_t* __restrict__ pairs, uint64_t n, uint32_t b, int both, int drop,
                                 uint64_t* __restrict__ keys)
 {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += stride) {
         const uint64_t s = pairs[2 * e], d = pairs[2 * e + 1];
         if (both) {
-            keys[2 * e] = (d << b) | s;
-            keys[2 * e + 1] = (s << b) | d;
+            keys[2 * e] = gz_edge_key(d, s, b, drop);
+            keys[2 * e + 1] = gz_edge_key(s, d, b, drop);
         } else {
-            keys[e] = (d << b) | s;
+            keys[e] = gz_edge_key(d, s, b, drop);
         }
     }
 }
 
-/* keep = first of its value and not a self-loop */
-__global__ void gz_k_mark_kept(const uint64_t* __restrict__ keys, uint64_t n, uint32_t b, uint8_t* __restrict__ keep)
+/* ---- sorted keys, tile by tile ------------------------------------------------
+ * The passes below walk a sorted key array in tiles of GZ_TILE keys, a
+ * wavefront taking GZ_TILE_ROWS rows of 64 consecutive keys with every row's
+ * load in flight at once.  A key needs its neighbours: they come from the
+ * next lanes, and from one extra load at each end of the wavefront's rows. */
+#define GZ_TILE_ROWS 16
+#define GZ_TILE_WAVE (GZ_TILE_ROWS * GZ_WAVE)
+#define GZ_TILE (GZ_WAVES_PER_BLOCK * GZ_TILE_WAVE)
+
+struct gz_tile_keys {
+    uint64_t k[GZ_TILE_ROWS], before, after; /* before: the key ahead of the rows; after: the one behind */
+};
+
+/* The wavefront's keys of tile `tile`; positions past n read as `pad`. */
+__device__ __forceinline__ uint64_t gz_tile_load(gz_tile_keys& t, const uint64_t* __restrict__ keys, uint64_t n,
+                                                 uint64_t tile, uint64_t pad)
+{
+    const uint64_t base = tile * GZ_TILE + (uint64_t)(threadIdx.x / GZ_WAVE) * GZ_TILE_WAVE;
+#pragma unroll
+    for (int r = 0; r < GZ_TILE_ROWS; ++r) {
+        const uint64_t i = base + (uint64_t)(r * GZ_WAVE + gz_lane());
+        t.k[r] = i < n ? keys[i] : pad;
+    }
+    t.before = (base > 0 && base <= n) ? keys[base - 1] : pad;
+    t.after = base + GZ_TILE_WAVE < n ? keys[base + GZ_TILE_WAVE] : pad;
+    return base;
+}
+
+/* The keys ahead of and behind each lane's key of row r. */
+__device__ __forceinline__ uint64_t gz_tile_prev(const gz_tile_keys& t, int r)
+{
+    const uint64_t x = (uint64_t)__shfl_up((unsigned long long)t.k[r], 1, GZ_WAVE);
+    const uint64_t edge = r == 0 ? t.before : gz_shfl_u64(t.k[r > 0 ? r - 1 : 0], GZ_WAVE - 1);
+    return gz_lane() == 0 ? edge : x;
+}
+
+__device__ __forceinline__ uint64_t gz_tile_next(const gz_tile_keys& t, int r)
+{
+    const uint64_t x = (uint64_t)__shfl_down((unsigned long long)t.k[r], 1, GZ_WAVE);
+    const uint64_t edge = r == GZ_TILE_ROWS - 1 ? t.after : gz_shfl_u64(t.k[r < GZ_TILE_ROWS - 1 ? r + 1 : r], 0);
+    return gz_lane() == GZ_WAVE - 1 ? edge : x;
+}
+
+/* Whether row r's keys count: kept (not all ones, not a duplicate), or, for
+ * kHeads, the first of their (key >> b). */
+template <bool kHeads>
+__device__ __forceinline__ bool gz_tile_flag(const gz_tile_keys& t, int r, uint64_t i, uint64_t n, uint32_t b,
+                                             uint64_t none)
+{
+    const uint64_t k = t.k[r], p = gz_tile_prev(t, r);
+    if (kHeads) return i < n && (i == 0 || (k >> b) != (p >> b));
+    return i < n && k != none && (i == 0 || k != p);
+}
+
+/* sums[tile] = keys of the tile that count. */
+template <bool kHeads>
+__global__ __launch_bounds__(GZ_BLOCK) void gz_k_tile_count(const uint64_t* __restrict__ keys, uint64_t n, uint32_t b,
+                                                            uint64_t none, uint64_t tiles, uint64_t* __restrict__ sums)
+{
+    __shared__ uint32_t lds[GZ_WAVES_PER_BLOCK];
+    for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        gz_tile_keys t;
+        const uint64_t base = gz_tile_load(t, keys, n, tile, none);
+        uint32_t c = 0;
+#pragma unroll
+        for (int r = 0; r < GZ_TILE_ROWS; ++r)
+            c += (uint32_t)__popcll(
+                __ballot(gz_tile_flag<kHeads>(t, r, base + (uint64_t)(r * GZ_WAVE + gz_lane()), n, b, none)));
+        if (gz_lane() == 0) lds[threadIdx.x / GZ_WAVE] = c;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            uint64_t x = 0;
+            for (int w = 0; w < GZ_WAVES_PER_BLOCK; ++w) x += lds[w];
+            sums[tile] = x;
+        }
+        __syncthreads();
+    }
+}
+
+/* Counting keys of the tile ahead of this wavefront's rows, given its own
+ * count (every thread of the workgroup calls it). */
+__device__ __forceinline__ uint64_t gz_tile_wave_base(uint32_t mine, uint32_t* lds)
+{
+    if (gz_lane() == 0) lds[threadIdx.x / GZ_WAVE] = mine;
+    __syncthreads();
+    uint64_t x = 0;
+    for (int w = 0; w < (int)(threadIdx.x / GZ_WAVE); ++w) x += lds[w];
+    __syncthreads();
+    return x;
+}
+
+/* Pass 2 of the dedupe: the kept keys to out, in order, and each group's
+ * first and end positions there (groups without kept keys keep their zeros).
+ * Equal keys are adjacent and self-loops are all ones, so a group's first raw
+ * key is kept and its last raw key ends it.  Bound by memory: 8 bytes read
+ * and 8 written per key (the flag array and the library's select it replaced
+ * moved 18 and took 2.2 ms for the 67 M keys of R-MAT s22; this and its count
+ * pass take 0.4). */
+__global__ __launch_bounds__(GZ_BLOCK) void gz_k_kept_write(const uint64_t* __restrict__ keys, uint64_t n, uint32_t b,
+                                                            uint64_t none, uint64_t tiles,
+                                                            const uint64_t* __restrict__ tile_base,
+                                                            uint64_t* __restrict__ out, uint64_t* __restrict__ first,
+                                                            uint64_t* __restrict__ end)
+{
+    __shared__ uint32_t lds[GZ_WAVES_PER_BLOCK];
+    const uint64_t below = (1ull << gz_lane()) - 1ull;
+    for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        gz_tile_keys t;
+        const uint64_t base = gz_tile_load(t, keys, n, tile, none);
+        uint64_t kept[GZ_TILE_ROWS];
+        uint32_t c = 0;
+#pragma unroll
+        for (int r = 0; r < GZ_TILE_ROWS; ++r) {
+            kept[r] = __ballot(gz_tile_flag<false>(t, r, base + (uint64_t)(r * GZ_WAVE + gz_lane()), n, b, none));
+            c += (uint32_t)__popcll(kept[r]);
+        }
+        uint64_t pos = tile_base[tile] + gz_tile_wave_base(c, lds);
+#pragma unroll
+        for (int r = 0; r < GZ_TILE_ROWS; ++r) {
+            const uint64_t k = t.k[r], g = k >> b;
+            const uint64_t at = pos + (uint64_t)__popcll(kept[r] & below);
+            const bool keep = (kept[r] >> gz_lane()) & 1ull;
+            const uint64_t p = gz_tile_prev(t, r), q = gz_tile_next(t, r);
+            if (keep) out[at] = k;
+            if (k != none) { /* padding reads as `none` */
+                const bool head = base + (uint64_t)(r * GZ_WAVE + gz_lane()) == 0 || (p >> b) != g;
+                if (head) first[g] = at;
+                if (q == none || (q >> b) != g) end[g] = at + (keep ? 1 : 0);
+            }
+            pos += (uint64_t)__popcll(kept[r]);
+        }
+    }
+}
+
+/* Group bounds of sorted keys without duplicates, the group being the low b
+ * bits (groups without keys keep their zeros). */
+__global__ void gz_k_low_bounds(const uint64_t* __restrict__ keys, uint64_t m, uint32_t b, uint64_t* __restrict__ first,
+                                uint64_t* __restrict__ end)
 {
     const uint64_t mask = (1ull << b) - 1ull;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const uint64_t k = keys[i];
-        const bool dup = (i > 0) && keys[i - 1] == k;
-        keep[i] = (!dup && (k >> b) != (k & mask)) ? 1 : 0;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += stride) {
+        const uint64_t g = keys[i] & mask;
+        if (i == 0 || (keys[i - 1] & mask) != g) first[g] = i;
+        if (i == m - 1 || (keys[i + 1] & mask) != g) end[g] = i + 1;
     }
 }
 
-__global__ void gz_k_swap_keys(const uint64_t* __restrict__ in, uint64_t n, uint32_t b, uint64_t* __restrict__ out)
-{
-    const uint64_t mask = (1ull << b) - 1ull;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const uint64_t k = in[i];
-        out[i] = ((k & mask) << b) | (k >> b);
-    }
-}
-
-/* eoff[v] = first i with keys[i] >> b >= v, for v in [0, V] (eoff[V] = m). */
-__global__ void gz_k_group_offsets(const uint64_t* __restrict__ keys, uint64_t m, uint32_t b, uint64_t nv,
-                                   uint64_t* __restrict__ eoff)
-{
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v <= nv; v += stride) {
-        if (v == nv) {
-            eoff[v] = m;
-            continue;
-        }
-        const uint64_t target = v << b;
-        uint64_t lo = 0, hi = m;
-        while (lo < hi) {
-            const uint64_t mid = lo + ((hi - lo) >> 1);
-            if (keys[mid] < target)
-                lo = mid + 1;
-            else
-                hi = mid;
-        }
-        eoff[v] = lo;
-    }
-}
-
-__global__ void gz_k_vector_counts(const uint64_t* __restrict__ eoff, uint64_t nv, uint64_t* __restrict__ cnt)
-{
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v <= nv; v += stride)
-        cnt[v] = (v < nv) ? (eoff[v + 1] - eoff[v] + 3) / 4 : 0;
-}
+/* Vectors of group v, 0 past the last group. */
+struct gz_group_vectors {
+    const uint64_t* first;
+    const uint64_t* end;
+    uint64_t nv;
+    __device__ uint64_t operator()(uint64_t v) const { return v < nv ? (end[v] - first[v] + 3) / 4 : 0; }
+};
 
 __device__ __forceinline__ uint64_t gz_piece(uint64_t g, int l)
 {
@@ -147,30 +266,33 @@ __device__ __forceinline__ uint64_t gz_piece(uint64_t g, int l)
     return ((g >> shift) & mask) << 48;
 }
 
-__global__ void gz_k_pack(const uint64_t* __restrict__ keys, uint64_t m, uint32_t b, const uint64_t* __restrict__ eoff,
+/* The group is the high bits of a key, or the low b bits when `low`. */
+__global__ void gz_k_pack(const uint64_t* __restrict__ keys, uint64_t m, uint32_t b, int low,
+                          const uint64_t* __restrict__ first, const uint64_t* __restrict__ end,
                           const uint64_t* __restrict__ voff, uint64_t* __restrict__ lanes)
 {
     const uint64_t mask = (1ull << b) - 1ull;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += stride) {
         const uint64_t k = keys[i];
-        const uint64_t g = k >> b;
-        const uint64_t r = i - eoff[g];
+        const uint64_t g = low ? k & mask : k >> b, nbr = low ? k >> b : k & mask;
+        const uint64_t r = i - first[g];
         const uint64_t j = voff[g] + r / 4;
         const int l = (int)(r & 3);
-        lanes[4 * j + l] = GZ_LANE_VALID_BIT | gz_piece(g, l) | (k & mask);
+        lanes[4 * j + l] = GZ_LANE_VALID_BIT | gz_piece(g, l) | nbr;
         if (l == 0) {
-            const uint64_t left = eoff[g + 1] - eoff[g] - r;
+            const uint64_t left = end[g] - i;
             for (int q = (left < 4 ? (int)left : 4); q < 4; ++q) lanes[4 * j + q] = gz_piece(g, q);
         }
     }
 }
 
-__global__ void gz_k_outdegrees(const uint64_t* __restrict__ eoff, uint64_t nv, double* __restrict__ outdeg)
+__global__ void gz_k_outdegrees(const uint64_t* __restrict__ first, const uint64_t* __restrict__ end, uint64_t nv,
+                                double* __restrict__ outdeg)
 {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv + 8; v += stride)
-        outdeg[v] = (v < nv) ? (double)(eoff[v + 1] - eoff[v]) : 0.0;
+        outdeg[v] = (v < nv) ? (double)(end[v] - first[v]) : 0.0;
 }
 
 unsigned gz_grid_for(uint64_t n)
@@ -195,49 +317,52 @@ uint32_t gz_id_bits(uint64_t nv)
     return b;
 }
 
-/* Sort keys[0, n) over bits [0, 2b); the sorted keys end in *sorted (one of a
- * or b_buf). */
-void gz_sort_keys(uint64_t* a, uint64_t* b_buf, uint64_t n, uint32_t bits, uint64_t** sorted)
+unsigned gz_tile_grid(uint64_t tiles) { return (unsigned)(tiles < 65536 ? tiles : 65536); }
+
+/* Sort keys[0, n) over bits [begin, end), stably; the sorted keys end in
+ * *sorted (one of a or b_buf). */
+void gz_sort_keys(uint64_t* a, uint64_t* b_buf, uint64_t n, uint32_t begin, uint32_t end, uint64_t** sorted)
 {
     rocprim::double_buffer<uint64_t> db(a, b_buf);
     size_t tmp_bytes = 0;
-    GZ_CHECK(rocprim::radix_sort_keys(nullptr, tmp_bytes, db, (size_t)n, 0, bits, gz_stream));
+    GZ_CHECK(rocprim::radix_sort_keys(nullptr, tmp_bytes, db, (size_t)n, begin, end, gz_stream));
     void* tmp = gz_device_malloc(tmp_bytes ? tmp_bytes : 1);
-    GZ_CHECK(rocprim::radix_sort_keys(tmp, tmp_bytes, db, (size_t)n, 0, bits, gz_stream));
+    GZ_CHECK(rocprim::radix_sort_keys(tmp, tmp_bytes, db, (size_t)n, begin, end, gz_stream));
     GZ_CHECK(hipStreamSynchronize(gz_stream));
     gz_device_free(tmp);
     *sorted = db.current();
 }
 
-/* Build one layout from sorted, duplicate-free keys[0, m). */
-void gz_build_layout(const uint64_t* keys, uint64_t m, uint32_t b, uint64_t nv, gz_vec_t** d_vecs,
-                     uint64_t** d_offsets, uint64_t* vector_count, uint64_t* eoff)
+/* out[0 .. n) = exclusive scan of in[0 .. n). */
+template <typename It>
+void gz_scan(It in, uint64_t* out, uint64_t n)
 {
-    const unsigned tb = GZ_BLOCK;
-    hipLaunchKernelGGL(gz_k_group_offsets, dim3(gz_grid_for(nv + 1)), dim3(tb), 0, gz_stream, keys, m, b, nv, eoff);
-    GZ_LAUNCH_CHECK();
-    uint64_t* cnt = (uint64_t*)gz_device_malloc((nv + 1) * sizeof(uint64_t));
-    uint64_t* voff = (uint64_t*)gz_device_malloc((nv + 1) * sizeof(uint64_t));
-    hipLaunchKernelGGL(gz_k_vector_counts, dim3(gz_grid_for(nv + 1)), dim3(tb), 0, gz_stream, eoff, nv, cnt);
-    GZ_LAUNCH_CHECK();
     size_t tmp_bytes = 0;
-    GZ_CHECK(rocprim::exclusive_scan(nullptr, tmp_bytes, cnt, voff, (uint64_t)0, (size_t)(nv + 1),
-                                     rocprim::plus<uint64_t>(), gz_stream));
+    GZ_CHECK(rocprim::exclusive_scan(nullptr, tmp_bytes, in, out, (uint64_t)0, (size_t)n, rocprim::plus<uint64_t>(),
+                                     gz_stream));
     void* tmp = gz_device_malloc(tmp_bytes ? tmp_bytes : 1);
-    GZ_CHECK(rocprim::exclusive_scan(tmp, tmp_bytes, cnt, voff, (uint64_t)0, (size_t)(nv + 1),
-                                     rocprim::plus<uint64_t>(), gz_stream));
-    uint64_t total = 0;
-    GZ_CHECK(hipMemcpyAsync(&total, voff + nv, sizeof(uint64_t), hipMemcpyDeviceToHost, gz_stream));
-    GZ_CHECK(hipStreamSynchronize(gz_stream));
+    GZ_CHECK(rocprim::exclusive_scan(tmp, tmp_bytes, in, out, (uint64_t)0, (size_t)n, rocprim::plus<uint64_t>(),
+                                     gz_stream));
     gz_device_free(tmp);
-    gz_device_free(cnt);
+}
+
+/* Build one layout from sorted, duplicate-free keys[0, m) and the bounds of
+ * their groups (the low key bits when `low`). */
+void gz_build_layout(const uint64_t* keys, uint64_t m, uint32_t b, int low, uint64_t nv, const uint64_t* first,
+                     const uint64_t* end, gz_vec_t** d_vecs, uint64_t** d_offsets, uint64_t* vector_count)
+{
+    uint64_t* voff = (uint64_t*)gz_device_malloc((nv + 1) * sizeof(uint64_t));
+    gz_scan(rocprim::make_transform_iterator(rocprim::make_counting_iterator<uint64_t>(0),
+                                             gz_group_vectors{first, end, nv}),
+            voff, nv + 1);
+    uint64_t total = 0;
+    gz_copy_to_host(&total, voff + nv, sizeof(uint64_t));
     gz_vec_t* vecs = (gz_vec_t*)gz_device_malloc((total ? total : 1) * sizeof(gz_vec_t));
     if (m) {
-        hipLaunchKernelGGL(gz_k_pack, dim3(gz_grid_for(m)), dim3(tb), 0, gz_stream, keys, m, b, eoff, voff,
-                           (uint64_t*)vecs);
+        hipLaunchKernelGGL(gz_k_pack, dim3(gz_grid_for(m)), dim3(GZ_BLOCK), 0, gz_stream, keys, m, b, low, first, end,
+                           voff, (uint64_t*)vecs);
         GZ_LAUNCH_CHECK();
     }
-    GZ_CHECK(hipStreamSynchronize(gz_stream));
     *d_vecs = vecs;
     *d_offsets = voff;
     *vector_count = total;
@@ -251,25 +376,26 @@ __global__ void gz_k_count_sources(const uint64_t* __restrict__ keys, uint64_t n
         atomicAdd(&cnt[keys[i] & mask], 1u);
 }
 
-/* sort key: out-degree descending, then id ascending */
-__global__ void gz_k_degree_order(const uint32_t* __restrict__ cnt, uint64_t nv, uint64_t* __restrict__ order)
+/* sort key: out-degree descending (as `most` less the degree), then id ascending */
+__global__ void gz_k_degree_order(const uint32_t* __restrict__ cnt, uint64_t nv, uint32_t b, uint64_t most,
+                                  uint64_t* __restrict__ order)
 {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv; v += stride)
-        order[v] = ((uint64_t)(0xffffffffu - cnt[v]) << 32) | v;
+        order[v] = ((most - cnt[v]) << b) | v;
 }
 
 /* Rank i of the degree order becomes id i, except that each of the first
  * `tiers` runs of 8*S ranks is dealt round robin into eight S-id windows:
  * rank t*8S + q -> t*8S + (q % 8) * S + q / 8. */
-__global__ void gz_k_permutation(const uint64_t* __restrict__ order, uint64_t nv, uint64_t slice_vertices,
-                                 uint32_t tiers, uint64_t* __restrict__ old_of_new, uint32_t* __restrict__ new_of_old)
+__global__ void gz_k_permutation(const uint64_t* __restrict__ order, uint64_t nv, uint32_t b,
+                                 uint64_t slice_vertices, uint32_t tiers, uint64_t* __restrict__ old_of_new, uint32_t* __restrict__ new_of_old)
 {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     const uint64_t tier = (uint64_t)GZ_XCDS * slice_vertices;
     const uint64_t hot = tier * tiers;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += stride) {
-        const uint64_t old = order[i] & 0xffffffffull;
+        const uint64_t old = order[i] & ((1ull << b) - 1ull);
         uint64_t id = i;
         if (i < hot) {
             const uint64_t t = i / tier, q = i - t * tier;
@@ -287,7 +413,7 @@ __global__ void gz_k_remap_keys(uint64_t* __restrict__ keys, uint64_t n, uint32_
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         const uint64_t k = keys[i];
-        keys[i] = ((uint64_t)new_of_old[k >> b] << b) | (uint64_t)new_of_old[k & mask];
+        keys[i] = gz_edge_key(new_of_old[k >> b], new_of_old[k & mask], b, 1);
     }
 }
 
@@ -305,15 +431,17 @@ uint64_t* gz_relabel_by_outdegree(uint64_t* keys, uint64_t n, uint32_t b, uint64
         hipLaunchKernelGGL(gz_k_count_sources, dim3(gz_grid_for(n)), dim3(GZ_BLOCK), 0, gz_stream, keys, n, b, cnt);
         GZ_LAUNCH_CHECK();
     }
+    const uint64_t most = n < 0xffffffffull ? n : 0xffffffffull; /* counts are 32-bit */
     uint64_t* order = (uint64_t*)gz_device_malloc(nv * sizeof(uint64_t));
     uint64_t* order_b = (uint64_t*)gz_device_malloc(nv * sizeof(uint64_t));
-    hipLaunchKernelGGL(gz_k_degree_order, dim3(gz_grid_for(nv)), dim3(GZ_BLOCK), 0, gz_stream, cnt, nv, order);
+    hipLaunchKernelGGL(gz_k_degree_order, dim3(gz_grid_for(nv)), dim3(GZ_BLOCK), 0, gz_stream, cnt, nv, b,
+                       most, order);
     GZ_LAUNCH_CHECK();
     uint64_t* sorted = order;
-    if (nv > 1) gz_sort_keys(order, order_b, nv, 64, &sorted);
+    if (nv > 1) gz_sort_keys(order, order_b, nv, 0, b + gz_id_bits(most + 1), &sorted);
     uint64_t* old_of_new = (uint64_t*)gz_device_malloc((nv + 8) * sizeof(uint64_t));
     uint32_t* new_of_old = cnt; /* counts are no longer needed */
-    hipLaunchKernelGGL(gz_k_permutation, dim3(gz_grid_for(nv)), dim3(GZ_BLOCK), 0, gz_stream, sorted, nv,
+    hipLaunchKernelGGL(gz_k_permutation, dim3(gz_grid_for(nv)), dim3(GZ_BLOCK), 0, gz_stream, sorted, nv, b,
                        slice_vertices, tiers, old_of_new, new_of_old);
     GZ_LAUNCH_CHECK();
     if (n) {
@@ -340,47 +468,56 @@ void gz_ingress_from_keys(uint64_t nv, uint64_t* a, uint64_t* b_buf, uint64_t n,
     if (flags & GZ_INGRESS_RELABEL_BY_OUTDEGREE)
         old_of_new = gz_relabel_by_outdegree(a, n, b, nv, slice_vertices, tiers);
     uint64_t* sorted = a;
-    if (n > 1) gz_sort_keys(a, b_buf, n, 2 * b, &sorted);
+    if (n > 1) gz_sort_keys(a, b_buf, n, 0, 2 * b, &sorted);
     uint64_t* other = (sorted == a) ? b_buf : a;
     uint64_t m = 0;
+    uint64_t* first = (uint64_t*)gz_device_malloc(nv * sizeof(uint64_t));
+    uint64_t* end = (uint64_t*)gz_device_malloc(nv * sizeof(uint64_t));
     if (n) {
-        uint8_t* keep = (uint8_t*)gz_device_malloc(n);
-        uint64_t* d_count = (uint64_t*)gz_device_malloc(sizeof(uint64_t));
-        hipLaunchKernelGGL(gz_k_mark_kept, dim3(gz_grid_for(n)), dim3(GZ_BLOCK), 0, gz_stream, sorted, n, b, keep);
+        const uint64_t none = gz_no_key(b);
+        const uint64_t tiles = (n + GZ_TILE - 1) / GZ_TILE;
+        uint64_t* sums = (uint64_t*)gz_device_malloc(2 * (tiles + 1) * sizeof(uint64_t)); /* sums[tiles] stays 0 */
+        uint64_t* base = sums + tiles + 1;
+        hipLaunchKernelGGL(gz_k_tile_count<false>, dim3(gz_tile_grid(tiles)), dim3(GZ_BLOCK), 0, gz_stream, sorted, n,
+                           b, none, tiles, sums);
         GZ_LAUNCH_CHECK();
-        size_t tmp_bytes = 0;
-        GZ_CHECK(rocprim::select(nullptr, tmp_bytes, sorted, keep, other, d_count, (size_t)n, gz_stream));
-        void* tmp = gz_device_malloc(tmp_bytes ? tmp_bytes : 1);
-        GZ_CHECK(rocprim::select(tmp, tmp_bytes, sorted, keep, other, d_count, (size_t)n, gz_stream));
-        GZ_CHECK(hipMemcpyAsync(&m, d_count, sizeof(uint64_t), hipMemcpyDeviceToHost, gz_stream));
-        GZ_CHECK(hipStreamSynchronize(gz_stream));
-        gz_device_free(tmp);
-        gz_device_free(keep);
-        gz_device_free(d_count);
+        gz_scan(sums, base, tiles + 1);
+        hipLaunchKernelGGL(gz_k_kept_write, dim3(gz_tile_grid(tiles)), dim3(GZ_BLOCK), 0, gz_stream, sorted, n, b,
+                           none, tiles, base, other, first, end);
+        GZ_LAUNCH_CHECK();
+        gz_copy_to_host(&m, base + tiles, sizeof(uint64_t));
+        gz_device_free(sums);
     }
 
     gz_device_layouts_t L;
     L.num_vertices = nv;
     L.num_edges = m;
     L.original_ids = old_of_new;
-    uint64_t* eoff = (uint64_t*)gz_device_malloc((nv + 1) * sizeof(uint64_t));
-    gz_build_layout(other, m, b, nv, &L.pull, &L.pull_offsets, &L.pull_count, eoff);
-    /* push layout: swap group and neighbour, sort again (still unique) */
+    gz_build_layout(other, m, b, 0, nv, first, end, &L.pull, &L.pull_offsets, &L.pull_count);
+    /* push layout: the kept keys by source (still unique) */
+    uint64_t* push_sorted = other;
+    if (m > 1) gz_sort_keys(other, sorted, m, 0, b, &push_sorted);
+    gz_device_zero(first, nv * sizeof(uint64_t));
+    gz_device_zero(end, nv * sizeof(uint64_t));
     if (m) {
-        hipLaunchKernelGGL(gz_k_swap_keys, dim3(gz_grid_for(m)), dim3(GZ_BLOCK), 0, gz_stream, other, m, b, sorted);
+        hipLaunchKernelGGL(gz_k_low_bounds, dim3(gz_grid_for(m)), dim3(GZ_BLOCK), 0, gz_stream, push_sorted, m, b, first,
+                           end);
         GZ_LAUNCH_CHECK();
     }
-    uint64_t* push_sorted = sorted;
-    if (m > 1) gz_sort_keys(sorted, other, m, 2 * b, &push_sorted);
-    gz_build_layout(push_sorted, m, b, nv, &L.push, &L.push_offsets, &L.push_count, eoff);
+    gz_build_layout(push_sorted, m, b, 1, nv, first, end, &L.push, &L.push_offsets, &L.push_count);
     L.outdeg = (double*)gz_device_malloc((nv + 8) * sizeof(double));
-    hipLaunchKernelGGL(gz_k_outdegrees, dim3(gz_grid_for(nv + 8)), dim3(GZ_BLOCK), 0, gz_stream, eoff, nv, L.outdeg);
+    hipLaunchKernelGGL(gz_k_outdegrees, dim3(gz_grid_for(nv + 8)), dim3(GZ_BLOCK), 0, gz_stream, first, end, nv,
+                       L.outdeg);
     GZ_LAUNCH_CHECK();
     GZ_CHECK(hipStreamSynchronize(gz_stream));
-    gz_device_free(eoff);
+    gz_device_free(first);
+    gz_device_free(end);
     gz_graph_adopt_device(&L);
     if (slice_log2) gz_graph_build_source_slices(1ull << slice_log2, tiers, blocks, GZ_SLICE_BLOCK_VERTICES);
 }
+
+/* Whether the key kernels drop self-loops (a renumbering counts them first). */
+int gz_drop_first(uint32_t flags) { return (flags & GZ_INGRESS_RELABEL_BY_OUTDEGREE) ? 0 : 1; }
 
 void gz_check_vertex_count(uint64_t nv)
 {
@@ -412,7 +549,7 @@ extern "C" int gz_graph_build_pairs_device(uint64_t num_vertices, uint64_t num_e
     uint64_t* bb = (uint64_t*)gz_device_malloc((n ? n : 1) * sizeof(uint64_t));
     if (num_edges) {
         hipLaunchKernelGGL(gz_k_pairs_keys, dim3(gz_grid_for(num_edges)), dim3(GZ_BLOCK), 0, gz_stream, d_pairs,
-                           num_edges, b, symmetrize, a);
+                           num_edges, b, symmetrize, gz_drop_first(flags), a);
         GZ_LAUNCH_CHECK();
     }
     GZ_CHECK(hipStreamSynchronize(gz_stream));
@@ -447,14 +584,15 @@ extern "C" int gz_graph_build_rmat_device(const gz_rmat_params_t* p, uint64_t nu
         const uint32_t tb = (uint32_t)((p->a + p->b) * 65536.0);
         const uint32_t tc = (uint32_t)((p->a + p->b + p->c) * 65536.0);
         hipLaunchKernelGGL(gz_k_rmat_keys, dim3(gz_grid_for(p->num_edges)), dim3(GZ_BLOCK), 0, gz_stream, p->seed,
-                           p->edge_offset, p->scale, rmat_nv, ta, tb, tc, p->num_edges, b, symmetrize, (uint64_t)0, a);
+                           p->edge_offset, p->scale, rmat_nv, ta, tb, tc, p->num_edges, b, symmetrize, gz_drop_first(flags),
+                           (uint64_t)0, a);
         GZ_LAUNCH_CHECK();
     }
     if (extra_edges) {
         uint64_t* d_pairs = (uint64_t*)gz_device_malloc(2 * extra_edges * sizeof(uint64_t));
         gz_copy_to_device(d_pairs, extra_pairs, 2 * extra_edges * sizeof(uint64_t));
         hipLaunchKernelGGL(gz_k_pairs_keys, dim3(gz_grid_for(extra_edges)), dim3(GZ_BLOCK), 0, gz_stream, d_pairs,
-                           extra_edges, b, symmetrize, a + per * p->num_edges);
+                           extra_edges, b, symmetrize, gz_drop_first(flags), a + per * p->num_edges);
         GZ_LAUNCH_CHECK();
         GZ_CHECK(hipStreamSynchronize(gz_stream));
         gz_device_free(d_pairs);
@@ -492,7 +630,7 @@ extern "C" int gz_graph_build_rmat_union_device(const gz_rmat_params_t* params, 
         const uint32_t tc = (uint32_t)((p->a + p->b + p->c) * 65536.0);
         const uint64_t gnv = vertex_bases[g + 1] - vertex_bases[g];
         hipLaunchKernelGGL(gz_k_rmat_keys, dim3(gz_grid_for(p->num_edges)), dim3(GZ_BLOCK), 0, gz_stream, p->seed,
-                           p->edge_offset, p->scale, gnv, ta, tb, tc, p->num_edges, b, symmetrize, vertex_bases[g],
+                           p->edge_offset, p->scale, gnv, ta, tb, tc, p->num_edges, b, symmetrize, 1, vertex_bases[g],
                            a + at);
         GZ_LAUNCH_CHECK();
         at += per * p->num_edges;
@@ -506,9 +644,17 @@ extern "C" int gz_graph_build_rmat_union_device(const gz_rmat_params_t* params, 
 
 /* ---- source-sliced pull layout ---------------------------------------------
  * From the loaded pull vectors: every valid lane becomes the key
- * (slice << 2b | dst << b | src) (invalid lanes all ones), a stable radix pass
- * over the 7 slice bits groups the keys by slice while keeping the (dst, src)
- * order, and each slice's keys are packed by the layout builder above. */
+ * (slice << 2b | dst << b | src) (invalid lanes all ones), and a stable radix
+ * pass over the 7 slice bits groups the keys by slice while keeping the
+ * (dst, src) order.  A run is the keys of one (slice, dst) pair: numbered in
+ * key order, run r is the slice accumulator r, and its number less its slice's
+ * first one is the destination's local rank.  All slices are then built
+ * together, in a number of launches that does not grow with theirs:
+ *   runs    each run's first key and destination (tile counts, then a write)
+ *   vectors the exclusive scan of the runs' ceil(length / 4)
+ *   pack    each vector's packed neighbours and local rank, in place
+ *   mask    per 64-vertex block, the slice bits of its vertices and the
+ *           number of its first run in each slice */
 namespace {
 
 __global__ void gz_k_slice_keys(const gz_vec_t* __restrict__ vecs, uint64_t nvec, uint32_t b, uint64_t slice_vertices,
@@ -551,168 +697,215 @@ __global__ void gz_k_slice_bounds(const uint64_t* __restrict__ keys, uint64_t n,
     first[x] = lo;
 }
 
-__global__ void gz_k_strip_slice(uint64_t* __restrict__ keys, uint64_t n, uint32_t b)
+/* Run r's first key (run_first[r], with run_first[runs] = n) and its
+ * destination; the runs ahead of each tile come from the tile counts. */
+__global__ __launch_bounds__(GZ_BLOCK) void gz_k_slice_runs(const uint64_t* __restrict__ keys, uint64_t n, uint32_t b,
+                                                            uint64_t tiles, const uint64_t* __restrict__ tile_base,
+                                                            uint64_t* __restrict__ run_first, uint32_t* __restrict__ gid)
 {
-    const uint64_t mask = (1ull << (2 * b)) - 1ull;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) keys[i] &= mask;
+    __shared__ uint32_t lds[GZ_WAVES_PER_BLOCK];
+    const uint64_t below = (1ull << gz_lane()) - 1ull, mask = (1ull << b) - 1ull;
+    for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        gz_tile_keys t;
+        const uint64_t base = gz_tile_load(t, keys, n, tile, ~0ull);
+        uint64_t heads[GZ_TILE_ROWS];
+        uint32_t c = 0;
+#pragma unroll
+        for (int r = 0; r < GZ_TILE_ROWS; ++r) {
+            heads[r] = __ballot(gz_tile_flag<true>(t, r, base + (uint64_t)(r * GZ_WAVE + gz_lane()), n, b, ~0ull));
+            c += (uint32_t)__popcll(heads[r]);
+        }
+        uint64_t at = tile_base[tile] + gz_tile_wave_base(c, lds);
+#pragma unroll
+        for (int r = 0; r < GZ_TILE_ROWS; ++r) {
+            if ((heads[r] >> gz_lane()) & 1ull) {
+                const uint64_t run = at + (uint64_t)__popcll(heads[r] & below);
+                run_first[run] = base + (uint64_t)(r * GZ_WAVE + gz_lane());
+                gid[run] = (uint32_t)((t.k[r] >> b) & mask);
+            }
+            at += (uint64_t)__popcll(heads[r]);
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) run_first[tile_base[tiles]] = n;
 }
 
-/* mask bit for slice `bit`, and has[v] = 1 when v has vectors in the slice
- * (has[nv] = 0, so its exclusive scan ends in the slice's vertex count) */
-template <typename M>
-__global__ void gz_k_slice_mask(const uint64_t* __restrict__ voff, uint64_t nv, uint32_t bit, M* __restrict__ mask,
-                                uint64_t* __restrict__ has)
+/* Vectors of run r, 0 past the last run. */
+struct gz_run_vectors {
+    const uint64_t* run_first;
+    uint64_t runs;
+    __device__ uint64_t operator()(uint64_t r) const { return r < runs ? (run_first[r + 1] - run_first[r] + 3) / 4 : 0; }
+};
+
+/* For slice x in [0, nslices]: its first run (first key lo[x] starts one) and
+ * its first vector. */
+__global__ void gz_k_slice_firsts(const uint64_t* __restrict__ lo, uint32_t nslices,
+                                  const uint64_t* __restrict__ run_first, uint64_t runs,
+                                  const uint64_t* __restrict__ run_vec, uint64_t* __restrict__ first_run,
+                                  uint64_t* __restrict__ first_vec)
 {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v <= nv; v += stride) {
-        const bool in = v < nv && voff[v + 1] > voff[v];
-        if (in) mask[v] |= (M)1 << bit;
-        has[v] = in ? 1 : 0;
+    const uint32_t x = threadIdx.x;
+    if (x > nslices) return;
+    uint64_t a = 0, z = runs;
+    while (a < z) {
+        const uint64_t mid = a + ((z - a) >> 1);
+        if (run_first[mid] < lo[x])
+            a = mid + 1;
+        else
+            z = mid;
+    }
+    first_run[x] = a;
+    first_vec[x] = run_vec[a];
+}
+
+struct gz_slice_pack_t {
+    uint64_t S, H;
+    uint32_t blocks, nslices;
+    uint64_t block_first, block_span, cold_first; /* first vector of the block slices, their count, and the cold slice's first */
+    const uint64_t* first_run;                    /* [nslices + 1], device */
+    uint32_t* nbr24;
+    uint64_t* nbr16;
+    gz_u32x4* nbr;
+    uint32_t* shared;
+};
+
+/* The packed vectors (gz_walk.h) of every slice: the lane that holds a
+ * vector's first key writes it.  Window slices: 12 bytes, four 24-bit offsets
+ * from the window's first vertex (empty lanes all ones), bit 23 of the first
+ * set on the first vector of each destination.  Block slices: 8 bytes, four
+ * 16-bit offsets from the block's first vertex (GZ_PACKED16_NONE for an empty
+ * lane), bit 15 of the first the flag.  The cold slice: 16 bytes, four 32-bit
+ * ids (GZ_PACKED_NONE), flag in bit 31.  shared: the local rank. */
+__global__ __launch_bounds__(GZ_BLOCK) void gz_k_slice_pack(const uint64_t* __restrict__ keys, uint64_t n, uint32_t b,
+                                                            uint64_t tiles, const uint64_t* __restrict__ tile_base,
+                                                            const uint64_t* __restrict__ run_first,
+                                                            const uint64_t* __restrict__ run_vec, gz_slice_pack_t p)
+{
+    __shared__ uint32_t lds[GZ_WAVES_PER_BLOCK];
+    const uint64_t upto = (2ull << gz_lane()) - 1ull, mask = (1ull << b) - 1ull;
+    for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        gz_tile_keys t;
+        const uint64_t base = gz_tile_load(t, keys, n, tile, ~0ull);
+        uint64_t heads[GZ_TILE_ROWS];
+        uint32_t c = 0;
+#pragma unroll
+        for (int r = 0; r < GZ_TILE_ROWS; ++r) {
+            heads[r] = __ballot(gz_tile_flag<true>(t, r, base + (uint64_t)(r * GZ_WAVE + gz_lane()), n, b, ~0ull));
+            c += (uint32_t)__popcll(heads[r]);
+        }
+        uint64_t at = tile_base[tile] + gz_tile_wave_base(c, lds);
+#pragma unroll
+        for (int r = 0; r < GZ_TILE_ROWS; ++r) {
+            const uint64_t i = base + (uint64_t)(r * GZ_WAVE + gz_lane());
+            /* the key's run: heads up to and including it, less one (a key
+             * that is no head has one ahead of it) */
+            const uint64_t run = at + (uint64_t)__popcll(heads[r] & upto) - 1;
+            at += (uint64_t)__popcll(heads[r]);
+            if (i >= n) continue;
+            const uint64_t rf = run_first[run], rank = i - rf;
+            if (rank & 3) continue;
+            const uint64_t j = run_vec[run] + rank / 4;
+            const uint64_t left = run_first[run + 1] - i;
+            const uint64_t k0 = t.k[r];
+            const uint32_t x = (uint32_t)(k0 >> (2 * b));
+            const uint64_t s0 = k0 & mask;
+            const uint64_t s1 = left > 1 ? keys[i + 1] & mask : 0, s2 = left > 2 ? keys[i + 2] & mask : 0,
+                           s3 = left > 3 ? keys[i + 3] & mask : 0;
+            const bool first = rank == 0;
+            p.shared[j] = (uint32_t)(run - p.first_run[x]);
+            if (x + 1 == p.nslices) {
+                gz_u32x4 a;
+                a.x = (uint32_t)s0 | (first ? 0x80000000u : 0u);
+                a.y = left > 1 ? (uint32_t)s1 : GZ_PACKED_NONE;
+                a.z = left > 2 ? (uint32_t)s2 : GZ_PACKED_NONE;
+                a.w = left > 3 ? (uint32_t)s3 : GZ_PACKED_NONE;
+                p.nbr[j - p.cold_first] = a;
+                continue;
+            }
+            const uint32_t level = x / GZ_XCDS;
+            const uint64_t window = gz_slice_window(x, p.S, p.blocks);
+            if (level >= 1 && level <= p.blocks) {
+                const uint64_t w = window + (uint64_t)level * p.H;
+                const uint64_t f0 = (s0 - w) | (first ? GZ_PACKED16_FIRST : 0u);
+                const uint64_t f1 = left > 1 ? s1 - w : GZ_PACKED16_NONE;
+                const uint64_t f2 = left > 2 ? s2 - w : GZ_PACKED16_NONE;
+                const uint64_t f3 = left > 3 ? s3 - w : GZ_PACKED16_NONE;
+                p.nbr16[j - p.block_first] = f0 | (f1 << 16) | (f2 << 32) | (f3 << 48);
+                continue;
+            }
+            const uint32_t f0 = (uint32_t)(s0 - window) | (first ? 0x800000u : 0u);
+            const uint32_t f1 = left > 1 ? (uint32_t)(s1 - window) : 0xffffffu;
+            const uint32_t f2 = left > 2 ? (uint32_t)(s2 - window) : 0xffffffu;
+            const uint32_t f3 = left > 3 ? (uint32_t)(s3 - window) : 0xffffffu;
+            uint32_t* w = p.nbr24 + 3 * (j - (level > p.blocks ? p.block_span : 0));
+            w[0] = f0 | (f1 << 24);
+            w[1] = (f1 >> 8) | (f2 << 16);
+            w[2] = (f2 >> 16) | (f3 << 8);
+        }
     }
 }
 
-/* gid[rank[v]] = v for the vertices with vectors in the slice */
-__global__ void gz_k_slice_gid(const uint64_t* __restrict__ has, const uint64_t* __restrict__ rank, uint64_t nv,
-                               uint32_t* __restrict__ gid)
+/* mask[v] bit x: v has vectors in slice x; rank_base[k * nslices + x]: the
+ * first run of slice x whose destination is not below 64 k.  A wavefront takes
+ * `per` consecutive 64-vertex blocks: lane x finds slice x's run at the first
+ * of them by binary search in the runs' destinations (ascending inside a
+ * slice) and steps it from block to block by the runs the block held. */
+template <typename M>
+__global__ __launch_bounds__(GZ_BLOCK) void gz_k_slice_mask(const uint32_t* __restrict__ gid, uint32_t nslices,
+                                                            const uint64_t* __restrict__ first_run, uint64_t nv,
+                                                            uint64_t nblocks, uint64_t per, M* __restrict__ mask,
+                                                            uint32_t* __restrict__ rank_base)
 {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv; v += stride)
-        if (has[v]) gid[rank[v]] = (uint32_t)v;
+    __shared__ unsigned long long bits[GZ_WAVES_PER_BLOCK][GZ_WAVE];
+    const int lane = gz_lane();
+    unsigned long long* mine = bits[threadIdx.x / GZ_WAVE];
+    const uint64_t wave = (uint64_t)blockIdx.x * GZ_WAVES_PER_BLOCK + threadIdx.x / GZ_WAVE;
+    const uint64_t k0 = wave * per;
+    if (k0 >= nblocks) return;
+    const uint64_t k1 = k0 + per < nblocks ? k0 + per : nblocks;
+    uint32_t at = 0, end = 0;
+    if ((uint32_t)lane < nslices) {
+        at = (uint32_t)first_run[lane];
+        end = (uint32_t)first_run[lane + 1];
+        uint32_t z = end;
+        while (at < z) {
+            const uint32_t mid = at + ((z - at) >> 1);
+            if ((uint64_t)gid[mid] < k0 * GZ_WAVE)
+                at = mid + 1;
+            else
+                z = mid;
+        }
+    }
+    for (uint64_t k = k0; k < k1; ++k) {
+        if ((uint32_t)lane < nslices) rank_base[k * nslices + (uint32_t)lane] = at;
+        mine[lane] = 0;
+        const uint64_t stop = (k + 1) * GZ_WAVE;
+        for (uint32_t x0 = 0; x0 < nslices; x0 += 8) {
+            uint32_t g[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) {
+                const uint32_t x = x0 + u; /* lanes from nslices on hold empty ranges; x stays below 64 */
+                const uint32_t i = (uint32_t)__builtin_amdgcn_readlane((int)at, (int)x) + (uint32_t)lane;
+                g[u] = i < (uint32_t)__builtin_amdgcn_readlane((int)end, (int)x) ? gid[i] : 0xffffffffu;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) {
+                const bool in = (uint64_t)g[u] < stop;
+                if (in) mine[g[u] & (GZ_WAVE - 1)] |= 1ull << (x0 + u); /* the lanes' vertices differ */
+                const uint32_t c = (uint32_t)__popcll(__ballot(in));
+                if ((uint32_t)lane == x0 + u) at += c;
+            }
+        }
+        const uint64_t v = k * GZ_WAVE + (uint64_t)lane;
+        if (v < nv) mask[v] = (M)mine[lane];
+    }
 }
 
-/* index in the concatenated slice accumulators (slice x's run starts at
- * `part_off`) of the first vertex of each 64-vertex block, at
- * out[block * nslices + x] */
 /* 32-bit copy of the FP64 out-degrees (integral, below 2^32: V <= 2^28 here). */
 __global__ void gz_k_outdeg32(const double* __restrict__ outdeg, uint64_t n, uint32_t* __restrict__ out)
 {
     /* grid-stride: gz_grid_for caps the grid at 65,536 workgroups */
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
         out[i] = (uint32_t)outdeg[i];
-}
-
-__global__ void gz_k_rank_base(const uint64_t* __restrict__ rank, uint64_t blocks, uint32_t x, uint32_t nslices,
-                               uint64_t part_off, uint32_t* __restrict__ out)
-{
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < blocks; k += stride)
-        out[k * nslices + x] = (uint32_t)(part_off + rank[k * GZ_WAVE]);
-}
-
-/* the shared vertex of every vector becomes the destination's local rank */
-__global__ void gz_k_local_dst(gz_vec_t* __restrict__ vecs, uint64_t n, const uint64_t* __restrict__ rank)
-{
-    const uint64_t clear = ~(0x7fffull << 48);
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += stride) {
-        gz_lanes w;
-        w.l0 = vecs[j].lane[0];
-        w.l1 = vecs[j].lane[1];
-        w.l2 = vecs[j].lane[2];
-        w.l3 = vecs[j].lane[3];
-        const uint64_t r = rank[gz_shared_vertex(w)];
-        vecs[j].lane[0] = (w.l0 & clear) | gz_piece(r, 0);
-        vecs[j].lane[1] = (w.l1 & clear) | gz_piece(r, 1);
-        vecs[j].lane[2] = (w.l2 & clear) | gz_piece(r, 2);
-        vecs[j].lane[3] = (w.l3 & clear) | gz_piece(r, 3);
-    }
-}
-
-/* Vector-Sparse vectors of one slice -> their 32-bit shared vertices, and
- * (nbr != nullptr) 16-byte packed vectors: 32-bit neighbour ids (empty lanes
- * GZ_PACKED_NONE), bit 31 of the first set on the first vector of each
- * destination. */
-__global__ void gz_k_pack_u32(const gz_vec_t* __restrict__ vecs, uint64_t n, gz_u32x4* __restrict__ nbr,
-                              uint32_t* __restrict__ shared)
-{
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += stride) {
-        gz_lanes w;
-        w.l0 = vecs[j].lane[0];
-        w.l1 = vecs[j].lane[1];
-        w.l2 = vecs[j].lane[2];
-        w.l3 = vecs[j].lane[3];
-        const uint64_t d = gz_shared_vertex(w);
-        bool first = true;
-        if (j > 0) {
-            gz_lanes p;
-            p.l0 = vecs[j - 1].lane[0];
-            p.l1 = vecs[j - 1].lane[1];
-            p.l2 = vecs[j - 1].lane[2];
-            p.l3 = vecs[j - 1].lane[3];
-            first = gz_shared_vertex(p) != d;
-        }
-        gz_u32x4 a;
-        a.x = (uint32_t)gz_lane_id(w.l0) | (first ? 0x80000000u : 0u); /* the first lane holds an edge */
-        a.y = gz_lane_valid(w.l1) ? (uint32_t)gz_lane_id(w.l1) : GZ_PACKED_NONE;
-        a.z = gz_lane_valid(w.l2) ? (uint32_t)gz_lane_id(w.l2) : GZ_PACKED_NONE;
-        a.w = gz_lane_valid(w.l3) ? (uint32_t)gz_lane_id(w.l3) : GZ_PACKED_NONE;
-        if (nbr) nbr[j] = a;
-        shared[j] = (uint32_t)d;
-    }
-}
-
-/* Vector-Sparse vectors of one block slice -> 8-byte packed vectors: four
- * 16-bit offsets from the block's first vertex (GZ_PACKED16_NONE for an empty
- * lane), bit 15 of the first set on the first vector of each destination. */
-__global__ void gz_k_pack_u16(const gz_vec_t* __restrict__ vecs, uint64_t n, uint64_t window,
-                              uint64_t* __restrict__ words)
-{
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += stride) {
-        gz_lanes w;
-        w.l0 = vecs[j].lane[0];
-        w.l1 = vecs[j].lane[1];
-        w.l2 = vecs[j].lane[2];
-        w.l3 = vecs[j].lane[3];
-        bool first = true;
-        if (j > 0) {
-            gz_lanes p;
-            p.l0 = vecs[j - 1].lane[0];
-            p.l1 = vecs[j - 1].lane[1];
-            p.l2 = vecs[j - 1].lane[2];
-            p.l3 = vecs[j - 1].lane[3];
-            first = gz_shared_vertex(p) != gz_shared_vertex(w);
-        }
-        const uint64_t f0 = (gz_lane_id(w.l0) - window) | (first ? GZ_PACKED16_FIRST : 0u);
-        const uint64_t f1 = gz_lane_valid(w.l1) ? gz_lane_id(w.l1) - window : GZ_PACKED16_NONE;
-        const uint64_t f2 = gz_lane_valid(w.l2) ? gz_lane_id(w.l2) - window : GZ_PACKED16_NONE;
-        const uint64_t f3 = gz_lane_valid(w.l3) ? gz_lane_id(w.l3) - window : GZ_PACKED16_NONE;
-        words[j] = f0 | (f1 << 16) | (f2 << 32) | (f3 << 48);
-    }
-}
-
-/* Vector-Sparse vectors of one window slice -> 12-byte packed vectors: four
- * 24-bit offsets from the window's first vertex (empty lanes all ones), bit
- * 23 of the first set on the first vector of each destination. */
-__global__ void gz_k_pack_u24(const gz_vec_t* __restrict__ vecs, uint64_t n, uint64_t window,
-                              uint32_t* __restrict__ words)
-{
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += stride) {
-        gz_lanes w;
-        w.l0 = vecs[j].lane[0];
-        w.l1 = vecs[j].lane[1];
-        w.l2 = vecs[j].lane[2];
-        w.l3 = vecs[j].lane[3];
-        bool first = true;
-        if (j > 0) {
-            gz_lanes p;
-            p.l0 = vecs[j - 1].lane[0];
-            p.l1 = vecs[j - 1].lane[1];
-            p.l2 = vecs[j - 1].lane[2];
-            p.l3 = vecs[j - 1].lane[3];
-            first = gz_shared_vertex(p) != gz_shared_vertex(w);
-        }
-        const uint32_t f0 = (uint32_t)(gz_lane_id(w.l0) - window) | (first ? 0x800000u : 0u);
-        const uint32_t f1 = gz_lane_valid(w.l1) ? (uint32_t)(gz_lane_id(w.l1) - window) : 0xffffffu;
-        const uint32_t f2 = gz_lane_valid(w.l2) ? (uint32_t)(gz_lane_id(w.l2) - window) : 0xffffffu;
-        const uint32_t f3 = gz_lane_valid(w.l3) ? (uint32_t)(gz_lane_id(w.l3) - window) : 0xffffffu;
-        words[3 * j] = f0 | (f1 << 24);
-        words[3 * j + 1] = (f1 >> 8) | (f2 << 16);
-        words[3 * j + 2] = (f2 >> 16) | (f3 << 8);
-    }
 }
 
 }  // namespace
@@ -754,133 +947,101 @@ extern "C" int gz_graph_build_source_slices(uint64_t slice_vertices, uint32_t ti
     const uint64_t n = 4 * nvec;
     uint64_t* a = (uint64_t*)gz_device_malloc((n ? n : 1) * sizeof(uint64_t));
     uint64_t* bb = (uint64_t*)gz_device_malloc((n ? n : 1) * sizeof(uint64_t));
-    uint64_t* first = (uint64_t*)gz_device_malloc((GZ_MAX_SLICES + 1) * sizeof(uint64_t));
-    uint64_t lo[GZ_MAX_SLICES + 1];
+    /* per slice: first key, first run, first vector (zero without edges) */
+    uint64_t* firsts = (uint64_t*)gz_device_malloc(3 * (GZ_MAX_SLICES + 1) * sizeof(uint64_t));
+    uint64_t* first_run = firsts + GZ_MAX_SLICES + 1;
+    uint64_t* first_vec = first_run + GZ_MAX_SLICES + 1;
     uint64_t* sorted = a;
+    uint64_t m = 0, runs = 0, tiles = 0;
+    uint64_t *tile_base = nullptr, *run_first = nullptr, *run_vec = nullptr;
     if (n) {
         hipLaunchKernelGGL(gz_k_slice_keys, dim3(gz_grid_for(n)), dim3(GZ_BLOCK), 0, gz_stream, gz_graph.pull_vectors,
                            nvec, b, S, tiers, blocks, H, a);
         GZ_LAUNCH_CHECK();
-        rocprim::double_buffer<uint64_t> db(a, bb);
-        size_t tmp_bytes = 0;
-        GZ_CHECK(rocprim::radix_sort_keys(nullptr, tmp_bytes, db, (size_t)n, 2 * b, 2 * b + GZ_SLICE_KEY_BITS,
-                                          gz_stream));
-        void* tmp = gz_device_malloc(tmp_bytes ? tmp_bytes : 1);
-        GZ_CHECK(rocprim::radix_sort_keys(tmp, tmp_bytes, db, (size_t)n, 2 * b, 2 * b + GZ_SLICE_KEY_BITS,
-                                          gz_stream));
-        GZ_CHECK(hipStreamSynchronize(gz_stream));
-        gz_device_free(tmp);
-        sorted = db.current();
-        hipLaunchKernelGGL(gz_k_slice_bounds, dim3(1), dim3(64), 0, gz_stream, sorted, n, b, ns, first);
+        gz_sort_keys(a, bb, n, 2 * b, 2 * b + GZ_SLICE_KEY_BITS, &sorted);
+        hipLaunchKernelGGL(gz_k_slice_bounds, dim3(1), dim3(64), 0, gz_stream, sorted, n, b, ns, firsts);
         GZ_LAUNCH_CHECK();
-        gz_copy_to_host(lo, first, (ns + 1) * sizeof(uint64_t));
-        hipLaunchKernelGGL(gz_k_strip_slice, dim3(gz_grid_for(lo[ns])), dim3(GZ_BLOCK), 0, gz_stream, sorted, lo[ns],
-                           b);
-        GZ_LAUNCH_CHECK();
-    } else {
-        for (uint32_t x = 0; x <= ns; ++x) lo[x] = 0;
+        gz_copy_to_host(&m, firsts + ns, sizeof(uint64_t));
+        tiles = (m + GZ_TILE - 1) / GZ_TILE;
     }
-    gz_slices.mask = gz_device_malloc((nv + 8) * (wide_mask ? sizeof(uint64_t) : sizeof(uint32_t)));
-    gz_slices.rank_blocks = (nv + GZ_WAVE - 1) / GZ_WAVE;
-    gz_slices.rank_base = (uint32_t*)gz_device_malloc(ns * gz_slices.rank_blocks * sizeof(uint32_t));
-    uint64_t* eoff = (uint64_t*)gz_device_malloc((nv + 1) * sizeof(uint64_t));
-    uint64_t* has = (uint64_t*)gz_device_malloc((nv + 1) * sizeof(uint64_t));
-    uint64_t* rank = (uint64_t*)gz_device_malloc((nv + 1) * sizeof(uint64_t));
-    size_t scan_bytes = 0;
-    GZ_CHECK(rocprim::exclusive_scan(nullptr, scan_bytes, has, rank, (uint64_t)0, (size_t)(nv + 1),
-                                     rocprim::plus<uint64_t>(), gz_stream));
-    void* scan_tmp = gz_device_malloc(scan_bytes ? scan_bytes : 1);
-    gz_vec_t* part_vecs[GZ_MAX_SLICES];
-    uint32_t* part_gid[GZ_MAX_SLICES];
-    uint64_t counts[GZ_MAX_SLICES], ranked[GZ_MAX_SLICES];
-    uint64_t part_off = 0;
-    for (uint32_t x = 0; x < ns; ++x) {
-        uint64_t* voff = nullptr;
-        gz_build_layout(sorted + lo[x], lo[x + 1] - lo[x], b, nv, &part_vecs[x], &voff, &counts[x], eoff);
-        if (wide_mask)
-            hipLaunchKernelGGL(gz_k_slice_mask<uint64_t>, dim3(gz_grid_for(nv + 1)), dim3(GZ_BLOCK), 0, gz_stream,
-                               voff, nv, x, (uint64_t*)gz_slices.mask, has);
-        else
-            hipLaunchKernelGGL(gz_k_slice_mask<uint32_t>, dim3(gz_grid_for(nv + 1)), dim3(GZ_BLOCK), 0, gz_stream,
-                               voff, nv, x, (uint32_t*)gz_slices.mask, has);
+    if (m) {
+        uint64_t* sums = (uint64_t*)gz_device_malloc(2 * (tiles + 1) * sizeof(uint64_t)); /* sums[tiles] stays 0 */
+        tile_base = sums + tiles + 1;
+        hipLaunchKernelGGL(gz_k_tile_count<true>, dim3(gz_tile_grid(tiles)), dim3(GZ_BLOCK), 0, gz_stream, sorted, m, b,
+                           ~0ull, tiles, sums);
         GZ_LAUNCH_CHECK();
-        GZ_CHECK(rocprim::exclusive_scan(scan_tmp, scan_bytes, has, rank, (uint64_t)0, (size_t)(nv + 1),
-                                         rocprim::plus<uint64_t>(), gz_stream));
-        hipLaunchKernelGGL(gz_k_rank_base, dim3(gz_grid_for(gz_slices.rank_blocks)), dim3(GZ_BLOCK), 0, gz_stream,
-                           rank, gz_slices.rank_blocks, x, ns, part_off, gz_slices.rank_base);
-        GZ_LAUNCH_CHECK();
-        if (counts[x]) {
-            hipLaunchKernelGGL(gz_k_local_dst, dim3(gz_grid_for(counts[x])), dim3(GZ_BLOCK), 0, gz_stream,
-                               part_vecs[x], counts[x], rank);
-            GZ_LAUNCH_CHECK();
-        }
-        gz_copy_to_host(&ranked[x], rank + nv, sizeof(uint64_t));
-        part_off += ranked[x];
-        if (part_off + 8 > 0xffffffffull) {
-            fprintf(stderr, "grazelle: the sliced layout needs fewer than 2^32 slice accumulators\n");
-            exit(65);
-        }
-        part_gid[x] = (uint32_t*)gz_device_malloc((ranked[x] ? ranked[x] : 1) * sizeof(uint32_t));
-        hipLaunchKernelGGL(gz_k_slice_gid, dim3(gz_grid_for(nv)), dim3(GZ_BLOCK), 0, gz_stream, has, rank, nv,
-                           part_gid[x]);
-        GZ_LAUNCH_CHECK();
-        GZ_CHECK(hipStreamSynchronize(gz_stream));
-        gz_device_free(voff);
+        gz_scan(sums, tile_base, tiles + 1);
+        gz_copy_to_host(&runs, tile_base + tiles, sizeof(uint64_t));
     }
-    gz_device_free(scan_tmp);
-    gz_device_free(rank);
-    gz_device_free(has);
-    gz_device_free(eoff);
-    gz_device_free(first);
-    gz_device_free(a);
-    gz_device_free(bb);
-    gz_slices.begin[0] = 0;
-    for (uint32_t x = 0; x < ns; ++x) gz_slices.begin[x + 1] = gz_slices.begin[x] + counts[x];
+    if (runs + 8 > 0xffffffffull) {
+        fprintf(stderr, "grazelle: the sliced layout needs fewer than 2^32 slice accumulators\n");
+        exit(65);
+    }
+    gz_slices.gid = (uint32_t*)gz_device_malloc((runs + 8) * sizeof(uint32_t));
+    if (m) {
+        run_first = (uint64_t*)gz_device_malloc((runs + 1) * sizeof(uint64_t));
+        run_vec = (uint64_t*)gz_device_malloc((runs + 1) * sizeof(uint64_t));
+        hipLaunchKernelGGL(gz_k_slice_runs, dim3(gz_tile_grid(tiles)), dim3(GZ_BLOCK), 0, gz_stream, sorted, m, b, tiles,
+                           tile_base, run_first, gz_slices.gid);
+        GZ_LAUNCH_CHECK();
+        gz_scan(rocprim::make_transform_iterator(rocprim::make_counting_iterator<uint64_t>(0),
+                                                 gz_run_vectors{run_first, runs}),
+                run_vec, runs + 1);
+        hipLaunchKernelGGL(gz_k_slice_firsts, dim3(1), dim3(64), 0, gz_stream, firsts, ns, run_first, runs, run_vec,
+                           first_run, first_vec);
+        GZ_LAUNCH_CHECK();
+    }
+    uint64_t host_firsts[3 * (GZ_MAX_SLICES + 1)];
+    gz_copy_to_host(host_firsts, firsts, sizeof(host_firsts));
+    memset(&gz_slices.part_base, 0, sizeof(gz_slices.part_base));
+    for (uint32_t x = 0; x <= ns; ++x) {
+        gz_slices.part_base.off[x] = host_firsts[GZ_MAX_SLICES + 1 + x];
+        gz_slices.begin[x] = host_firsts[2 * (GZ_MAX_SLICES + 1) + x];
+    }
     const uint64_t total = gz_slices.begin[ns];
+    const uint64_t cold = total - gz_slices.begin[ns - 1];
     const uint64_t block_first = gz_slices.begin[GZ_XCDS];
     const uint64_t block_span = gz_slices.begin[GZ_XCDS * (blocks + 1)] - block_first;
     const uint64_t window_total = gz_slices.begin[ns - 1] - block_span;
     gz_slices.nbr24 = (uint32_t*)gz_device_malloc((window_total ? 3 * window_total : 1) * sizeof(uint32_t));
     gz_slices.nbr16 = (uint64_t*)gz_device_malloc((block_span ? block_span : 1) * sizeof(uint64_t));
     gz_slices.block_span = block_span;
-    gz_slices.nbr = (gz_u32x4*)gz_device_malloc((counts[ns - 1] ? counts[ns - 1] : 1) * sizeof(gz_u32x4));
+    gz_slices.nbr = (gz_u32x4*)gz_device_malloc((cold ? cold : 1) * sizeof(gz_u32x4));
     gz_slices.shared = (uint32_t*)gz_device_malloc((total ? total : 1) * sizeof(uint32_t));
-    for (uint32_t x = 0; x < ns; ++x) {
-        if (counts[x]) {
-            /* the shared vertices of every slice, then the packed neighbours */
-            hipLaunchKernelGGL(gz_k_pack_u32, dim3(gz_grid_for(counts[x])), dim3(GZ_BLOCK), 0, gz_stream, part_vecs[x],
-                               counts[x], x + 1 == ns ? gz_slices.nbr : (gz_u32x4*)nullptr,
-                               gz_slices.shared + gz_slices.begin[x]);
-            GZ_LAUNCH_CHECK();
-            const uint32_t level = x / GZ_XCDS;
-            if (x + 1 < ns && level >= 1 && level <= blocks) {
-                hipLaunchKernelGGL(gz_k_pack_u16, dim3(gz_grid_for(counts[x])), dim3(GZ_BLOCK), 0, gz_stream,
-                                   part_vecs[x], counts[x], gz_slice_window(x, S, blocks) + (uint64_t)level * H,
-                                   gz_slices.nbr16 + (gz_slices.begin[x] - block_first));
-                GZ_LAUNCH_CHECK();
-            } else if (x + 1 < ns) {
-                const uint64_t at = gz_slices.begin[x] - (level > blocks ? block_span : 0);
-                hipLaunchKernelGGL(gz_k_pack_u24, dim3(gz_grid_for(counts[x])), dim3(GZ_BLOCK), 0, gz_stream,
-                                   part_vecs[x], counts[x], gz_slice_window(x, S, blocks), gz_slices.nbr24 + 3 * at);
-                GZ_LAUNCH_CHECK();
-            }
-        }
-        GZ_CHECK(hipStreamSynchronize(gz_stream));
-        gz_device_free(part_vecs[x]);
+    if (m) {
+        const gz_slice_pack_t pack{S,         H,          blocks,    ns, block_first, block_span, gz_slices.begin[ns - 1],
+                                   first_run, gz_slices.nbr24, gz_slices.nbr16, gz_slices.nbr, gz_slices.shared};
+        hipLaunchKernelGGL(gz_k_slice_pack, dim3(gz_tile_grid(tiles)), dim3(GZ_BLOCK), 0, gz_stream, sorted, m, b, tiles,
+                           tile_base, run_first, run_vec, pack);
+        GZ_LAUNCH_CHECK();
     }
-    memset(&gz_slices.part_base, 0, sizeof(gz_slices.part_base));
-    for (uint32_t x = 0; x < ns; ++x) gz_slices.part_base.off[x + 1] = gz_slices.part_base.off[x] + ranked[x];
-    gz_slices.parts = (double*)gz_device_malloc((gz_slices.part_base.off[ns] + 8) * sizeof(double));
-    gz_slices.gid = (uint32_t*)gz_device_malloc((gz_slices.part_base.off[ns] + 8) * sizeof(uint32_t));
-    for (uint32_t x = 0; x < ns; ++x) {
-        if (ranked[x]) gz_device_copy(gz_slices.gid + gz_slices.part_base.off[x], part_gid[x], ranked[x] * sizeof(uint32_t));
-        GZ_CHECK(hipStreamSynchronize(gz_stream));
-        gz_device_free(part_gid[x]);
-    }
+    gz_slices.mask = gz_device_malloc((nv + 8) * (wide_mask ? sizeof(uint64_t) : sizeof(uint32_t)));
+    gz_slices.rank_blocks = (nv + GZ_WAVE - 1) / GZ_WAVE;
+    gz_slices.rank_base = (uint32_t*)gz_device_malloc(ns * gz_slices.rank_blocks * sizeof(uint32_t));
+    /* consecutive blocks per wavefront: few enough that the chip is full */
+    uint64_t per = gz_slices.rank_blocks / ((uint64_t)gz_cu_count * 32);
+    per = per < 1 ? 1 : per > 64 ? 64 : per;
+    const uint64_t mask_waves = (gz_slices.rank_blocks + per - 1) / per;
+    const unsigned mask_grid = (unsigned)((mask_waves + GZ_WAVES_PER_BLOCK - 1) / GZ_WAVES_PER_BLOCK);
+    if (wide_mask)
+        hipLaunchKernelGGL(gz_k_slice_mask<uint64_t>, dim3(mask_grid), dim3(GZ_BLOCK), 0, gz_stream, gz_slices.gid, ns,
+                           first_run, nv, gz_slices.rank_blocks, per, (uint64_t*)gz_slices.mask, gz_slices.rank_base);
+    else
+        hipLaunchKernelGGL(gz_k_slice_mask<uint32_t>, dim3(mask_grid), dim3(GZ_BLOCK), 0, gz_stream, gz_slices.gid, ns,
+                           first_run, nv, gz_slices.rank_blocks, per, (uint32_t*)gz_slices.mask, gz_slices.rank_base);
+    GZ_LAUNCH_CHECK();
+    gz_slices.parts = (double*)gz_device_malloc((runs + 8) * sizeof(double));
     gz_slices.outdeg32 = (uint32_t*)gz_device_malloc((nv + 8) * sizeof(uint32_t));
     hipLaunchKernelGGL(gz_k_outdeg32, dim3(gz_grid_for(nv)), dim3(GZ_BLOCK), 0, gz_stream, gz_graph.vertex_outdegrees,
                        nv, gz_slices.outdeg32);
     GZ_LAUNCH_CHECK();
+    GZ_CHECK(hipStreamSynchronize(gz_stream));
+    gz_device_free(run_vec);
+    gz_device_free(run_first);
+    if (tile_base) gz_device_free(tile_base - (tiles + 1));
+    gz_device_free(firsts);
+    gz_device_free(a);
+    gz_device_free(bb);
     gz_slices.base_list = gz_graph.pull_vectors;
     gz_slices.base_count = nvec;
     gz_slices.slice_vertices = S;

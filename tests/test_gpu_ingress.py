@@ -168,3 +168,36 @@ def test_relabel_bfs_depths_and_tree(gz, orc, device, engine):
         p, d = gz.bfs_result()
         assert np.array_equal(d, dep)
         _bfs_tree_ok(g, root, p, d)
+
+
+TILE = 4096  # keys per workgroup of the dedupe passes, 1024 per wavefront
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1024, 1025, TILE - 1, TILE, TILE + 1, 3 * TILE + 17])
+@pytest.mark.parametrize("V", [1, 2, 64, 1000, 1 << 20])
+def test_dedupe_tiles(gz, device, n, V):
+    """Raw lists around the tile and wavefront sizes, with duplicates and
+    self-loops on both sides of every border: the highest vertex has
+    self-loops and in-edges (its group ends where the dropped keys begin),
+    and one destination spans tiles."""
+    rng = np.random.default_rng(n * 7 + V)
+    p = rng.integers(0, V, size=(n, 2), dtype=np.uint64)
+    p[rng.random(n) < 0.2, 1] = V - 1
+    loops = rng.random(n) < 0.1
+    p[loops, 0] = p[loops, 1]
+    p[n // 3:n // 2] = p[0]
+    p[n // 2:n // 2 + n // 4, 1] = V // 2
+    host = _host_state(gz, gz.make_graph(p, V))
+    gz.load_pairs_device(V, p)
+    _assert_same(_state(gz), host)
+    host = _host_state(gz, gz.make_graph(p, V, symmetrize=True))
+    gz.load_pairs_device(V, p, symmetrize=True)
+    _assert_same(_state(gz), host)
+    gz.load_pairs_device(V, p, relabel=True)
+    old = gz.original_ids()
+    order = np.lexsort((np.arange(V), -np.bincount(p[:, 0].astype(np.int64), minlength=V)))
+    assert np.array_equal(old, order.astype(np.uint64))
+    new = np.empty(V, np.uint64)
+    new[old.astype(np.int64)] = np.arange(V, dtype=np.uint64)
+    dev = _state(gz)
+    _assert_same(dev, _host_state(gz, gz.make_graph(new[p.astype(np.int64)], V)))
