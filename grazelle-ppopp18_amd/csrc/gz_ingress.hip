@@ -376,6 +376,198 @@ __global__ void gz_k_count_sources(const uint64_t* __restrict__ keys, uint64_t n
         atomicAdd(&cnt[keys[i] & mask], 1u);
 }
 
+/* Fewest keys, and most id bits, of the bucketed count below.  A renumbering
+ * load of R-MAT with edge factor 16, atomics / buckets: 2^18 keys 1022 / 1011
+ * us, 2^20 1426 / 1210, 2^21 2122 / 1716, 2^24 12.2 / 10.2 ms; each id bit
+ * above 24 doubles the times a bucket's ids are read back. */
+#define GZ_COUNT_BUCKET_KEYS (1ull << 19)
+#define GZ_COUNT_BUCKET_BITS 28
+
+/* ---- counting sources by buckets -------------------------------------------
+ * One atomic per key on a count per vertex runs at 7 G keys/s here (67 M keys
+ * of R-MAT s22: 9.24 ms): atomics from different XCDs on one line take turns.
+ * Instead the sources are partitioned by their high bits into at most 1024
+ * buckets, staged through LDS so that a bucket's ids leave in runs, and each
+ * bucket is then counted in LDS, 2^14 ids at a time.  Memory-bound: 8 bytes
+ * per key read twice, 4 written, 4 read back per 2^14 ids of a bucket: 0.58 ms
+ * for those 67 M keys (sizes 0.14, scatter 0.31, count 0.13), and 16.1 ms in
+ * place of 128.8 for 1.49 G keys over 41.7 M ids. */
+#define GZ_COUNT_BUCKETS 1024
+#define GZ_COUNT_IDS_LOG2 14
+#define GZ_COUNT_THREADS 1024
+#define GZ_COUNT_TILE 16384                      /* keys a workgroup partitions at a time */
+#define GZ_COUNT_SEGMENT 131072                  /* partitioned ids a workgroup counts */
+#define GZ_COUNT_PAD 64                          /* words between bucket cursors: a line of their own each */
+
+__global__ __launch_bounds__(GZ_COUNT_THREADS) void gz_k_bucket_sizes(const uint64_t* __restrict__ keys, uint64_t n,
+                                                                      uint64_t mask, uint32_t shift,
+                                                                      uint32_t buckets,
+                                                                      unsigned long long* __restrict__ sizes)
+{
+    __shared__ uint32_t hist[GZ_COUNT_BUCKETS];
+    hist[threadIdx.x] = 0;
+    __syncthreads();
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+        atomicAdd(&hist[(keys[i] & mask) >> shift], 1u);
+    __syncthreads();
+    if (threadIdx.x < buckets && hist[threadIdx.x])
+        atomicAdd(&sizes[(uint64_t)threadIdx.x * GZ_COUNT_PAD], (unsigned long long)hist[threadIdx.x]);
+}
+
+/* One workgroup: base[k] = ids of the buckets before k (base[buckets] = n),
+ * and the cursors, which held the sizes, start there. */
+__global__ __launch_bounds__(GZ_COUNT_THREADS) void gz_k_bucket_bases(unsigned long long* __restrict__ cursors,
+                                                                      uint32_t buckets, uint64_t* __restrict__ base)
+{
+    __shared__ uint64_t waves[GZ_COUNT_THREADS / GZ_WAVE];
+    const uint32_t k = threadIdx.x;
+    const uint64_t size = k < buckets ? (uint64_t)cursors[(uint64_t)k * GZ_COUNT_PAD] : 0;
+    uint64_t incl = size;
+#pragma unroll
+    for (int o = 1; o < GZ_WAVE; o <<= 1) {
+        const uint64_t t = (uint64_t)__shfl_up((unsigned long long)incl, o, GZ_WAVE);
+        if (gz_lane() >= o) incl += t;
+    }
+    if (gz_lane() == GZ_WAVE - 1) waves[k / GZ_WAVE] = incl;
+    __syncthreads();
+    for (uint32_t w = 0; w < k / GZ_WAVE; ++w) incl += waves[w];
+    if (k < buckets) {
+        base[k] = incl - size;
+        cursors[(uint64_t)k * GZ_COUNT_PAD] = incl - size;
+        if (k == buckets - 1) base[buckets] = incl;
+    }
+}
+
+__global__ __launch_bounds__(GZ_COUNT_THREADS) void gz_k_bucket_scatter(const uint64_t* __restrict__ keys, uint64_t n,
+                                                                        uint64_t mask, uint32_t shift,
+                                                                        uint64_t tiles,
+                                                                        unsigned long long* __restrict__ cursors,
+                                                                        uint32_t* __restrict__ ids)
+{
+    constexpr int kPer = GZ_COUNT_TILE / GZ_COUNT_THREADS;
+    __shared__ uint32_t stage[GZ_COUNT_TILE];  /* ids in bucket order */
+    __shared__ uint16_t owner[GZ_COUNT_TILE];  /* their buckets */
+    __shared__ uint32_t hist[GZ_COUNT_BUCKETS], start[GZ_COUNT_BUCKETS];
+    __shared__ uint64_t out[GZ_COUNT_BUCKETS]; /* where the bucket's first staged id goes */
+    __shared__ uint32_t waves[GZ_COUNT_THREADS / GZ_WAVE];
+    const uint32_t t = threadIdx.x, low = (1u << shift) - 1u;
+    for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const uint64_t first = tile * GZ_COUNT_TILE;
+        const uint32_t count = (uint32_t)(n - first < GZ_COUNT_TILE ? n - first : GZ_COUNT_TILE);
+        hist[t] = 0;
+        __syncthreads();
+        uint32_t id[kPer], rank[kPer];
+#pragma unroll
+        for (int r = 0; r < kPer; ++r) {
+            const uint32_t i = (uint32_t)r * GZ_COUNT_THREADS + t;
+            id[r] = i < count ? (uint32_t)(keys[first + i] & mask) : 0u;
+        }
+#pragma unroll
+        for (int r = 0; r < kPer; ++r)
+            rank[r] = (uint32_t)r * GZ_COUNT_THREADS + t < count ? atomicAdd(&hist[id[r] >> shift], 1u) : 0u;
+        __syncthreads();
+        const uint32_t size = hist[t];
+        uint32_t incl = size;
+#pragma unroll
+        for (int o = 1; o < GZ_WAVE; o <<= 1) {
+            const uint32_t x = __shfl_up(incl, o, GZ_WAVE);
+            if (gz_lane() >= o) incl += x;
+        }
+        if (gz_lane() == GZ_WAVE - 1) waves[t / GZ_WAVE] = incl;
+        __syncthreads();
+        for (uint32_t w = 0; w < t / GZ_WAVE; ++w) incl += waves[w];
+        start[t] = incl - size;
+        if (size) out[t] = atomicAdd(&cursors[(uint64_t)t * GZ_COUNT_PAD], (unsigned long long)size);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kPer; ++r) {
+            if ((uint32_t)r * GZ_COUNT_THREADS + t >= count) continue;
+            const uint32_t k = id[r] >> shift, at = start[k] + rank[r];
+            stage[at] = id[r] & low;
+            owner[at] = (uint16_t)k;
+        }
+        __syncthreads();
+        for (uint32_t i = t; i < count; i += GZ_COUNT_THREADS) {
+            const uint32_t k = owner[i];
+            ids[out[k] + (i - start[k])] = stage[i];
+        }
+        __syncthreads();
+    }
+}
+
+/* cnt[v] += the ids of v among a segment of the partitioned ids, bucket by
+ * bucket (a segment holds a part of a large bucket or several small ones). */
+__global__ __launch_bounds__(GZ_COUNT_THREADS) void gz_k_bucket_count(const uint32_t* __restrict__ ids, uint64_t n,
+                                                                      uint32_t shift, uint32_t buckets,
+                                                                      const uint64_t* __restrict__ base, uint64_t nv,
+                                                                      uint32_t* __restrict__ cnt)
+{
+    __shared__ uint32_t hist[1 << GZ_COUNT_IDS_LOG2];
+    const uint64_t lo = (uint64_t)blockIdx.x * GZ_COUNT_SEGMENT;
+    const uint64_t hi = lo + GZ_COUNT_SEGMENT < n ? lo + GZ_COUNT_SEGMENT : n;
+    uint32_t k = 0; /* the last bucket that starts at or before lo */
+    for (uint32_t z = buckets; z - k > 1;) {
+        const uint32_t mid = (k + z) / 2;
+        if (base[mid] <= lo)
+            k = mid;
+        else
+            z = mid;
+    }
+    for (; k < buckets && base[k] < hi; ++k) {
+        const uint64_t b = base[k] > lo ? base[k] : lo, e = base[k + 1] < hi ? base[k + 1] : hi;
+        if (b >= e) continue;
+        for (uint32_t part = 0; part < 1u << (shift - GZ_COUNT_IDS_LOG2); ++part) {
+            const uint64_t v0 = ((uint64_t)k << shift) + ((uint64_t)part << GZ_COUNT_IDS_LOG2);
+            if (v0 >= nv) break;
+            for (uint32_t i = threadIdx.x; i < 1u << GZ_COUNT_IDS_LOG2; i += GZ_COUNT_THREADS) hist[i] = 0;
+            __syncthreads();
+            for (uint64_t i = b + threadIdx.x; i < e; i += GZ_COUNT_THREADS) {
+                const uint32_t id = ids[i];
+                if (id >> GZ_COUNT_IDS_LOG2 == part) atomicAdd(&hist[id & ((1u << GZ_COUNT_IDS_LOG2) - 1u)], 1u);
+            }
+            __syncthreads();
+            for (uint32_t i = threadIdx.x; i < 1u << GZ_COUNT_IDS_LOG2; i += GZ_COUNT_THREADS)
+                if (hist[i]) atomicAdd(&cnt[v0 + i], hist[i]); /* an id counted is below nv */
+            __syncthreads();
+        }
+    }
+}
+
+/* cnt[s] = keys whose source is s, cnt cleared beforehand; `ids` holds n words
+ * of scratch. */
+void gz_count_sources(const uint64_t* keys, uint64_t n, uint32_t b, uint64_t nv, uint32_t* ids, uint32_t* cnt)
+{
+    if (n == 0) return;
+    if (n < GZ_COUNT_BUCKET_KEYS || b > GZ_COUNT_BUCKET_BITS) {
+        hipLaunchKernelGGL(gz_k_count_sources, dim3(gz_grid_for(n)), dim3(GZ_BLOCK), 0, gz_stream, keys, n, b, cnt);
+        GZ_LAUNCH_CHECK();
+        return;
+    }
+    const uint32_t shift = b > GZ_COUNT_IDS_LOG2 + 10 ? b - 10 : GZ_COUNT_IDS_LOG2;
+    const uint32_t buckets = (uint32_t)((nv - 1) >> shift) + 1;
+    const uint64_t mask = (1ull << b) - 1ull;
+    const uint64_t tiles = (n + GZ_COUNT_TILE - 1) / GZ_COUNT_TILE;
+    const uint64_t segments = (n + GZ_COUNT_SEGMENT - 1) / GZ_COUNT_SEGMENT;
+    const size_t cursor_words = (size_t)buckets * GZ_COUNT_PAD;
+    unsigned long long* cursors =
+        (unsigned long long*)gz_device_malloc((cursor_words + buckets + 1) * sizeof(uint64_t)); /* zero-filled */
+    uint64_t* base = (uint64_t*)cursors + cursor_words;
+    hipLaunchKernelGGL(gz_k_bucket_sizes, dim3((unsigned)(tiles < 1024 ? tiles : 1024)), dim3(GZ_COUNT_THREADS), 0,
+                       gz_stream, keys, n, mask, shift, buckets, cursors);
+    GZ_LAUNCH_CHECK();
+    hipLaunchKernelGGL(gz_k_bucket_bases, dim3(1), dim3(GZ_COUNT_THREADS), 0, gz_stream, cursors, buckets, base);
+    GZ_LAUNCH_CHECK();
+    hipLaunchKernelGGL(gz_k_bucket_scatter, dim3((unsigned)(tiles < 4096 ? tiles : 4096)), dim3(GZ_COUNT_THREADS), 0,
+                       gz_stream, keys, n, mask, shift, tiles, cursors, ids);
+    GZ_LAUNCH_CHECK();
+    hipLaunchKernelGGL(gz_k_bucket_count, dim3((unsigned)segments), dim3(GZ_COUNT_THREADS), 0, gz_stream, ids, n, shift,
+                       buckets, base, nv, cnt);
+    GZ_LAUNCH_CHECK();
+    GZ_CHECK(hipStreamSynchronize(gz_stream));
+    gz_device_free(cursors);
+}
+
 /* sort key: out-degree descending (as `most` less the degree), then id ascending */
 __global__ void gz_k_degree_order(const uint32_t* __restrict__ cnt, uint64_t nv, uint32_t b, uint64_t most,
                                   uint64_t* __restrict__ order)
@@ -418,19 +610,16 @@ __global__ void gz_k_remap_keys(uint64_t* __restrict__ keys, uint64_t n, uint32_
 }
 
 /* Renumber the vertices by raw out-degree, descending (ties by id), and
- * rewrite the keys in place.  Returns the device array of original ids,
+ * rewrite the keys in place (`scratch`: n words).  Returns the device array of original ids,
  * indexed by new id.  The hot sources of a power-law graph then share cache
  * lines, which is what the pull gathers need once the vertex array no longer
  * fits in the caches. */
-uint64_t* gz_relabel_by_outdegree(uint64_t* keys, uint64_t n, uint32_t b, uint64_t nv, uint64_t slice_vertices,
-                                  uint32_t tiers)
+uint64_t* gz_relabel_by_outdegree(uint64_t* keys, uint64_t* scratch, uint64_t n, uint32_t b, uint64_t nv,
+                                  uint64_t slice_vertices, uint32_t tiers)
 {
     uint32_t* cnt = (uint32_t*)gz_device_malloc(nv * sizeof(uint32_t));
     GZ_CHECK(hipMemsetAsync(cnt, 0, nv * sizeof(uint32_t), gz_stream));
-    if (n) {
-        hipLaunchKernelGGL(gz_k_count_sources, dim3(gz_grid_for(n)), dim3(GZ_BLOCK), 0, gz_stream, keys, n, b, cnt);
-        GZ_LAUNCH_CHECK();
-    }
+    gz_count_sources(keys, n, b, nv, (uint32_t*)scratch, cnt);
     const uint64_t most = n < 0xffffffffull ? n : 0xffffffffull; /* counts are 32-bit */
     uint64_t* order = (uint64_t*)gz_device_malloc(nv * sizeof(uint64_t));
     uint64_t* order_b = (uint64_t*)gz_device_malloc(nv * sizeof(uint64_t));
@@ -466,7 +655,7 @@ void gz_ingress_from_keys(uint64_t nv, uint64_t* a, uint64_t* b_buf, uint64_t n,
     const uint64_t slice_vertices = slice_log2 ? gz_slices_effective(1ull << slice_log2, tiers, nv) : 0;
     uint64_t* old_of_new = nullptr;
     if (flags & GZ_INGRESS_RELABEL_BY_OUTDEGREE)
-        old_of_new = gz_relabel_by_outdegree(a, n, b, nv, slice_vertices, tiers);
+        old_of_new = gz_relabel_by_outdegree(a, b_buf, n, b, nv, slice_vertices, tiers);
     uint64_t* sorted = a;
     if (n > 1) gz_sort_keys(a, b_buf, n, 0, 2 * b, &sorted);
     uint64_t* other = (sorted == a) ? b_buf : a;

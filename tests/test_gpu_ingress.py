@@ -201,3 +201,20 @@ def test_dedupe_tiles(gz, device, n, V):
     new[old.astype(np.int64)] = np.arange(V, dtype=np.uint64)
     dev = _state(gz)
     _assert_same(dev, _host_state(gz, gz.make_graph(new[p.astype(np.int64)], V)))
+
+
+@pytest.mark.parametrize("V", [3, 1 << 14, (1 << 14) + 1, 300007, (1 << 24) + 5, 41_700_000])
+@pytest.mark.parametrize("hot", [0, 1])
+def test_source_counts_by_buckets(gz, device, V, hot):
+    """The renumbering's counts on lists long enough for the bucketed count:
+    one bucket, two, many, and ids counted in several parts (V above 2^24); a
+    source in half of all edges fills a bucket over many segments."""
+    n = (1 << 19) + 4097
+    rng = np.random.default_rng(V)
+    p = rng.integers(0, V, size=(n, 2), dtype=np.uint64)
+    if hot:
+        p[rng.random(n) < 0.5, 0] = V - 1
+    gz.load_pairs_device(V, p, relabel=True)
+    cnt = np.bincount(p[:, 0].astype(np.int64), minlength=V)
+    order = np.argsort(-cnt, kind="stable")
+    assert np.array_equal(gz.original_ids(), order.astype(np.uint64))
