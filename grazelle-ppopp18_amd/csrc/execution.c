@@ -100,9 +100,9 @@ void gz_execution_prepare(const gz_run_options_t* o)
                     (unsigned long long)o->root, (unsigned long long)V);
             exit(66);
         }
-        const uint64_t r = gz_graph_device_vertex(o->root);
         gz_dev_bfs_reset((uint64_t*)gz_graph.vertex_props, V, (uint64_t*)gz_graph.vertex_accumulators,
-                         gz_graph.frontier_has_info, gz_graph.frontier_wants_info, fwords, r);
+                         gz_graph.frontier_has_info, gz_graph.frontier_wants_info, fwords, o->root,
+                         gz_graph_device_ids_device(), gz_graph.vertex_outdegrees);
         break;
     }
     default:
@@ -554,10 +554,22 @@ static void gz_run_hybrid(const gz_run_options_t* o, gz_run_result_t* r)
 {
     const int bfs = (o->algorithm == GZ_ALG_BFS);
     const uint64_t V = gz_graph.num_vertices, E = gz_graph.num_edges;
-    uint64_t vote = 0;
+    uint64_t vote = 0, device_root = V, root_outdeg = 0;
     if (bfs) {
-        const double* od = gz_graph_outdegrees_host();
-        if (o->stat_mode != GZ_STAT_COUNT_ONLY) vote += (uint64_t)od[gz_graph_device_vertex(o->root)];
+        /* noted by the start's launch (the stream has drained); a root other
+         * than the prepared one is looked up */
+        if (!gz_dev_bfs_start_info(o->root, &device_root, &root_outdeg)) {
+            uint64_t info[2];
+            if (o->root >= V) {
+                fprintf(stderr, "grazelle: BFS root %llu is not a vertex of a %llu-vertex graph\n",
+                        (unsigned long long)o->root, (unsigned long long)V);
+                exit(66);
+            }
+            gz_graph_vertex_info(&o->root, 1, info);
+            device_root = info[0];
+            root_outdeg = info[1];
+        }
+        if (o->stat_mode != GZ_STAT_COUNT_ONLY) vote += root_outdeg;
         if (o->stat_mode != GZ_STAT_OUTDEG_ONLY) vote += 1;
     } else {
         if (o->stat_mode != GZ_STAT_COUNT_ONLY) vote += E;
@@ -584,7 +596,7 @@ static void gz_run_hybrid(const gz_run_options_t* o, gz_run_result_t* r)
     uint64_t sel_unvisited = V, sel_unvisited_in = E;
     if (features) {
         /* features of the first iteration: the initial frontier */
-        const uint64_t root = bfs ? gz_graph_device_vertex(o->root) : V;
+        const uint64_t root = device_root;
         const int host_first = learned && bfs && root < V;
         /* with the first decision on the host, the device counts start past
          * the root and no first step runs */
@@ -595,9 +607,8 @@ static void gz_run_hybrid(const gz_run_options_t* o, gz_run_result_t* r)
         if (host_first) {
             /* the first frontier is the root alone, so the host knows the
              * features and takes the first decision itself */
-            const double* od = gz_graph_outdegrees_host();
             sel.features[0] = logf(1.f + 1.f);
-            sel.features[1] = logf(1.f + (float)(uint64_t)od[root]);
+            sel.features[1] = logf(1.f + (float)root_outdeg);
             sel.features[2] = logf(1.f + (float)(V - 1));
             sel.features[3] = gz_selector_feature_used(3) ? logf(1.f + (float)(E - gz_graph_indegree_host(root))) : 0.f;
             sel.features[4] = 1.f;

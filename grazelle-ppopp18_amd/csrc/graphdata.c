@@ -239,7 +239,7 @@ void gz_count_outdegrees(const uint64_t* pairs, uint64_t num_edges, uint64_t num
 typedef struct gz_host_graph_t {
     uint64_t num_vertices, num_edges;
     uint64_t pull_vectors, push_vectors;
-    double* outdeg;              /* host mirror */
+    double* outdeg;              /* host mirror, made when first asked for */
     /* device allocations */
     gz_vec_t* d_pull;
     gz_vec_t* d_push;
@@ -252,8 +252,8 @@ typedef struct gz_host_graph_t {
     uint64_t* d_wants;
     /* renumbered graphs only (else NULL) */
     uint64_t* d_original_ids;    /* original id by device vertex */
-    uint64_t* original_ids;      /* host mirror of the above */
-    uint64_t* device_ids;        /* device vertex by original id */
+    uint32_t* d_device_ids;      /* device vertex by original id */
+    uint32_t* device_ids;        /* host mirror of the above, made when first asked for */
     uint32_t* d_indeg;           /* in-degrees, built on first use */
     uint32_t* h_indeg;           /* host copy of d_indeg, made on first use */
 } gz_host_graph_t;
@@ -276,7 +276,19 @@ void gz_graph_reset_roles(void)
 uint64_t gz_graph_num_edges(void) { return G.num_edges; }
 uint64_t gz_graph_pull_vector_count(void) { return G.pull_vectors; }
 uint64_t gz_graph_push_vector_count(void) { return G.push_vectors; }
-const double* gz_graph_outdegrees_host(void) { return G.outdeg; }
+
+/* The host mirrors serve callers that ask for them (this function and
+ * gz_graph_device_vertex); loading, running and the result getters read the
+ * device arrays. */
+const double* gz_graph_outdegrees_host(void)
+{
+    if (G.outdeg == NULL && G.d_outdeg != NULL) {
+        const size_t bytes = (G.num_vertices + 8) * sizeof(double);
+        G.outdeg = (double*)malloc(bytes);
+        gz_copy_to_host(G.outdeg, G.d_outdeg, bytes);
+    }
+    return G.outdeg;
+}
 
 void gz_graph_release(void)
 {
@@ -285,6 +297,7 @@ void gz_graph_release(void)
     gz_pr_release();
     gz_bfs_batch_release();
     gz_bfs_pending_release();
+    gz_dev_bfs_start_forget();
     gz_device_free(G.d_pull);
     gz_device_free(G.d_push);
     gz_device_free(G.d_pull_offsets);
@@ -295,9 +308,9 @@ void gz_graph_release(void)
     gz_device_free(G.d_has);
     gz_device_free(G.d_wants);
     gz_device_free(G.d_original_ids);
+    gz_device_free(G.d_device_ids);
     gz_device_free(G.d_indeg);
     free(G.h_indeg);
-    free(G.original_ids);
     free(G.device_ids);
     free(G.outdeg);
     memset(&G, 0, sizeof(G));
@@ -358,16 +371,8 @@ void gz_graph_adopt_device(const gz_device_layouts_t* L)
     G.d_push_offsets = L->push_offsets;
     G.push_vectors = L->push_count;
     G.d_outdeg = L->outdeg;
-    G.outdeg = (double*)malloc((L->num_vertices + 8) * sizeof(double));
-    gz_copy_to_host(G.outdeg, G.d_outdeg, (L->num_vertices + 8) * sizeof(double));
-    if (L->original_ids != NULL) {
-        const uint64_t n = L->num_vertices;
-        G.d_original_ids = L->original_ids;
-        G.original_ids = (uint64_t*)malloc(n * sizeof(uint64_t));
-        G.device_ids = (uint64_t*)malloc(n * sizeof(uint64_t));
-        gz_copy_to_host(G.original_ids, G.d_original_ids, n * sizeof(uint64_t));
-        for (uint64_t i = 0; i < n; ++i) G.device_ids[G.original_ids[i]] = i;
-    }
+    G.d_original_ids = L->original_ids;
+    G.d_device_ids = L->device_ids;
     gz_graph_finish();
 }
 
@@ -403,24 +408,28 @@ void gz_graph_indegrees(uint32_t* out)
 
 uint64_t gz_graph_device_vertex(uint64_t original)
 {
-    if (G.device_ids == NULL || original >= G.num_vertices) return original;
+    if (G.d_device_ids == NULL || original >= G.num_vertices) return original;
+    if (G.device_ids == NULL) {
+        G.device_ids = (uint32_t*)malloc(G.num_vertices * sizeof(uint32_t));
+        gz_copy_to_host(G.device_ids, G.d_device_ids, G.num_vertices * sizeof(uint32_t));
+    }
     return G.device_ids[original];
+}
+
+const uint32_t* gz_graph_device_ids_device(void) { return G.d_device_ids; }
+
+void gz_graph_vertex_info(const uint64_t* vertices, uint32_t count, uint64_t* info)
+{
+    gz_dev_vertex_info(vertices, count, G.d_device_ids, G.d_outdeg, info);
 }
 
 void gz_graph_original_ids(uint64_t* out)
 {
-    for (uint64_t v = 0; v < G.num_vertices; ++v) out[v] = G.original_ids != NULL ? G.original_ids[v] : v;
-}
-
-/* out[original id] = in[device vertex] for V words (identity copy when the
- * graph is not renumbered). */
-static void gz_to_original_order(uint64_t* out, const uint64_t* in)
-{
-    if (G.device_ids == NULL) {
-        if (out != in) memcpy(out, in, G.num_vertices * sizeof(uint64_t));
+    if (G.d_original_ids != NULL) {
+        gz_copy_to_host(out, G.d_original_ids, G.num_vertices * sizeof(uint64_t));
         return;
     }
-    for (uint64_t v = 0; v < G.num_vertices; ++v) out[v] = in[G.device_ids[v]];
+    for (uint64_t v = 0; v < G.num_vertices; ++v) out[v] = v;
 }
 
 /* Allocate the vertex arrays and frontiers and publish the graph record. */
@@ -500,58 +509,24 @@ void gz_graph_download_offsets(int pull, uint64_t* out)
 
 /* ---- results -------------------------------------------------------------- */
 
-/* Device vertex words in original-id order (a fresh malloc'd array). */
-static uint64_t* gz_download_vertex_words(void)
-{
-    const uint64_t n = G.num_vertices;
-    uint64_t* w = (uint64_t*)malloc((n ? n : 1) * sizeof(uint64_t));
-    gz_copy_to_host(w, gz_graph.vertex_props, n * sizeof(uint64_t));
-    if (G.device_ids != NULL) {
-        uint64_t* o = (uint64_t*)malloc((n ? n : 1) * sizeof(uint64_t));
-        gz_to_original_order(o, w);
-        free(w);
-        w = o;
-    }
-    return w;
-}
-
 void gz_result_pr_props(double* out)
 {
-    uint64_t* w = gz_download_vertex_words();
-    memcpy(out, w, G.num_vertices * sizeof(double));
-    free(w);
+    gz_dev_result_words(gz_graph.vertex_props, NULL, G.d_original_ids, G.num_vertices, (uint64_t*)out);
 }
 
 void gz_result_pr_ranks(double* out)
 {
-    gz_result_pr_props(out);
-    const double nv = (double)G.num_vertices;
-    for (uint64_t i = 0; i < G.num_vertices; ++i) {
-        const double od = G.outdeg[gz_graph_device_vertex(i)];
-        out[i] = out[i] * (0.0 == od ? nv : od);
-    }
+    gz_dev_result_words(gz_graph.vertex_props, G.d_outdeg, G.d_original_ids, G.num_vertices, (uint64_t*)out);
 }
 
 void gz_result_cc_labels(uint64_t* out)
 {
-    uint64_t* w = gz_download_vertex_words();
-    memcpy(out, w, G.num_vertices * sizeof(uint64_t));
-    free(w);
+    gz_dev_result_words(gz_graph.vertex_props, NULL, G.d_original_ids, G.num_vertices, out);
 }
 
 void gz_result_bfs(int64_t* parents, uint64_t* depths)
 {
-    uint64_t* w = gz_download_vertex_words();
-    for (uint64_t i = 0; i < G.num_vertices; ++i) {
-        int64_t p = -1;
-        if (w[i] != GZ_BFS_UNVISITED && gz_bfs_parent(w[i]) >= 0) {
-            p = gz_bfs_parent(w[i]);
-            if (G.original_ids != NULL) p = (int64_t)G.original_ids[p];
-        }
-        if (parents) parents[i] = p;
-        if (depths) depths[i] = (w[i] == GZ_BFS_UNVISITED) ? UINT64_MAX : gz_bfs_depth(w[i]);
-    }
-    free(w);
+    gz_dev_result_bfs(gz_graph.vertex_props, G.d_original_ids, G.num_vertices, parents, depths);
 }
 
 int graph_data_write_ranks_to_file(const char* filename, uint32_t algorithm)

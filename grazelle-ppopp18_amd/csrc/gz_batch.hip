@@ -434,13 +434,33 @@ extern "C" double gz_batch_time_pull(const gz_batch_config_t* cfg, uint32_t buck
     return best;
 }
 
+/* rank = props * outdeg', outdeg' = the vertex count of the vertex's graph
+ * for sinks. */
+__global__ __launch_bounds__(GZ_BLOCK) void gz_k_batch_ranks(const double* __restrict__ props,
+                                                             const double* __restrict__ outdeg,
+                                                             const uint16_t* __restrict__ gid,
+                                                             const uint64_t* __restrict__ base, uint64_t n,
+                                                             double* __restrict__ out)
+{
+    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (uint64_t)gridDim.x * blockDim.x) {
+        const double od = outdeg[v];
+        const uint32_t g = gid[v];
+        out[v] = props[v] * (0.0 == od ? (double)(base[g + 1] - base[g]) : od);
+    }
+}
+
 extern "C" void gz_batch_pr_ranks(double* out)
 {
     const uint64_t V = gz_graph.num_vertices;
-    gz_copy_to_host(out, gz_graph.vertex_props, V * sizeof(double));
-    const double* od = gz_graph_outdegrees_host();
-    for (uint32_t g = 0; g < B.count; ++g) {
-        const double n = (double)(B.base[g + 1] - B.base[g]);
-        for (uint64_t v = B.base[g]; v < B.base[g + 1]; ++v) out[v] = out[v] * (0.0 == od[v] ? n : od[v]);
+    if (B.count == 0) {
+        gz_copy_to_host(out, gz_graph.vertex_props, V * sizeof(double));
+        return;
     }
+    double* d = (double*)gz_device_malloc((V ? V : 1) * sizeof(double));
+    hipLaunchKernelGGL(gz_k_batch_ranks, dim3(gz_grid(V, GZ_BLOCK)), dim3(GZ_BLOCK), 0, gz_stream,
+                       (const double*)gz_graph.vertex_props, gz_graph.vertex_outdegrees, (const uint16_t*)B.d_gid,
+                       (const uint64_t*)B.d_base, V, d);
+    GZ_LAUNCH_CHECK();
+    gz_copy_to_host(out, d, V * sizeof(double));
+    gz_device_free(d);
 }

@@ -207,21 +207,23 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_msbfs_level_end(uint64_t num_ve
     if (lane == 0) partials[gw] = total;
 }
 
-/* Depths of search r as words (UINT64_MAX unreached) and parents (device
- * ids, ~0 for the root and unreached vertices): the smallest in-neighbour one
- * level up, in the pull list's source order. */
+/* Depths of search r as words (UINT64_MAX unreached) and parents (original
+ * ids, -1 for the root and unreached vertices: the in-neighbour one level up
+ * that is first in the pull list's source order), in original-id order. */
 __global__ __launch_bounds__(GZ_BLOCK) void gz_k_msbfs_result(const gz_vec_t* __restrict__ pull,
                                                               const uint64_t* __restrict__ offsets,
                                                               uint64_t num_vertices, uint32_t r,
                                                               const uint8_t* __restrict__ depth,
+                                                              const uint64_t* __restrict__ original,
                                                               uint64_t* __restrict__ out_depth,
-                                                              uint64_t* __restrict__ out_parent, int want_parents)
+                                                              int64_t* __restrict__ out_parent)
 {
     for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < num_vertices;
          v += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t d = depth[v * 64 + r];
-        out_depth[v] = (d == GZ_MSBFS_UNREACHED) ? ~0ull : (uint64_t)d;
-        if (!want_parents) continue;
+        const uint64_t at = original != nullptr ? original[v] : v;
+        if (out_depth != nullptr) out_depth[at] = (d == GZ_MSBFS_UNREACHED) ? ~0ull : (uint64_t)d;
+        if (out_parent == nullptr) continue;
         uint64_t parent = ~0ull;
         if (d != GZ_MSBFS_UNREACHED && d != 0) {
             for (uint64_t i = offsets[v]; i < offsets[v + 1] && parent == ~0ull; ++i) {
@@ -235,7 +237,7 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_msbfs_result(const gz_vec_t* __
                 }
             }
         }
-        out_parent[v] = parent;
+        out_parent[at] = parent == ~0ull ? -1 : (int64_t)(original != nullptr ? original[parent] : parent);
     }
 }
 
@@ -288,8 +290,10 @@ extern "C" int gz_bfs_batch_run(const uint64_t* roots, uint32_t count, gz_run_re
                     (unsigned long long)roots[r], (unsigned long long)V);
             return -1;
         }
-        dev_roots[r] = gz_graph_device_vertex(roots[r]);
     }
+    uint64_t info[2 * GZ_BFS_BATCH_MAX_ROOTS];
+    gz_graph_vertex_info(roots, count, info);
+    for (uint32_t r = 0; r < count; ++r) dev_roots[r] = info[2 * r];
     gz_msbfs_reserve(V);
     gz_scratch_reserve(GZ_PERSISTENT_BLOCKS * GZ_WAVES_PER_BLOCK, V);
     const uint64_t words = (V + 63) / 64;
@@ -302,12 +306,11 @@ extern "C" int gz_bfs_batch_run(const uint64_t* roots, uint32_t count, gz_run_re
     M.count = count;
     const uint64_t full = count >= 64 ? ~0ull : ((1ull << count) - 1ull);
     /* the roots' frontier statistic: 1 + outdeg for each distinct root */
-    const double* od = gz_graph_outdegrees_host();
     uint64_t vote = 0;
     for (uint32_t r = 0; r < count; ++r) {
         int dup = 0;
         for (uint32_t q = 0; q < r; ++q) dup |= dev_roots[q] == dev_roots[r];
-        if (!dup) vote += 1 + (uint64_t)od[dev_roots[r]];
+        if (!dup) vote += 1 + info[2 * r + 1];
     }
     uint64_t* reduce = gz_scratch.reduce_tmp + 2032; /* one word the vote reduction writes */
     gz_synchronize();
@@ -385,27 +388,16 @@ extern "C" void gz_bfs_batch_result(uint32_t search, int64_t* parents, uint64_t*
         fprintf(stderr, "grazelle: no BFS batch result for search %u\n", search);
         exit(66);
     }
-    uint64_t* d_depth = (uint64_t*)gz_device_malloc((V + 8) * sizeof(uint64_t));
-    uint64_t* d_parent = parents ? (uint64_t*)gz_device_malloc((V + 8) * sizeof(uint64_t)) : nullptr;
+    uint64_t* d_depth = depths ? (uint64_t*)gz_device_malloc((V + 8) * sizeof(uint64_t)) : nullptr;
+    int64_t* d_parent = parents ? (int64_t*)gz_device_malloc((V + 8) * sizeof(int64_t)) : nullptr;
     uint64_t blocks = (V + GZ_BLOCK - 1) / GZ_BLOCK;
     if (blocks > 16384) blocks = 16384;
     hipLaunchKernelGGL(gz_k_msbfs_result, dim3((unsigned)blocks), dim3(GZ_BLOCK), 0, gz_stream, gz_graph.pull_vectors,
-                       gz_graph.pull_vertex_offsets, V, search, M.depth, d_depth, d_parent, parents != nullptr);
+                       gz_graph.pull_vertex_offsets, V, search, M.depth, gz_graph_original_ids_device(), d_depth,
+                       d_parent);
     GZ_LAUNCH_CHECK();
-    uint64_t* h = (uint64_t*)malloc((V ? V : 1) * sizeof(uint64_t));
-    uint64_t* hp = parents ? (uint64_t*)malloc((V ? V : 1) * sizeof(uint64_t)) : nullptr;
-    gz_copy_to_host(h, d_depth, V * sizeof(uint64_t));
-    if (parents) gz_copy_to_host(hp, d_parent, V * sizeof(uint64_t));
+    if (depths) gz_copy_to_host(depths, d_depth, V * sizeof(uint64_t));
+    if (parents) gz_copy_to_host(parents, d_parent, V * sizeof(int64_t));
     gz_device_free(d_depth);
     gz_device_free(d_parent);
-    /* original-id order: result[original id] = value at its device vertex */
-    uint64_t* orig = (uint64_t*)malloc((V ? V : 1) * sizeof(uint64_t));
-    gz_graph_original_ids(orig);
-    for (uint64_t v = 0; v < V; ++v) {
-        if (depths) depths[orig[v]] = h[v];
-        if (parents) parents[orig[v]] = (hp[v] == ~0ull) ? -1 : (int64_t)orig[hp[v]];
-    }
-    free(orig);
-    free(h);
-    free(hp);
 }

@@ -25,22 +25,40 @@ typedef struct gz_device_layouts_t {
     uint64_t push_count;
     double* outdeg;              /* [V+8] */
     uint64_t* original_ids;      /* [V+8] original id of each device vertex, or NULL (not renumbered) */
+    uint32_t* device_ids;        /* [V] its inverse, or NULL */
 } gz_device_layouts_t;
 
 /* Take ownership of device layouts and allocate the vertex arrays. */
 void gz_graph_adopt_device(const gz_device_layouts_t* layouts);
 /* Device array of original ids by device vertex, NULL when not renumbered. */
 const uint64_t* gz_graph_original_ids_device(void);
+/* Its inverse: device vertex by original id, NULL when not renumbered. */
+const uint32_t* gz_graph_device_ids_device(void);
+/* Device vertex and out-degree of up to 64 original vertices of the loaded
+ * graph, as pairs in info (one launch and one copy). */
+void gz_graph_vertex_info(const uint64_t* vertices, uint32_t count, uint64_t* info);
+
+/* Results into host arrays, in original-id order (gz_results.hip). */
+void gz_dev_result_words(const uint64_t* words, const double* outdeg, const uint64_t* original, uint64_t n,
+                         uint64_t* out);
+void gz_dev_result_bfs(const uint64_t* words, const uint64_t* original, uint64_t n, int64_t* parents,
+                       uint64_t* depths);
+void gz_dev_vertex_info(const uint64_t* vertices, uint32_t count, const uint32_t* device_ids, const double* outdeg,
+                        uint64_t* info);
 
 void gz_dev_init_pr(double* props, double* acc, const double* outdeg, uint64_t n);
 void gz_dev_fill_u64(uint64_t* p, uint64_t value, uint64_t n);
 void gz_dev_iota_u64(uint64_t* p, uint64_t n);
 void gz_dev_store_u64(uint64_t* p, uint64_t index, uint64_t value);
-/* A BFS start from device vertex `root` in one launch: words[0..n) unvisited
- * but the root's (no parent), acc[0..fwords) = 0, has = {root}, wants = all
- * but root. */
+/* A BFS start from original vertex `root` in one launch: words[0..n)
+ * unvisited but the root's (no parent), acc[0..fwords) = 0, has = {root},
+ * wants = all but root.  The launch also notes the root's device vertex and
+ * out-degree in pinned memory: gz_dev_bfs_start_info, once the stream has
+ * drained, gives them for the root of the last start (0 for another root). */
 void gz_dev_bfs_reset(uint64_t* words, uint64_t n, uint64_t* acc, uint64_t* has, uint64_t* wants, uint64_t fwords,
-                      uint64_t root);
+                      uint64_t root, const uint32_t* device_ids, const double* outdeg);
+int gz_dev_bfs_start_info(uint64_t root, uint64_t* device_root, uint64_t* outdeg);
+void gz_dev_bfs_start_forget(void); /* the graph is released */
 void gz_graph_reset_roles(void);
 void gz_dev_indegrees(const gz_vec_t* vecs, uint64_t count, int pull_layout, uint32_t* indeg, uint64_t n);
 /* In-degrees of the loaded graph (u32[V+8]), built on first use. */

@@ -610,12 +610,12 @@ __global__ void gz_k_remap_keys(uint64_t* __restrict__ keys, uint64_t n, uint32_
 }
 
 /* Renumber the vertices by raw out-degree, descending (ties by id), and
- * rewrite the keys in place (`scratch`: n words).  Returns the device array of original ids,
- * indexed by new id.  The hot sources of a power-law graph then share cache
- * lines, which is what the pull gathers need once the vertex array no longer
- * fits in the caches. */
+ * rewrite the keys in place (`scratch`: n words).  Returns the device array of
+ * original ids, indexed by new id, and its inverse in *device_ids.  The hot
+ * sources of a power-law graph then share cache lines, which is what the pull
+ * gathers need once the vertex array no longer fits in the caches. */
 uint64_t* gz_relabel_by_outdegree(uint64_t* keys, uint64_t* scratch, uint64_t n, uint32_t b, uint64_t nv,
-                                  uint64_t slice_vertices, uint32_t tiers)
+                                  uint64_t slice_vertices, uint32_t tiers, uint32_t** device_ids)
 {
     uint32_t* cnt = (uint32_t*)gz_device_malloc(nv * sizeof(uint32_t));
     GZ_CHECK(hipMemsetAsync(cnt, 0, nv * sizeof(uint32_t), gz_stream));
@@ -640,7 +640,7 @@ uint64_t* gz_relabel_by_outdegree(uint64_t* keys, uint64_t* scratch, uint64_t n,
     GZ_CHECK(hipStreamSynchronize(gz_stream));
     gz_device_free(order);
     gz_device_free(order_b);
-    gz_device_free(cnt);
+    *device_ids = new_of_old;
     return old_of_new;
 }
 
@@ -654,8 +654,9 @@ void gz_ingress_from_keys(uint64_t nv, uint64_t* a, uint64_t* b_buf, uint64_t n,
     const uint32_t blocks = (flags >> 16) & 0x7u;
     const uint64_t slice_vertices = slice_log2 ? gz_slices_effective(1ull << slice_log2, tiers, nv) : 0;
     uint64_t* old_of_new = nullptr;
+    uint32_t* new_of_old = nullptr;
     if (flags & GZ_INGRESS_RELABEL_BY_OUTDEGREE)
-        old_of_new = gz_relabel_by_outdegree(a, b_buf, n, b, nv, slice_vertices, tiers);
+        old_of_new = gz_relabel_by_outdegree(a, b_buf, n, b, nv, slice_vertices, tiers, &new_of_old);
     uint64_t* sorted = a;
     if (n > 1) gz_sort_keys(a, b_buf, n, 0, 2 * b, &sorted);
     uint64_t* other = (sorted == a) ? b_buf : a;
@@ -682,6 +683,7 @@ void gz_ingress_from_keys(uint64_t nv, uint64_t* a, uint64_t* b_buf, uint64_t n,
     L.num_vertices = nv;
     L.num_edges = m;
     L.original_ids = old_of_new;
+    L.device_ids = new_of_old;
     gz_build_layout(other, m, b, 0, nv, first, end, &L.pull, &L.pull_offsets, &L.pull_count);
     /* push layout: the kept keys by source (still unique) */
     uint64_t* push_sorted = other;

@@ -40,12 +40,21 @@ __global__ void gz_k_store(uint64_t* __restrict__ p, uint64_t index, uint64_t va
 
 /* The start of a BFS from `root` in one launch (execution_bfs.c:106-116 and
  * :70-102): every word unvisited but the root's (no parent), HasInfo* clear,
- * HasInfo = {root}, WantsInfo = every vertex but the root. */
+ * HasInfo = {root}, WantsInfo = every vertex but the root.  `original` is the
+ * root's original id; its device vertex and out-degree go to info. */
 __global__ __launch_bounds__(GZ_BLOCK) void gz_k_bfs_reset(uint64_t* __restrict__ words, uint64_t n,
                                                            uint64_t* __restrict__ acc, uint64_t* __restrict__ has,
                                                            uint64_t* __restrict__ wants, uint64_t fwords,
-                                                           uint64_t root)
+                                                           uint64_t original,
+                                                           const uint32_t* __restrict__ device_ids,
+                                                           const double* __restrict__ outdeg,
+                                                           uint64_t* __restrict__ info)
 {
+    const uint64_t root = device_ids != nullptr ? (uint64_t)device_ids[original] : original;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        info[0] = root;
+        info[1] = (uint64_t)outdeg[root];
+    }
     const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t i = first; i < n; i += stride) words[i] = (i == root) ? GZ_BFS_PARENT_NONE : GZ_BFS_UNVISITED;
     const uint64_t rw = root >> 6, rbit = 1ull << (root & 63);
@@ -64,12 +73,32 @@ static unsigned gz_blocks_for(uint64_t n)
     return (unsigned)b;
 }
 
+/* Pinned, mapped: the device vertex and out-degree of the last start's root. */
+static uint64_t* gz_bfs_info = nullptr;
+static uint64_t* gz_bfs_info_dev = nullptr;
+static uint64_t gz_bfs_info_root = ~0ull;
+
 void gz_dev_bfs_reset(uint64_t* words, uint64_t n, uint64_t* acc, uint64_t* has, uint64_t* wants, uint64_t fwords,
-                      uint64_t root)
+                      uint64_t root, const uint32_t* device_ids, const double* outdeg)
 {
+    if (gz_bfs_info == nullptr) {
+        GZ_CHECK(hipHostMalloc((void**)&gz_bfs_info, 2 * sizeof(uint64_t), hipHostMallocMapped | hipHostMallocCoherent));
+        GZ_CHECK(hipHostGetDevicePointer((void**)&gz_bfs_info_dev, gz_bfs_info, 0));
+    }
+    gz_bfs_info_root = root;
     hipLaunchKernelGGL(gz_k_bfs_reset, dim3(gz_blocks_for(n > fwords ? n : fwords)), dim3(GZ_BLOCK), 0, gz_stream, words,
-                       n, acc, has, wants, fwords, root);
+                       n, acc, has, wants, fwords, root, device_ids, outdeg, gz_bfs_info_dev);
     GZ_LAUNCH_CHECK();
+}
+
+void gz_dev_bfs_start_forget(void) { gz_bfs_info_root = ~0ull; }
+
+int gz_dev_bfs_start_info(uint64_t root, uint64_t* device_root, uint64_t* outdeg)
+{
+    if (gz_bfs_info == nullptr || root != gz_bfs_info_root) return 0;
+    *device_root = gz_bfs_info[0];
+    *outdeg = gz_bfs_info[1];
+    return 1;
 }
 
 extern "C" void gz_dev_init_pr(double* props, double* acc, const double* outdeg, uint64_t n)
