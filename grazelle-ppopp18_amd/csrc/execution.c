@@ -185,18 +185,18 @@ static void gz_snapshot_alloc(gz_snapshot_t* s)
     const uint64_t V = gz_graph.num_vertices;
     s->vbytes = V * sizeof(uint64_t);
     s->fbytes = ((V + 63) / 64) * sizeof(uint64_t);
-    s->props = gz_device_malloc(s->vbytes ? s->vbytes : 8);
-    s->has = gz_device_malloc(s->fbytes ? s->fbytes : 8);
-    s->wants = gz_device_malloc(s->fbytes ? s->fbytes : 8);
-    s->next = gz_device_malloc(s->fbytes ? s->fbytes : 8);
+    s->props = gz_pool_malloc(s->vbytes ? s->vbytes : 8, 1);
+    s->has = gz_pool_malloc(s->fbytes ? s->fbytes : 8, 1);
+    s->wants = gz_pool_malloc(s->fbytes ? s->fbytes : 8, 1);
+    s->next = gz_pool_malloc(s->fbytes ? s->fbytes : 8, 1);
 }
 
 static void gz_snapshot_free(gz_snapshot_t* s)
 {
-    gz_device_free(s->props);
-    gz_device_free(s->has);
-    gz_device_free(s->wants);
-    gz_device_free(s->next);
+    gz_pool_free(s->props);
+    gz_pool_free(s->has);
+    gz_pool_free(s->wants);
+    gz_pool_free(s->next);
 }
 
 static void gz_snapshot_take(gz_snapshot_t* s)
@@ -491,7 +491,7 @@ static int gz_cc_device_loop(const gz_run_options_t* o, uint64_t vote, uint64_t 
     const uint64_t waves = gz_cc_loop_waves(&pull_waves, &push_waves);
     /* every buffer the launches use exists before any capture */
     gz_scratch_reserve_public(waves, V);
-    if (gz_cc_ctrl == NULL) gz_cc_ctrl = (uint64_t*)gz_device_malloc(GZ_LOOP_WORDS(GZ_CC_LOOP_LOG) * sizeof(uint64_t));
+    if (gz_cc_ctrl == NULL) gz_cc_ctrl = (uint64_t*)gz_pool_malloc(GZ_LOOP_WORDS(GZ_CC_LOOP_LOG) * sizeof(uint64_t), 1);
     uint64_t ctrl[16];
     memset(ctrl, 0, sizeof(ctrl));
     const int first_pull = o->engine == GZ_ENGINE_PULL ? 1 : o->engine == GZ_ENGINE_PUSH ? 0 : vote > threshold;

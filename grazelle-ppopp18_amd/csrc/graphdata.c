@@ -292,24 +292,27 @@ const double* gz_graph_outdegrees_host(void)
 
 void gz_graph_release(void)
 {
+    /* a caller's own streams may still read the arrays, which the next load
+     * may be handed at once */
+    if (G.num_vertices) gz_device_wait();
     gz_source_slices_release();
     gz_frontier_counts_release();
     gz_pr_release();
     gz_bfs_batch_release();
     gz_bfs_pending_release();
     gz_dev_bfs_start_forget();
-    gz_device_free(G.d_pull);
-    gz_device_free(G.d_push);
-    gz_device_free(G.d_pull_offsets);
-    gz_device_free(G.d_push_offsets);
-    gz_device_free(G.d_outdeg);
-    gz_device_free(G.d_props);
-    gz_device_free(G.d_acc);
-    gz_device_free(G.d_has);
-    gz_device_free(G.d_wants);
-    gz_device_free(G.d_original_ids);
-    gz_device_free(G.d_device_ids);
-    gz_device_free(G.d_indeg);
+    gz_pool_free(G.d_pull);
+    gz_pool_free(G.d_push);
+    gz_pool_free(G.d_pull_offsets);
+    gz_pool_free(G.d_push_offsets);
+    gz_pool_free(G.d_outdeg);
+    gz_pool_free(G.d_props);
+    gz_pool_free(G.d_acc);
+    gz_pool_free(G.d_has);
+    gz_pool_free(G.d_wants);
+    gz_pool_free(G.d_original_ids);
+    gz_pool_free(G.d_device_ids);
+    gz_pool_free(G.d_indeg);
     free(G.h_indeg);
     free(G.device_ids);
     free(G.outdeg);
@@ -326,9 +329,9 @@ static void gz_upload_layout(const uint64_t* pairs, uint64_t num_edges, uint64_t
     const uint64_t nv = gz_pack_vectors(pairs, num_edges, by_dst, vecs);
     uint64_t* offs = (uint64_t*)malloc((num_vertices + 1) * sizeof(uint64_t));
     gz_build_vertex_offsets(vecs, nv, num_vertices, offs);
-    *d_vecs = (gz_vec_t*)gz_device_malloc((nv ? nv : 1) * sizeof(gz_vec_t));
+    *d_vecs = (gz_vec_t*)gz_pool_malloc((nv ? nv : 1) * sizeof(gz_vec_t), 0);
     gz_copy_to_device(*d_vecs, vecs, nv * sizeof(gz_vec_t));
-    *d_offsets = (uint64_t*)gz_device_malloc((num_vertices + 1) * sizeof(uint64_t));
+    *d_offsets = (uint64_t*)gz_pool_malloc((num_vertices + 1) * sizeof(uint64_t), 0);
     gz_copy_to_device(*d_offsets, offs, (num_vertices + 1) * sizeof(uint64_t));
     *count = nv;
     free(offs);
@@ -354,7 +357,7 @@ int gz_graph_load_pairs(uint64_t num_vertices, uint64_t pull_edges, const uint64
     if (pull_pairs) gz_upload_layout(pull_pairs, pull_edges, num_vertices, 1, &G.d_pull, &G.d_pull_offsets, &G.pull_vectors);
     if (push_pairs) gz_upload_layout(push_pairs, push_edges, num_vertices, 0, &G.d_push, &G.d_push_offsets, &G.push_vectors);
     const size_t vbytes = (num_vertices + 8) * sizeof(uint64_t);
-    G.d_outdeg = (double*)gz_device_malloc(vbytes);
+    G.d_outdeg = (double*)gz_pool_malloc(vbytes, 0);
     gz_copy_to_device(G.d_outdeg, G.outdeg, vbytes);
     gz_graph_finish();
     return 0;
@@ -381,7 +384,7 @@ const uint64_t* gz_graph_original_ids_device(void) { return G.d_original_ids; }
 const uint32_t* gz_graph_indegrees_device(void)
 {
     if (G.d_indeg == NULL && G.num_vertices) {
-        G.d_indeg = (uint32_t*)gz_device_malloc((G.num_vertices + 8) * sizeof(uint32_t));
+        G.d_indeg = (uint32_t*)gz_pool_malloc((G.num_vertices + 8) * sizeof(uint32_t), 1);
         if (G.d_pull != NULL)
             gz_dev_indegrees(G.d_pull, G.pull_vectors, 1, G.d_indeg, G.num_vertices);
         else
@@ -441,10 +444,10 @@ static void gz_graph_finish(void)
     gz_frontier_counts_release();
     const size_t vbytes = (num_vertices + 8) * sizeof(uint64_t);
     const size_t fwords = (num_vertices + 63) / 64 + 8;
-    G.d_props = gz_device_malloc(vbytes);
-    G.d_acc = gz_device_malloc(vbytes);
-    G.d_has = (uint64_t*)gz_device_malloc(fwords * sizeof(uint64_t));
-    G.d_wants = (uint64_t*)gz_device_malloc(fwords * sizeof(uint64_t));
+    G.d_props = gz_pool_malloc(vbytes, 1);
+    G.d_acc = gz_pool_malloc(vbytes, 1);
+    G.d_has = (uint64_t*)gz_pool_malloc(fwords * sizeof(uint64_t), 1);
+    G.d_wants = (uint64_t*)gz_pool_malloc(fwords * sizeof(uint64_t), 1);
 
     gz_graph.num_vertices = num_vertices;
     gz_graph.num_edges = G.num_edges;

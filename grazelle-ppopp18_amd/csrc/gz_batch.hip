@@ -172,10 +172,10 @@ void gz_batch_free_graph(void)
 void gz_batch_free_chunks(void)
 {
     gz_batch_free_graph();
-    gz_device_free(B.d_chunks);
-    gz_device_free(B.d_cbase);
-    gz_device_free(B.d_merge);
-    gz_device_free(B.d_partials);
+    gz_pool_free(B.d_chunks);
+    gz_pool_free(B.d_cbase);
+    gz_pool_free(B.d_merge);
+    gz_pool_free(B.d_partials);
     B.d_chunks = nullptr;
     B.d_cbase = nullptr;
     B.d_merge = nullptr;
@@ -218,12 +218,12 @@ void gz_batch_build_chunks(uint32_t mask)
         }
     }
     B.nchunks = n;
-    B.d_chunks = (uint64_t*)gz_device_malloc((2 * n + 2) * sizeof(uint64_t));
+    B.d_chunks = (uint64_t*)gz_pool_malloc((2 * n + 2) * sizeof(uint64_t), 1);
     if (n) gz_copy_to_device(B.d_chunks, pairs, 2 * n * sizeof(uint64_t));
-    B.d_cbase = (uint64_t*)gz_device_malloc((B.count + 1) * sizeof(uint64_t));
+    B.d_cbase = (uint64_t*)gz_pool_malloc((B.count + 1) * sizeof(uint64_t), 1);
     gz_copy_to_device(B.d_cbase, cbase, (B.count + 1) * sizeof(uint64_t));
-    B.d_merge = (mergeaccum_t*)gz_device_malloc((n ? n : 1) * sizeof(mergeaccum_t));
-    B.d_partials = (double*)gz_device_malloc((n ? n : 1) * sizeof(double));
+    B.d_merge = (mergeaccum_t*)gz_pool_malloc((n ? n : 1) * sizeof(mergeaccum_t), 1);
+    B.d_partials = (double*)gz_pool_malloc((n ? n : 1) * sizeof(double), 1);
     free(pairs);
     free(cbase);
 }
@@ -285,9 +285,9 @@ bool gz_batch_config_valid(const gz_batch_config_t* c)
 extern "C" void gz_batch_release(void)
 {
     gz_batch_free_chunks();
-    gz_device_free(B.d_base);
-    gz_device_free(B.d_gid);
-    gz_device_free(B.d_c);
+    gz_pool_free(B.d_base);
+    gz_pool_free(B.d_gid);
+    gz_pool_free(B.d_c);
     free(B.base);
     free(B.vec_base);
     free(B.bucket);
@@ -313,22 +313,22 @@ extern "C" int gz_batch_attach(const uint64_t* vertex_bases, uint32_t count)
     B.count = count;
     B.base = (uint64_t*)malloc((count + 1) * sizeof(uint64_t));
     memcpy(B.base, vertex_bases, (count + 1) * sizeof(uint64_t));
-    B.d_base = (uint64_t*)gz_device_malloc((count + 1) * sizeof(uint64_t));
+    B.d_base = (uint64_t*)gz_pool_malloc((count + 1) * sizeof(uint64_t), 1);
     gz_copy_to_device(B.d_base, B.base, (count + 1) * sizeof(uint64_t));
-    B.d_gid = (uint16_t*)gz_device_malloc((V ? V : 1) * sizeof(uint16_t));
+    B.d_gid = (uint16_t*)gz_pool_malloc((V ? V : 1) * sizeof(uint16_t), 1);
     hipLaunchKernelGGL(gz_k_batch_gid, dim3(gz_grid(V, GZ_BLOCK)), dim3(GZ_BLOCK), 0, gz_stream,
                        (const uint64_t*)B.d_base, count, V, B.d_gid);
     GZ_LAUNCH_CHECK();
-    uint64_t* d_vb = (uint64_t*)gz_device_malloc((count + 1) * sizeof(uint64_t));
+    uint64_t* d_vb = (uint64_t*)gz_pool_malloc((count + 1) * sizeof(uint64_t), 1);
     hipLaunchKernelGGL(gz_k_batch_gather_offsets, dim3((count + 1 + 255) / 256), dim3(256), 0, gz_stream,
                        (const uint64_t*)gz_graph.pull_vertex_offsets, (const uint64_t*)B.d_base, count + 1, d_vb);
     GZ_LAUNCH_CHECK();
     B.vec_base = (uint64_t*)malloc((count + 1) * sizeof(uint64_t));
     gz_copy_to_host(B.vec_base, d_vb, (count + 1) * sizeof(uint64_t));
-    gz_device_free(d_vb);
+    gz_pool_free(d_vb);
     B.bucket = (uint32_t*)malloc(count * sizeof(uint32_t));
     for (uint32_t g = 0; g < count; ++g) B.bucket[g] = gz_bucket_of(B.base[g + 1] - B.base[g]);
-    B.d_c = (double*)gz_device_malloc(count * sizeof(double));
+    B.d_c = (double*)gz_pool_malloc(count * sizeof(double), 1);
     gz_batch_build_chunks(~0u);
     return 0;
 }
@@ -405,7 +405,7 @@ extern "C" double gz_batch_time_pull(const gz_batch_config_t* cfg, uint32_t buck
     if (B.nchunks) {
         gz_timer_t* t = gz_timer_create();
         double* props = (double*)gz_graph.vertex_props;
-        double* scratch_acc = (double*)gz_device_malloc((gz_graph.num_vertices + 8) * sizeof(double));
+        double* scratch_acc = (double*)gz_pool_malloc((gz_graph.num_vertices + 8) * sizeof(double), 1);
         for (uint32_t r = 0; r < reps + 1; ++r) {
             const unsigned blocks = gz_batch_pull_blocks(B.nchunks, B.cfg.workgroup_size);
             gz_timer_start(t);
@@ -424,7 +424,7 @@ extern "C" double gz_batch_time_pull(const gz_batch_config_t* cfg, uint32_t buck
             const double ms = gz_timer_elapsed_ms(t);
             if (r > 0 && (best < 0.0 || ms < best)) best = ms; /* the first run warms up */
         }
-        gz_device_free(scratch_acc);
+        gz_pool_free(scratch_acc);
         gz_timer_destroy(t);
     } else {
         best = 0.0;
@@ -456,11 +456,11 @@ extern "C" void gz_batch_pr_ranks(double* out)
         gz_copy_to_host(out, gz_graph.vertex_props, V * sizeof(double));
         return;
     }
-    double* d = (double*)gz_device_malloc((V ? V : 1) * sizeof(double));
+    double* d = (double*)gz_pool_malloc((V ? V : 1) * sizeof(double), 0);
     hipLaunchKernelGGL(gz_k_batch_ranks, dim3(gz_grid(V, GZ_BLOCK)), dim3(GZ_BLOCK), 0, gz_stream,
                        (const double*)gz_graph.vertex_props, gz_graph.vertex_outdegrees, (const uint16_t*)B.d_gid,
                        (const uint64_t*)B.d_base, V, d);
     GZ_LAUNCH_CHECK();
     gz_copy_to_host(out, d, V * sizeof(double));
-    gz_device_free(d);
+    gz_pool_free(d);
 }

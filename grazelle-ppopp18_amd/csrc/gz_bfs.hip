@@ -453,26 +453,26 @@ static struct {
 static void gz_bfs_pending_reserve(uint64_t V)
 {
     if (gz_bfs_pend.vertices >= V && gz_bfs_pend.bits != nullptr) return;
-    gz_device_free(gz_bfs_pend.bits);
-    gz_device_free(gz_bfs_pend.out.list);
-    gz_device_free(gz_bfs_pend.out.prefix);
-    gz_device_free(gz_bfs_pend.out.block_sums);
-    gz_device_free(gz_bfs_pend.out.totals);
-    gz_bfs_pend.bits = (uint64_t*)gz_device_malloc(((V + 63) / 64 + 8) * sizeof(uint64_t));
-    gz_bfs_pend.out.list = (uint64_t*)gz_device_malloc((V + 8) * sizeof(uint64_t));
-    gz_bfs_pend.out.prefix = (uint64_t*)gz_device_malloc((V + 8) * sizeof(uint64_t));
-    gz_bfs_pend.out.block_sums = (uint64_t*)gz_device_malloc((2 * (gz_compact_blocks(V) + 1) + 8) * sizeof(uint64_t));
-    gz_bfs_pend.out.totals = (uint64_t*)gz_device_malloc(8 * sizeof(uint64_t));
+    gz_pool_free(gz_bfs_pend.bits);
+    gz_pool_free(gz_bfs_pend.out.list);
+    gz_pool_free(gz_bfs_pend.out.prefix);
+    gz_pool_free(gz_bfs_pend.out.block_sums);
+    gz_pool_free(gz_bfs_pend.out.totals);
+    gz_bfs_pend.bits = (uint64_t*)gz_pool_malloc(((V + 63) / 64 + 8) * sizeof(uint64_t), 1);
+    gz_bfs_pend.out.list = (uint64_t*)gz_pool_malloc((V + 8) * sizeof(uint64_t), 1);
+    gz_bfs_pend.out.prefix = (uint64_t*)gz_pool_malloc((V + 8) * sizeof(uint64_t), 1);
+    gz_bfs_pend.out.block_sums = (uint64_t*)gz_pool_malloc((2 * (gz_compact_blocks(V) + 1) + 8) * sizeof(uint64_t), 1);
+    gz_bfs_pend.out.totals = (uint64_t*)gz_pool_malloc(8 * sizeof(uint64_t), 1);
     gz_bfs_pend.vertices = V;
 }
 
 extern "C" void gz_bfs_pending_release(void)
 {
-    gz_device_free(gz_bfs_pend.bits);
-    gz_device_free(gz_bfs_pend.out.list);
-    gz_device_free(gz_bfs_pend.out.prefix);
-    gz_device_free(gz_bfs_pend.out.block_sums);
-    gz_device_free(gz_bfs_pend.out.totals);
+    gz_pool_free(gz_bfs_pend.bits);
+    gz_pool_free(gz_bfs_pend.out.list);
+    gz_pool_free(gz_bfs_pend.out.prefix);
+    gz_pool_free(gz_bfs_pend.out.block_sums);
+    gz_pool_free(gz_bfs_pend.out.totals);
     memset(&gz_bfs_pend, 0, sizeof(gz_bfs_pend));
 }
 

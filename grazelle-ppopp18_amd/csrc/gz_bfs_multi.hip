@@ -243,12 +243,12 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_msbfs_result(const gz_vec_t* __
 
 void gz_msbfs_release_buffers()
 {
-    gz_device_free(M.seen);
-    gz_device_free(M.front);
-    gz_device_free(M.next);
-    gz_device_free(M.depth);
-    gz_device_free(M.fbits);
-    gz_device_free(M.roots);
+    gz_pool_free(M.seen);
+    gz_pool_free(M.front);
+    gz_pool_free(M.next);
+    gz_pool_free(M.depth);
+    gz_pool_free(M.fbits);
+    gz_pool_free(M.roots);
     memset(&M, 0, sizeof(M));
 }
 
@@ -257,12 +257,12 @@ void gz_msbfs_reserve(uint64_t V)
     if (M.seen != nullptr && M.vertices == V) return;
     gz_msbfs_release_buffers();
     const uint64_t words = (V + 63) / 64 + 8;
-    M.seen = (uint64_t*)gz_device_malloc((V + 8) * sizeof(uint64_t));
-    M.front = (uint64_t*)gz_device_malloc((V + 8) * sizeof(uint64_t));
-    M.next = (uint64_t*)gz_device_malloc((V + 8) * sizeof(uint64_t));
-    M.depth = (uint8_t*)gz_device_malloc((V + 8) * 64);
-    M.fbits = (uint64_t*)gz_device_malloc(words * sizeof(uint64_t));
-    M.roots = (uint64_t*)gz_device_malloc(64 * sizeof(uint64_t));
+    M.seen = (uint64_t*)gz_pool_malloc((V + 8) * sizeof(uint64_t), 1);
+    M.front = (uint64_t*)gz_pool_malloc((V + 8) * sizeof(uint64_t), 1);
+    M.next = (uint64_t*)gz_pool_malloc((V + 8) * sizeof(uint64_t), 1);
+    M.depth = (uint8_t*)gz_pool_malloc((V + 8) * 64, 1);
+    M.fbits = (uint64_t*)gz_pool_malloc(words * sizeof(uint64_t), 1);
+    M.roots = (uint64_t*)gz_pool_malloc(64 * sizeof(uint64_t), 1);
     M.vertices = V;
 }
 
@@ -388,8 +388,8 @@ extern "C" void gz_bfs_batch_result(uint32_t search, int64_t* parents, uint64_t*
         fprintf(stderr, "grazelle: no BFS batch result for search %u\n", search);
         exit(66);
     }
-    uint64_t* d_depth = depths ? (uint64_t*)gz_device_malloc((V + 8) * sizeof(uint64_t)) : nullptr;
-    int64_t* d_parent = parents ? (int64_t*)gz_device_malloc((V + 8) * sizeof(int64_t)) : nullptr;
+    uint64_t* d_depth = depths ? (uint64_t*)gz_pool_malloc((V + 8) * sizeof(uint64_t), 0) : nullptr;
+    int64_t* d_parent = parents ? (int64_t*)gz_pool_malloc((V + 8) * sizeof(int64_t), 0) : nullptr;
     uint64_t blocks = (V + GZ_BLOCK - 1) / GZ_BLOCK;
     if (blocks > 16384) blocks = 16384;
     hipLaunchKernelGGL(gz_k_msbfs_result, dim3((unsigned)blocks), dim3(GZ_BLOCK), 0, gz_stream, gz_graph.pull_vectors,
@@ -398,6 +398,6 @@ extern "C" void gz_bfs_batch_result(uint32_t search, int64_t* parents, uint64_t*
     GZ_LAUNCH_CHECK();
     if (depths) gz_copy_to_host(depths, d_depth, V * sizeof(uint64_t));
     if (parents) gz_copy_to_host(parents, d_parent, V * sizeof(int64_t));
-    gz_device_free(d_depth);
-    gz_device_free(d_parent);
+    gz_pool_free(d_depth);
+    gz_pool_free(d_parent);
 }

@@ -10,6 +10,7 @@
  * from one block scan of the per-thread counts, in vertex order.
  */
 #include "gz_frontier.h"
+#include "gz_host_internal.h"
 
 /* Vertices v0 .. v0+GZ_COMPACT_VPT-1 (v0 a multiple of GZ_COMPACT_VPT):
  * vector counts c[k] of the vertices whose bit is set, 0 otherwise; a vertex
@@ -461,12 +462,12 @@ static int gz_hasvec_next;
 extern "C" void gz_frontier_counts_release(void)
 {
     for (auto& e : gz_counts_cache) {
-        gz_device_free(e.counts);
+        gz_pool_free(e.counts);
         e = {nullptr, 0, 0, nullptr};
     }
     gz_counts_next = 0;
     for (auto& e : gz_hasvec_cache) {
-        gz_device_free(e.bits);
+        gz_pool_free(e.bits);
         e = {nullptr, 0, 0, nullptr};
     }
     gz_hasvec_next = 0;
@@ -480,9 +481,9 @@ static const uint64_t* gz_frontier_hasvec(const uint64_t* offsets, uint64_t num_
             return e.bits;
     auto& e = gz_hasvec_cache[gz_hasvec_next];
     gz_hasvec_next ^= 1;
-    gz_device_free(e.bits);
+    gz_pool_free(e.bits);
     const uint64_t words = (num_vertices + 63) / 64;
-    e.bits = (uint64_t*)gz_device_malloc((words + 8) * sizeof(uint64_t));
+    e.bits = (uint64_t*)gz_pool_malloc((words + 8) * sizeof(uint64_t), 1);
     uint64_t blocks = (words * GZ_WAVE + GZ_BLOCK - 1) / GZ_BLOCK;
     if (blocks > 4096) blocks = 4096;
     hipLaunchKernelGGL(gz_k_has_vectors, dim3((unsigned)blocks), dim3(GZ_BLOCK), 0, gz_stream, offsets, num_vertices,
@@ -512,9 +513,9 @@ static const uint32_t* gz_frontier_counts(const uint64_t* offsets, uint64_t num_
             return e.counts;
     auto& e = gz_counts_cache[gz_counts_next];
     gz_counts_next ^= 1;
-    gz_device_free(e.counts);
+    gz_pool_free(e.counts);
     const uint64_t padded = (num_vertices + GZ_COMPACT_VPT - 1) / GZ_COMPACT_VPT * GZ_COMPACT_VPT;
-    e.counts = (uint32_t*)gz_device_malloc(padded * sizeof(uint32_t));
+    e.counts = (uint32_t*)gz_pool_malloc(padded * sizeof(uint32_t), 1);
     uint64_t blocks = (padded + GZ_BLOCK - 1) / GZ_BLOCK;
     if (blocks > 4096) blocks = 4096;
     hipLaunchKernelGGL(gz_k_vector_counts, dim3((unsigned)blocks), dim3(GZ_BLOCK), 0, gz_stream, offsets,
@@ -541,7 +542,7 @@ static bool gz_seg_take(unsigned long long** bank, unsigned long long** other)
     if (status != hipStreamCaptureStatusNone) return false;
     const size_t words = (size_t)GZ_SEGMENTS * GZ_SEG_STRIDE;
     if (gz_seg_banks == nullptr) {
-        gz_seg_banks = (unsigned long long*)gz_device_malloc(2 * words * sizeof(uint64_t));
+        gz_seg_banks = (unsigned long long*)gz_pool_malloc(2 * words * sizeof(uint64_t), 1);
         gz_device_zero(gz_seg_banks, 2 * words * sizeof(uint64_t));
     }
     *bank = gz_seg_banks + (size_t)gz_seg_parity * words;

@@ -14,6 +14,14 @@
 extern "C" {
 #endif
 
+/* Device memory for the library's own buffers, from blocks kept between
+ * requests (gz_runtime.hip), zero-filled when `zero`; used on the library's
+ * stream only. */
+void* gz_pool_malloc(size_t bytes, int zero);
+void gz_pool_free(void* ptr);
+/* Waits for the whole device (nothing before the runtime is up). */
+void gz_device_wait(void);
+
 /* Device-built layouts handed to the graph record (device ingress). */
 typedef struct gz_device_layouts_t {
     uint64_t num_vertices, num_edges;

@@ -88,12 +88,16 @@ __global__ void gz_k_rmat_keys(uint64_t seed, uint64_t edge_offset, uint32_t sca
     }
 }
 
-__global__ void gz_k_pairs_keys(const uint64_t* __restrict__ pairs, uint64_t n, uint32_t b, int both, int drop,
-                                uint64_t* __restrict__ keys)
+/* The same for uploaded (src, dst) pairs; *bad becomes the smallest index of
+ * an endpoint (word of `pairs`) that is not below nv. */
+__global__ void gz_k_pairs_keys(const gz_u64x2* __restrict__ pairs, uint64_t n, uint32_t b, int both, int drop,
+                                uint64_t nv, uint64_t* __restrict__ keys, unsigned long long* __restrict__ bad)
 {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += stride) {
-        const uint64_t s = pairs[2 * e], d = pairs[2 * e + 1];
+        const gz_u64x2 sd = pairs[e];
+        const uint64_t s = sd.x, d = sd.y;
+        if (s >= nv || d >= nv) atomicMin(bad, (unsigned long long)(2 * e + (s >= nv ? 0 : 1)));
         if (both) {
             keys[2 * e] = gz_edge_key(d, s, b, drop);
             keys[2 * e + 1] = gz_edge_key(s, d, b, drop);
@@ -326,10 +330,9 @@ void gz_sort_keys(uint64_t* a, uint64_t* b_buf, uint64_t n, uint32_t begin, uint
     rocprim::double_buffer<uint64_t> db(a, b_buf);
     size_t tmp_bytes = 0;
     GZ_CHECK(rocprim::radix_sort_keys(nullptr, tmp_bytes, db, (size_t)n, begin, end, gz_stream));
-    void* tmp = gz_device_malloc(tmp_bytes ? tmp_bytes : 1);
+    void* tmp = gz_pool_malloc(tmp_bytes ? tmp_bytes : 1, 0);
     GZ_CHECK(rocprim::radix_sort_keys(tmp, tmp_bytes, db, (size_t)n, begin, end, gz_stream));
-    GZ_CHECK(hipStreamSynchronize(gz_stream));
-    gz_device_free(tmp);
+    gz_pool_free(tmp);
     *sorted = db.current();
 }
 
@@ -340,10 +343,10 @@ void gz_scan(It in, uint64_t* out, uint64_t n)
     size_t tmp_bytes = 0;
     GZ_CHECK(rocprim::exclusive_scan(nullptr, tmp_bytes, in, out, (uint64_t)0, (size_t)n, rocprim::plus<uint64_t>(),
                                      gz_stream));
-    void* tmp = gz_device_malloc(tmp_bytes ? tmp_bytes : 1);
+    void* tmp = gz_pool_malloc(tmp_bytes ? tmp_bytes : 1, 0);
     GZ_CHECK(rocprim::exclusive_scan(tmp, tmp_bytes, in, out, (uint64_t)0, (size_t)n, rocprim::plus<uint64_t>(),
                                      gz_stream));
-    gz_device_free(tmp);
+    gz_pool_free(tmp);
 }
 
 /* Build one layout from sorted, duplicate-free keys[0, m) and the bounds of
@@ -351,13 +354,13 @@ void gz_scan(It in, uint64_t* out, uint64_t n)
 void gz_build_layout(const uint64_t* keys, uint64_t m, uint32_t b, int low, uint64_t nv, const uint64_t* first,
                      const uint64_t* end, gz_vec_t** d_vecs, uint64_t** d_offsets, uint64_t* vector_count)
 {
-    uint64_t* voff = (uint64_t*)gz_device_malloc((nv + 1) * sizeof(uint64_t));
+    uint64_t* voff = (uint64_t*)gz_pool_malloc((nv + 1) * sizeof(uint64_t), 0);
     gz_scan(rocprim::make_transform_iterator(rocprim::make_counting_iterator<uint64_t>(0),
                                              gz_group_vectors{first, end, nv}),
             voff, nv + 1);
     uint64_t total = 0;
     gz_copy_to_host(&total, voff + nv, sizeof(uint64_t));
-    gz_vec_t* vecs = (gz_vec_t*)gz_device_malloc((total ? total : 1) * sizeof(gz_vec_t));
+    gz_vec_t* vecs = (gz_vec_t*)gz_pool_malloc((total ? total : 1) * sizeof(gz_vec_t), 0);
     if (m) {
         hipLaunchKernelGGL(gz_k_pack, dim3(gz_grid_for(m)), dim3(GZ_BLOCK), 0, gz_stream, keys, m, b, low, first, end,
                            voff, (uint64_t*)vecs);
@@ -551,7 +554,7 @@ void gz_count_sources(const uint64_t* keys, uint64_t n, uint32_t b, uint64_t nv,
     const uint64_t segments = (n + GZ_COUNT_SEGMENT - 1) / GZ_COUNT_SEGMENT;
     const size_t cursor_words = (size_t)buckets * GZ_COUNT_PAD;
     unsigned long long* cursors =
-        (unsigned long long*)gz_device_malloc((cursor_words + buckets + 1) * sizeof(uint64_t)); /* zero-filled */
+        (unsigned long long*)gz_pool_malloc((cursor_words + buckets + 1) * sizeof(uint64_t), 1); /* zero-filled */
     uint64_t* base = (uint64_t*)cursors + cursor_words;
     hipLaunchKernelGGL(gz_k_bucket_sizes, dim3((unsigned)(tiles < 1024 ? tiles : 1024)), dim3(GZ_COUNT_THREADS), 0,
                        gz_stream, keys, n, mask, shift, buckets, cursors);
@@ -564,8 +567,7 @@ void gz_count_sources(const uint64_t* keys, uint64_t n, uint32_t b, uint64_t nv,
     hipLaunchKernelGGL(gz_k_bucket_count, dim3((unsigned)segments), dim3(GZ_COUNT_THREADS), 0, gz_stream, ids, n, shift,
                        buckets, base, nv, cnt);
     GZ_LAUNCH_CHECK();
-    GZ_CHECK(hipStreamSynchronize(gz_stream));
-    gz_device_free(cursors);
+    gz_pool_free(cursors);
 }
 
 /* sort key: out-degree descending (as `most` less the degree), then id ascending */
@@ -617,18 +619,17 @@ __global__ void gz_k_remap_keys(uint64_t* __restrict__ keys, uint64_t n, uint32_
 uint64_t* gz_relabel_by_outdegree(uint64_t* keys, uint64_t* scratch, uint64_t n, uint32_t b, uint64_t nv,
                                   uint64_t slice_vertices, uint32_t tiers, uint32_t** device_ids)
 {
-    uint32_t* cnt = (uint32_t*)gz_device_malloc(nv * sizeof(uint32_t));
-    GZ_CHECK(hipMemsetAsync(cnt, 0, nv * sizeof(uint32_t), gz_stream));
+    uint32_t* cnt = (uint32_t*)gz_pool_malloc(nv * sizeof(uint32_t), 1);
     gz_count_sources(keys, n, b, nv, (uint32_t*)scratch, cnt);
     const uint64_t most = n < 0xffffffffull ? n : 0xffffffffull; /* counts are 32-bit */
-    uint64_t* order = (uint64_t*)gz_device_malloc(nv * sizeof(uint64_t));
-    uint64_t* order_b = (uint64_t*)gz_device_malloc(nv * sizeof(uint64_t));
+    uint64_t* order = (uint64_t*)gz_pool_malloc(nv * sizeof(uint64_t), 0);
+    uint64_t* order_b = (uint64_t*)gz_pool_malloc(nv * sizeof(uint64_t), 0);
     hipLaunchKernelGGL(gz_k_degree_order, dim3(gz_grid_for(nv)), dim3(GZ_BLOCK), 0, gz_stream, cnt, nv, b,
                        most, order);
     GZ_LAUNCH_CHECK();
     uint64_t* sorted = order;
     if (nv > 1) gz_sort_keys(order, order_b, nv, 0, b + gz_id_bits(most + 1), &sorted);
-    uint64_t* old_of_new = (uint64_t*)gz_device_malloc((nv + 8) * sizeof(uint64_t));
+    uint64_t* old_of_new = (uint64_t*)gz_pool_malloc((nv + 8) * sizeof(uint64_t), 0);
     uint32_t* new_of_old = cnt; /* counts are no longer needed */
     hipLaunchKernelGGL(gz_k_permutation, dim3(gz_grid_for(nv)), dim3(GZ_BLOCK), 0, gz_stream, sorted, nv, b,
                        slice_vertices, tiers, old_of_new, new_of_old);
@@ -637,9 +638,8 @@ uint64_t* gz_relabel_by_outdegree(uint64_t* keys, uint64_t* scratch, uint64_t n,
         hipLaunchKernelGGL(gz_k_remap_keys, dim3(gz_grid_for(n)), dim3(GZ_BLOCK), 0, gz_stream, keys, n, b, new_of_old);
         GZ_LAUNCH_CHECK();
     }
-    GZ_CHECK(hipStreamSynchronize(gz_stream));
-    gz_device_free(order);
-    gz_device_free(order_b);
+    gz_pool_free(order);
+    gz_pool_free(order_b);
     *device_ids = new_of_old;
     return old_of_new;
 }
@@ -661,12 +661,12 @@ void gz_ingress_from_keys(uint64_t nv, uint64_t* a, uint64_t* b_buf, uint64_t n,
     if (n > 1) gz_sort_keys(a, b_buf, n, 0, 2 * b, &sorted);
     uint64_t* other = (sorted == a) ? b_buf : a;
     uint64_t m = 0;
-    uint64_t* first = (uint64_t*)gz_device_malloc(nv * sizeof(uint64_t));
-    uint64_t* end = (uint64_t*)gz_device_malloc(nv * sizeof(uint64_t));
+    uint64_t* first = (uint64_t*)gz_pool_malloc(nv * sizeof(uint64_t), 1);
+    uint64_t* end = (uint64_t*)gz_pool_malloc(nv * sizeof(uint64_t), 1);
     if (n) {
         const uint64_t none = gz_no_key(b);
         const uint64_t tiles = (n + GZ_TILE - 1) / GZ_TILE;
-        uint64_t* sums = (uint64_t*)gz_device_malloc(2 * (tiles + 1) * sizeof(uint64_t)); /* sums[tiles] stays 0 */
+        uint64_t* sums = (uint64_t*)gz_pool_malloc(2 * (tiles + 1) * sizeof(uint64_t), 1); /* sums[tiles] stays 0 */
         uint64_t* base = sums + tiles + 1;
         hipLaunchKernelGGL(gz_k_tile_count<false>, dim3(gz_tile_grid(tiles)), dim3(GZ_BLOCK), 0, gz_stream, sorted, n,
                            b, none, tiles, sums);
@@ -676,7 +676,7 @@ void gz_ingress_from_keys(uint64_t nv, uint64_t* a, uint64_t* b_buf, uint64_t n,
                            none, tiles, base, other, first, end);
         GZ_LAUNCH_CHECK();
         gz_copy_to_host(&m, base + tiles, sizeof(uint64_t));
-        gz_device_free(sums);
+        gz_pool_free(sums);
     }
 
     gz_device_layouts_t L;
@@ -696,15 +696,15 @@ void gz_ingress_from_keys(uint64_t nv, uint64_t* a, uint64_t* b_buf, uint64_t n,
         GZ_LAUNCH_CHECK();
     }
     gz_build_layout(push_sorted, m, b, 1, nv, first, end, &L.push, &L.push_offsets, &L.push_count);
-    L.outdeg = (double*)gz_device_malloc((nv + 8) * sizeof(double));
+    L.outdeg = (double*)gz_pool_malloc((nv + 8) * sizeof(double), 0);
     hipLaunchKernelGGL(gz_k_outdegrees, dim3(gz_grid_for(nv + 8)), dim3(GZ_BLOCK), 0, gz_stream, first, end, nv,
                        L.outdeg);
     GZ_LAUNCH_CHECK();
-    GZ_CHECK(hipStreamSynchronize(gz_stream));
-    gz_device_free(first);
-    gz_device_free(end);
+    gz_pool_free(first);
+    gz_pool_free(end);
     gz_graph_adopt_device(&L);
     if (slice_log2) gz_graph_build_source_slices(1ull << slice_log2, tiers, blocks, GZ_SLICE_BLOCK_VERTICES);
+    gz_synchronize();
 }
 
 /* Whether the key kernels drop self-loops (a renumbering counts them first). */
@@ -720,34 +720,45 @@ void gz_check_vertex_count(uint64_t nv)
 
 }  // namespace
 
+/* Upload n host pairs and append their keys; dies with `what` and the first
+ * endpoint that is not below nv.  The check rides on the key kernel's reads: a
+ * host loop over the endpoints cost more than the upload (a load of 3 M pairs,
+ * CC and its labels: 4.00 ms with the loop, 2.59 without). */
+static void gz_upload_keys(const uint64_t* pairs, uint64_t n, uint32_t b, int both, int drop, uint64_t nv,
+                           uint64_t* keys, const char* what)
+{
+    if (n == 0) return;
+    uint64_t* d = (uint64_t*)gz_pool_malloc((2 * n + 2) * sizeof(uint64_t), 0);
+    unsigned long long* bad = (unsigned long long*)(d + 2 * n);
+    gz_dev_fill_u64((uint64_t*)bad, ~0ull, 1);
+    gz_copy_to_device(d, pairs, 2 * n * sizeof(uint64_t));
+    hipLaunchKernelGGL(gz_k_pairs_keys, dim3(gz_grid_for(n)), dim3(GZ_BLOCK), 0, gz_stream, (const gz_u64x2*)d, n, b,
+                       both, drop, nv, keys, bad);
+    GZ_LAUNCH_CHECK();
+    uint64_t at = 0;
+    gz_copy_to_host(&at, bad, sizeof(at));
+    gz_pool_free(d);
+    if (at != ~0ull) {
+        fprintf(stderr, "grazelle: %s %llu is not below V = %llu\n", what, (unsigned long long)pairs[at],
+                (unsigned long long)nv);
+        exit(65);
+    }
+}
+
 extern "C" int gz_graph_build_pairs_device(uint64_t num_vertices, uint64_t num_edges, const uint64_t* pairs,
                                            int symmetrize, uint32_t flags)
 {
     gz_runtime_init(0);
     gz_graph_release();
     gz_check_vertex_count(num_vertices);
-    for (uint64_t i = 0; i < 2 * num_edges; ++i)
-        if (pairs[i] >= num_vertices) {
-            fprintf(stderr, "grazelle: edge endpoint %llu is not below V = %llu\n", (unsigned long long)pairs[i],
-                    (unsigned long long)num_vertices);
-            exit(65);
-        }
     const uint32_t b = gz_id_bits(num_vertices);
     const uint64_t n = symmetrize ? 2 * num_edges : num_edges;
-    uint64_t* d_pairs = (uint64_t*)gz_device_malloc((num_edges ? 2 * num_edges : 2) * sizeof(uint64_t));
-    if (num_edges) gz_copy_to_device(d_pairs, pairs, 2 * num_edges * sizeof(uint64_t));
-    uint64_t* a = (uint64_t*)gz_device_malloc((n ? n : 1) * sizeof(uint64_t));
-    uint64_t* bb = (uint64_t*)gz_device_malloc((n ? n : 1) * sizeof(uint64_t));
-    if (num_edges) {
-        hipLaunchKernelGGL(gz_k_pairs_keys, dim3(gz_grid_for(num_edges)), dim3(GZ_BLOCK), 0, gz_stream, d_pairs,
-                           num_edges, b, symmetrize, gz_drop_first(flags), a);
-        GZ_LAUNCH_CHECK();
-    }
-    GZ_CHECK(hipStreamSynchronize(gz_stream));
-    gz_device_free(d_pairs);
+    uint64_t* a = (uint64_t*)gz_pool_malloc((n ? n : 1) * sizeof(uint64_t), 0);
+    uint64_t* bb = (uint64_t*)gz_pool_malloc((n ? n : 1) * sizeof(uint64_t), 0);
+    gz_upload_keys(pairs, num_edges, b, symmetrize, gz_drop_first(flags), num_vertices, a, "edge endpoint");
     gz_ingress_from_keys(num_vertices, a, bb, n, b, flags);
-    gz_device_free(a);
-    gz_device_free(bb);
+    gz_pool_free(a);
+    gz_pool_free(bb);
     return 0;
 }
 
@@ -758,18 +769,12 @@ extern "C" int gz_graph_build_rmat_device(const gz_rmat_params_t* p, uint64_t nu
     gz_graph_release();
     const uint64_t rmat_nv = p->num_vertices ? p->num_vertices : (1ull << p->scale);
     uint64_t nv = num_vertices > rmat_nv ? num_vertices : rmat_nv;
-    for (uint64_t i = 0; i < 2 * extra_edges; ++i)
-        if (extra_pairs[i] >= nv) {
-            fprintf(stderr, "grazelle: extra edge endpoint %llu is not below V = %llu\n",
-                    (unsigned long long)extra_pairs[i], (unsigned long long)nv);
-            exit(65);
-        }
     gz_check_vertex_count(nv);
     const uint32_t b = gz_id_bits(nv);
     const uint64_t per = symmetrize ? 2 : 1;
     const uint64_t n = per * (p->num_edges + extra_edges);
-    uint64_t* a = (uint64_t*)gz_device_malloc((n ? n : 1) * sizeof(uint64_t));
-    uint64_t* bb = (uint64_t*)gz_device_malloc((n ? n : 1) * sizeof(uint64_t));
+    uint64_t* a = (uint64_t*)gz_pool_malloc((n ? n : 1) * sizeof(uint64_t), 0);
+    uint64_t* bb = (uint64_t*)gz_pool_malloc((n ? n : 1) * sizeof(uint64_t), 0);
     if (p->num_edges) {
         const uint32_t ta = (uint32_t)(p->a * 65536.0);
         const uint32_t tb = (uint32_t)((p->a + p->b) * 65536.0);
@@ -779,19 +784,11 @@ extern "C" int gz_graph_build_rmat_device(const gz_rmat_params_t* p, uint64_t nu
                            (uint64_t)0, a);
         GZ_LAUNCH_CHECK();
     }
-    if (extra_edges) {
-        uint64_t* d_pairs = (uint64_t*)gz_device_malloc(2 * extra_edges * sizeof(uint64_t));
-        gz_copy_to_device(d_pairs, extra_pairs, 2 * extra_edges * sizeof(uint64_t));
-        hipLaunchKernelGGL(gz_k_pairs_keys, dim3(gz_grid_for(extra_edges)), dim3(GZ_BLOCK), 0, gz_stream, d_pairs,
-                           extra_edges, b, symmetrize, gz_drop_first(flags), a + per * p->num_edges);
-        GZ_LAUNCH_CHECK();
-        GZ_CHECK(hipStreamSynchronize(gz_stream));
-        gz_device_free(d_pairs);
-    }
-    GZ_CHECK(hipStreamSynchronize(gz_stream));
+    gz_upload_keys(extra_pairs, extra_edges, b, symmetrize, gz_drop_first(flags), nv, a + per * p->num_edges,
+                   "extra edge endpoint");
     gz_ingress_from_keys(nv, a, bb, n, b, flags);
-    gz_device_free(a);
-    gz_device_free(bb);
+    gz_pool_free(a);
+    gz_pool_free(bb);
     return 0;
 }
 
@@ -810,8 +807,8 @@ extern "C" int gz_graph_build_rmat_union_device(const gz_rmat_params_t* params, 
     vertex_bases[count] = nv;
     gz_check_vertex_count(nv);
     const uint32_t b = gz_id_bits(nv);
-    uint64_t* a = (uint64_t*)gz_device_malloc((n ? n : 1) * sizeof(uint64_t));
-    uint64_t* bb = (uint64_t*)gz_device_malloc((n ? n : 1) * sizeof(uint64_t));
+    uint64_t* a = (uint64_t*)gz_pool_malloc((n ? n : 1) * sizeof(uint64_t), 0);
+    uint64_t* bb = (uint64_t*)gz_pool_malloc((n ? n : 1) * sizeof(uint64_t), 0);
     uint64_t at = 0;
     for (uint32_t g = 0; g < count; ++g) {
         const gz_rmat_params_t* p = &params[g];
@@ -826,10 +823,9 @@ extern "C" int gz_graph_build_rmat_union_device(const gz_rmat_params_t* params, 
         GZ_LAUNCH_CHECK();
         at += per * p->num_edges;
     }
-    GZ_CHECK(hipStreamSynchronize(gz_stream));
     gz_ingress_from_keys(nv, a, bb, n, b, 0);
-    gz_device_free(a);
-    gz_device_free(bb);
+    gz_pool_free(a);
+    gz_pool_free(bb);
     return 0;
 }
 
@@ -1136,10 +1132,10 @@ extern "C" int gz_graph_build_source_slices(uint64_t slice_vertices, uint32_t ti
     const uint32_t ns = GZ_XCDS * (tiers + blocks) + 1;
     const bool wide_mask = ns > 32;
     const uint64_t n = 4 * nvec;
-    uint64_t* a = (uint64_t*)gz_device_malloc((n ? n : 1) * sizeof(uint64_t));
-    uint64_t* bb = (uint64_t*)gz_device_malloc((n ? n : 1) * sizeof(uint64_t));
+    uint64_t* a = (uint64_t*)gz_pool_malloc((n ? n : 1) * sizeof(uint64_t), 0);
+    uint64_t* bb = (uint64_t*)gz_pool_malloc((n ? n : 1) * sizeof(uint64_t), 0);
     /* per slice: first key, first run, first vector (zero without edges) */
-    uint64_t* firsts = (uint64_t*)gz_device_malloc(3 * (GZ_MAX_SLICES + 1) * sizeof(uint64_t));
+    uint64_t* firsts = (uint64_t*)gz_pool_malloc(3 * (GZ_MAX_SLICES + 1) * sizeof(uint64_t), 1);
     uint64_t* first_run = firsts + GZ_MAX_SLICES + 1;
     uint64_t* first_vec = first_run + GZ_MAX_SLICES + 1;
     uint64_t* sorted = a;
@@ -1156,7 +1152,7 @@ extern "C" int gz_graph_build_source_slices(uint64_t slice_vertices, uint32_t ti
         tiles = (m + GZ_TILE - 1) / GZ_TILE;
     }
     if (m) {
-        uint64_t* sums = (uint64_t*)gz_device_malloc(2 * (tiles + 1) * sizeof(uint64_t)); /* sums[tiles] stays 0 */
+        uint64_t* sums = (uint64_t*)gz_pool_malloc(2 * (tiles + 1) * sizeof(uint64_t), 1); /* sums[tiles] stays 0 */
         tile_base = sums + tiles + 1;
         hipLaunchKernelGGL(gz_k_tile_count<true>, dim3(gz_tile_grid(tiles)), dim3(GZ_BLOCK), 0, gz_stream, sorted, m, b,
                            ~0ull, tiles, sums);
@@ -1168,10 +1164,10 @@ extern "C" int gz_graph_build_source_slices(uint64_t slice_vertices, uint32_t ti
         fprintf(stderr, "grazelle: the sliced layout needs fewer than 2^32 slice accumulators\n");
         exit(65);
     }
-    gz_slices.gid = (uint32_t*)gz_device_malloc((runs + 8) * sizeof(uint32_t));
+    gz_slices.gid = (uint32_t*)gz_pool_malloc((runs + 8) * sizeof(uint32_t), 1);
     if (m) {
-        run_first = (uint64_t*)gz_device_malloc((runs + 1) * sizeof(uint64_t));
-        run_vec = (uint64_t*)gz_device_malloc((runs + 1) * sizeof(uint64_t));
+        run_first = (uint64_t*)gz_pool_malloc((runs + 1) * sizeof(uint64_t), 0);
+        run_vec = (uint64_t*)gz_pool_malloc((runs + 1) * sizeof(uint64_t), 0);
         hipLaunchKernelGGL(gz_k_slice_runs, dim3(gz_tile_grid(tiles)), dim3(GZ_BLOCK), 0, gz_stream, sorted, m, b, tiles,
                            tile_base, run_first, gz_slices.gid);
         GZ_LAUNCH_CHECK();
@@ -1194,11 +1190,11 @@ extern "C" int gz_graph_build_source_slices(uint64_t slice_vertices, uint32_t ti
     const uint64_t block_first = gz_slices.begin[GZ_XCDS];
     const uint64_t block_span = gz_slices.begin[GZ_XCDS * (blocks + 1)] - block_first;
     const uint64_t window_total = gz_slices.begin[ns - 1] - block_span;
-    gz_slices.nbr24 = (uint32_t*)gz_device_malloc((window_total ? 3 * window_total : 1) * sizeof(uint32_t));
-    gz_slices.nbr16 = (uint64_t*)gz_device_malloc((block_span ? block_span : 1) * sizeof(uint64_t));
+    gz_slices.nbr24 = (uint32_t*)gz_pool_malloc((window_total ? 3 * window_total : 1) * sizeof(uint32_t), 0);
+    gz_slices.nbr16 = (uint64_t*)gz_pool_malloc((block_span ? block_span : 1) * sizeof(uint64_t), 0);
     gz_slices.block_span = block_span;
-    gz_slices.nbr = (gz_u32x4*)gz_device_malloc((cold ? cold : 1) * sizeof(gz_u32x4));
-    gz_slices.shared = (uint32_t*)gz_device_malloc((total ? total : 1) * sizeof(uint32_t));
+    gz_slices.nbr = (gz_u32x4*)gz_pool_malloc((cold ? cold : 1) * sizeof(gz_u32x4), 0);
+    gz_slices.shared = (uint32_t*)gz_pool_malloc((total ? total : 1) * sizeof(uint32_t), 0);
     if (m) {
         const gz_slice_pack_t pack{S,         H,          blocks,    ns, block_first, block_span, gz_slices.begin[ns - 1],
                                    first_run, gz_slices.nbr24, gz_slices.nbr16, gz_slices.nbr, gz_slices.shared};
@@ -1206,9 +1202,9 @@ extern "C" int gz_graph_build_source_slices(uint64_t slice_vertices, uint32_t ti
                            tile_base, run_first, run_vec, pack);
         GZ_LAUNCH_CHECK();
     }
-    gz_slices.mask = gz_device_malloc((nv + 8) * (wide_mask ? sizeof(uint64_t) : sizeof(uint32_t)));
+    gz_slices.mask = gz_pool_malloc((nv + 8) * (wide_mask ? sizeof(uint64_t) : sizeof(uint32_t)), 1);
     gz_slices.rank_blocks = (nv + GZ_WAVE - 1) / GZ_WAVE;
-    gz_slices.rank_base = (uint32_t*)gz_device_malloc(ns * gz_slices.rank_blocks * sizeof(uint32_t));
+    gz_slices.rank_base = (uint32_t*)gz_pool_malloc(ns * gz_slices.rank_blocks * sizeof(uint32_t), 0);
     /* consecutive blocks per wavefront: few enough that the chip is full */
     uint64_t per = gz_slices.rank_blocks / ((uint64_t)gz_cu_count * 32);
     per = per < 1 ? 1 : per > 64 ? 64 : per;
@@ -1221,18 +1217,18 @@ extern "C" int gz_graph_build_source_slices(uint64_t slice_vertices, uint32_t ti
         hipLaunchKernelGGL(gz_k_slice_mask<uint32_t>, dim3(mask_grid), dim3(GZ_BLOCK), 0, gz_stream, gz_slices.gid, ns,
                            first_run, nv, gz_slices.rank_blocks, per, (uint32_t*)gz_slices.mask, gz_slices.rank_base);
     GZ_LAUNCH_CHECK();
-    gz_slices.parts = (double*)gz_device_malloc((runs + 8) * sizeof(double));
-    gz_slices.outdeg32 = (uint32_t*)gz_device_malloc((nv + 8) * sizeof(uint32_t));
+    gz_slices.parts = (double*)gz_pool_malloc((runs + 8) * sizeof(double), 1);
+    gz_slices.outdeg32 = (uint32_t*)gz_pool_malloc((nv + 8) * sizeof(uint32_t), 1);
     hipLaunchKernelGGL(gz_k_outdeg32, dim3(gz_grid_for(nv)), dim3(GZ_BLOCK), 0, gz_stream, gz_graph.vertex_outdegrees,
                        nv, gz_slices.outdeg32);
     GZ_LAUNCH_CHECK();
     GZ_CHECK(hipStreamSynchronize(gz_stream));
-    gz_device_free(run_vec);
-    gz_device_free(run_first);
-    if (tile_base) gz_device_free(tile_base - (tiles + 1));
-    gz_device_free(firsts);
-    gz_device_free(a);
-    gz_device_free(bb);
+    gz_pool_free(run_vec);
+    gz_pool_free(run_first);
+    if (tile_base) gz_pool_free(tile_base - (tiles + 1));
+    gz_pool_free(firsts);
+    gz_pool_free(a);
+    gz_pool_free(bb);
     gz_slices.base_list = gz_graph.pull_vectors;
     gz_slices.base_count = nvec;
     gz_slices.slice_vertices = S;

@@ -17,6 +17,7 @@
  * of all gathered values; each wavefront writes its share to the partials.
  * No floating-point atomics, so results are reproducible run to run.
  */
+#include "gz_host_internal.h"
 #include "gz_pr_ops.h"
 #include "gz_walk.h"
 
@@ -397,11 +398,11 @@ static uint64_t gz_pr_fixed_vertices = 0;
 
 extern "C" void gz_pr_release(void)
 {
-    gz_device_free(gz_pr_fixed_acc);
+    gz_pool_free(gz_pr_fixed_acc);
     gz_pr_fixed_acc = nullptr;
     gz_pr_fixed_vertices = 0;
     gz_pr_acc_is_fixed = 0;
-    gz_device_free(gz_pr_run_head);
+    gz_pool_free(gz_pr_run_head);
     gz_pr_run_head = nullptr;
     gz_pr_run_head_cap = 0;
 }
@@ -410,8 +411,8 @@ extern "C" void gz_pr_release(void)
 static uint64_t* gz_pr_fixed_reserve(uint64_t num_vertices)
 {
     if (gz_pr_fixed_acc == nullptr || gz_pr_fixed_vertices != num_vertices) {
-        gz_device_free(gz_pr_fixed_acc);
-        gz_pr_fixed_acc = (uint64_t*)gz_device_malloc((num_vertices + 8) * 2 * sizeof(uint64_t));
+        gz_pool_free(gz_pr_fixed_acc);
+        gz_pr_fixed_acc = (uint64_t*)gz_pool_malloc((num_vertices + 8) * 2 * sizeof(uint64_t), 1);
         gz_pr_fixed_vertices = num_vertices;
     }
     return gz_pr_fixed_acc;
@@ -712,8 +713,8 @@ extern "C" void gz_pr_fused_tail(int on) { gz_pr_fused_tail_on = on ? 1 : 0; }
 static uint32_t* gz_pr_run_heads_reserve(uint64_t V)
 {
     if (gz_pr_run_head_cap < V) {
-        gz_device_free(gz_pr_run_head);
-        gz_pr_run_head = (uint32_t*)gz_device_malloc(V * sizeof(uint32_t));
+        gz_pool_free(gz_pr_run_head);
+        gz_pr_run_head = (uint32_t*)gz_pool_malloc(V * sizeof(uint32_t), 1);
         gz_pr_run_head_cap = V;
     }
     return gz_pr_run_head;
@@ -893,7 +894,7 @@ extern "C" int gz_pr_run_persistent(uint64_t iterations, uint64_t* reduce_buffer
     gz_pr_acc_in_slices = 0;
     gz_pr_acc_is_fixed = 0;
     if (gz_pr_bar == nullptr) {
-        gz_pr_bar = (gz_grid_bar_t*)gz_device_malloc(sizeof(gz_grid_bar_t));
+        gz_pr_bar = (gz_grid_bar_t*)gz_pool_malloc(sizeof(gz_grid_bar_t), 1);
         GZ_CHECK(hipHostMalloc((void**)&gz_pr_bar_host, sizeof(uint32_t)));
     }
     GZ_CHECK(hipMemsetAsync(gz_pr_bar, 0, sizeof(gz_grid_bar_t), gz_stream));

@@ -15,6 +15,13 @@
 
 #include <string.h>
 
+#include <atomic>
+#include <map>
+#include <mutex>
+#include <system_error>
+#include <thread>
+#include <unordered_map>
+
 gz_phase_graph_t gz_graph;
 gz_phase_config_t gz_phase_config = {
     0.875,                    /* damping: const_damping_factor, constants.asm:75-79 */
@@ -121,6 +128,99 @@ extern "C" void gz_device_free(void* ptr)
     }
 }
 
+/* ---- pooled device memory ----------------------------------------------------
+ * The library's own buffers (graph arrays, ingress temporaries, scratch).  A
+ * load makes some 40 of them, and hipMalloc and hipFree cost 6 to 120 us each
+ * here (44 of the 140 ms of a sliced R-MAT s22 load with 426 calls, 0.3 of the
+ * 1.3 ms of a 20 K-vertex one), so a freed block is kept for the next request
+ * of about its size.  All of the library's work is on one stream, so a block
+ * handed out again is written only after its last use there; a caller's own
+ * streams are covered by gz_graph_release, which waits for the device.  At most
+ * GZ_POOL_IDLE_MAX bytes are kept idle; a request that the device cannot
+ * satisfy and gz_runtime_shutdown give them back. */
+#define GZ_POOL_IDLE_MAX (8ull << 30)
+
+static struct {
+    std::mutex lock;
+    std::multimap<size_t, void*> idle;         /* by size */
+    std::unordered_map<void*, size_t> in_use;
+    size_t idle_bytes;
+} gz_pool;
+
+/* Sizes are rounded so that requests of about the same size share blocks. */
+static size_t gz_pool_round(size_t bytes)
+{
+    const size_t unit = bytes < (1u << 20) ? 4096 : (size_t)2 << 20;
+    return (bytes + unit - 1) / unit * unit;
+}
+
+static void gz_pool_trim_locked(void)
+{
+    for (auto& b : gz_pool.idle) GZ_CHECK(hipFree(b.second));
+    gz_pool.idle.clear();
+    gz_pool.idle_bytes = 0;
+}
+
+extern "C" void* gz_pool_malloc(size_t bytes, int zero)
+{
+    gz_require_runtime();
+    if (bytes == 0) bytes = 256;
+    const size_t size = gz_pool_round(bytes);
+    void* p = nullptr;
+    {
+        std::lock_guard<std::mutex> hold(gz_pool.lock);
+        ++gz_alloc_generation;
+        /* the smallest idle block that fits, unless it wastes over a quarter */
+        auto b = gz_pool.idle.lower_bound(size);
+        size_t got = size;
+        if (b != gz_pool.idle.end() && b->first <= size + size / 4 + (64u << 10)) {
+            p = b->second;
+            got = b->first;
+            gz_pool.idle_bytes -= got;
+            gz_pool.idle.erase(b);
+        } else {
+            hipError_t err = hipMalloc(&p, size);
+            if (err != hipSuccess && !gz_pool.idle.empty()) {
+                (void)hipGetLastError();
+                gz_pool_trim_locked();
+                err = hipMalloc(&p, size);
+            }
+            if (err != hipSuccess) {
+                fprintf(stderr, "grazelle: device allocation of %zu bytes failed: %s\n", bytes, hipGetErrorString(err));
+                exit(71);
+            }
+        }
+        gz_pool.in_use[p] = got;
+    }
+    if (zero) gz_device_zero(p, bytes);
+    return p;
+}
+
+extern "C" void gz_pool_free(void* ptr)
+{
+    if (ptr == nullptr) return;
+    std::lock_guard<std::mutex> hold(gz_pool.lock);
+    ++gz_alloc_generation;
+    const auto b = gz_pool.in_use.find(ptr);
+    if (b == gz_pool.in_use.end()) {
+        fprintf(stderr, "grazelle: freeing a device block the pool did not hand out\n");
+        exit(71);
+    }
+    const size_t size = b->second;
+    gz_pool.in_use.erase(b);
+    if (gz_pool.idle_bytes + size > GZ_POOL_IDLE_MAX) {
+        GZ_CHECK(hipFree(ptr));
+        return;
+    }
+    gz_pool.idle.emplace(size, ptr);
+    gz_pool.idle_bytes += size;
+}
+
+extern "C" void gz_device_wait(void)
+{
+    if (gz_stream != nullptr) GZ_CHECK(hipDeviceSynchronize());
+}
+
 extern "C" uint64_t gz_device_allocation_events(void) { return gz_alloc_generation; }
 
 /* ---- replay of a captured launch sequence ----------------------------------
@@ -219,10 +319,79 @@ extern "C" int gz_graph_replay_cached(const uint64_t* key, size_t n, void (*enqu
     return gz_graph_replay_cached_slot(0, key, n, enqueue, ctx, times);
 }
 
+/* ---- copies between the device and pageable host memory -----------------------
+ * Given a large pageable buffer, the runtime pins it for the copy: into a
+ * freshly mapped result array that took up to 95 ms for 33 MB here, against
+ * under 1 ms of transfer.  Large copies therefore go through pinned staging
+ * chunks of the library's own, several host threads each moving chunks of
+ * their own through their own buffer, so that transfers, host copies and page
+ * faults overlap.  The buffers (GZ_STAGE_THREADS chunks) are kept until
+ * gz_runtime_shutdown; one large copy runs at a time. */
+#define GZ_STAGE_THREADS 4
+#define GZ_STAGE_CHUNK ((size_t)2 << 20)
+
+static struct {
+    std::mutex lock;
+    void* buf[GZ_STAGE_THREADS];
+    hipEvent_t done[GZ_STAGE_THREADS];
+} gz_stage;
+
+static void gz_stage_chunks(int t, int threads, char* host, char* dev, size_t bytes, bool to_host)
+{
+    GZ_CHECK(hipSetDevice(gz_device_id));
+    const size_t chunks = (bytes + GZ_STAGE_CHUNK - 1) / GZ_STAGE_CHUNK;
+    for (size_t c = (size_t)t; c < chunks; c += (size_t)threads) {
+        const size_t at = c * GZ_STAGE_CHUNK;
+        const size_t n = bytes - at < GZ_STAGE_CHUNK ? bytes - at : GZ_STAGE_CHUNK;
+        if (to_host) {
+            GZ_CHECK(hipMemcpyAsync(gz_stage.buf[t], dev + at, n, hipMemcpyDeviceToHost, gz_stream));
+            GZ_CHECK(hipEventRecord(gz_stage.done[t], gz_stream));
+            GZ_CHECK(hipEventSynchronize(gz_stage.done[t]));
+            memcpy(host + at, gz_stage.buf[t], n);
+        } else {
+            memcpy(gz_stage.buf[t], host + at, n);
+            GZ_CHECK(hipMemcpyAsync(dev + at, gz_stage.buf[t], n, hipMemcpyHostToDevice, gz_stream));
+            GZ_CHECK(hipEventRecord(gz_stage.done[t], gz_stream));
+            GZ_CHECK(hipEventSynchronize(gz_stage.done[t]));
+        }
+    }
+}
+
+static void gz_copy_staged(void* host, void* dev, size_t bytes, bool to_host)
+{
+    std::lock_guard<std::mutex> hold(gz_stage.lock);
+    for (int t = 0; t < GZ_STAGE_THREADS; ++t) {
+        if (gz_stage.buf[t] != nullptr) continue;
+        GZ_CHECK(hipHostMalloc(&gz_stage.buf[t], GZ_STAGE_CHUNK, hipHostMallocDefault));
+        GZ_CHECK(hipEventCreateWithFlags(&gz_stage.done[t], hipEventDisableTiming));
+    }
+    std::thread helpers[GZ_STAGE_THREADS];
+    int threads = 1; /* a helper that cannot start leaves its chunks to fewer threads */
+    const size_t chunks = (bytes + GZ_STAGE_CHUNK - 1) / GZ_STAGE_CHUNK;
+    const int want = chunks < GZ_STAGE_THREADS ? (int)chunks : GZ_STAGE_THREADS;
+    std::atomic<int> go(0); /* the thread count, once it is known */
+    const auto body = [&](int t) {
+        int n;
+        while ((n = go.load(std::memory_order_acquire)) == 0) std::this_thread::yield();
+        gz_stage_chunks(t, n, (char*)host, (char*)dev, bytes, to_host);
+    };
+    try {
+        for (; threads < want; ++threads) helpers[threads] = std::thread(body, threads);
+    } catch (const std::system_error&) {
+    }
+    go.store(threads, std::memory_order_release);
+    body(0);
+    for (int t = 1; t < threads; ++t) helpers[t].join();
+}
+
 extern "C" void gz_copy_to_device(void* dst, const void* src, size_t bytes)
 {
     gz_require_runtime();
     if (bytes == 0) return;
+    if (bytes >= 2 * GZ_STAGE_CHUNK) {
+        gz_copy_staged(const_cast<void*>(src), dst, bytes, false);
+        return;
+    }
     GZ_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, gz_stream));
     GZ_CHECK(hipStreamSynchronize(gz_stream));
 }
@@ -231,6 +400,10 @@ extern "C" void gz_copy_to_host(void* dst, const void* src, size_t bytes)
 {
     gz_require_runtime();
     if (bytes == 0) return;
+    if (bytes >= 2 * GZ_STAGE_CHUNK) {
+        gz_copy_staged(dst, const_cast<void*>(src), bytes, true);
+        return;
+    }
     GZ_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, gz_stream));
     GZ_CHECK(hipStreamSynchronize(gz_stream));
 }
@@ -445,33 +618,33 @@ void gz_scratch_reserve(uint64_t waves, uint64_t num_vertices)
     gz_require_runtime();
     if (waves < (uint64_t)GZ_PERSISTENT_BLOCKS * GZ_WAVES_PER_BLOCK) waves = (uint64_t)GZ_PERSISTENT_BLOCKS * GZ_WAVES_PER_BLOCK;
     if (waves > gz_scratch.partials_capacity) {
-        gz_device_free(gz_scratch.partials);
-        gz_device_free(gz_scratch.stats);
-        gz_device_free(gz_scratch.features);
-        gz_scratch.partials = gz_device_malloc(waves * sizeof(uint64_t));
-        gz_scratch.stats = (uint64_t*)gz_device_malloc(waves * 2 * sizeof(uint64_t));
-        gz_scratch.features = (uint64_t*)gz_device_malloc(waves * 3 * sizeof(uint64_t));
+        gz_pool_free(gz_scratch.partials);
+        gz_pool_free(gz_scratch.stats);
+        gz_pool_free(gz_scratch.features);
+        gz_scratch.partials = gz_pool_malloc(waves * sizeof(uint64_t), 1);
+        gz_scratch.stats = (uint64_t*)gz_pool_malloc(waves * 2 * sizeof(uint64_t), 1);
+        gz_scratch.features = (uint64_t*)gz_pool_malloc(waves * 3 * sizeof(uint64_t), 1);
         gz_scratch.partials_capacity = waves;
     }
-    if (gz_scratch.reduce_tmp == nullptr) gz_scratch.reduce_tmp = (uint64_t*)gz_device_malloc(2048 * sizeof(uint64_t));
+    if (gz_scratch.reduce_tmp == nullptr) gz_scratch.reduce_tmp = (uint64_t*)gz_pool_malloc(2048 * sizeof(uint64_t), 1);
     if (gz_scratch.push_queue == nullptr) {
-        gz_scratch.push_pieces = (uint64_t*)gz_device_malloc((size_t)GZ_PUSH_QUEUE_PIECES * 3 * sizeof(uint64_t));
-        gz_scratch.push_queue = (uint64_t*)gz_device_malloc(2 * sizeof(uint64_t));
+        gz_scratch.push_pieces = (uint64_t*)gz_pool_malloc((size_t)GZ_PUSH_QUEUE_PIECES * 3 * sizeof(uint64_t), 1);
+        gz_scratch.push_queue = (uint64_t*)gz_pool_malloc(2 * sizeof(uint64_t), 1);
         GZ_CHECK(hipMemsetAsync(gz_scratch.push_queue, 0, 2 * sizeof(uint64_t), gz_stream));
         gz_scratch.push_queue_parity = 0;
     }
     if (num_vertices > gz_scratch.scratch_vertices) {
-        gz_device_free(gz_scratch.active_vertices);
-        gz_device_free(gz_scratch.active_prefix);
-        gz_device_free(gz_scratch.bfs_first_vector);
-        gz_scratch.active_vertices = (uint64_t*)gz_device_malloc(num_vertices * sizeof(uint64_t));
-        gz_scratch.active_prefix = (uint64_t*)gz_device_malloc((num_vertices + 1) * sizeof(uint64_t));
-        gz_scratch.bfs_first_vector = (uint64_t*)gz_device_malloc(num_vertices * sizeof(uint64_t));
+        gz_pool_free(gz_scratch.active_vertices);
+        gz_pool_free(gz_scratch.active_prefix);
+        gz_pool_free(gz_scratch.bfs_first_vector);
+        gz_scratch.active_vertices = (uint64_t*)gz_pool_malloc(num_vertices * sizeof(uint64_t), 1);
+        gz_scratch.active_prefix = (uint64_t*)gz_pool_malloc((num_vertices + 1) * sizeof(uint64_t), 1);
+        gz_scratch.bfs_first_vector = (uint64_t*)gz_pool_malloc(num_vertices * sizeof(uint64_t), 1);
         GZ_CHECK(hipMemsetAsync(gz_scratch.bfs_first_vector, 0xff, num_vertices * sizeof(uint64_t), gz_stream));
         const uint64_t blocks = gz_compact_blocks(num_vertices) + 1;
-        gz_device_free(gz_scratch.active_block_sums);
-        gz_scratch.active_block_sums = (uint64_t*)gz_device_malloc((2 * blocks + 8) * sizeof(uint64_t));
-        if (gz_scratch.active_totals == nullptr) gz_scratch.active_totals = (uint64_t*)gz_device_malloc(8 * sizeof(uint64_t));
+        gz_pool_free(gz_scratch.active_block_sums);
+        gz_scratch.active_block_sums = (uint64_t*)gz_pool_malloc((2 * blocks + 8) * sizeof(uint64_t), 1);
+        if (gz_scratch.active_totals == nullptr) gz_scratch.active_totals = (uint64_t*)gz_pool_malloc(8 * sizeof(uint64_t), 1);
         gz_scratch.scratch_vertices = num_vertices;
         gz_scratch.active_capacity = num_vertices;
     }
@@ -484,8 +657,8 @@ extern "C" void gz_merge_buffer_allocate(uint64_t units)
     gz_require_runtime();
     if (units == 0) units = 1;
     if (units > gz_merge_buffer_count) {
-        gz_device_free(gz_merge_buffer);
-        gz_merge_buffer = (mergeaccum_t*)gz_device_malloc(units * sizeof(mergeaccum_t));
+        gz_pool_free(gz_merge_buffer);
+        gz_merge_buffer = (mergeaccum_t*)gz_pool_malloc(units * sizeof(mergeaccum_t), 1);
     }
     gz_merge_buffer_count = units;
     /* graph_data_allocate_merge_buffers initialises every record to ~0 / 0.0 */
@@ -822,21 +995,31 @@ extern "C" void gz_runtime_shutdown(void)
     if (gz_stream == nullptr) return;
     GZ_CHECK(hipStreamSynchronize(gz_stream));
     gz_replay_release();
-    gz_device_free(gz_scratch.partials);
-    gz_device_free(gz_scratch.stats);
-    gz_device_free(gz_scratch.features);
-    gz_device_free(gz_scratch.reduce_tmp);
-    gz_device_free(gz_scratch.active_vertices);
-    gz_device_free(gz_scratch.active_prefix);
-    gz_device_free(gz_scratch.active_block_sums);
-    gz_device_free(gz_scratch.active_totals);
-    gz_device_free(gz_scratch.bfs_first_vector);
-    gz_device_free(gz_scratch.push_pieces);
-    gz_device_free(gz_scratch.push_queue);
-    gz_device_free(gz_merge_buffer);
+    gz_pool_free(gz_scratch.partials);
+    gz_pool_free(gz_scratch.stats);
+    gz_pool_free(gz_scratch.features);
+    gz_pool_free(gz_scratch.reduce_tmp);
+    gz_pool_free(gz_scratch.active_vertices);
+    gz_pool_free(gz_scratch.active_prefix);
+    gz_pool_free(gz_scratch.active_block_sums);
+    gz_pool_free(gz_scratch.active_totals);
+    gz_pool_free(gz_scratch.bfs_first_vector);
+    gz_pool_free(gz_scratch.push_pieces);
+    gz_pool_free(gz_scratch.push_queue);
+    gz_pool_free(gz_merge_buffer);
     gz_merge_buffer = nullptr;
     gz_merge_buffer_count = 0;
     memset(&gz_scratch, 0, sizeof(gz_scratch));
+    {
+        std::lock_guard<std::mutex> hold(gz_pool.lock);
+        gz_pool_trim_locked();
+    }
+    for (int t = 0; t < GZ_STAGE_THREADS; ++t) {
+        if (gz_stage.buf[t] == nullptr) continue;
+        GZ_CHECK(hipHostFree(gz_stage.buf[t]));
+        GZ_CHECK(hipEventDestroy(gz_stage.done[t]));
+        gz_stage.buf[t] = nullptr;
+    }
     if (gz_reduce_mirror != nullptr) GZ_CHECK(hipHostFree(gz_reduce_mirror));
     gz_reduce_mirror = nullptr;
     GZ_CHECK(hipStreamDestroy(gz_stream));

@@ -155,18 +155,18 @@ extern "C" void gz_slices_settings(uint32_t* out3)
 
 extern "C" void gz_source_slices_release(void)
 {
-    gz_device_free(gz_slices.nbr24);
-    gz_device_free(gz_slices.nbr16);
-    gz_device_free(gz_slices.nbr);
-    gz_device_free(gz_slices.shared);
-    gz_device_free(gz_slices.mask);
-    gz_device_free(gz_slices.parts);
-    gz_device_free(gz_slices.rank_base);
-    gz_device_free(gz_slices.outdeg32);
-    gz_device_free(gz_slices.gid);
-    gz_device_free(gz_slices.table);
-    gz_device_free(gz_slices.merge);
-    gz_device_free(gz_slices.counters);
+    gz_pool_free(gz_slices.nbr24);
+    gz_pool_free(gz_slices.nbr16);
+    gz_pool_free(gz_slices.nbr);
+    gz_pool_free(gz_slices.shared);
+    gz_pool_free(gz_slices.mask);
+    gz_pool_free(gz_slices.parts);
+    gz_pool_free(gz_slices.rank_base);
+    gz_pool_free(gz_slices.outdeg32);
+    gz_pool_free(gz_slices.gid);
+    gz_pool_free(gz_slices.table);
+    gz_pool_free(gz_slices.merge);
+    gz_pool_free(gz_slices.counters);
     memset(&gz_slices, 0, sizeof(gz_slices));
 }
 
@@ -272,17 +272,17 @@ static void gz_slices_prepare_table(uint64_t chunk_len)
     uint64_t records = 0;
     for (uint32_t x = 0; x < ns; ++x) records += (vectors[x] + chunk_len - 1) / chunk_len;
     GZ_CHECK(hipStreamSynchronize(gz_stream));
-    gz_device_free(gz_slices.table);
-    gz_device_free(gz_slices.merge);
-    gz_slices.table = (gz_slice_chunk_t*)gz_device_malloc((slots ? slots : 1) * sizeof(gz_slice_chunk_t));
+    gz_pool_free(gz_slices.table);
+    gz_pool_free(gz_slices.merge);
+    gz_slices.table = (gz_slice_chunk_t*)gz_pool_malloc((slots ? slots : 1) * sizeof(gz_slice_chunk_t), 1);
     gz_copy_to_device(gz_slices.table, h, slots * sizeof(gz_slice_chunk_t));
-    gz_slices.merge = (mergeaccum_t*)gz_device_malloc((records ? records : 1) * sizeof(mergeaccum_t));
+    gz_slices.merge = (mergeaccum_t*)gz_pool_malloc((records ? records : 1) * sizeof(mergeaccum_t), 1);
     gz_slices.records = records;
     for (int x = 0; x < GZ_XCDS; ++x) gz_slices.xcd_chunks[x] = 0;
     for (uint64_t i = 0; i < slots; ++i)
         if (h[i].count) gz_slices.xcd_chunks[(i / GZ_WAVES_PER_BLOCK) % GZ_XCDS] += 1;
     if (gz_slices.counters == nullptr)
-        gz_slices.counters = (uint32_t*)gz_device_malloc(GZ_XCDS * GZ_COUNTER_STRIDE * sizeof(uint32_t));
+        gz_slices.counters = (uint32_t*)gz_pool_malloc(GZ_XCDS * GZ_COUNTER_STRIDE * sizeof(uint32_t), 1);
     free(h);
     gz_slices.slots = slots;
     gz_slices.table_chunk_len = chunk_len;

@@ -1,0 +1,69 @@
+"""Loads and read-backs: copies through the staging chunks, the endpoint check
+on the uploaded pairs, and buffers handed out again after a release.
+
+Bars: bytes equal; the same message and exit status for a bad endpoint.
+"""
+import pathlib
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CHUNK = 2 << 20  # a staging chunk; copies of two chunks and more are staged
+
+
+@pytest.mark.parametrize("size", [8, 2 * CHUNK - 1, 2 * CHUNK, 2 * CHUNK + 1, 3 * CHUNK, 5 * CHUNK + 4093])
+def test_copies_at_chunk_edges(gz, device, size):
+    src = np.random.default_rng(size).integers(0, 256, size=size + 1, dtype=np.uint8)[1:]  # odd address
+    dst = np.zeros(size + 9, np.uint8)
+    gz.lib.gz_device_malloc.restype = gz.vp
+    d = gz.vp(gz.lib.gz_device_malloc(gz.C.c_size_t(size)))
+    try:
+        gz.lib.gz_copy_to_device(d, src.ctypes.data_as(gz.vp), gz.C.c_size_t(size))
+        gz.lib.gz_copy_to_host(dst[1:].ctypes.data_as(gz.vp), d, gz.C.c_size_t(size))
+    finally:
+        gz.lib.gz_device_free(d)
+    assert np.array_equal(dst[1 : size + 1], src)
+    assert dst[0] == 0 and not dst[size + 1 :].any()
+
+
+def test_graphs_of_other_sizes_share_buffers(gz, device):
+    # blocks of a released graph serve the next one, also a smaller one
+    def answers(V, seed):
+        pairs = np.random.default_rng(seed).integers(0, V, size=(6 * V, 2), dtype=np.uint64)
+        gz.load_pairs_device(V, pairs, relabel=True)
+        gz.run(gz.options("cc"))
+        labels = gz.cc_labels().copy()
+        gz.run(gz.options("pr", iterations=4))
+        return labels, gz.pr_ranks().copy()
+
+    sizes = [(30011, 1), (29000, 2), (517, 3), (70001, 4), (30011, 1)]
+    first = {}
+    for V, seed in sizes + sizes:
+        got = answers(V, seed)
+        want = first.setdefault((V, seed), got)
+        assert np.array_equal(got[0], want[0])
+        assert np.allclose(got[1], want[1], rtol=1e-12, atol=0)
+    
+
+@pytest.mark.parametrize("at", [0, 1, 2 * 999 + 1])
+def test_bad_endpoint_ends_the_process(gz, device, at):
+    # the bad endpoint with the smallest index is the one named
+    code = f"""
+import sys
+sys.path.insert(0, {str(pathlib.Path(gz.__file__).parent)!r})
+import numpy as np, grazelle as gz
+pairs = np.arange(2000, dtype=np.uint64).reshape(-1, 2) % np.uint64(77)
+words = pairs.reshape(-1)
+words[{at}] = 77
+words[{at} + 1 :: 5] = 999
+gz.load_pairs_device(77, pairs)
+print("loaded")
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 65
+    assert "edge endpoint 77 is not below V = 77" in r.stderr
+    assert "loaded" not in r.stdout
