@@ -306,6 +306,7 @@ typedef struct gz_pr_iteration_t {
     int use_push;
     uint32_t pull_variant;
     int fused_tail; /* merge, sum and vertex phase in one launch (gz_pr_vertex_merged) */
+    int short_tail; /* ... in two (gz_pr_tail_two_launches) */
 } gz_pr_iteration_t;
 
 /* One PageRank iteration's launches, as the loop below makes them. */
@@ -316,6 +317,11 @@ static void gz_pr_enqueue_iteration(void* p)
     if (c->fused_tail) {
         perform_edge_pull_phase_pr(gz_graph.pull_vectors, gz_graph.pull_vector_count);
         gz_pr_vertex_merged(gz_reduce_buffer);
+        return;
+    }
+    if (c->short_tail) {
+        perform_edge_pull_phase_pr(gz_graph.pull_vectors, gz_graph.pull_vector_count);
+        gz_pr_tail_two_launches(gz_reduce_buffer);
         return;
     }
     if (!c->use_push) {
@@ -343,6 +349,7 @@ static size_t gz_pr_iteration_key(const gz_pr_iteration_t* c, uint64_t* k)
     k[n++] = (uint64_t)c->use_push;
     k[n++] = c->pull_variant;
     k[n++] = (uint64_t)c->fused_tail;
+    k[n++] = (uint64_t)c->short_tail;
     k[n++] = damping;
     k[n++] = gz_phase_config.stat_mode;
     k[n++] = gz_phase_config.pull_variant;
@@ -385,6 +392,8 @@ static void gz_run_pr(const gz_run_options_t* o, gz_run_result_t* r)
     /* with few enough chunks, the merge, the sum of S and the vertex phase
      * run as one launch (gz_pr_vertex_merged) */
     const int fused_tail = plain && gz_pr_fused_tail_applies();
+    /* with more, as two */
+    const int short_tail = plain && !fused_tail && gz_pr_short_tail_applies();
     /* every iteration in one launch (gz_pr_run_persistent), when switched on */
     if (plain) {
         const int one = gz_pr_run_persistent(o->iterations, gz_reduce_buffer);
@@ -400,7 +409,7 @@ static void gz_run_pr(const gz_run_options_t* o, gz_run_result_t* r)
     uint64_t ctr;
     for (ctr = 0; ctr < o->iterations; ++ctr) {
         if (replay && ctr == 1) {
-            gz_pr_iteration_t c = {use_push, o->pull_variant, fused_tail};
+            gz_pr_iteration_t c = {use_push, o->pull_variant, fused_tail, short_tail};
             uint64_t key[32];
             const size_t n = gz_pr_iteration_key(&c, key);
             const uint64_t rest = o->iterations - 1;
@@ -418,6 +427,13 @@ static void gz_run_pr(const gz_run_options_t* o, gz_run_result_t* r)
             perform_edge_pull_phase_pr(gz_graph.pull_vectors, gz_graph.pull_vector_count);
             if (ctr == 0) gz_pr_run_heads_build(); /* the first pull's records fix the runs */
             gz_pr_vertex_merged(gz_reduce_buffer);
+            r->pull_iterations += 1;
+            continue;
+        }
+        if (short_tail) {
+            phase_op_reset_global_accum();
+            perform_edge_pull_phase_pr(gz_graph.pull_vectors, gz_graph.pull_vector_count);
+            gz_pr_tail_two_launches(gz_reduce_buffer);
             r->pull_iterations += 1;
             continue;
         }

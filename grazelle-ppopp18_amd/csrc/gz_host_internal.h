@@ -172,6 +172,9 @@ int gz_pr_run_persistent(uint64_t iterations, uint64_t* reduce_buffer);
 int gz_pr_fused_tail_applies(void);
 void gz_pr_run_heads_build(void);
 void gz_pr_vertex_merged(uint64_t* reduce_buffer);
+/* The same in two launches on a longer list. */
+void gz_pr_tail_two_launches(uint64_t* reduce_buffer);
+int gz_pr_short_tail_applies(void);
 void gz_pr_clear_fixed(void);
 /* The source-sliced pull's settings: hot cache, cold spread, cold stream. */
 void gz_slices_settings(uint32_t* out3);

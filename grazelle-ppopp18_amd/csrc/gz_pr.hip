@@ -700,6 +700,59 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_vertex_pr_merged(double* __rest
                                       nv);
 }
 
+/* The tail of an iteration over a longer list in two launches in place of
+ * three: the merge of the records, with the first stage of S's sum in the
+ * first workgroups of the same grid, then the vertex phase, whose workgroups
+ * each do the second stage (at most 1024 slice sums) themselves.  The same
+ * additions in gz_k_reduce's order: bit-identical to gz_k_merge_sum +
+ * gz_k_reduce + gz_k_vertex_pr.  Bound by the vertex phase's streams; the
+ * launch saved is 4.5 us an iteration (1.5 M vertices, 20 iterations: 3510 ->
+ * 3423 us). */
+__global__ __launch_bounds__(GZ_BLOCK) void gz_k_merge_and_slices(const mergeaccum_t* __restrict__ merge,
+                                                                  uint64_t nchunks, double* __restrict__ acc,
+                                                                  const double* __restrict__ partials,
+                                                                  uint32_t reduce_blocks, double* __restrict__ slots)
+{
+    __shared__ double lds[GZ_WAVES_PER_BLOCK];
+    if (blockIdx.x < reduce_blocks) {
+        const uint64_t per = (nchunks + reduce_blocks - 1) / reduce_blocks;
+        const uint64_t lo = (uint64_t)blockIdx.x * per;
+        const uint64_t hi = (lo + per < nchunks) ? lo + per : nchunks;
+        double x = 0.0;
+        for (uint64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) x += partials[i];
+        const double r = gz_block_sum<double>(x, lds);
+        if (threadIdx.x == 0) slots[blockIdx.x] = r;
+        return;
+    }
+    const uint64_t u = (uint64_t)(blockIdx.x - reduce_blocks) * blockDim.x + threadIdx.x;
+    if (u < nchunks) gz_merge_sum_record(merge, nchunks, u, acc);
+}
+
+__global__ __launch_bounds__(GZ_BLOCK) void gz_k_vertex_pr_slices(double* __restrict__ props,
+                                                                  const double* __restrict__ acc,
+                                                                  const double* __restrict__ outdeg,
+                                                                  uint64_t num_vertices,
+                                                                  const double* __restrict__ slots,
+                                                                  uint32_t reduce_blocks,
+                                                                  uint64_t* __restrict__ reduce_buffer, double damping)
+{
+    __shared__ double lds[GZ_WAVES_PER_BLOCK];
+    __shared__ double s_total;
+    double y = 0.0;
+    for (uint32_t i = threadIdx.x; i < reduce_blocks; i += blockDim.x) y += slots[i];
+    const double total = gz_block_sum<double>(y, lds);
+    if (threadIdx.x == 0) s_total = total;
+    __syncthreads();
+    const double S = s_total;
+    if (blockIdx.x == 0 && threadIdx.x == 0) reduce_buffer[0] = (uint64_t)__double_as_longlong(S);
+    const double nv = (double)num_vertices;
+    const double c = (1.0 - S) / nv;
+    const double k = (1.0 - damping) / nv;
+    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < num_vertices;
+         v += (uint64_t)gridDim.x * blockDim.x)
+        props[v] = gz_pr_vertex_value(acc[v], outdeg[v], c, k, damping, nv);
+}
+
 __global__ __launch_bounds__(GZ_BLOCK) void gz_k_pr_clear_u32(uint32_t* __restrict__ p, uint64_t n)
 {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
@@ -730,6 +783,16 @@ extern "C" int gz_pr_fused_tail_applies(void)
     return nchunks <= GZ_PR_FUSED_TAIL_CHUNKS && gz_merge_buffer_count >= nchunks;
 }
 
+/* Every longer list: R-MAT s19 1402 -> 1303 us for 20 iterations, s20 2540 ->
+ * 2432, s22 9474 -> 9390, s24 65450 -> 65330.  (One launch up to 4096 chunks
+ * is faster still, s18 in 760 us.) */
+extern "C" int gz_pr_short_tail_applies(void)
+{
+    const uint64_t nvec = gz_graph.pull_vector_count;
+    return gz_pr_fused_tail_on && gz_graph.pull_vectors != nullptr && nvec != 0 && gz_graph.num_vertices != 0 &&
+           gz_merge_buffer_count >= gz_chunks_for(nvec) && !gz_pr_fused_tail_applies();
+}
+
 extern "C" void gz_pr_run_heads_build(void)
 {
     const uint64_t V = gz_graph.num_vertices, nchunks = gz_chunks_for(gz_graph.pull_vector_count);
@@ -756,6 +819,27 @@ extern "C" void gz_pr_vertex_merged(uint64_t* reduce_buffer)
                        (uint32_t)gz_reduce_blocks(nchunks), gz_pr_run_head, reduce_buffer, gz_phase_config.damping);
     GZ_LAUNCH_CHECK();
     gz_ktimer_end(GZ_K_VERTEX_PR);
+}
+
+/* After a scheduler-aware pull of the loaded graph's pull list. */
+extern "C" void gz_pr_tail_two_launches(uint64_t* reduce_buffer)
+{
+    gz_reduce_mirror_stale();
+    const uint64_t V = gz_graph.num_vertices, nchunks = gz_chunks_for(gz_graph.pull_vector_count);
+    const uint32_t reduce_blocks = (uint32_t)gz_reduce_blocks(nchunks);
+    const uint64_t merge_blocks = (nchunks + GZ_BLOCK - 1) / GZ_BLOCK;
+    double* slots = (double*)gz_scratch.reduce_tmp;
+    hipLaunchKernelGGL(gz_k_merge_and_slices, dim3((unsigned)(reduce_blocks + merge_blocks)), dim3(GZ_BLOCK), 0,
+                       gz_stream, gz_merge_buffer, nchunks, (double*)gz_graph.vertex_accumulators,
+                       (const double*)gz_scratch.partials, reduce_blocks, slots);
+    GZ_LAUNCH_CHECK();
+    uint64_t blocks = (V + GZ_BLOCK - 1) / GZ_BLOCK;
+    if (blocks > 8192) blocks = 8192;
+    hipLaunchKernelGGL(gz_k_vertex_pr_slices, dim3((unsigned)blocks), dim3(GZ_BLOCK), 0, gz_stream,
+                       (double*)gz_graph.vertex_props, (const double*)gz_graph.vertex_accumulators,
+                       gz_graph.vertex_outdegrees, V, (const double*)slots, reduce_blocks, reduce_buffer,
+                       gz_phase_config.damping);
+    GZ_LAUNCH_CHECK();
 }
 
 template <int VPL>

@@ -180,8 +180,8 @@ void gz_pr_graph_replay(int on);
 /* PageRank runs that record nothing per iteration and use the
  * scheduler-aware pull, on a pull list of at most 4096 chunks, run the merge,
  * the sum of S and the vertex phase as one launch after each pull (two
- * launches per iteration instead of four; results bit-identical).  On by
- * default; 0 switches it off. */
+ * launches per iteration instead of four; results bit-identical), and on a
+ * longer list as two.  On by default; 0 switches both off. */
 void gz_pr_fused_tail(int on);
 /* PageRank runs that record nothing per iteration and use the
  * scheduler-aware pull can run all their iterations in one cooperative

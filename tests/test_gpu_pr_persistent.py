@@ -174,3 +174,29 @@ def test_barrier_that_gives_up_restarts_per_phase(gz, orc, device):
     assert np.array_equal(gz.pr_props().view(np.uint64), want)
     # and the next run takes the one-launch path again
     assert np.array_equal(_one_launch(gz, opts), want)
+
+@pytest.mark.parametrize("scale", [16, 17, 18])
+def test_two_launch_tail_equals_per_phase(gz, device, scale):
+    # about 4100, 8200 and 16500 chunks of 64 vectors: one to five slices of
+    # S's first stage; eager, captured and replayed
+    g = gz.rmat_graph(scale, 16, seed=6)
+    try:
+        gz.set_chunk_vectors(64)
+        gz.load(g)
+        for iters in (1, 6, 6, 6, 3):
+            opts = gz.options("pr", iterations=iters, damping=0.85)
+            want = _per_phase(gz, opts)
+            r = gz.run(opts)
+            assert r.iterations == r.pull_iterations == iters
+            assert np.array_equal(gz.pr_props().view(np.uint64), want), (scale, iters)
+    finally:
+        gz.set_chunk_vectors(512)
+
+
+def test_list_without_edges(gz, device):
+    # no pull vectors: neither fused tail runs
+    gz.load_pairs_device(100, np.zeros((0, 2), np.uint64))
+    opts = gz.options("pr", iterations=3, damping=0.85)
+    want = _per_phase(gz, opts)
+    gz.run(opts)
+    assert np.array_equal(gz.pr_props().view(np.uint64), want)
