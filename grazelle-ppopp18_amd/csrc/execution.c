@@ -72,27 +72,28 @@ void gz_execution_prepare(const gz_run_options_t* o)
     gz_phase_config.collect_stats = o->collect_stats;
     gz_graph_reset_roles();
     if (gz_reduce_buffer == NULL) gz_reduce_buffer = gz_reduce_buffer_create();
-    gz_device_zero(gz_reduce_buffer, 8 * sizeof(uint64_t));
     gz_reduce_mirror_stale();
-    if (gz_graph.pull_vectors != NULL) gz_merge_buffer_allocate(gz_pull_units_for(gz_graph.pull_vector_count));
+    if (gz_graph.pull_vectors != NULL) {
+        /* only PageRank and the merge-buffer CC write and read records */
+        const uint64_t units = gz_pull_units_for(gz_graph.pull_vector_count);
+        if (o->algorithm == GZ_ALG_PR || o->pull_variant == GZ_PULL_MERGE_BUFFER)
+            gz_merge_buffer_allocate(units);
+        else
+            gz_merge_buffer_reserve(units);
+    }
 
     switch (o->algorithm) {
     case GZ_ALG_PR:
-        gz_dev_init_pr((double*)gz_graph.vertex_props, (double*)gz_graph.vertex_accumulators,
-                       gz_graph.vertex_outdegrees, V);
+        gz_dev_pr_reset((double*)gz_graph.vertex_props, (double*)gz_graph.vertex_accumulators,
+                        gz_graph.vertex_outdegrees, V, gz_graph.frontier_has_info, gz_graph.frontier_wants_info, fwords,
+                        gz_reduce_buffer);
         gz_pr_clear_fixed();
-        gz_dev_fill_u64(gz_graph.frontier_has_info, ~0ull, fwords);
-        gz_dev_fill_u64(gz_graph.frontier_wants_info, ~0ull, fwords);
         break;
     case GZ_ALG_CC:
         /* labels start at the original ids, also on a renumbered graph */
-        if (gz_graph_original_ids_device() != NULL)
-            gz_device_copy(gz_graph.vertex_props, gz_graph_original_ids_device(), V * sizeof(uint64_t));
-        else
-            gz_dev_iota_u64((uint64_t*)gz_graph.vertex_props, V);
-        gz_dev_fill_u64((uint64_t*)gz_graph.vertex_accumulators, 0, fwords);
-        gz_dev_fill_u64(gz_graph.frontier_has_info, ~0ull, fwords);
-        gz_dev_fill_u64(gz_graph.frontier_wants_info, ~0ull, fwords);
+        gz_dev_cc_reset((uint64_t*)gz_graph.vertex_props, V, gz_graph_original_ids_device(),
+                        (uint64_t*)gz_graph.vertex_accumulators, gz_graph.frontier_has_info,
+                        gz_graph.frontier_wants_info, fwords, gz_reduce_buffer);
         break;
     case GZ_ALG_BFS: {
         if (o->root >= V) {
@@ -102,7 +103,7 @@ void gz_execution_prepare(const gz_run_options_t* o)
         }
         gz_dev_bfs_reset((uint64_t*)gz_graph.vertex_props, V, (uint64_t*)gz_graph.vertex_accumulators,
                          gz_graph.frontier_has_info, gz_graph.frontier_wants_info, fwords, o->root,
-                         gz_graph_device_ids_device(), gz_graph.vertex_outdegrees);
+                         gz_graph_device_ids_device(), gz_graph.vertex_outdegrees, gz_reduce_buffer);
         break;
     }
     default:
@@ -403,8 +404,8 @@ static void gz_run_pr(const gz_run_options_t* o, gz_run_result_t* r)
             return;
         }
         if (one < 0) /* a barrier gave up mid-run: start again from the initial ranks */
-            gz_dev_init_pr((double*)gz_graph.vertex_props, (double*)gz_graph.vertex_accumulators,
-                           gz_graph.vertex_outdegrees, V);
+            gz_dev_pr_reset((double*)gz_graph.vertex_props, (double*)gz_graph.vertex_accumulators,
+                            gz_graph.vertex_outdegrees, V, NULL, NULL, 0, NULL);
     }
     uint64_t ctr;
     for (ctr = 0; ctr < o->iterations; ++ctr) {
@@ -767,12 +768,12 @@ void gz_execution_run(const gz_run_options_t* o, gz_run_result_t* r)
 {
     memset(r, 0, sizeof(*r));
     gz_records_count = 0;
-    gz_synchronize();
+    gz_stream_wait();
     const double t0 = gz_now_ms();
     if (o->algorithm == GZ_ALG_PR)
         gz_run_pr(o, r);
     else
         gz_run_hybrid(o, r);
-    gz_synchronize();
+    gz_stream_wait();
     r->elapsed_ms = gz_now_ms() - t0;
 }

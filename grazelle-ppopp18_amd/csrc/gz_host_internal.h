@@ -54,17 +54,26 @@ void gz_dev_result_bfs(const uint64_t* words, const uint64_t* original, uint64_t
 void gz_dev_vertex_info(const uint64_t* vertices, uint32_t count, const uint32_t* device_ids, const double* outdeg,
                         uint64_t* info);
 
-void gz_dev_init_pr(double* props, double* acc, const double* outdeg, uint64_t n);
+/* The start of a PageRank or CC run in one launch: vertex arrays, frontier
+ * bitmaps of fwords words (0: none) and the reduce buffer (NULL: none). */
+void gz_dev_pr_reset(double* props, double* acc, const double* outdeg, uint64_t n, uint64_t* has, uint64_t* wants,
+                     uint64_t fwords, uint64_t* reduce);
+void gz_dev_cc_reset(uint64_t* labels, uint64_t n, const uint64_t* original, uint64_t* next, uint64_t* has,
+                     uint64_t* wants, uint64_t fwords, uint64_t* reduce);
+/* Waits for the work enqueued so far, at less cost than a stream
+ * synchronisation when it is short (gz_runtime.hip). */
+void gz_stream_wait(void);
+/* gz_merge_buffer_allocate without re-marking the records of a buffer that is
+ * there already. */
+void gz_merge_buffer_reserve(uint64_t units);
 void gz_dev_fill_u64(uint64_t* p, uint64_t value, uint64_t n);
-void gz_dev_iota_u64(uint64_t* p, uint64_t n);
-void gz_dev_store_u64(uint64_t* p, uint64_t index, uint64_t value);
 /* A BFS start from original vertex `root` in one launch: words[0..n)
  * unvisited but the root's (no parent), acc[0..fwords) = 0, has = {root},
  * wants = all but root.  The launch also notes the root's device vertex and
  * out-degree in pinned memory: gz_dev_bfs_start_info, once the stream has
  * drained, gives them for the root of the last start (0 for another root). */
 void gz_dev_bfs_reset(uint64_t* words, uint64_t n, uint64_t* acc, uint64_t* has, uint64_t* wants, uint64_t fwords,
-                      uint64_t root, const uint32_t* device_ids, const double* outdeg);
+                      uint64_t root, const uint32_t* device_ids, const double* outdeg, uint64_t* reduce);
 int gz_dev_bfs_start_info(uint64_t root, uint64_t* device_root, uint64_t* outdeg);
 void gz_dev_bfs_start_forget(void); /* the graph is released */
 void gz_graph_reset_roles(void);

@@ -9,11 +9,25 @@
 #include "gz_internal.h"
 #include "gz_host_internal.h"
 
-__global__ __launch_bounds__(GZ_BLOCK) void gz_k_init_pr(double* __restrict__ props, double* __restrict__ acc,
-                                                         const double* __restrict__ outdeg, uint64_t n)
+/* The start of a run in one launch each: the vertex arrays, the frontier
+ * bitmaps (fwords words each; 0: left alone) and the reduce buffer's eight
+ * words.  Separate fills were four to six launches of 2 us with gaps of 5 us,
+ * 20 of the 370 us of a CC run on R-MAT s16. */
+__device__ __forceinline__ void gz_reset_reduce(uint64_t* __restrict__ reduce)
 {
+    if (reduce != nullptr && blockIdx.x == 0 && threadIdx.x < 8) reduce[threadIdx.x] = 0;
+}
+
+/* PageRank: props = (1/V) / outdeg', accumulators 0, every frontier bit set. */
+__global__ __launch_bounds__(GZ_BLOCK) void gz_k_pr_reset(double* __restrict__ props, double* __restrict__ acc,
+                                                          const double* __restrict__ outdeg, uint64_t n,
+                                                          uint64_t* __restrict__ has, uint64_t* __restrict__ wants,
+                                                          uint64_t fwords, uint64_t* __restrict__ reduce)
+{
+    const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
     const double nv = (double)n;
-    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n + 8; v += (uint64_t)gridDim.x * blockDim.x) {
+    gz_reset_reduce(reduce);
+    for (uint64_t v = first; v < n + 8; v += stride) {
         if (v < n) {
             const double od = outdeg[v];
             props[v] = (1.0 / nv) / (0.0 == od ? nv : od);
@@ -22,6 +36,28 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_init_pr(double* __restrict__ pr
         }
         acc[v] = 0.0;
     }
+    for (uint64_t w = first; w < fwords; w += stride) {
+        has[w] = ~0ull;
+        wants[w] = ~0ull;
+    }
+}
+
+/* CC: each vertex labelled with its original id, HasInfo* clear, every other
+ * frontier bit set. */
+__global__ __launch_bounds__(GZ_BLOCK) void gz_k_cc_reset(uint64_t* __restrict__ labels, uint64_t n,
+                                                          const uint64_t* __restrict__ original,
+                                                          uint64_t* __restrict__ next, uint64_t* __restrict__ has,
+                                                          uint64_t* __restrict__ wants, uint64_t fwords,
+                                                          uint64_t* __restrict__ reduce)
+{
+    const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
+    gz_reset_reduce(reduce);
+    for (uint64_t v = first; v < n; v += stride) labels[v] = original != nullptr ? original[v] : v;
+    for (uint64_t w = first; w < fwords; w += stride) {
+        next[w] = 0;
+        has[w] = ~0ull;
+        wants[w] = ~0ull;
+    }
 }
 
 __global__ __launch_bounds__(GZ_BLOCK) void gz_k_fill(uint64_t* __restrict__ p, uint64_t value, uint64_t n)
@@ -29,14 +65,6 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_fill(uint64_t* __restrict__ p, 
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
         p[i] = value;
 }
-
-__global__ __launch_bounds__(GZ_BLOCK) void gz_k_iota(uint64_t* __restrict__ p, uint64_t n)
-{
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        p[i] = i;
-}
-
-__global__ void gz_k_store(uint64_t* __restrict__ p, uint64_t index, uint64_t value) { p[index] = value; }
 
 /* The start of a BFS from `root` in one launch (execution_bfs.c:106-116 and
  * :70-102): every word unvisited but the root's (no parent), HasInfo* clear,
@@ -48,12 +76,14 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_bfs_reset(uint64_t* __restrict_
                                                            uint64_t original,
                                                            const uint32_t* __restrict__ device_ids,
                                                            const double* __restrict__ outdeg,
-                                                           uint64_t* __restrict__ info)
+                                                           uint64_t* __restrict__ info,
+                                                           uint64_t* __restrict__ reduce)
 {
+    gz_reset_reduce(reduce);
     const uint64_t root = device_ids != nullptr ? (uint64_t)device_ids[original] : original;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        info[0] = root;
-        info[1] = (uint64_t)outdeg[root];
+        __hip_atomic_store(&info[0], root, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&info[1], (uint64_t)outdeg[root], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t i = first; i < n; i += stride) words[i] = (i == root) ? GZ_BFS_PARENT_NONE : GZ_BFS_UNVISITED;
@@ -79,7 +109,7 @@ static uint64_t* gz_bfs_info_dev = nullptr;
 static uint64_t gz_bfs_info_root = ~0ull;
 
 void gz_dev_bfs_reset(uint64_t* words, uint64_t n, uint64_t* acc, uint64_t* has, uint64_t* wants, uint64_t fwords,
-                      uint64_t root, const uint32_t* device_ids, const double* outdeg)
+                      uint64_t root, const uint32_t* device_ids, const double* outdeg, uint64_t* reduce)
 {
     if (gz_bfs_info == nullptr) {
         GZ_CHECK(hipHostMalloc((void**)&gz_bfs_info, 2 * sizeof(uint64_t), hipHostMallocMapped | hipHostMallocCoherent));
@@ -87,7 +117,8 @@ void gz_dev_bfs_reset(uint64_t* words, uint64_t n, uint64_t* acc, uint64_t* has,
     }
     gz_bfs_info_root = root;
     hipLaunchKernelGGL(gz_k_bfs_reset, dim3(gz_blocks_for(n > fwords ? n : fwords)), dim3(GZ_BLOCK), 0, gz_stream, words,
-                       n, acc, has, wants, fwords, root, device_ids, outdeg, gz_bfs_info_dev);
+                       n, acc, has, wants, fwords, root, device_ids, outdeg, gz_bfs_info_dev,
+                       reduce);
     GZ_LAUNCH_CHECK();
 }
 
@@ -101,9 +132,19 @@ int gz_dev_bfs_start_info(uint64_t root, uint64_t* device_root, uint64_t* outdeg
     return 1;
 }
 
-extern "C" void gz_dev_init_pr(double* props, double* acc, const double* outdeg, uint64_t n)
+extern "C" void gz_dev_pr_reset(double* props, double* acc, const double* outdeg, uint64_t n, uint64_t* has,
+                                uint64_t* wants, uint64_t fwords, uint64_t* reduce)
 {
-    hipLaunchKernelGGL(gz_k_init_pr, dim3(gz_blocks_for(n + 8)), dim3(GZ_BLOCK), 0, gz_stream, props, acc, outdeg, n);
+    hipLaunchKernelGGL(gz_k_pr_reset, dim3(gz_blocks_for(n + 8)), dim3(GZ_BLOCK), 0, gz_stream, props, acc, outdeg, n,
+                       has, wants, fwords, reduce);
+    GZ_LAUNCH_CHECK();
+}
+
+extern "C" void gz_dev_cc_reset(uint64_t* labels, uint64_t n, const uint64_t* original, uint64_t* next, uint64_t* has,
+                                uint64_t* wants, uint64_t fwords, uint64_t* reduce)
+{
+    hipLaunchKernelGGL(gz_k_cc_reset, dim3(gz_blocks_for(n > fwords ? n : fwords)), dim3(GZ_BLOCK), 0, gz_stream, labels,
+                       n, original, next, has, wants, fwords, reduce);
     GZ_LAUNCH_CHECK();
 }
 
@@ -111,19 +152,6 @@ extern "C" void gz_dev_fill_u64(uint64_t* p, uint64_t value, uint64_t n)
 {
     if (n == 0) return;
     hipLaunchKernelGGL(gz_k_fill, dim3(gz_blocks_for(n)), dim3(GZ_BLOCK), 0, gz_stream, p, value, n);
-    GZ_LAUNCH_CHECK();
-}
-
-extern "C" void gz_dev_iota_u64(uint64_t* p, uint64_t n)
-{
-    if (n == 0) return;
-    hipLaunchKernelGGL(gz_k_iota, dim3(gz_blocks_for(n)), dim3(GZ_BLOCK), 0, gz_stream, p, n);
-    GZ_LAUNCH_CHECK();
-}
-
-extern "C" void gz_dev_store_u64(uint64_t* p, uint64_t index, uint64_t value)
-{
-    hipLaunchKernelGGL(gz_k_store, dim3(1), dim3(1), 0, gz_stream, p, index, value);
     GZ_LAUNCH_CHECK();
 }
 

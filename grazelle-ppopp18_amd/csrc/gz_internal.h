@@ -259,7 +259,14 @@ void gz_frontier_compact_to(const uint64_t* bitmap, const uint64_t* offsets, uin
  * (gz_mirror_words, after its own writes to rb), so that
  * phase_op_combine_global_var_from_buf(rb) needs no copy; a launcher that
  * writes a reduce buffer otherwise calls gz_reduce_mirror_stale. */
-extern "C" uint64_t* gz_reduce_mirror_target(const uint64_t* reduce_buffer);
+struct gz_mirror_t {
+    uint64_t* words;  /* device address of the copy, GZ_MIRROR_WORDS words */
+    uint64_t ticket;  /* goes to word GZ_MIRROR_TICKET once the copy is written */
+};
+#define GZ_MIRROR_TICKET 8
+#define GZ_MIRROR_DRAIN 9  /* the tickets of gz_stream_wait */
+#define GZ_MIRROR_WORDS 16
+gz_mirror_t gz_reduce_mirror_target(const uint64_t* reduce_buffer);
 extern "C" void gz_reduce_mirror_stale(void);
 
 /* ---- device helpers ------------------------------------------------------- */
@@ -416,12 +423,12 @@ struct gz_feature_acc {
 };
 
 /* Copy the eight reduce-buffer words to the pinned host copy (one thread,
- * after it wrote its own words of `out`); nothing when mirror is null. */
-__device__ __forceinline__ void gz_mirror_words(uint64_t* __restrict__ mirror, const uint64_t* out)
+ * after it wrote its own words of `out`), then the ticket the host polls for. */
+__device__ __forceinline__ void gz_mirror_words(const gz_mirror_t& mirror, const uint64_t* out)
 {
-    if (mirror == nullptr) return;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) mirror[i] = out[i];
+    for (int i = 0; i < 8; ++i) mirror.words[i] = out[i];
+    __hip_atomic_store(&mirror.words[GZ_MIRROR_TICKET], mirror.ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 /* The frontier words at the end of a CC or BFS iteration, done by the

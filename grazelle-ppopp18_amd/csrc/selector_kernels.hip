@@ -224,7 +224,7 @@ __global__ __launch_bounds__(1024) void gz_k_sel_decide(const uint64_t* __restri
                                                             float iteration, float prev_engine, float prev_ms,
                                                             float clock_khz, uint64_t* __restrict__ out,
                                                             int out_from_vote, int with_in,
-                                                            uint64_t* __restrict__ mirror)
+                                                            gz_mirror_t mirror)
 {
     __shared__ uint64_t red[4][1024 / GZ_WAVE];
     __shared__ float x[GZ_SEL_IN], xn[GZ_SEL_IN], h1[GZ_SEL_H], h2[GZ_SEL_H], y[GZ_SEL_OUT];
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(1024) void gz_k_sel_sums(const uint64_t* __restrict
                                                           uint64_t stride, const uint64_t* __restrict__ votes,
                                                           const gz_sel_dev_state* __restrict__ st, float clock_khz,
                                                           int out_from_vote, int with_in, uint64_t* __restrict__ out,
-                                                          uint64_t* __restrict__ mirror, gz_end_words end)
+                                                          gz_mirror_t mirror, gz_end_words end)
 {
     if (blockIdx.x > 0) {
         gz_end_words_do(end);
@@ -554,7 +554,7 @@ extern "C" void gz_sel_dev_step(const uint64_t* frontier, const uint32_t* indeg,
     if (votes != nullptr && gz_phase_config.stat_mode == GZ_STAT_COUNT_AND_OUTDEG) out_from_vote = 1;
     if (votes != nullptr && gz_phase_config.stat_mode == GZ_STAT_OUTDEG_ONLY) out_from_vote = 2;
     const int with_in = indeg != nullptr || source != GZ_SEL_FROM_EDGE_PHASE;
-    uint64_t* mirror = gz_reduce_mirror_target(reduce_buffer);
+    const gz_mirror_t mirror = gz_reduce_mirror_target(reduce_buffer);
     /* timed as the vote reduction it replaces */
     gz_ktimer_begin(GZ_K_REDUCE);
     hipLaunchKernelGGL(gz_k_sel_decide, dim3(1), dim3(1024), 0, gz_stream, feat, blocks, stride, votes, gz_sel_dev_st,
@@ -569,7 +569,7 @@ extern "C" void gz_sel_dev_sums(uint64_t* reduce_buffer, const uint32_t* indeg)
     int out_from_vote = 0;
     if (gz_phase_config.stat_mode == GZ_STAT_COUNT_AND_OUTDEG) out_from_vote = 1;
     if (gz_phase_config.stat_mode == GZ_STAT_OUTDEG_ONLY) out_from_vote = 2;
-    uint64_t* mirror = gz_reduce_mirror_target(reduce_buffer);
+    const gz_mirror_t mirror = gz_reduce_mirror_target(reduce_buffer);
     const gz_end_words end = gz_iteration_end_words(1);
     gz_ktimer_begin(GZ_K_REDUCE);
     hipLaunchKernelGGL(gz_k_sel_sums, dim3(gz_end_blocks(end)), dim3(1024), 0, gz_stream, gz_scratch.features, gz_scratch.partials_count,
