@@ -681,12 +681,12 @@ static void gz_run_hybrid(const gz_run_options_t* o, gz_run_result_t* r)
         memcpy(rec.predicted, sel.predicted, sizeof(rec.predicted));
         gz_phase_config.bfs_level = (uint32_t)ctr;
         float prev_ms = -1.0f;
-        /* a small CC frontier: its push iterations run on the device back to
-         * back (gz_cc_launch_push_tail); the vote comes back with their count */
-        const int tail = !bfs && !use_pull && !features && !o->profile && !o->collect_stats &&
+        /* a small frontier: its push iterations run on the device back to back
+         * (gz_{cc,bfs}_launch_push_tail); the vote comes back with their count */
+        const int tail = !use_pull && !features && !o->profile && !o->collect_stats &&
                          (o->engine == GZ_ENGINE_PUSH || o->engine == GZ_ENGINE_HYBRID ||
                           o->engine == GZ_ENGINE_LEARNED) &&
-                         gz_cc_push_tail_applies(vote);
+                         (bfs ? gz_bfs_push_tail_applies(vote) : gz_cc_push_tail_applies(vote));
         const int fused_end = !features && !tail;
         if (probe) {
             /* the chosen engine runs last, so its result is what continues */
@@ -708,7 +708,10 @@ static void gz_run_hybrid(const gz_run_options_t* o, gz_run_result_t* r)
             if (tail) {
                 const uint64_t cap = o->engine == GZ_ENGINE_PUSH ? ~0ull : threshold;
                 const uint64_t rounds = o->max_iterations ? o->max_iterations - ctr + 1 : ~0ull;
-                gz_cc_launch_push_tail(cap, rounds, gz_reduce_buffer);
+                if (bfs)
+                    gz_bfs_launch_push_tail(ctr == 1 ? device_root : V, cap, rounds, gz_reduce_buffer);
+                else
+                    gz_cc_launch_push_tail(cap, rounds, gz_reduce_buffer);
             } else {
                 gz_push_hint(bfs, use_pull, vote);
                 gz_edge_phase(bfs, use_pull);
@@ -739,7 +742,7 @@ static void gz_run_hybrid(const gz_run_options_t* o, gz_run_result_t* r)
             const uint64_t rounds = gz_reduce_words()[7];
             ctr += rounds - 1;
             r->push_iterations += rounds - 1;
-            gz_cc_tail_rounds += rounds;
+            if (!bfs) gz_cc_tail_rounds += rounds;
         }
         if (host_decides)
             gz_selector_host_step(&sel, &sel_unvisited, &sel_unvisited_in, V, E, (float)(ctr + 1), (float)rec.engine);

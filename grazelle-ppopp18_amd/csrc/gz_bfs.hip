@@ -514,6 +514,221 @@ static void gz_bfs_retire(void)
     GZ_LAUNCH_CHECK();
 }
 
+/* ---- push tail: small-frontier levels in one workgroup -----------------------
+ * A search's first and last levels visit a handful of vertices, and each costs
+ * its launches and the host's read of the vote whatever its size (35 us or
+ * more; no reference counterpart, execution_bfs.c:146-169 returns to the host
+ * after every level).  While the frontier statistic stays at most `vote_cap`
+ * (<= GZ_BFS_TAIL_CAP), gz_k_bfs_push_tail runs these push levels ("rounds")
+ * back to back in one workgroup, with the frontier listed in LDS.
+ *
+ * The words alone say whether an edge (s, d) visits d: unvisited words are all
+ * ones, a word of an earlier level is below this level's key (level << 48 | s),
+ * and one of this level is replaced by a smaller key only, so every source of
+ * the level competes and the smallest one stays, as in gz_k_edge_push_bfs.  The
+ * lane that sees the unvisited word lists the vertex and counts its statistic,
+ * once.  WantsInfo loses each round's vertices as they are listed (nothing here
+ * reads it), and HasInfo* gets the last round's.  (A destination's word is read
+ * plainly: a stale one is an older, larger value and only costs an atomic.)
+ *
+ * A round's list holds targets of the round before's edges, at most that
+ * frontier's out-degrees, which its statistic counts and vote_cap bounds;
+ * activations past the list (a push list that disagrees with the out-degrees)
+ * go to HasInfo* at once and the round is the last.
+ *
+ * The workgroup stops after a round that activates nothing, whose statistic
+ * exceeds vote_cap, or after max_rounds, and leaves what one push level and
+ * its retirement leave, the statistic in out[0] and the rounds in out[7].
+ * Bound by a round's chain of dependent memory steps (offsets, vector, words,
+ * atomic min), about 4 us.  Four searches on R-MAT s17 (two tail launches
+ * each, for the first level and the last two or three): 910 -> 845 us. */
+#define GZ_BFS_TAIL_THREADS 1024
+#define GZ_BFS_TAIL_CAP 16384
+/* Entry bound (as the CC tail's): larger rounds are faster on the whole grid. */
+#define GZ_BFS_TAIL_VOTE 4096
+/* Up to this many vertices the workgroup reads the HasInfo bitmap itself. */
+#define GZ_BFS_TAIL_DIRECT_VERTICES (1ull << 20)
+
+__global__ __launch_bounds__(GZ_BFS_TAIL_THREADS) void gz_k_bfs_push_tail(
+    uint64_t* __restrict__ words, uint64_t* __restrict__ wants_info, uint64_t* __restrict__ next_frontier,
+    const gz_vec_t* __restrict__ vecs, const uint64_t* __restrict__ offsets, const double* __restrict__ outdeg,
+    uint32_t stat_mode, uint64_t level, uint64_t root, uint64_t* __restrict__ first_list,
+    const uint64_t* __restrict__ first_count, const uint64_t* __restrict__ first_bits, uint64_t num_vertices,
+    uint64_t vote_cap, uint64_t max_rounds, uint64_t* __restrict__ out, gz_mirror_t mirror)
+{
+    constexpr uint32_t T = GZ_BFS_TAIL_THREADS;
+    constexpr int kWaves = GZ_BFS_TAIL_THREADS / GZ_WAVE;
+    __shared__ uint32_t lists[2][GZ_BFS_TAIL_CAP];
+    __shared__ uint32_t incl[T];  /* inclusive vector counts of the chunk's sources */
+    __shared__ uint32_t first[T]; /* their first push vector */
+    __shared__ uint32_t srcv[T];  /* the sources */
+    __shared__ uint64_t wave_tot[kWaves];
+    __shared__ uint32_t next_count;
+    __shared__ unsigned long long round_vote;
+    const uint32_t tid = threadIdx.x;
+    const int lane = gz_lane(), wave = (int)(tid / GZ_WAVE);
+    uint64_t n, first_in_lds = GZ_BFS_TAIL_CAP;
+    if (root < num_vertices) {
+        n = 1;
+        if (tid == 0) lists[0][0] = (uint32_t)root;
+    } else if (first_bits != nullptr) {
+        if (tid == 0) next_count = 0;
+        __syncthreads();
+        const uint64_t nwords = (num_vertices + 63) >> 6;
+        for (uint64_t w = tid; w < nwords; w += T) {
+            uint64_t bits = first_bits[w];
+            if (w == nwords - 1 && (num_vertices & 63)) bits &= (1ull << (num_vertices & 63)) - 1;
+            while (bits) {
+                const uint64_t v = (w << 6) + (uint64_t)(__ffsll((unsigned long long)bits) - 1);
+                bits &= bits - 1;
+                if (offsets[v + 1] == offsets[v]) continue;
+                const uint32_t at = atomicAdd(&next_count, 1u);
+                if (at < GZ_BFS_TAIL_CAP)
+                    lists[0][at] = (uint32_t)v;
+                else
+                    first_list[at] = v;
+            }
+        }
+        __syncthreads();
+        n = next_count;
+    } else {
+        n = *first_count;
+        first_in_lds = 0;
+    }
+    __syncthreads();
+    const uint64_t with_count = stat_mode != GZ_STAT_OUTDEG_ONLY ? 1 : 0;
+    uint32_t cur = 0;
+    uint64_t rounds = 0, vote = 0;
+    for (;;) {
+        if (tid == 0) {
+            next_count = 0;
+            round_vote = 0;
+        }
+        __syncthreads();
+        const uint64_t level_key = (level + rounds) << 48;
+        uint64_t my_vote = 0;
+        for (uint64_t base = 0; base < n; base += T) {
+            const uint64_t i = base + tid;
+            uint64_t c = 0, f = 0, v = 0;
+            if (i < n) {
+                v = rounds == 0 && i >= first_in_lds ? first_list[i] : (uint64_t)lists[cur][i];
+                f = offsets[v];
+                c = offsets[v + 1] - f;
+            }
+            const uint64_t wincl = gz_wave_inclusive_sum(c, lane);
+            if (lane == GZ_WAVE - 1) wave_tot[wave] = wincl;
+            __syncthreads();
+            uint64_t before = 0, total = 0;
+            for (int w = 0; w < kWaves; ++w) {
+                const uint64_t x = wave_tot[w];
+                if (w < wave) before += x;
+                total += x;
+            }
+            incl[tid] = (uint32_t)(before + wincl);
+            first[tid] = (uint32_t)f;
+            srcv[tid] = (uint32_t)v;
+            __syncthreads();
+            const uint32_t nsrc = (uint32_t)(n - base < T ? n - base : T);
+            for (uint64_t slot = tid; slot < total; slot += T) {
+                /* the first source whose inclusive count exceeds the slot */
+                uint32_t lo = 0, hi = nsrc - 1;
+                while (lo < hi) {
+                    const uint32_t mid = (lo + hi) >> 1;
+                    if ((uint64_t)incl[mid] > slot)
+                        hi = mid;
+                    else
+                        lo = mid + 1;
+                }
+                const uint64_t excl = lo ? incl[lo - 1] : 0;
+                const gz_lanes vec = gz_load_vector(vecs, (uint64_t)first[lo] + (slot - excl));
+                const uint64_t key = level_key | (uint64_t)srcv[lo];
+                const uint64_t l[4] = {vec.l0, vec.l1, vec.l2, vec.l3};
+                uint64_t g[4], od[4], old[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint64_t d = gz_lane_valid(l[k]) ? gz_lane_id(l[k]) : 0;
+                    g[k] = words[d];
+                    od[k] = (uint64_t)__double_as_longlong(outdeg[d]);
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    old[k] = 0;
+                    if (gz_lane_valid(l[k]) && key < g[k])
+                        old[k] = atomicMin((unsigned long long*)&words[gz_lane_id(l[k])], (unsigned long long)key);
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    if (old[k] != GZ_BFS_UNVISITED) continue;
+                    const uint64_t d = gz_lane_id(l[k]);
+                    my_vote += with_count + (uint64_t)llrint(__longlong_as_double((long long)od[k]));
+                    atomicAnd(reinterpret_cast<unsigned int*>(wants_info) + (d >> 5), ~(1u << (d & 31)));
+                    const uint32_t at = atomicAdd(&next_count, 1u);
+                    if (at < GZ_BFS_TAIL_CAP)
+                        lists[cur ^ 1u][at] = (uint32_t)d;
+                    else
+                        gz_bit_set(next_frontier, d); /* the round is the last */
+                }
+            }
+            __syncthreads(); /* the next chunk rewrites incl, first, srcv, wave_tot */
+        }
+        const uint64_t wv = gz_wave_sum_u64(my_vote);
+        if (lane == 0 && wv) atomicAdd(&round_vote, (unsigned long long)wv);
+        __syncthreads();
+        rounds += 1;
+        vote = round_vote;
+        const uint64_t listed = next_count;
+        cur ^= 1u;
+        n = listed < GZ_BFS_TAIL_CAP ? listed : GZ_BFS_TAIL_CAP;
+        /* an activated vertex may have no out-edges and, with out-degrees alone
+         * in the statistic, add nothing to it: the vote decides, as on the host */
+        if (vote == 0 || vote > vote_cap || listed > GZ_BFS_TAIL_CAP || rounds >= max_rounds) break;
+        __syncthreads(); /* every wavefront has read round_vote and next_count */
+    }
+    for (uint64_t i = tid; i < n; i += T) gz_bit_set(next_frontier, lists[cur][i]);
+    if (tid == 0) {
+        out[0] = vote;
+        out[7] = rounds;
+        gz_mirror_words(mirror, out);
+    }
+}
+
+static uint64_t gz_bfs_tail_vote = GZ_BFS_TAIL_VOTE;
+
+extern "C" void gz_bfs_push_tail(uint64_t max_vote)
+{
+    gz_bfs_tail_vote = max_vote < GZ_BFS_TAIL_CAP ? max_vote : GZ_BFS_TAIL_CAP;
+}
+
+extern "C" int gz_bfs_push_tail_applies(uint64_t vote)
+{
+    return vote <= gz_bfs_tail_vote && gz_bfs_tail_vote > 0 && gz_phase_config.push_frontier_skip &&
+           gz_graph.push_vertex_offsets != nullptr && gz_graph.push_vectors != nullptr &&
+           gz_phase_config.stat_mode != GZ_STAT_COUNT_ONLY && gz_graph.num_vertices > 0 &&
+           gz_graph.num_vertices < (1ull << 32) && gz_graph.push_vector_count < (1ull << 32);
+}
+
+extern "C" void gz_bfs_launch_push_tail(uint64_t root, uint64_t vote_cap, uint64_t max_rounds, uint64_t* reduce_buffer)
+{
+    const uint64_t V = gz_graph.num_vertices;
+    if (vote_cap > gz_bfs_tail_vote) vote_cap = gz_bfs_tail_vote;
+    if (max_rounds == 0) max_rounds = 1;
+    gz_scratch_reserve(0, V);
+    const bool direct = V <= GZ_BFS_TAIL_DIRECT_VERTICES;
+    if (root >= V && !direct)
+        gz_frontier_list(gz_graph.frontier_has_info, gz_graph.push_vertex_offsets, V, gz_graph.push_vector_count);
+    const gz_mirror_t mirror = gz_reduce_mirror_target(reduce_buffer);
+    gz_ktimer_begin(GZ_K_PUSH_BFS);
+    hipLaunchKernelGGL(gz_k_bfs_push_tail, dim3(1), dim3(GZ_BFS_TAIL_THREADS), 0, gz_stream,
+                       (uint64_t*)gz_graph.vertex_props, gz_graph.frontier_wants_info,
+                       (uint64_t*)gz_graph.vertex_accumulators, gz_graph.push_vectors, gz_graph.push_vertex_offsets,
+                       gz_graph.vertex_outdegrees, gz_phase_config.stat_mode, (uint64_t)gz_phase_config.bfs_level, root,
+                       gz_scratch.active_vertices, gz_scratch.active_totals,
+                       direct ? (const uint64_t*)gz_graph.frontier_has_info : (const uint64_t*)nullptr, V, vote_cap,
+                       max_rounds, reduce_buffer, mirror);
+    GZ_LAUNCH_CHECK();
+    gz_ktimer_end(GZ_K_PUSH_BFS);
+}
+
 extern "C" void perform_edge_push_phase_bfs(const gz_vec_t* edge_list, uint64_t edge_list_count)
 {
     const uint64_t chunk_len = 256;

@@ -223,6 +223,13 @@ void gz_cc_graph_replay(int on);
 void gz_cc_push_tail(uint64_t max_vote);
 /* Push iterations run that way since the library was loaded. */
 uint64_t gz_cc_push_tail_rounds(void);
+/* BFS runs that record nothing per iteration, with the fixed threshold or a
+ * forced push, run their push levels over a frontier whose statistic is at
+ * most `max_vote` (clamped to 16384; 0 switches it off) back to back in one
+ * workgroup (default 4096; no reference counterpart, execution_bfs.c:146-169
+ * returns to the host after each level).  Depths and parents are the same;
+ * iterations keep their count, one per level. */
+void gz_bfs_push_tail(uint64_t max_vote);
 /* Graph captures and graph launches made so far (no reference counterpart). */
 void gz_graph_replay_counts(uint64_t* captures, uint64_t* launches);
 

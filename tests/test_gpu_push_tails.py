@@ -1,0 +1,89 @@
+"""BFS push levels over small frontiers run back to back in one workgroup
+(gz_bfs_push_tail) against one launch per level (execution_bfs.c:146-169: the
+host reads the vote after every level).
+
+Bars: depths equal those of the paths, parents bit-exact against the
+per-level launches, as many levels of each engine.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+DEFAULT_TAIL = 4096  # the library's default entry bound
+DIRECT = 1 << 20
+
+
+def _strands(V, lengths, seed):
+    """Disjoint paths over random vertices, the last vertex among them;
+    returns the edges and each path's vertices in order."""
+    rng = np.random.default_rng(seed)
+    ids = rng.choice(V, size=sum(lengths), replace=False).astype(np.uint64)
+    if V - 1 not in ids:
+        ids[-1] = V - 1
+    paths = np.split(ids, np.cumsum(lengths)[:-1])
+    pairs = np.concatenate([np.stack([p[:-1], p[1:]], axis=1) for p in paths])
+    return pairs, paths
+
+
+def _bfs(gz, opts, max_vote):
+    gz.bfs_push_tail(max_vote)
+    try:
+        r = gz.run(opts)
+        parents, depths = gz.bfs_result()
+        return parents.copy(), depths.copy(), r
+    finally:
+        gz.bfs_push_tail(DEFAULT_TAIL)
+
+
+@pytest.mark.parametrize("V", [65, 4097, DIRECT - 1, DIRECT, DIRECT + 1])
+def test_bfs_tail_on_paths(gz, device, V):
+    # every level is one or two vertices wide: the whole search is one launch
+    n = min(V // 3, 400)
+    pairs, paths = _strands(V, [n, n // 2, 2], V + 1)
+    gz.load_pairs_device(V, pairs, symmetrize=True, relabel=True)
+    for p, at in ((paths[0], n // 3), (paths[1], 0), (paths[2], 1)):
+        p = p.astype(np.int64)
+        want = np.full(V, 2**64 - 1, np.uint64)
+        want[p] = np.abs(np.arange(len(p)) - at)
+        for engine in ("push", "hybrid"):
+            for cap in (0, 3, DEFAULT_TAIL):
+                parents, depths, r = _bfs(gz, gz.options("bfs", engine=engine, root=int(p[at])), cap)
+                assert np.array_equal(depths, want), (engine, cap)
+                assert r.pull_iterations + r.push_iterations == r.iterations
+                assert r.iterations == max(at, len(p) - 1 - at) + 1
+                seen = np.nonzero(want != np.uint64(2**64 - 1))[0]
+                up = seen[want[seen] > 0]
+                assert np.all(want[parents[up]] + np.uint64(1) == want[up])
+
+
+@pytest.mark.parametrize("stat", ["both", "outdeg", "count"])
+@pytest.mark.parametrize("scale", [10, 13, 16])
+def test_bfs_tail_equals_per_level(gz, device, scale, stat):
+    # levels that leave the workgroup above the cap and come back below it:
+    # the same depths, the same (smallest) parents among push levels, the
+    # same number of levels
+    gz.load_rmat_device(scale, 16 << scale, 5, relabel=True)
+    deg = gz.outdegrees()[np.argsort(gz.original_ids())]
+    for root in np.random.default_rng(scale).choice(np.nonzero(deg > 0)[0], 4, replace=False):
+        for engine in ("push", "hybrid"):
+            opts = gz.options("bfs", engine=engine, root=int(root), stat=stat)
+            p0, d0, r0 = _bfs(gz, opts, 0)
+            for cap in (16384, DEFAULT_TAIL, 100, 3):
+                p, d, r = _bfs(gz, opts, cap)
+                assert np.array_equal(d, d0), (engine, cap)
+                assert r.iterations == r0.iterations
+                assert (r.pull_iterations, r.push_iterations) == (r0.pull_iterations, r0.push_iterations)
+                if engine == "push":
+                    assert np.array_equal(p, p0), cap
+
+
+@pytest.mark.parametrize("limit", [1, 2, 5, 40])
+def test_bfs_tail_respects_max_iterations(gz, device, limit):
+    V = 200
+    pairs = np.stack([np.arange(V - 1), np.arange(1, V)], axis=1).astype(np.uint64)
+    gz.load_pairs_device(V, pairs, symmetrize=True)
+    _, depths, r = _bfs(gz, gz.options("bfs", engine="push", root=0, max_iterations=limit), DEFAULT_TAIL)
+    assert r.iterations == limit
+    reached = depths != np.uint64(2**64 - 1)
+    assert np.array_equal(reached, np.arange(V) <= limit)
