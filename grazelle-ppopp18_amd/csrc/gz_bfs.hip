@@ -140,9 +140,10 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_push_bfs(const gz_vec_t* _
     }
 }
 
-/* The BFS push's per-edge work for the sparse push: the key (level << 48 |
- * source), the destination's WantsInfo word and its state read ahead, and the
- * atomic min, as in gz_k_edge_push_bfs. */
+/* The BFS push's per-edge work for the sparse push (gz_sparse_push.h): the key
+ * (level << 48 | source), the destination's WantsInfo word and its state read
+ * ahead, and the atomic min; the lane that sees the unvisited word activates
+ * the vertex. */
 struct gz_bfs_push_op {
     const uint64_t* wants_info;
     uint64_t* words;
@@ -157,18 +158,31 @@ struct gz_bfs_push_op {
         g[0] = wants_info[d >> 6];
         g[1] = __hip_atomic_load(&words[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    __device__ __forceinline__ void apply(uint64_t d, uint64_t key, const uint64_t* g, uint64_t& vote,
-                                          gz_feature_acc& feat) const
+    /* words only decrease: a value already <= key means a source no larger
+     * than this one reached d at this level */
+    __device__ __forceinline__ bool tries(uint64_t d, uint64_t key, const uint64_t* g) const
     {
-        if (!((g[0] >> (d & 63)) & 1ull)) return;
-        /* words only decrease: a value already <= key means a source no
-         * larger than this one reached d at this level */
-        if (g[1] <= key) return;
-        const unsigned long long old = atomicMin((unsigned long long*)&words[d], (unsigned long long)key);
-        if (old == GZ_BFS_UNVISITED) {
-            gz_bit_set(next_frontier, d);
-            vote += gz_activate_stat(feat, sink, outdeg, d, stat_mode);
+        return ((g[0] >> (d & 63)) & 1ull) && g[1] > key;
+    }
+    __device__ __forceinline__ uint64_t update(uint64_t d, uint64_t key) const
+    {
+        return atomicMin((unsigned long long*)&words[d], (unsigned long long)key);
+    }
+    __device__ __forceinline__ bool activated(uint64_t old, uint64_t) const { return old == GZ_BFS_UNVISITED; }
+    __device__ __forceinline__ gz_push_stat stat_gather(uint64_t d) const
+    {
+        return gz_push_stat{(sink.out != nullptr || stat_mode != GZ_STAT_COUNT_ONLY) ? outdeg[d] : 0.0,
+                            (sink.out != nullptr && sink.indeg != nullptr) ? sink.indeg[d] : 0u};
+    }
+    __device__ __forceinline__ uint64_t stat(const gz_push_stat& s, gz_feature_acc& feat) const
+    {
+        if (sink.out != nullptr) {
+            feat.count += 1;
+            feat.out_edges += (uint64_t)s.outdeg;
+            feat.in_edges += s.indeg;
         }
+        return (stat_mode != GZ_STAT_OUTDEG_ONLY ? 1 : 0) +
+               (stat_mode != GZ_STAT_COUNT_ONLY ? (uint64_t)llrint(s.outdeg) : 0);
     }
     __device__ __forceinline__ void finish(uint64_t wave, const gz_feature_acc& feat) const
     {

@@ -343,16 +343,19 @@ struct gz_cc_push_op {
     uint32_t stat_mode;
     __device__ __forceinline__ uint64_t message(uint64_t s) const { return labels[s]; }
     __device__ __forceinline__ void gather(uint64_t d, uint64_t* g) const { g[0] = labels[d]; }
-    __device__ __forceinline__ void apply(uint64_t d, uint64_t m, const uint64_t* g, uint64_t& vote,
-                                          gz_feature_acc&) const
+    __device__ __forceinline__ bool tries(uint64_t, uint64_t m, const uint64_t* g) const { return m < g[0]; }
+    __device__ __forceinline__ uint64_t update(uint64_t d, uint64_t m) const
     {
-        if (m < g[0]) {
-            const unsigned long long old = atomicMin((unsigned long long*)&labels[d], (unsigned long long)m);
-            if (old > m) {
-                gz_bit_set(next_frontier, d);
-                vote += gz_frontier_stat(outdeg, d, stat_mode);
-            }
-        }
+        return atomicMin((unsigned long long*)&labels[d], (unsigned long long)m);
+    }
+    __device__ __forceinline__ bool activated(uint64_t old, uint64_t m) const { return old > m; }
+    __device__ __forceinline__ gz_push_stat stat_gather(uint64_t d) const
+    {
+        return gz_push_stat{stat_mode != GZ_STAT_COUNT_ONLY ? outdeg[d] : 0.0, 0u};
+    }
+    __device__ __forceinline__ uint64_t stat(const gz_push_stat& s, gz_feature_acc&) const
+    {
+        return (stat_mode != GZ_STAT_OUTDEG_ONLY ? 1 : 0) + (uint64_t)llrint(s.outdeg);
     }
     __device__ __forceinline__ void finish(uint64_t, const gz_feature_acc&) const {}
 };
