@@ -52,6 +52,7 @@ struct gz_cc_pull_op {
     const double* __restrict__ outdeg;
     uint32_t stat_mode;
     uint64_t vote;
+    uint64_t first_d; /* the chunk's first destination */
     __device__ __forceinline__ uint64_t identity() const { return ~0ull; }
     __device__ __forceinline__ uint64_t combine(uint64_t a, uint64_t b) const { return a < b ? a : b; }
     __device__ __forceinline__ uint64_t gather(const gz_lanes& v, bool in_range, uint32_t& edges) const
@@ -70,7 +71,23 @@ struct gz_cc_pull_op {
         }
         return m;
     }
+    /* A run that starts and ends inside the chunk is its destination's only
+     * one, so no other wavefront writes the label and a store does (at device
+     * scope: other XCDs read the lower label sooner).  The atomic min's round
+     * trip was in every step's chain: the first two sweeps of R-MAT s16 (0.5 M
+     * vectors) took 43 and 39 us, now 33 and 28 with the chunks below. */
     __device__ __forceinline__ void store(uint64_t d, uint64_t m)
+    {
+        if (d == first_d) {
+            store_shared(d, m);
+        } else if (m < labels[d]) {
+            __hip_atomic_store(&labels[d], m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            gz_bit_set(next_frontier, d);
+            vote += gz_frontier_stat(outdeg, d, stat_mode);
+        }
+    }
+    /* the chunk's first and last runs may go on in the neighbouring chunks */
+    __device__ __forceinline__ void store_shared(uint64_t d, uint64_t m)
     {
         gz_cc_apply(labels, next_frontier, outdeg, stat_mode, d, m, vote);
     }
@@ -90,11 +107,11 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_pull_cc(const gz_vec_t* __
     if (chunk >= nchunks) return;
     const uint64_t b = chunk * chunk_len;
     const uint64_t e = (b + chunk_len < nvec) ? b + chunk_len : nvec;
-    gz_cc_pull_op op{labels, next_frontier, outdeg, stat_mode, 0};
-    uint64_t first_d, carry_d, carry_m;
+    gz_cc_pull_op op{labels, next_frontier, outdeg, stat_mode, 0, 0};
+    uint64_t carry_d, carry_m;
     uint32_t edges = 0;
-    gz_walk_chunk<VPL, uint64_t>(vecs, b, e, op, first_d, carry_d, carry_m, edges);
-    if (lane == 0) op.store(carry_d, carry_m);
+    gz_walk_chunk<VPL, uint64_t>(vecs, b, e, op, op.first_d, carry_d, carry_m, edges);
+    if (lane == 0) op.store_shared(carry_d, carry_m);
     const uint64_t total = gz_wave_sum_u64(op.vote);
     if (lane == 0) partials[chunk] = total;
     if (collect) {
@@ -247,23 +264,39 @@ static void gz_pull_cc_merge(const gz_vec_t* edge_list, uint64_t edge_list_count
     gz_ktimer_end(GZ_K_MERGE);
 }
 
+/* Chunk length of the in-place pull: the configured one, halved while the
+ * list gives fewer than GZ_CC_PULL_WAVES wavefronts.  Its units meet in atomic
+ * mins alone (no records), so they may be as short as a step; on a small list
+ * the sweep is the latency of a chunk's chain of steps.  CC on R-MAT s14 109 us
+ * at the configured length, 97 so; s16 with trees 310 and 297.  With 4096
+ * wavefronts more of the runs are shared and the latter takes 325. */
+#define GZ_CC_PULL_WAVES 2048
+static uint64_t gz_cc_pull_chunk(uint64_t nvec)
+{
+    const uint64_t step = (uint64_t)GZ_WAVE * gz_vectors_per_lane();
+    uint64_t len = gz_chunk_len();
+    while (len > step && nvec < len * GZ_CC_PULL_WAVES) len = (len / 2 + step - 1) / step * step;
+    return len;
+}
+
 extern "C" void perform_edge_pull_phase_cc(const gz_vec_t* edge_list, uint64_t edge_list_count)
 {
     if (gz_phase_config.pull_variant == GZ_PULL_SOURCE_SLICED && edge_list_count > 0) {
         gz_pull_cc_sliced(edge_list, edge_list_count);
         return;
     }
-    const uint64_t nchunks = gz_chunks_for(edge_list_count);
+    const bool merged = gz_phase_config.pull_variant == GZ_PULL_MERGE_BUFFER;
+    const uint64_t chunk_len = merged ? gz_chunk_len() : gz_cc_pull_chunk(edge_list_count);
+    const uint64_t nchunks = (edge_list_count + chunk_len - 1) / chunk_len;
     gz_scratch_reserve(nchunks, gz_graph.num_vertices);
     gz_scratch.partials_is_double = 0;
     gz_scratch.partials_count = nchunks;
     gz_scratch.stats_count = gz_phase_config.collect_stats ? nchunks : 0;
     if (nchunks == 0) return;
-    if (gz_phase_config.pull_variant == GZ_PULL_MERGE_BUFFER) {
+    if (merged) {
         gz_pull_cc_merge(edge_list, edge_list_count);
         return;
     }
-    const uint64_t chunk_len = gz_chunk_len();
     const uint64_t blocks = (nchunks + GZ_WAVES_PER_BLOCK - 1) / GZ_WAVES_PER_BLOCK;
     const uint32_t vpl = gz_vectors_per_lane();
 #define GZ_PULL_CC_ARGS                                                                                       \
@@ -717,7 +750,7 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_pull_cc_loop(const gz_vec_
 {
     if (gz_guard_off(guard)) return;
     const uint64_t gw = (uint64_t)blockIdx.x * GZ_WAVES_PER_BLOCK + (threadIdx.x / GZ_WAVE);
-    gz_cc_pull_op op{labels, next_frontier, outdeg, stat_mode, 0};
+    gz_cc_pull_op op{labels, next_frontier, outdeg, stat_mode, 0, 0};
     while (true) {
         uint64_t chunk = 0;
         if (gz_lane() == 0) chunk = atomicAdd((unsigned long long*)counter, 1ull);
@@ -725,10 +758,10 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_pull_cc_loop(const gz_vec_
         if (chunk >= nchunks) break;
         const uint64_t b = chunk * chunk_len;
         const uint64_t e = (b + chunk_len < nvec) ? b + chunk_len : nvec;
-        uint64_t first_d, carry_d, carry_m;
+        uint64_t carry_d, carry_m;
         uint32_t edges = 0;
-        gz_walk_chunk<VPL, uint64_t>(vecs, b, e, op, first_d, carry_d, carry_m, edges);
-        if (gz_lane() == 0) op.store(carry_d, carry_m);
+        gz_walk_chunk<VPL, uint64_t>(vecs, b, e, op, op.first_d, carry_d, carry_m, edges);
+        if (gz_lane() == 0) op.store_shared(carry_d, carry_m);
     }
     const uint64_t total = gz_wave_sum_u64(op.vote);
     if (gz_lane() == 0) partials[gw] = total;

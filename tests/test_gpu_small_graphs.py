@@ -117,3 +117,36 @@ def test_iteration_end_past_one_workgroup_sum(gz, orc, device):
     finally:
         gz.set_chunk_vectors(512)
     assert np.array_equal(got, orc.cc(orc.Graph(g.num_vertices, g.pull, g.push), orc.options(threads=8))[0])
+
+
+@pytest.mark.parametrize("vpl", [1, 2, 4])
+@pytest.mark.parametrize("edges", [3, 255, 256, 257, 4095, 70000, 1200000])
+def test_cc_pull_runs_across_chunks(gz, device, edges, vpl):
+    # one destination over many chunks, destinations of one vector, and chunk
+    # lengths from a step to the configured one (about 2048 wavefronts at
+    # 131072 vectors): a label written by the wrong unit would stay too high
+    rng = np.random.default_rng(edges + vpl)
+    V = max(4, edges // 2)
+    hubs = rng.choice(V, size=2, replace=False)
+    half = edges // 2
+    src = np.concatenate([rng.integers(0, V, size=half), rng.integers(0, V, size=edges - half)])
+    dst = np.concatenate([hubs[rng.integers(0, 2, size=half)], rng.integers(0, V, size=edges - half)])
+    pairs = np.stack([src, dst], axis=1).astype(np.uint64)
+    want = np.arange(V)
+    while True:  # smallest id of each component, by sweeps
+        low = np.minimum(want[src], want[dst])
+        new = want.copy()
+        np.minimum.at(new, src, low)
+        np.minimum.at(new, dst, low)
+        new = new[new]
+        if np.array_equal(new, want):
+            break
+        want = new
+    gz.set_vectors_per_lane(vpl)
+    try:
+        gz.load_pairs_device(V, pairs, symmetrize=True)
+        for engine in ("pull", "hybrid"):
+            gz.run(gz.options("cc", engine=engine))
+            assert np.array_equal(gz.cc_labels(), want.astype(np.uint64)), engine
+    finally:
+        gz.set_vectors_per_lane(1)
