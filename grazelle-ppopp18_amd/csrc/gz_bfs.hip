@@ -145,6 +145,7 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_push_bfs(const gz_vec_t* _
  * ahead, and the atomic min; the lane that sees the unvisited word activates
  * the vertex. */
 struct gz_bfs_push_op {
+    static constexpr bool kInPlace = false;
     const uint64_t* wants_info;
     uint64_t* words;
     uint64_t* next_frontier;
@@ -751,7 +752,7 @@ extern "C" void perform_edge_push_phase_bfs(const gz_vec_t* edge_list, uint64_t 
     gz_scratch_reserve(0, gz_graph.num_vertices);
     if (gz_push_sparse_eligible(hint)) {
         /* reserve first: the feature sink points into the per-wave scratch */
-        gz_scratch_reserve(gz_push_sparse_waves(hint), gz_graph.num_vertices);
+        gz_scratch_reserve(gz_push_sparse_waves(hint, gz_bfs_push_op::kInPlace), gz_graph.num_vertices);
         const gz_bfs_push_op op{gz_graph.frontier_wants_info,
                                 (uint64_t*)gz_graph.vertex_props,
                                 (uint64_t*)gz_graph.vertex_accumulators,

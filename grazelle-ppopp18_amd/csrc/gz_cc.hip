@@ -370,6 +370,7 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_push_cc(const gz_vec_t* __
 /* The CC push's per-edge work for the sparse push (gz_sparse_push.h): the
  * source's label, the destination's label read ahead, and the atomic min. */
 struct gz_cc_push_op {
+    static constexpr bool kInPlace = true;
     uint64_t* labels;
     uint64_t* next_frontier;
     const double* outdeg;

@@ -19,6 +19,7 @@
  *  - gz_k_push_pieces: wavefront gw pushes pieces gw, gw + W, ... of the queue.
  *
  * The per-edge work is the Op's (one struct per algorithm):
+ *   kInPlace                                the message may change during the push;
  *   uint64_t message(uint64_t s)            the source's message, per vector;
  *   void gather(uint64_t d, uint64_t g[2])  reads for edge (s, d), issued for a
  *                                           whole batch before any update;
@@ -321,12 +322,18 @@ static inline bool gz_push_sparse_eligible(uint64_t hint)
  * wavefront that holds the most sources, so at most 16 and the overflow
  * queue.  On a small graph those widths leave most SIMDs idle (64 wavefronts
  * of 16 words at 2^16 vertices, each with a chain of several rounds), so the
- * width shrinks by four until there are GZ_SPARSE_PUSH_MIN_WAVES wavefronts. */
-static inline uint64_t gz_push_sparse_words(uint64_t hint)
+ * width shrinks by four until there are GZ_SPARSE_PUSH_MIN_WAVES wavefronts.
+ * Below 2^16 vertices a push in place (CC) keeps four words: its wavefront's
+ * rounds pass labels on within an iteration, so paths take fewer iterations
+ * on the whole grid (a 200-vertex path before a star of 20,000: 40 of its 202
+ * iterations in the one-workgroup tail instead of one or none), and one word
+ * is no faster there (R-MAT s14 98 and 100 us). */
+static inline uint64_t gz_push_sparse_words(uint64_t hint, bool in_place)
 {
     const uint64_t nwords = (gz_graph.num_vertices + 63) >> 6;
     uint64_t words = hint <= GZ_SPARSE_PUSH_WIDE_VOTE ? 64 : 16;
-    while (words > 1 && nwords < words * GZ_SPARSE_PUSH_MIN_WAVES) words /= 4;
+    const uint64_t least = in_place && nwords < 1024 ? 4 : 1;
+    while (words > least && nwords < words * GZ_SPARSE_PUSH_MIN_WAVES) words /= 4;
     return words;
 }
 
@@ -334,9 +341,9 @@ static inline uint64_t gz_push_sparse_words(uint64_t hint)
 static inline bool gz_push_sparse_queued(uint64_t hint) { return hint > GZ_SPARSE_PUSH_WIDE_VOTE; }
 
 /* Per-wave partials the sparse push writes for a vote of `hint`. */
-static inline uint64_t gz_push_sparse_waves(uint64_t hint)
+static inline uint64_t gz_push_sparse_waves(uint64_t hint, bool in_place)
 {
-    const uint64_t words = gz_push_sparse_words(hint);
+    const uint64_t words = gz_push_sparse_words(hint, in_place);
     const uint64_t waves = (((gz_graph.num_vertices + 63) >> 6) + words - 1) / words;
     const uint64_t blocks = (waves + GZ_WAVES_PER_BLOCK - 1) / GZ_WAVES_PER_BLOCK;
     const uint64_t qblocks = gz_push_sparse_queued(hint) ? GZ_PERSISTENT_BLOCKS / 4 : 0;
@@ -353,7 +360,7 @@ template <class Op>
 static void gz_launch_push_sparse(const Op& op, const gz_vec_t* edge_list, uint64_t hint, uint64_t* stamp)
 {
     const uint64_t V = gz_graph.num_vertices;
-    const uint64_t words = gz_push_sparse_words(hint);
+    const uint64_t words = gz_push_sparse_words(hint, Op::kInPlace);
     const bool queued = gz_push_sparse_queued(hint);
     const uint64_t waves = (((V + 63) >> 6) + words - 1) / words;
     const uint64_t blocks = (waves + GZ_WAVES_PER_BLOCK - 1) / GZ_WAVES_PER_BLOCK;
