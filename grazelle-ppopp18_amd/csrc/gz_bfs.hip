@@ -76,9 +76,42 @@ __device__ __forceinline__ bool gz_vec_has_frontier_source(const gz_lanes& v, co
     return q;
 }
 
+/* gz_activate_stat in two steps: the reads, and the sums. */
+__device__ __forceinline__ gz_push_stat gz_bfs_stat_gather(const double* __restrict__ outdeg,
+                                                           const gz_feature_sink& sink, uint32_t stat_mode, uint64_t d)
+{
+    return gz_push_stat{(sink.out != nullptr || stat_mode != GZ_STAT_COUNT_ONLY) ? outdeg[d] : 0.0,
+                        (sink.out != nullptr && sink.indeg != nullptr) ? sink.indeg[d] : 0u};
+}
+
+__device__ __forceinline__ uint64_t gz_bfs_stat(const gz_push_stat& s, const gz_feature_sink& sink, uint32_t stat_mode,
+                                                gz_feature_acc& feat)
+{
+    if (sink.out != nullptr) {
+        feat.count += 1;
+        feat.out_edges += (uint64_t)s.outdeg;
+        feat.in_edges += s.indeg;
+    }
+    return (stat_mode != GZ_STAT_OUTDEG_ONLY ? 1 : 0) +
+           (stat_mode != GZ_STAT_COUNT_ONLY ? (uint64_t)llrint(s.outdeg) : 0);
+}
+
+/* The push over any frontier, slots [from, to) of GZ_BFS_PUSH_SLICES equal
+ * slices of its sources' vectors.  A large frontier is pushed in parts, and
+ * the vertices that a part visits leave WantsInfo before the next one: later
+ * sources are larger, so their edges to those vertices change nothing and stop
+ * at the bitmap, which stays in L2, instead of reading the vertex's word, a
+ * line from beyond it.  A level of 38.6 M edges on R-MAT s24 (134 MB of words)
+ * is bound by those lines: 965 us edge by edge, 868 with a vector's accesses
+ * issued together, 670 in three parts (four, from a sixteenth: 682; six: 706).
+ * Below a sixteenth of the edges most late levels find few vertices to visit
+ * and the parts' launches cost as much as they save. */
+#define GZ_BFS_PUSH_SLICES 16
+#define GZ_BFS_PUSH_PARTED_VERTICES (1ull << 20)
+
 template <bool kActive>
 __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_push_bfs(const gz_vec_t* __restrict__ vecs, gz_slot_source src,
-                                                               uint64_t chunk_len,
+                                                               uint64_t chunk_len, uint32_t from, uint32_t to,
                                                                const uint64_t* __restrict__ has_info,
                                                                uint64_t* __restrict__ wants_info,
                                                                uint64_t* __restrict__ words,
@@ -91,12 +124,13 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_push_bfs(const gz_vec_t* _
     const int lane = gz_lane();
     const uint64_t gw = (uint64_t)blockIdx.x * GZ_WAVES_PER_BLOCK + (threadIdx.x / GZ_WAVE);
     const uint64_t W = (uint64_t)gridDim.x * GZ_WAVES_PER_BLOCK;
-    const uint64_t T = gz_slot_total<kActive>(src);
+    const uint64_t all = gz_slot_total<kActive>(src);
+    const uint64_t first = all * from / GZ_BFS_PUSH_SLICES, T = all * to / GZ_BFS_PUSH_SLICES;
     uint64_t vote = 0;
     gz_feature_acc feat{0, 0, 0};
     uint32_t vectors = 0, edges = 0;
-    for (uint64_t chunk = gw; chunk * chunk_len < T; chunk += W) {
-        const uint64_t j0 = chunk * chunk_len;
+    for (uint64_t chunk = gw; first + chunk * chunk_len < T; chunk += W) {
+        const uint64_t j0 = first + chunk * chunk_len;
         const uint64_t jend = (j0 + chunk_len < T) ? j0 + chunk_len : T;
         uint64_t a = gz_slot_begin<kActive>(src, j0);
         for (uint64_t base = j0; base < jend; base += GZ_WAVE) {
@@ -110,22 +144,42 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_push_bfs(const gz_vec_t* _
             vectors += 1;
             const unsigned long long key = ((unsigned long long)level << 48) | (unsigned long long)s;
             const uint64_t l[4] = {v.l0, v.l1, v.l2, v.l3};
+            /* each kind of access for the four edges before any result is
+             * used: the WantsInfo words, the states, the updates, the degrees */
+            uint32_t wants[4];
+            uint64_t state[4], old[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                if (!gz_lane_valid(l[k])) continue;
-                edges += 1;
+                const uint64_t d = gz_lane_valid(l[k]) ? gz_lane_id(l[k]) : 0;
+                wants[k] = reinterpret_cast<const uint32_t*>(wants_info)[d >> 5];
+                edges += gz_lane_valid(l[k]) ? 1u : 0u;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
                 const uint64_t d = gz_lane_id(l[k]);
-                if (!gz_bit_test(wants_info, d)) continue;
+                state[k] = 0;
+                if (gz_lane_valid(l[k]) && ((wants[k] >> (d & 31)) & 1u))
+                    state[k] = __hip_atomic_load(&words[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
                 /* words only decrease: a value already <= key means a source
                  * no larger than s reached d at this level, and the atomic
                  * would change nothing */
-                if (__hip_atomic_load(&words[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <= key) continue;
-                const unsigned long long old = atomicMin((unsigned long long*)&words[d], key);
-                if (old == GZ_BFS_UNVISITED) {
-                    gz_bit_set(next_frontier, d);
-                    vote += gz_activate_stat(feat, sink, outdeg, d, stat_mode);
-                }
+                old[k] = 0;
+                if (state[k] > key) old[k] = atomicMin((unsigned long long*)&words[gz_lane_id(l[k])], key);
             }
+            gz_push_stat st[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                st[k] = gz_push_stat{0.0, 0u};
+                if (old[k] != GZ_BFS_UNVISITED) continue;
+                st[k] = gz_bfs_stat_gather(outdeg, sink, stat_mode, gz_lane_id(l[k]));
+                gz_bit_set(next_frontier, gz_lane_id(l[k]));
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (old[k] == GZ_BFS_UNVISITED) vote += gz_bfs_stat(st[k], sink, stat_mode, feat);
         }
     }
     const uint64_t total = gz_wave_sum_u64(vote);
@@ -172,18 +226,11 @@ struct gz_bfs_push_op {
     __device__ __forceinline__ bool activated(uint64_t old, uint64_t) const { return old == GZ_BFS_UNVISITED; }
     __device__ __forceinline__ gz_push_stat stat_gather(uint64_t d) const
     {
-        return gz_push_stat{(sink.out != nullptr || stat_mode != GZ_STAT_COUNT_ONLY) ? outdeg[d] : 0.0,
-                            (sink.out != nullptr && sink.indeg != nullptr) ? sink.indeg[d] : 0u};
+        return gz_bfs_stat_gather(outdeg, sink, stat_mode, d);
     }
     __device__ __forceinline__ uint64_t stat(const gz_push_stat& s, gz_feature_acc& feat) const
     {
-        if (sink.out != nullptr) {
-            feat.count += 1;
-            feat.out_edges += (uint64_t)s.outdeg;
-            feat.in_edges += s.indeg;
-        }
-        return (stat_mode != GZ_STAT_OUTDEG_ONLY ? 1 : 0) +
-               (stat_mode != GZ_STAT_COUNT_ONLY ? (uint64_t)llrint(s.outdeg) : 0);
+        return gz_bfs_stat(s, sink, stat_mode, feat);
     }
     __device__ __forceinline__ void finish(uint64_t wave, const gz_feature_acc& feat) const
     {
@@ -515,18 +562,22 @@ extern "C" int gz_bfs_take_deferred_retire(void)
     return due;
 }
 
-static void gz_bfs_retire(void)
+static void gz_bfs_retire_now(void)
 {
-    if (gz_bfs_retire_deferred) {
-        gz_bfs_retire_due = 1;
-        return;
-    }
     const uint64_t words = (gz_graph.num_vertices + 63) / 64;
     uint64_t rblocks = (words + GZ_BLOCK - 1) / GZ_BLOCK;
     if (rblocks > 4096) rblocks = 4096;
     hipLaunchKernelGGL(gz_k_bfs_retire_wants, dim3((unsigned)rblocks), dim3(GZ_BLOCK), 0, gz_stream,
                        gz_graph.frontier_wants_info, (const uint64_t*)gz_graph.vertex_accumulators, words);
     GZ_LAUNCH_CHECK();
+}
+
+static void gz_bfs_retire(void)
+{
+    if (gz_bfs_retire_deferred)
+        gz_bfs_retire_due = 1;
+    else
+        gz_bfs_retire_now();
 }
 
 /* ---- push tail: small-frontier levels in one workgroup -----------------------
@@ -781,23 +832,38 @@ extern "C" void perform_edge_push_phase_bfs(const gz_vec_t* edge_list, uint64_t 
         if (blocks == 0) blocks = 1;
     }
     const uint64_t waves = blocks * GZ_WAVES_PER_BLOCK;
-    gz_scratch_reserve(waves, gz_graph.num_vertices);
+    /* parts for at least a sixteenth of the edges (up to four a vector), and
+     * for words that outgrow one XCD's 4 MB of L2: on R-MAT s17, 1 MB of
+     * words, the parts' launches cost 15 us of 42 */
+    static const uint32_t cuts[] = {0, 2, 6, GZ_BFS_PUSH_SLICES};
+    const bool parted = active && hint != ~0ull && hint >= edge_list_count / 4 &&
+                        gz_graph.num_vertices >= GZ_BFS_PUSH_PARTED_VERTICES;
+    const int parts = parted ? 3 : 1;
+    gz_scratch_reserve(waves * parts, gz_graph.num_vertices);
     gz_scratch.partials_is_double = 0;
-    gz_scratch.partials_count = waves;
-    gz_scratch.stats_count = gz_phase_config.collect_stats ? waves : 0;
+    gz_scratch.partials_count = waves * parts;
+    gz_scratch.stats_count = gz_phase_config.collect_stats ? waves * parts : 0;
     const uint64_t level = gz_phase_config.bfs_level;
     const gz_feature_sink sink{gz_scratch.features_on ? gz_scratch.features : nullptr, gz_scratch.features_indeg,
                                  gz_scratch.partials_capacity};
     gz_ktimer_begin(GZ_K_PUSH_BFS);
-    if (active)
-        hipLaunchKernelGGL(gz_k_edge_push_bfs<true>, dim3((unsigned)blocks), dim3(GZ_BLOCK), 0, gz_stream, edge_list,
-                           src, chunk_len, gz_graph.frontier_has_info, gz_graph.frontier_wants_info,
-                           (uint64_t*)gz_graph.vertex_props, (uint64_t*)gz_graph.vertex_accumulators,
-                           gz_graph.vertex_outdegrees, gz_phase_config.stat_mode, level,
-                           (uint64_t*)gz_scratch.partials, gz_scratch.stats, gz_phase_config.collect_stats, sink);
+    if (active) {
+        for (int p = 0; p < parts; ++p) {
+            const gz_feature_sink psink{sink.out ? sink.out + waves * p : nullptr, sink.indeg, sink.stride};
+            if (p > 0) gz_bfs_retire_now();
+            hipLaunchKernelGGL(gz_k_edge_push_bfs<true>, dim3((unsigned)blocks), dim3(GZ_BLOCK), 0, gz_stream, edge_list,
+                               src, parted ? chunk_len / 2 : chunk_len, parted ? cuts[p] : 0u,
+                               parted ? cuts[p + 1] : (uint32_t)GZ_BFS_PUSH_SLICES, gz_graph.frontier_has_info,
+                               gz_graph.frontier_wants_info, (uint64_t*)gz_graph.vertex_props,
+                               (uint64_t*)gz_graph.vertex_accumulators, gz_graph.vertex_outdegrees,
+                               gz_phase_config.stat_mode, level, (uint64_t*)gz_scratch.partials + waves * p,
+                               gz_scratch.stats + 2 * waves * p, gz_phase_config.collect_stats, psink);
+            GZ_LAUNCH_CHECK();
+        }
+    }
     else
         hipLaunchKernelGGL(gz_k_edge_push_bfs<false>, dim3((unsigned)blocks), dim3(GZ_BLOCK), 0, gz_stream, edge_list,
-                           src, chunk_len, gz_graph.frontier_has_info, gz_graph.frontier_wants_info,
+                           src, chunk_len, 0u, (uint32_t)GZ_BFS_PUSH_SLICES, gz_graph.frontier_has_info, gz_graph.frontier_wants_info,
                            (uint64_t*)gz_graph.vertex_props, (uint64_t*)gz_graph.vertex_accumulators,
                            gz_graph.vertex_outdegrees, gz_phase_config.stat_mode, level,
                            (uint64_t*)gz_scratch.partials, gz_scratch.stats, gz_phase_config.collect_stats, sink);

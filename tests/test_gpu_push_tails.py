@@ -87,3 +87,32 @@ def test_bfs_tail_respects_max_iterations(gz, device, limit):
     assert r.iterations == limit
     reached = depths != np.uint64(2**64 - 1)
     assert np.array_equal(reached, np.arange(V) <= limit)
+
+
+@pytest.mark.parametrize("V", [1 << 16, (1 << 20) - 1, 1 << 20, (1 << 20) + 77])
+def test_bfs_push_in_parts_keeps_smallest_parents(gz, device, V):
+    # from 2^20 vertices, levels of at least a sixteenth of the edges are
+    # pushed in parts: every parent is the smallest in-neighbour one level up
+    pairs = np.random.default_rng(V).integers(0, V, size=(5 * V, 2), dtype=np.uint64)
+    pairs[:, 0] = pairs[:, 0] * pairs[:, 0] // np.uint64(V)  # skewed towards low ids
+    gz.load_pairs_device(V, pairs)
+    src, dst = pairs[:, 0].astype(np.int64), pairs[:, 1].astype(np.int64)
+    for root in (int(src[0]), int(src[-1])):
+        for stat in ("both", "outdeg"):
+            gz.run(gz.options("bfs", engine="push", root=root, stat=stat))
+            parents, depths = gz.bfs_result()
+            depth = np.full(V, -1, np.int64)
+            depth[root], level = 0, 0
+            want = np.full(V, V, np.int64)
+            while True:
+                hit = (depth[src] == level) & ((depth[dst] < 0) | (depth[dst] == level + 1))
+                if not hit.any():
+                    break
+                np.minimum.at(want, dst[hit], src[hit])
+                depth[dst[hit]] = level + 1
+                level += 1
+            seen = depth >= 0
+            assert np.array_equal(depths[seen].astype(np.int64), depth[seen])
+            assert np.all(depths[~seen] == np.uint64(2**64 - 1))
+            below = depth > 0
+            assert np.array_equal(parents[below], want[below])
