@@ -7,9 +7,9 @@
  *   perform_vertex_phase_cc     phase_vertex_cc.asm:64-170
  *
  * Pull: the same wavefront chunking and segmented scan as the PageRank pull,
- * with min in place of sum.  Every run of a destination (including the runs
- * cut by chunk boundaries) is applied with a 64-bit atomic min, the GPU form
- * of the asm's lock cmpxchg at each destination change; a label that
+ * with min in place of sum.  A run inside a chunk is its destination's only
+ * one and lowers the label with a store; the chunk's first and last runs use a
+ * 64-bit atomic min, the GPU form of the asm's lock cmpxchg; a label that
  * actually drops sets the destination's HasInfo* bit and adds
  * phase_helper_add_frontier_stat to the wavefront's vote.  Gathers read the
  * labels in place, so updates made earlier in the sweep propagate within it,
