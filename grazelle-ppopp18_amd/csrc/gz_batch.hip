@@ -456,11 +456,10 @@ extern "C" void gz_batch_pr_ranks(double* out)
         gz_copy_to_host(out, gz_graph.vertex_props, V * sizeof(double));
         return;
     }
-    double* d = (double*)gz_pool_malloc((V ? V : 1) * sizeof(double), 0);
+    double* d = (double*)gz_result_buffer(0);
     hipLaunchKernelGGL(gz_k_batch_ranks, dim3(gz_grid(V, GZ_BLOCK)), dim3(GZ_BLOCK), 0, gz_stream,
                        (const double*)gz_graph.vertex_props, gz_graph.vertex_outdegrees, (const uint16_t*)B.d_gid,
                        (const uint64_t*)B.d_base, V, d);
     GZ_LAUNCH_CHECK();
     gz_copy_to_host(out, d, V * sizeof(double));
-    gz_pool_free(d);
 }

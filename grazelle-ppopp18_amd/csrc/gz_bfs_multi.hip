@@ -388,8 +388,8 @@ extern "C" void gz_bfs_batch_result(uint32_t search, int64_t* parents, uint64_t*
         fprintf(stderr, "grazelle: no BFS batch result for search %u\n", search);
         exit(66);
     }
-    uint64_t* d_depth = depths ? (uint64_t*)gz_pool_malloc((V + 8) * sizeof(uint64_t), 0) : nullptr;
-    int64_t* d_parent = parents ? (int64_t*)gz_pool_malloc((V + 8) * sizeof(int64_t), 0) : nullptr;
+    uint64_t* d_depth = depths ? gz_result_buffer(0) : nullptr;
+    int64_t* d_parent = parents ? (int64_t*)gz_result_buffer(1) : nullptr;
     uint64_t blocks = (V + GZ_BLOCK - 1) / GZ_BLOCK;
     if (blocks > 16384) blocks = 16384;
     hipLaunchKernelGGL(gz_k_msbfs_result, dim3((unsigned)blocks), dim3(GZ_BLOCK), 0, gz_stream, gz_graph.pull_vectors,
@@ -398,6 +398,4 @@ extern "C" void gz_bfs_batch_result(uint32_t search, int64_t* parents, uint64_t*
     GZ_LAUNCH_CHECK();
     if (depths) gz_copy_to_host(depths, d_depth, V * sizeof(uint64_t));
     if (parents) gz_copy_to_host(parents, d_parent, V * sizeof(int64_t));
-    gz_pool_free(d_depth);
-    gz_pool_free(d_parent);
 }

@@ -215,6 +215,11 @@ uint64_t gz_chunks_for(uint64_t n);
 /* Chunk length in vectors (a multiple of 64 x vectors per lane). */
 uint64_t gz_chunk_len(void);
 uint32_t gz_vectors_per_lane(void);
+/* V words for a result on its way to the host (which: 0 or 1, two at once):
+ * the scratch's frontier lists, which every phase builds before it reads them.
+ * A getter thus takes no memory beyond what a run has, and leaves the
+ * allocation generation, so captured launches stay valid. */
+uint64_t* gz_result_buffer(int which);
 /* Reduce gz_scratch.partials[0..count) into dst[0] (bit pattern). */
 void gz_reduce_partials(uint64_t* dst);
 /* The frontier words of the iteration that ends (gz_runtime.hip). */

@@ -74,6 +74,12 @@ __global__ void gz_k_vertex_info(gz_vertex_list list, uint32_t count, const uint
 
 }  // namespace
 
+uint64_t* gz_result_buffer(int which)
+{
+    gz_scratch_reserve(0, gz_graph.num_vertices);
+    return which ? gz_scratch.active_prefix : gz_scratch.active_vertices;
+}
+
 extern "C" void gz_dev_result_words(const uint64_t* words, const double* outdeg, const uint64_t* original, uint64_t n,
                                     uint64_t* out)
 {
@@ -82,27 +88,24 @@ extern "C" void gz_dev_result_words(const uint64_t* words, const double* outdeg,
         gz_copy_to_host(out, words, n * sizeof(uint64_t));
         return;
     }
-    uint64_t* d = (uint64_t*)gz_pool_malloc(n * sizeof(uint64_t), 0);
+    uint64_t* d = gz_result_buffer(0);
     hipLaunchKernelGGL(gz_k_result_words, dim3(gz_result_blocks(n)), dim3(GZ_BLOCK), 0, gz_stream, words, outdeg,
                        original, n, d);
     GZ_LAUNCH_CHECK();
     gz_copy_to_host(out, d, n * sizeof(uint64_t));
-    gz_pool_free(d);
 }
 
 extern "C" void gz_dev_result_bfs(const uint64_t* words, const uint64_t* original, uint64_t n, int64_t* parents,
                                   uint64_t* depths)
 {
     if (n == 0 || (parents == nullptr && depths == nullptr)) return;
-    int64_t* dp = parents ? (int64_t*)gz_pool_malloc(n * sizeof(int64_t), 0) : nullptr;
-    uint64_t* dd = depths ? (uint64_t*)gz_pool_malloc(n * sizeof(uint64_t), 0) : nullptr;
+    uint64_t* dd = depths ? gz_result_buffer(0) : nullptr;
+    int64_t* dp = parents ? (int64_t*)gz_result_buffer(1) : nullptr;
     hipLaunchKernelGGL(gz_k_result_bfs, dim3(gz_result_blocks(n)), dim3(GZ_BLOCK), 0, gz_stream, words, original, n, dp,
                        dd);
     GZ_LAUNCH_CHECK();
     if (parents) gz_copy_to_host(parents, dp, n * sizeof(int64_t));
     if (depths) gz_copy_to_host(depths, dd, n * sizeof(uint64_t));
-    gz_pool_free(dp);
-    gz_pool_free(dd);
 }
 
 extern "C" void gz_dev_vertex_info(const uint64_t* vertices, uint32_t count, const uint32_t* device_ids,
@@ -111,9 +114,9 @@ extern "C" void gz_dev_vertex_info(const uint64_t* vertices, uint32_t count, con
     if (count == 0 || count > 64) return;
     gz_vertex_list list;
     for (uint32_t i = 0; i < count; ++i) list.v[i] = vertices[i];
-    uint64_t* d = (uint64_t*)gz_pool_malloc(2 * 64 * sizeof(uint64_t), 0);
+    gz_scratch_reserve(0, gz_graph.num_vertices);
+    uint64_t* d = gz_scratch.reduce_tmp + 1024; /* past the reduction slots, 128 words */
     hipLaunchKernelGGL(gz_k_vertex_info, dim3(1), dim3(64), 0, gz_stream, list, count, device_ids, outdeg, d);
     GZ_LAUNCH_CHECK();
     gz_copy_to_host(info, d, 2 * (size_t)count * sizeof(uint64_t));
-    gz_pool_free(d);
 }

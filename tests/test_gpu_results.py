@@ -46,3 +46,31 @@ def test_getters_in_original_order(gz, device, V, relabel):
     up = batch_parents >= 0
     assert np.array_equal(up, parents >= 0)
     assert np.array_equal(depths[batch_parents[up]] + np.uint64(1), depths[up])
+
+
+@pytest.mark.parametrize("relabel", [False, True])
+def test_getters_leave_captures_valid(gz, device, relabel):
+    # a run whose results are read between repeats is captured the second
+    # time and replayed from then on: no getter allocates
+    gz.load_rmat_device(12, 16 << 12, 9, relabel=relabel)
+    root = int(gz.original_ids()[int(np.argmax(gz.outdegrees()))])
+    gz.run(gz.options("bfs", root=root))  # the allocations of the runs below
+    gz.run(gz.options("cc"))
+    gz.bfs_batch([root])
+    pr = gz.options("pr", iterations=6)
+    gz.run(pr)
+    (c0, l0), a0 = gz.graph_replay_counts(), gz.lib.gz_device_allocation_events()
+    first = gz.pr_ranks().copy()
+    for _ in range(3):
+        gz.run(gz.options("bfs", root=root))
+        gz.bfs_result()
+        gz.run(gz.options("cc"))
+        gz.cc_labels()
+        gz.bfs_batch([root])
+        gz.bfs_batch_result(0)
+        gz.run(pr)
+        gz.pr_props()
+        assert np.array_equal(gz.pr_ranks().view(np.uint64), first.view(np.uint64))
+    c1, l1 = gz.graph_replay_counts()
+    assert (c1 - c0, l1 - l0) == (1, 3)
+    assert gz.lib.gz_device_allocation_events() == a0
