@@ -715,7 +715,7 @@ static void gz_run_hybrid(const gz_run_options_t* o, gz_run_result_t* r)
                 const uint64_t cap = o->engine == GZ_ENGINE_PUSH ? ~0ull : threshold;
                 const uint64_t rounds = o->max_iterations ? o->max_iterations - ctr + 1 : ~0ull;
                 if (bfs)
-                    gz_bfs_launch_push_tail(ctr == 1 ? device_root : V, cap, rounds, gz_reduce_buffer);
+                    gz_bfs_launch_push_tail(cap, rounds, gz_reduce_buffer);
                 else
                     gz_cc_launch_push_tail(cap, rounds, gz_reduce_buffer);
             } else {

@@ -588,37 +588,45 @@ static void gz_bfs_retire(void)
  * (<= GZ_BFS_TAIL_CAP), gz_k_bfs_push_tail runs these push levels ("rounds")
  * back to back in one workgroup, with the frontier listed in LDS.
  *
- * The words alone say whether an edge (s, d) visits d: unvisited words are all
- * ones, a word of an earlier level is below this level's key (level << 48 | s),
- * and one of this level is replaced by a smaller key only, so every source of
- * the level competes and the smallest one stays, as in gz_k_edge_push_bfs.  The
- * lane that sees the unvisited word lists the vertex and counts its statistic,
- * once.  WantsInfo loses each round's vertices as they are listed (nothing here
- * reads it), and HasInfo* gets the last round's.  (A destination's word is read
- * plainly: a stale one is an older, larger value and only costs an atomic.)
+ * The first round's sources are the HasInfo bits, whatever set them.  An edge
+ * (s, d) visits d while d is in WantsInfo and its word exceeds this level's key
+ * (level << 48 | s): unvisited words are all ones, a word of an earlier level
+ * is below the key (levels stay below 2^16 here), and one of this level is
+ * replaced by a smaller key only, so every source of the level competes and the
+ * smallest one stays, as in gz_k_edge_push_bfs.  The lane that sees the
+ * unvisited word lists the vertex and counts its statistic, once.  A round's
+ * vertices leave WantsInfo after its barrier, and HasInfo* gets the last
+ * round's.  (Both words are read plainly: a stale one is an older, larger
+ * value or a bit of a visited vertex and only costs an atomic.)
  *
  * A round's list holds targets of the round before's edges, at most that
  * frontier's out-degrees, which its statistic counts and vote_cap bounds;
- * activations past the list (a push list that disagrees with the out-degrees)
- * go to HasInfo* at once and the round is the last.
+ * activations past the list (a first frontier beyond its statistic, or a push
+ * list that disagrees with the out-degrees) go to `spill`, and the round is the
+ * last.
  *
  * The workgroup stops after a round that activates nothing, whose statistic
  * exceeds vote_cap, or after max_rounds, and leaves what one push level and
  * its retirement leave, the statistic in out[0] and the rounds in out[7].
  * Bound by a round's chain of dependent memory steps (offsets, vector, words,
  * atomic min), about 4 us.  Four searches on R-MAT s17 (two tail launches
- * each, for the first level and the last two or three): 910 -> 845 us. */
+ * each, for the first level and the last two or three): 910 -> 845 us.  Listing
+ * a first frontier that is the root alone costs a search 0 us on s17, 5 on s20,
+ * 8 on s22 and 12 of 986 on s24; a check of the bitmap in the run's first wait
+ * (so that the root may stand for it) costs as much. */
 #define GZ_BFS_TAIL_THREADS 1024
 #define GZ_BFS_TAIL_CAP 16384
 /* Entry bound (as the CC tail's): larger rounds are faster on the whole grid. */
 #define GZ_BFS_TAIL_VOTE 4096
+/* Levels from here on wrap in the words; their pushes go by WantsInfo alone. */
+#define GZ_BFS_TAIL_LEVELS (1u << 16)
 /* Up to this many vertices the workgroup reads the HasInfo bitmap itself. */
 #define GZ_BFS_TAIL_DIRECT_VERTICES (1ull << 20)
 
 __global__ __launch_bounds__(GZ_BFS_TAIL_THREADS) void gz_k_bfs_push_tail(
     uint64_t* __restrict__ words, uint64_t* __restrict__ wants_info, uint64_t* __restrict__ next_frontier,
     const gz_vec_t* __restrict__ vecs, const uint64_t* __restrict__ offsets, const double* __restrict__ outdeg,
-    uint32_t stat_mode, uint64_t level, uint64_t root, uint64_t* __restrict__ first_list,
+    uint32_t stat_mode, uint64_t level, uint64_t* __restrict__ first_list, uint64_t* __restrict__ spill,
     const uint64_t* __restrict__ first_count, const uint64_t* __restrict__ first_bits, uint64_t num_vertices,
     uint64_t vote_cap, uint64_t max_rounds, uint64_t* __restrict__ out, gz_mirror_t mirror)
 {
@@ -634,10 +642,7 @@ __global__ __launch_bounds__(GZ_BFS_TAIL_THREADS) void gz_k_bfs_push_tail(
     const uint32_t tid = threadIdx.x;
     const int lane = gz_lane(), wave = (int)(tid / GZ_WAVE);
     uint64_t n, first_in_lds = GZ_BFS_TAIL_CAP;
-    if (root < num_vertices) {
-        n = 1;
-        if (tid == 0) lists[0][0] = (uint32_t)root;
-    } else if (first_bits != nullptr) {
+    if (first_bits != nullptr) {
         if (tid == 0) next_count = 0;
         __syncthreads();
         const uint64_t nwords = (num_vertices + 63) >> 6;
@@ -709,17 +714,19 @@ __global__ __launch_bounds__(GZ_BFS_TAIL_THREADS) void gz_k_bfs_push_tail(
                 const gz_lanes vec = gz_load_vector(vecs, (uint64_t)first[lo] + (slot - excl));
                 const uint64_t key = level_key | (uint64_t)srcv[lo];
                 const uint64_t l[4] = {vec.l0, vec.l1, vec.l2, vec.l3};
+                uint32_t wants[4];
                 uint64_t g[4], od[4], old[4];
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     const uint64_t d = gz_lane_valid(l[k]) ? gz_lane_id(l[k]) : 0;
+                    wants[k] = reinterpret_cast<const uint32_t*>(wants_info)[d >> 5] >> (d & 31);
                     g[k] = words[d];
                     od[k] = (uint64_t)__double_as_longlong(outdeg[d]);
                 }
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     old[k] = 0;
-                    if (gz_lane_valid(l[k]) && key < g[k])
+                    if (gz_lane_valid(l[k]) && (wants[k] & 1u) && key < g[k])
                         old[k] = atomicMin((unsigned long long*)&words[gz_lane_id(l[k])], (unsigned long long)key);
                 }
 #pragma unroll
@@ -727,12 +734,11 @@ __global__ __launch_bounds__(GZ_BFS_TAIL_THREADS) void gz_k_bfs_push_tail(
                     if (old[k] != GZ_BFS_UNVISITED) continue;
                     const uint64_t d = gz_lane_id(l[k]);
                     my_vote += with_count + (uint64_t)llrint(__longlong_as_double((long long)od[k]));
-                    atomicAnd(reinterpret_cast<unsigned int*>(wants_info) + (d >> 5), ~(1u << (d & 31)));
                     const uint32_t at = atomicAdd(&next_count, 1u);
                     if (at < GZ_BFS_TAIL_CAP)
                         lists[cur ^ 1u][at] = (uint32_t)d;
                     else
-                        gz_bit_set(next_frontier, d); /* the round is the last */
+                        spill[at - GZ_BFS_TAIL_CAP] = d; /* the round is the last */
                 }
             }
             __syncthreads(); /* the next chunk rewrites incl, first, srcv, wave_tot */
@@ -745,6 +751,11 @@ __global__ __launch_bounds__(GZ_BFS_TAIL_THREADS) void gz_k_bfs_push_tail(
         const uint64_t listed = next_count;
         cur ^= 1u;
         n = listed < GZ_BFS_TAIL_CAP ? listed : GZ_BFS_TAIL_CAP;
+        for (uint64_t i = tid; i < listed; i += T) {
+            const uint32_t d = i < n ? lists[cur][i] : (uint32_t)spill[i - n];
+            atomicAnd(reinterpret_cast<unsigned int*>(wants_info) + (d >> 5), ~(1u << (d & 31)));
+            if (i >= n) gz_bit_set(next_frontier, d);
+        }
         /* an activated vertex may have no out-edges and, with out-degrees alone
          * in the statistic, add nothing to it: the vote decides, as on the host */
         if (vote == 0 || vote > vote_cap || listed > GZ_BFS_TAIL_CAP || rounds >= max_rounds) break;
@@ -767,28 +778,30 @@ extern "C" void gz_bfs_push_tail(uint64_t max_vote)
 
 extern "C" int gz_bfs_push_tail_applies(uint64_t vote)
 {
-    return vote <= gz_bfs_tail_vote && gz_bfs_tail_vote > 0 && gz_phase_config.push_frontier_skip &&
+    return vote <= gz_bfs_tail_vote && gz_bfs_tail_vote > 0 && gz_phase_config.bfs_level < GZ_BFS_TAIL_LEVELS &&
+           gz_phase_config.push_frontier_skip &&
            gz_graph.push_vertex_offsets != nullptr && gz_graph.push_vectors != nullptr &&
            gz_phase_config.stat_mode != GZ_STAT_COUNT_ONLY && gz_graph.num_vertices > 0 &&
            gz_graph.num_vertices < (1ull << 32) && gz_graph.push_vector_count < (1ull << 32);
 }
 
-extern "C" void gz_bfs_launch_push_tail(uint64_t root, uint64_t vote_cap, uint64_t max_rounds, uint64_t* reduce_buffer)
+extern "C" void gz_bfs_launch_push_tail(uint64_t vote_cap, uint64_t max_rounds, uint64_t* reduce_buffer)
 {
-    const uint64_t V = gz_graph.num_vertices;
+    const uint64_t V = gz_graph.num_vertices, level = gz_phase_config.bfs_level;
     if (vote_cap > gz_bfs_tail_vote) vote_cap = gz_bfs_tail_vote;
+    if (max_rounds > GZ_BFS_TAIL_LEVELS - level) max_rounds = GZ_BFS_TAIL_LEVELS - level;
     if (max_rounds == 0) max_rounds = 1;
     gz_scratch_reserve(0, V);
     const bool direct = V <= GZ_BFS_TAIL_DIRECT_VERTICES;
-    if (root >= V && !direct)
+    if (!direct)
         gz_frontier_list(gz_graph.frontier_has_info, gz_graph.push_vertex_offsets, V, gz_graph.push_vector_count);
     const gz_mirror_t mirror = gz_reduce_mirror_target(reduce_buffer);
     gz_ktimer_begin(GZ_K_PUSH_BFS);
     hipLaunchKernelGGL(gz_k_bfs_push_tail, dim3(1), dim3(GZ_BFS_TAIL_THREADS), 0, gz_stream,
                        (uint64_t*)gz_graph.vertex_props, gz_graph.frontier_wants_info,
                        (uint64_t*)gz_graph.vertex_accumulators, gz_graph.push_vectors, gz_graph.push_vertex_offsets,
-                       gz_graph.vertex_outdegrees, gz_phase_config.stat_mode, (uint64_t)gz_phase_config.bfs_level, root,
-                       gz_scratch.active_vertices, gz_scratch.active_totals,
+                       gz_graph.vertex_outdegrees, gz_phase_config.stat_mode, level, gz_scratch.active_vertices,
+                       gz_scratch.active_prefix, gz_scratch.active_totals,
                        direct ? (const uint64_t*)gz_graph.frontier_has_info : (const uint64_t*)nullptr, V, vote_cap,
                        max_rounds, reduce_buffer, mirror);
     GZ_LAUNCH_CHECK();

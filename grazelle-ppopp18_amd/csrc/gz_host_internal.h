@@ -107,10 +107,9 @@ void gz_cc_push_vote_hint(uint64_t vote);
  * to reduce_buffer[7]. */
 int gz_cc_push_tail_applies(uint64_t vote);
 void gz_cc_launch_push_tail(uint64_t vote_cap, uint64_t max_rounds, uint64_t* reduce_buffer);
-/* The same for BFS (gz_bfs_push_tail); the first frontier is the root alone
- * when root < V, else HasInfo. */
+/* The same for BFS (gz_bfs_push_tail), from gz_phase_config.bfs_level on. */
 int gz_bfs_push_tail_applies(uint64_t vote);
-void gz_bfs_launch_push_tail(uint64_t root, uint64_t vote_cap, uint64_t max_rounds, uint64_t* reduce_buffer);
+void gz_bfs_launch_push_tail(uint64_t vote_cap, uint64_t max_rounds, uint64_t* reduce_buffer);
 /* Control words of a device-driven iteration loop (CC, and the log of
  * (engine, vote) pairs from GZ_LOOP_LOG on). */
 #define GZ_LOOP_ENGINE 0          /* engine of the iteration about to run: 0 stop, 1 pull, 2 push over the

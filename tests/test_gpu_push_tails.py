@@ -116,3 +116,101 @@ def test_bfs_push_in_parts_keeps_smallest_parents(gz, device, V):
             assert np.all(depths[~seen] == np.uint64(2**64 - 1))
             below = depth > 0
             assert np.array_equal(parents[below], want[below])
+
+
+def _bits(gz, at):
+    """HasInfo or WantsInfo (a device pointer) as booleans, and how to write them back."""
+    n = (gz.num_vertices() + 63) // 64
+    words = np.empty(n, np.uint64)
+    gz.lib.gz_copy_to_host(words.ctypes.data_as(gz.vp), gz.vp(at), gz.C.c_size_t(8 * n))
+    bits = np.unpackbits(words.view(np.uint8), bitorder="little").astype(bool)
+
+    def write():
+        w = np.packbits(bits, bitorder="little").view(np.uint64)
+        gz.lib.gz_copy_to_device(gz.vp(at), w.ctypes.data_as(gz.vp), gz.C.c_size_t(8 * n))
+
+    return bits, write
+
+
+def _execute(gz, opts, max_vote):
+    r = gz.RunResult()
+    gz.bfs_push_tail(max_vote)
+    try:
+        gz.lib.gz_execution_run(gz.C.byref(opts), gz.C.byref(r))
+    finally:
+        gz.bfs_push_tail(DEFAULT_TAIL)
+    return (*(x.copy() for x in gz.bfs_result()), r)
+
+
+@pytest.mark.parametrize("extra", [2, 500])
+@pytest.mark.parametrize("V", [5000, DIRECT, DIRECT + 1])
+def test_bfs_tail_takes_the_frontier_it_is_given(gz, device, V, extra):
+    # sources added to HasInfo after the start are searched from too, vertices
+    # taken out of WantsInfo are not visited, and a run asked for another root
+    # goes on from the prepared one
+    edges = np.random.default_rng(V).integers(0, V, size=(2 * V, 2), dtype=np.uint64)
+    gz.load_pairs_device(V, edges)
+    src, dst = edges[:, 0].astype(np.int64), edges[:, 1].astype(np.int64)
+    picked = np.random.default_rng(extra).choice(np.unique(src), extra + 40, replace=False)
+    sources, barred = picked[:extra], picked[extra:]
+    G = gz.phase_graph
+    for engine in ("push", "hybrid"):
+        depth = np.full(V, -1, np.int64)
+        depth[sources], level = 0, 0
+        depth[barred] = -2
+        while True:
+            hit = (depth[src] == level) & (depth[dst] == -1)
+            if not hit.any():
+                break
+            level += 1
+            depth[dst[hit]] = level
+        want = np.where(depth > 0, depth.astype(np.uint64), np.uint64(2**64 - 1))
+        want[sources[0]] = 0
+        for cap in (0, 3, DEFAULT_TAIL):
+            opts = gz.options("bfs", engine=engine, root=int(sources[0]))
+            gz.lib.gz_execution_prepare(gz.C.byref(opts))
+            has, put_has = _bits(gz, G.frontier_has_info)
+            wants, put_wants = _bits(gz, G.frontier_wants_info)
+            has[sources] = True
+            wants[sources] = wants[barred] = False
+            put_has()
+            put_wants()
+            opts.root = int(sources[-1])
+            _, got, r = _execute(gz, opts, cap)
+            assert np.array_equal(got, want), (engine, cap)
+            assert r.iterations == level + 1
+            left, _ = _bits(gz, G.frontier_wants_info)
+            assert np.array_equal(left[:V], depth == -1), (engine, cap)
+
+
+def test_bfs_tail_levels_beyond_the_words(gz, device):
+    # a word holds 16 bits of level: from level 65,536 on a vertex of an
+    # earlier level is told by WantsInfo alone
+    V = 65536 + 300
+    pairs = np.stack([np.arange(V - 1), np.arange(1, V)], axis=1).astype(np.uint64)
+    gz.load_pairs_device(V, pairs, symmetrize=True)
+    opts = gz.options("bfs", engine="push", root=0)
+    parents, depths, r = _bfs(gz, opts, DEFAULT_TAIL)
+    assert r.iterations == V
+    assert np.array_equal(parents, np.arange(V) - 1)
+    assert np.array_equal(depths, np.arange(V, dtype=np.uint64) % np.uint64(1 << 16))
+
+
+def test_bfs_tail_frontier_past_its_list(gz, device):
+    # a first frontier far beyond its root's statistic lists more vertices
+    # than the workgroup holds: all of them reach the next level
+    hubs, fan = 400, 100
+    V = hubs * (fan + 1)
+    hub = np.repeat(np.arange(hubs), fan)
+    pairs = np.stack([hub, hubs + np.arange(hubs * fan)], axis=1).astype(np.uint64)
+    gz.load_pairs_device(V, pairs)
+    opts = gz.options("bfs", engine="push", root=0)
+    gz.lib.gz_execution_prepare(gz.C.byref(opts))
+    has, put = _bits(gz, gz.phase_graph.frontier_has_info)
+    has[:hubs] = True
+    put()
+    parents, depths, r = _execute(gz, opts, DEFAULT_TAIL)
+    assert r.iterations == 2
+    assert np.all(depths[hubs:] == 1) and np.array_equal(parents[hubs:], hub)
+    left, _ = _bits(gz, gz.phase_graph.frontier_wants_info)
+    assert not left[hubs:V].any()
