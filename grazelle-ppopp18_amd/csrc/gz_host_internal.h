@@ -19,6 +19,8 @@ extern "C" {
  * stream only. */
 void* gz_pool_malloc(size_t bytes, int zero);
 void gz_pool_free(void* ptr);
+/* The idle blocks go back to the device. */
+void gz_pool_trim(void);
 /* Waits for the whole device (nothing before the runtime is up). */
 void gz_device_wait(void);
 

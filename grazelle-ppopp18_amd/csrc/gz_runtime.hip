@@ -114,6 +114,11 @@ extern "C" void* gz_device_malloc(size_t bytes)
     if (bytes == 0) bytes = 256;
     hipError_t err = hipMalloc(&p, bytes);
     if (err != hipSuccess) {
+        (void)hipGetLastError();
+        gz_pool_trim(); /* the library's idle blocks may be what is missing */
+        err = hipMalloc(&p, bytes);
+    }
+    if (err != hipSuccess) {
         fprintf(stderr, "grazelle: device allocation of %zu bytes failed: %s\n", bytes, hipGetErrorString(err));
         exit(71);
     }
@@ -160,6 +165,12 @@ static void gz_pool_trim_locked(void)
     for (auto& b : gz_pool.idle) GZ_CHECK(hipFree(b.second));
     gz_pool.idle.clear();
     gz_pool.idle_bytes = 0;
+}
+
+extern "C" void gz_pool_trim(void)
+{
+    std::lock_guard<std::mutex> hold(gz_pool.lock);
+    gz_pool_trim_locked();
 }
 
 extern "C" void* gz_pool_malloc(size_t bytes, int zero)

@@ -67,3 +67,32 @@ print("loaded")
     assert r.returncode == 65
     assert "edge endpoint 77 is not below V = 77" in r.stderr
     assert "loaded" not in r.stdout
+
+
+def _in_a_process(gz, body):
+    """Runs body in a process of its own, after a load of R-MAT s23 whose
+    temporaries (two arrays of 2^27 words and more) leave the pool idle blocks;
+    free() is the device's free memory."""
+    code = f"""
+import sys, torch
+sys.path.insert(0, {str(pathlib.Path(gz.__file__).parent)!r})
+import grazelle as gz
+gz.init()
+free = lambda: torch.cuda.mem_get_info()[0]
+gz.load_rmat_device(10, 16 << 10, 1)
+before = free()
+gz.load_rmat_device(23, 16 << 23, 1)
+{body}
+print("done")
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "done" in r.stdout, r.stderr
+
+
+def test_allocation_takes_back_idle_blocks(gz, device):
+    # a request beyond what is free, by less than the idle blocks hold
+    _in_a_process(gz, """
+gz.lib.gz_device_malloc.restype, gz.lib.gz_device_malloc.argtypes = gz.vp, [gz.C.c_size_t]
+gz.lib.gz_device_free.argtypes = [gz.vp]
+gz.lib.gz_device_free(gz.lib.gz_device_malloc(free() + (512 << 20)))
+""")
