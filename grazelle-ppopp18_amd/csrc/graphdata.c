@@ -290,7 +290,7 @@ const double* gz_graph_outdegrees_host(void)
     return G.outdeg;
 }
 
-void gz_graph_release(void)
+void gz_graph_drop(void)
 {
     /* a caller's own streams may still read the arrays, which the next load
      * may be handed at once */
@@ -320,6 +320,12 @@ void gz_graph_release(void)
     memset(&gz_graph, 0, sizeof(gz_graph));
 }
 
+void gz_graph_release(void)
+{
+    gz_graph_drop();
+    gz_pool_trim();
+}
+
 static void gz_graph_finish(void);
 
 static void gz_upload_layout(const uint64_t* pairs, uint64_t num_edges, uint64_t num_vertices, int by_dst,
@@ -342,7 +348,7 @@ int gz_graph_load_pairs(uint64_t num_vertices, uint64_t pull_edges, const uint64
                         const uint64_t* push_pairs)
 {
     gz_runtime_init(0);
-    gz_graph_release();
+    gz_graph_drop();
     if (num_vertices == 0 || num_vertices > GZ_MAX_VERTEX_ID) {
         fprintf(stderr, "grazelle: vertex count %llu is outside [1, 2^48)\n", (unsigned long long)num_vertices);
         exit(65);

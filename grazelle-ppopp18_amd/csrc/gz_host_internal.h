@@ -23,6 +23,8 @@ void gz_pool_free(void* ptr);
 void gz_pool_trim(void);
 /* Waits for the whole device (nothing before the runtime is up). */
 void gz_device_wait(void);
+/* gz_graph_release for a load: the blocks stay with the pool. */
+void gz_graph_drop(void);
 
 /* Device-built layouts handed to the graph record (device ingress). */
 typedef struct gz_device_layouts_t {

@@ -749,7 +749,7 @@ extern "C" int gz_graph_build_pairs_device(uint64_t num_vertices, uint64_t num_e
                                            int symmetrize, uint32_t flags)
 {
     gz_runtime_init(0);
-    gz_graph_release();
+    gz_graph_drop();
     gz_check_vertex_count(num_vertices);
     const uint32_t b = gz_id_bits(num_vertices);
     const uint64_t n = symmetrize ? 2 * num_edges : num_edges;
@@ -766,7 +766,7 @@ extern "C" int gz_graph_build_rmat_device(const gz_rmat_params_t* p, uint64_t nu
                                           uint64_t extra_edges, const uint64_t* extra_pairs, uint32_t flags)
 {
     gz_runtime_init(0);
-    gz_graph_release();
+    gz_graph_drop();
     const uint64_t rmat_nv = p->num_vertices ? p->num_vertices : (1ull << p->scale);
     uint64_t nv = num_vertices > rmat_nv ? num_vertices : rmat_nv;
     gz_check_vertex_count(nv);
@@ -796,7 +796,7 @@ extern "C" int gz_graph_build_rmat_union_device(const gz_rmat_params_t* params, 
                                                 uint64_t* vertex_bases)
 {
     gz_runtime_init(0);
-    gz_graph_release();
+    gz_graph_drop();
     uint64_t nv = 0, n = 0;
     const uint64_t per = symmetrize ? 2 : 1;
     for (uint32_t g = 0; g < count; ++g) {

@@ -141,9 +141,10 @@ extern "C" void gz_device_free(void* ptr)
  * 1.3 ms of a 20 K-vertex one), so a freed block is kept for the next request
  * of about its size.  All of the library's work is on one stream, so a block
  * handed out again is written only after its last use there; a caller's own
- * streams are covered by gz_graph_release, which waits for the device.  At most
- * GZ_POOL_IDLE_MAX bytes are kept idle; a request that the device cannot
- * satisfy and gz_runtime_shutdown give them back. */
+ * streams are covered by gz_graph_drop, which waits for the device.  At most
+ * GZ_POOL_IDLE_MAX bytes are kept idle; a request of the library's that the
+ * device cannot satisfy, gz_graph_release and gz_runtime_shutdown give them
+ * back. */
 #define GZ_POOL_IDLE_MAX (8ull << 30)
 
 static struct {

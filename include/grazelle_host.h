@@ -274,6 +274,11 @@ double gz_batch_time_pull(const gz_batch_config_t* cfg, uint32_t bucket, uint32_
 /* PageRank ranks of the whole union (rank = props * outdeg', outdeg' = V of
  * the vertex's graph for sinks), V entries. */
 void gz_batch_pr_ranks(double* out);
+/* Frees the loaded graph.  A load frees the graph before it by itself and keeps
+ * up to 8 GiB of that graph's and its own freed device memory for the next
+ * load; gz_graph_release gives this memory back to the device as well (for
+ * other allocators of the process), and so does a device allocation of the
+ * library's that would fail without it.  No reference counterpart. */
 void gz_graph_release(void);
 
 /* Host mirrors filled at load time (for output, statistics and tests). */

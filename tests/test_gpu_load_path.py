@@ -96,3 +96,11 @@ gz.lib.gz_device_malloc.restype, gz.lib.gz_device_malloc.argtypes = gz.vp, [gz.C
 gz.lib.gz_device_free.argtypes = [gz.vp]
 gz.lib.gz_device_free(gz.lib.gz_device_malloc(free() + (512 << 20)))
 """)
+
+
+def test_release_gives_idle_blocks_back(gz, device):
+    # what stays is the scratch of the larger graph (by its 2^23 vertices)
+    _in_a_process(gz, """
+gz.release()
+assert before - free() < 512 << 20, (before, free())
+""")
