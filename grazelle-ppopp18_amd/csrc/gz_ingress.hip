@@ -1035,7 +1035,8 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_slice_pack(const uint64_t* __re
  * first run of slice x whose destination is not below 64 k.  A wavefront takes
  * `per` consecutive 64-vertex blocks: lane x finds slice x's run at the first
  * of them by binary search in the runs' destinations (ascending inside a
- * slice) and steps it from block to block by the runs the block held. */
+ * slice) and steps it from block to block by the runs the block held.  The
+ * lanes meet in a row of LDS words of their wavefront's own. */
 template <typename M>
 __global__ __launch_bounds__(GZ_BLOCK) void gz_k_slice_mask(const uint32_t* __restrict__ gid, uint32_t nslices,
                                                             const uint64_t* __restrict__ first_run, uint64_t nv,
@@ -1065,6 +1066,7 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_slice_mask(const uint32_t* __re
     for (uint64_t k = k0; k < k1; ++k) {
         if ((uint32_t)lane < nslices) rank_base[k * nslices + (uint32_t)lane] = at;
         mine[lane] = 0;
+        gz_wave_lds_sync();
         const uint64_t stop = (k + 1) * GZ_WAVE;
         for (uint32_t x0 = 0; x0 < nslices; x0 += 8) {
             uint32_t g[8];
@@ -1077,11 +1079,12 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_slice_mask(const uint32_t* __re
 #pragma unroll
             for (uint32_t u = 0; u < 8; ++u) {
                 const bool in = (uint64_t)g[u] < stop;
-                if (in) mine[g[u] & (GZ_WAVE - 1)] |= 1ull << (x0 + u); /* the lanes' vertices differ */
+                if (in) atomicOr(&mine[g[u] & (GZ_WAVE - 1)], 1ull << (x0 + u));
                 const uint32_t c = (uint32_t)__popcll(__ballot(in));
                 if ((uint32_t)lane == x0 + u) at += c;
             }
         }
+        gz_wave_lds_sync();
         const uint64_t v = k * GZ_WAVE + (uint64_t)lane;
         if (v < nv) mask[v] = (M)mine[lane];
     }

@@ -306,6 +306,16 @@ __device__ __forceinline__ uint64_t gz_lane_id(uint64_t l) { return l & GZ_LANE_
 
 __device__ __forceinline__ int gz_lane() { return (int)(threadIdx.x & (GZ_WAVE - 1)); }
 
+/* Orders the wavefront's LDS accesses before it ahead of those after it, for
+ * values that pass between its lanes (no instruction of its own: a wavefront's
+ * LDS accesses run in order). */
+__device__ __forceinline__ void gz_wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 /* Index of the segment head at or below `lane`, given the ballot of heads. */
 __device__ __forceinline__ int gz_segment_start(uint64_t heads, int lane)
 {
