@@ -49,6 +49,7 @@ struct gz_batch_t {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     uint32_t graph_iters = 0;
+    double graph_damping = 0.0; /* an argument of the captured launches */
 };
 
 gz_batch_t B;
@@ -370,7 +371,7 @@ extern "C" double gz_batch_pr_run(uint32_t iterations, int use_graph)
     gz_timer_t* t = gz_timer_create();
     const int timing = gz_kernel_timing_enabled();
     if (use_graph) {
-        if (B.exec == nullptr || B.graph_iters != iterations) {
+        if (B.exec == nullptr || B.graph_iters != iterations || B.graph_damping != B.damping) {
             gz_batch_free_graph();
             gz_kernel_timing_enable(0); /* no event records inside the capture */
             GZ_CHECK(hipStreamBeginCapture(gz_stream, hipStreamCaptureModeThreadLocal));
@@ -378,6 +379,7 @@ extern "C" double gz_batch_pr_run(uint32_t iterations, int use_graph)
             GZ_CHECK(hipStreamEndCapture(gz_stream, &B.graph));
             GZ_CHECK(hipGraphInstantiate(&B.exec, B.graph, nullptr, nullptr, 0));
             B.graph_iters = iterations;
+            B.graph_damping = B.damping;
             gz_kernel_timing_enable(timing);
         }
         gz_timer_start(t);

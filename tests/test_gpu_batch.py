@@ -106,3 +106,15 @@ def test_autotuner_probe(gz, device):
     gz.batch_set_config(vectors_per_lane=2, workgroup_size=128, chunk=(256, 512, 512, 1024))
     gz.batch_time_pull(1, 64, (64, 64, 64, 64), 1)
     assert gz.batch_get_config() == {"vectors_per_lane": 2, "workgroup_size": 128, "chunk": [256, 512, 512, 1024]}
+
+
+def test_replay_follows_the_damping(gz, device):
+    # captured launches hold the damping they were captured with
+    gz.load_batch_device(SPECS)
+    gz.batch_set_config()
+    for damping in (0.85, 0.875, 0.6, 0.85):
+        gz.batch_pr(5, damping=damping, use_graph=False)
+        eager = gz.batch_pr_ranks()
+        for _ in range(2):
+            gz.batch_pr(5, damping=damping, use_graph=True)
+            assert np.array_equal(gz.batch_pr_ranks().view(np.uint64), eager.view(np.uint64)), damping
