@@ -255,12 +255,31 @@ static int gz_probe_wide_on = 0;
  * gz_sel_above * threshold; outside, the fixed rule's choice stands (pull
  * above, push below).  A factor of 0 lifts that side of the band. */
 static double gz_sel_above = 1.0, gz_sel_below = 32.0;
-#define GZ_SEL_TIE 0.5f
+/* A near tie (log times) on a large level of a search goes to the pull, whose
+ * time varies less.  On the 41.7 M-vertex graph levels of half to two thirds of
+ * the threshold are predicted within 0.4, and run in a search of 3.0 to 3.2 ms
+ * pulled, 3.2 to 3.6 pushed.  CC levels have no such figures and go by the
+ * model. */
+static float gz_sel_tie = 0.5f;
 
 void gz_selector_set_trust(double above, double below)
 {
     gz_sel_above = (above >= 1.0) ? above : 0.0;
     gz_sel_below = (below >= 1.0) ? below : 0.0;
+}
+
+void gz_selector_set_tie(double margin) { gz_sel_tie = margin > 0.0 ? (float)margin : 0.0f; }
+
+int gz_selector_choose(int bfs, uint64_t vote, uint64_t threshold, int choice, const float* predicted)
+{
+    int use_pull = (choice == 1);
+    if (bfs && !use_pull && gz_sel_tie > 0.0f && vote >= threshold / 4 && predicted[1] > predicted[0] - gz_sel_tie)
+        use_pull = 1;
+    if (gz_sel_above > 0.0 && (double)vote > gz_sel_above * (double)threshold)
+        use_pull = 1;
+    else if (gz_sel_below > 0.0 && (double)vote * gz_sel_below < (double)threshold)
+        use_pull = 0;
+    return use_pull;
 }
 
 void gz_probe_wide(int on) { gz_probe_wide_on = on ? 1 : 0; }
@@ -661,18 +680,8 @@ static void gz_run_hybrid(const gz_run_options_t* o, gz_run_result_t* r)
             use_pull = 1;
         else if (o->engine == GZ_ENGINE_PUSH)
             use_pull = 0;
-        else if (learned) {
-            use_pull = (sel.choice == 1);
-            /* a near tie (log times) on a large level goes to the pull: its
-             * time varies less.  On the 41.7 M-vertex graph levels of half to
-             * two thirds of the threshold are predicted within 0.4, and run
-             * in a search of 3.0 to 3.2 ms pulled, 3.2 to 3.6 pushed */
-            if (!use_pull && vote >= threshold / 4 && sel.predicted[1] > sel.predicted[0] - GZ_SEL_TIE) use_pull = 1;
-            if (gz_sel_above > 0.0 && (double)vote > gz_sel_above * (double)threshold)
-                use_pull = 1;
-            else if (gz_sel_below > 0.0 && (double)vote * gz_sel_below < (double)threshold)
-                use_pull = 0;
-        }
+        else if (learned)
+            use_pull = gz_selector_choose(bfs, vote, threshold, sel.choice, sel.predicted);
         else
             use_pull = vote > threshold;
         if (use_pull && gz_graph.pull_vectors == NULL) use_pull = 0;

@@ -163,6 +163,10 @@ void gz_bfs_push_vote_hint(uint64_t vote);
  * BFS pushes leave WantsInfo to it. */
 void gz_iteration_end(int bfs, uint64_t* reduce_buffer);
 void gz_bfs_defer_retire(int on);
+/* The learned engine's choice (1 pull, 0 push) for a level: the model's choice
+ * (1 pull) and predicted log times (pull, push) within the bounds of
+ * gz_selector_set_trust and gz_selector_set_tie. */
+int gz_selector_choose(int bfs, uint64_t vote, uint64_t threshold, int choice, const float* predicted);
 /* Whether the last BFS push left its visited vertices in WantsInfo; clears
  * the mark. */
 int gz_bfs_take_deferred_retire(void);

@@ -147,6 +147,7 @@ _sig("gz_selector_save_file", C.c_int, C.c_char_p)
 _sig("gz_selector_loaded", C.c_int)
 _sig("gz_selector_feature_used", C.c_int, u32)
 _sig("gz_selector_set_trust", None, C.c_double, C.c_double)
+_sig("gz_selector_set_tie", None, C.c_double)
 _sig("gz_selector_forward_batch", C.c_int, vp, vp, vp, u64)
 _sig("gz_selector_gradient", C.c_float, vp, vp, vp, u64, vp)
 _sig("gz_selector_train", C.c_int, vp, vp, vp, u64, u32, C.c_float, vp)
@@ -763,6 +764,16 @@ def selector_set_trust(above: float, below: float | None = None) -> None:
     one factor sets both)."""
     init()
     lib.gz_selector_set_trust(float(above), float(above if below is None else below))
+
+
+TIE = 0.5  # the engine's default margin
+
+
+def selector_set_tie(margin: float = TIE) -> None:
+    """In a learned search, from a quarter of the threshold up, a push must be
+    predicted e^margin cheaper than the pull to be followed (0: no margin)."""
+    init()
+    lib.gz_selector_set_tie(float(margin))
 
 
 def selector_feature_used(i: int) -> bool:

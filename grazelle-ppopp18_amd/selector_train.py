@@ -177,7 +177,7 @@ def fit(data: dict, steps: int = 6000, lr: float = 1e-3, seed: int = 7, per_edge
 TRUST = (gz.TRUST_ABOVE, gz.TRUST_BELOW)  # the engine's default band (gz_selector_set_trust)
 
 
-def policy_times(data: dict, params=None, mean=None, std=None, trust: tuple = TRUST) -> dict:
+def policy_times(data: dict, params=None, mean=None, std=None, trust: tuple = TRUST, tie: float = gz.TIE) -> dict:
     """Total edge-phase ms of the fixed threshold, the learned selector and
     the per-level best, summed over the probed runs.  The learned policy sees
     its own previous choice and time (features 5 and 6): where it chose what
@@ -186,7 +186,8 @@ def policy_times(data: dict, params=None, mean=None, std=None, trust: tuple = TR
     clock overhead stands in for it.  As in the engine, the model decides
     only while the level's vote (vertices plus out-edges of the frontier,
     features 0 and 1) lies in [E/5 / below, above * E/5], with (above, below)
-    = `trust`; a factor below 1 lifts that side."""
+    = `trust` (a factor below 1 lifts that side), and from a quarter of E/5 up
+    a push must be predicted e^tie cheaper (gz_selector_set_tie)."""
     X = data["features"].astype(np.float32)
     tp, ts = data["pull_ms"], data["push_ms"]
     fixed = np.where(data["fixed"] == 1, tp, ts)
@@ -211,6 +212,8 @@ def policy_times(data: dict, params=None, mean=None, std=None, trust: tuple = TR
                 above, below = trust
                 vote = float(np.expm1(X[i][0]) + np.expm1(X[i][1]))
                 threshold = float(data["edges"][i] // 5)
+                if not pull and tie > 0 and vote >= threshold // 4 and y[1] > y[0] - np.float32(tie):
+                    pull = True
                 if above >= 1.0 and vote > above * threshold:
                     pull = True
                 elif below >= 1.0 and vote * below < threshold:

@@ -48,6 +48,11 @@ int gz_selector_feature_used(uint32_t i);
  * above the threshold, and the pull often beat the push down to about a
  * 32nd of it.  A factor below 1 lifts that side of the band. */
 void gz_selector_set_trust(double above, double below);
+/* In a search (not in CC), inside the band and from a quarter of the threshold
+ * up, the model's push is followed only when it is predicted cheaper than the
+ * pull by a factor of e^margin (default 0.5; 0: whenever it is predicted
+ * cheaper). */
+void gz_selector_set_tie(double margin);
 
 /* Weights: GZ_SEL_PARAMS floats plus feature normalisation (mean[8], std[8]). */
 int gz_selector_set_weights(const float* params, const float* feat_mean, const float* feat_std);
