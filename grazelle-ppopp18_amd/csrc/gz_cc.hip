@@ -73,9 +73,10 @@ struct gz_cc_pull_op {
     }
     /* A run that starts and ends inside the chunk is its destination's only
      * one, so no other wavefront writes the label and a store does (at device
-     * scope: other XCDs read the lower label sooner).  The atomic min's round
-     * trip was in every step's chain: the first two sweeps of R-MAT s16 (0.5 M
-     * vectors) took 43 and 39 us, now 33 and 28 with the chunks below. */
+     * scope: other XCDs read the lower label sooner), which keeps the atomic
+     * min's round trip out of the chunk's chain of steps: the first two sweeps
+     * of R-MAT s14 with trees take 33 and 30 us (36 and 33 by atomics), of s16
+     * 37 and 33 (39 and 35). */
     __device__ __forceinline__ void store(uint64_t d, uint64_t m)
     {
         if (d == first_d) {
@@ -264,39 +265,28 @@ static void gz_pull_cc_merge(const gz_vec_t* edge_list, uint64_t edge_list_count
     gz_ktimer_end(GZ_K_MERGE);
 }
 
-/* Chunk length of the in-place pull: the configured one, halved while the
- * list gives fewer than GZ_CC_PULL_WAVES wavefronts.  Its units meet in atomic
- * mins alone (no records), so they may be as short as a step; on a small list
- * the sweep is the latency of a chunk's chain of steps.  CC on R-MAT s14 109 us
- * at the configured length, 97 so; s16 with trees 310 and 297.  With 4096
- * wavefronts more of the runs are shared and the latter takes 325. */
-#define GZ_CC_PULL_WAVES 2048
-static uint64_t gz_cc_pull_chunk(uint64_t nvec)
-{
-    const uint64_t step = (uint64_t)GZ_WAVE * gz_vectors_per_lane();
-    uint64_t len = gz_chunk_len();
-    while (len > step && nvec < len * GZ_CC_PULL_WAVES) len = (len / 2 + step - 1) / step * step;
-    return len;
-}
-
 extern "C" void perform_edge_pull_phase_cc(const gz_vec_t* edge_list, uint64_t edge_list_count)
 {
     if (gz_phase_config.pull_variant == GZ_PULL_SOURCE_SLICED && edge_list_count > 0) {
         gz_pull_cc_sliced(edge_list, edge_list_count);
         return;
     }
-    const bool merged = gz_phase_config.pull_variant == GZ_PULL_MERGE_BUFFER;
-    const uint64_t chunk_len = merged ? gz_chunk_len() : gz_cc_pull_chunk(edge_list_count);
-    const uint64_t nchunks = (edge_list_count + chunk_len - 1) / chunk_len;
+    const uint64_t nchunks = gz_chunks_for(edge_list_count);
     gz_scratch_reserve(nchunks, gz_graph.num_vertices);
     gz_scratch.partials_is_double = 0;
     gz_scratch.partials_count = nchunks;
     gz_scratch.stats_count = gz_phase_config.collect_stats ? nchunks : 0;
     if (nchunks == 0) return;
-    if (merged) {
+    if (gz_phase_config.pull_variant == GZ_PULL_MERGE_BUFFER) {
         gz_pull_cc_merge(edge_list, edge_list_count);
         return;
     }
+    /* A label passes along a chunk step by step within a sweep, so the chunk
+     * stays as long as configured on a small list too.  Halved until there are
+     * 2048 wavefronts, R-MAT s14 with trees takes 241 us instead of 266 and s16
+     * 248 instead of 263, but 1024 chains of 64 vertices on a spine 24.2 ms
+     * (1084 iterations) instead of 7.5 (192). */
+    const uint64_t chunk_len = gz_chunk_len();
     const uint64_t blocks = (nchunks + GZ_WAVES_PER_BLOCK - 1) / GZ_WAVES_PER_BLOCK;
     const uint32_t vpl = gz_vectors_per_lane();
 #define GZ_PULL_CC_ARGS                                                                                       \

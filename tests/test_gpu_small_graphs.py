@@ -122,9 +122,9 @@ def test_iteration_end_past_one_workgroup_sum(gz, orc, device):
 @pytest.mark.parametrize("vpl", [1, 2, 4])
 @pytest.mark.parametrize("edges", [3, 255, 256, 257, 4095, 70000, 1200000])
 def test_cc_pull_runs_across_chunks(gz, device, edges, vpl):
-    # one destination over many chunks, destinations of one vector, and chunk
-    # lengths from a step to the configured one (about 2048 wavefronts at
-    # 131072 vectors): a label written by the wrong unit would stay too high
+    # one destination over many chunks, destinations of one vector, and lists
+    # from a step to hundreds of chunks: a label written by the wrong unit
+    # would stay too high
     rng = np.random.default_rng(edges + vpl)
     V = max(4, edges // 2)
     hubs = rng.choice(V, size=2, replace=False)
@@ -150,3 +150,20 @@ def test_cc_pull_runs_across_chunks(gz, device, edges, vpl):
             assert np.array_equal(gz.cc_labels(), want.astype(np.uint64)), engine
     finally:
         gz.set_vectors_per_lane(1)
+
+
+@pytest.mark.parametrize("chains", [39, 312])
+def test_pull_passes_labels_along_a_chunk(gz, device, chains):
+    # chains of 64 consecutive vertices hang off a spine of their first ones,
+    # a vector each: a sweep's step holds one chain, so the smallest label
+    # passes the spine by the chunk's eight steps in a sweep, then one vertex
+    # of the last chain per sweep, whatever the list's length
+    L = 64
+    a = np.arange(chains * L, dtype=np.uint64).reshape(chains, L)
+    pairs = np.concatenate([np.stack([a[:, :-1].ravel(), a[:, 1:].ravel()], axis=1),
+                            np.stack([a[:-1, 0], a[1:, 0]], axis=1)])
+    gz.load_pairs_device(chains * L, pairs, symmetrize=True)
+    gz.set_chunk_vectors(512)
+    r = gz.run(gz.options("cc", engine="pull"))
+    assert not gz.cc_labels().any()
+    assert r.iterations == r.pull_iterations <= (chains + 7) // 8 + L + 2
