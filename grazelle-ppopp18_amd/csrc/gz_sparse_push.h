@@ -323,16 +323,20 @@ static inline bool gz_push_sparse_eligible(uint64_t hint)
  * queue.  On a small graph those widths leave most SIMDs idle (64 wavefronts
  * of 16 words at 2^16 vertices, each with a chain of several rounds), so the
  * width shrinks by four until there are GZ_SPARSE_PUSH_MIN_WAVES wavefronts.
- * Below 2^16 vertices a push in place (CC) keeps four words: its wavefront's
- * rounds pass labels on within an iteration, so paths take fewer iterations
- * on the whole grid (a 200-vertex path before a star of 20,000: 40 of its 202
- * iterations in the one-workgroup tail instead of one or none), and one word
- * is no faster there (R-MAT s14 98 and 100 us). */
+ * A push in place (CC) keeps four words while the statistic of the whole graph
+ * is within the sparse push's bound, so that all of its pushes may be sparse:
+ * a wavefront's rounds pass labels on within an iteration, and long paths need
+ * the iterations that this saves (312 chains of 64 vertices on a spine, pushed:
+ * 4.1 ms and 141 iterations with four words, 7.0 and 369 with one).  On a
+ * larger graph the first pushes are not sparse, the iterations are the same
+ * either way (703 such chains 15.2 and 14.3 ms), and one word is faster: 40
+ * chains of 500 in a random graph of 65,000 vertices 13.8 and 10.8 ms, R-MAT
+ * s13, s15, s16, s18 with trees 272, 263, 271, 379 and 231, 231, 248, 362 us. */
 static inline uint64_t gz_push_sparse_words(uint64_t hint, bool in_place)
 {
     const uint64_t nwords = (gz_graph.num_vertices + 63) >> 6;
     uint64_t words = hint <= GZ_SPARSE_PUSH_WIDE_VOTE ? 64 : 16;
-    const uint64_t least = in_place && nwords < 1024 ? 4 : 1;
+    const uint64_t least = in_place && gz_graph.num_edges + gz_graph.num_vertices <= GZ_SPARSE_PUSH_VOTE ? 4 : 1;
     while (words > least && nwords < words * GZ_SPARSE_PUSH_MIN_WAVES) words /= 4;
     return words;
 }

@@ -167,3 +167,27 @@ def test_pull_passes_labels_along_a_chunk(gz, device, chains):
     r = gz.run(gz.options("cc", engine="pull"))
     assert not gz.cc_labels().any()
     assert r.iterations == r.pull_iterations <= (chains + 7) // 8 + L + 2
+
+
+@pytest.mark.parametrize("chains", [64, 313, 341, 342])
+def test_cc_sparse_push_on_both_sides_of_four_words(gz, device, chains):
+    # the same graph: up to 341 chains its edges and vertices are within the
+    # sparse push's bound of 2^16, a wavefront takes four chains, and a label
+    # passes the spine by four of them an iteration
+    L = 64
+    a = np.arange(chains * L, dtype=np.uint64).reshape(chains, L)
+    pairs = np.concatenate([np.stack([a[:, :-1].ravel(), a[:, 1:].ravel()], axis=1),
+                            np.stack([a[:-1, 0], a[1:, 0]], axis=1)])
+    gz.load_pairs_device(chains * L, pairs, symmetrize=True)
+    within = gz.num_edges() + gz.num_vertices() <= 1 << 16
+    assert within == (chains <= 341)
+    for tail in (0, 4096):
+        gz.cc_push_tail(tail)
+        try:
+            r = gz.run(gz.options("cc", engine="push"))
+        finally:
+            gz.cc_push_tail()
+        assert not gz.cc_labels().any()
+        assert r.iterations == r.push_iterations
+        if within and tail == 0:
+            assert r.iterations <= (chains + 3) // 4 + L + 2
