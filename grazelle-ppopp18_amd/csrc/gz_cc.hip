@@ -337,31 +337,18 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_push_cc(const gz_vec_t* __
             vectors += 1;
             const uint64_t msg = labels[s];
             const uint64_t l[4] = {v.l0, v.l1, v.l2, v.l3};
-            /* each kind of access for the four edges before any result is
-             * used: the labels, the updates, the degrees */
-            uint64_t cur[4], old[4];
-            double od[4];
+            /* one edge after the other: a label read just before its update is
+             * fresher, which saves atomics on labels that many sources lower.
+             * With the four edges' reads issued together, random graphs pushed
+             * were up to 7% faster (1 M vertices, degree 8: 1123 -> 1043 us),
+             * 300,000 vertices joined to six hubs 244 -> 457 us. */
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                cur[k] = labels[gz_lane_valid(l[k]) ? gz_lane_id(l[k]) : 0];
-                edges += gz_lane_valid(l[k]) ? 1u : 0u;
+                if (gz_lane_valid(l[k])) {
+                    edges += 1;
+                    gz_cc_apply(labels, next_frontier, outdeg, stat_mode, gz_lane_id(l[k]), msg, vote);
+                }
             }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                old[k] = 0;
-                if (gz_lane_valid(l[k]) && msg < cur[k])
-                    old[k] = atomicMin((unsigned long long*)&labels[gz_lane_id(l[k])], (unsigned long long)msg);
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                od[k] = 0.0;
-                if (old[k] <= msg) continue;
-                if (stat_mode != GZ_STAT_COUNT_ONLY) od[k] = outdeg[gz_lane_id(l[k])];
-                gz_bit_set(next_frontier, gz_lane_id(l[k]));
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (old[k] > msg) vote += (stat_mode != GZ_STAT_OUTDEG_ONLY ? 1 : 0) + (uint64_t)llrint(od[k]);
         }
     }
     const uint64_t total = gz_wave_sum_u64(vote);
