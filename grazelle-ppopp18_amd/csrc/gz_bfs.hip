@@ -105,9 +105,15 @@ __device__ __forceinline__ uint64_t gz_bfs_stat(const gz_push_stat& s, const gz_
  * is bound by those lines: 965 us edge by edge, 868 with a vector's accesses
  * issued together, 670 in three parts (four, from a sixteenth: 682; six: 706).
  * Below a sixteenth of the edges most late levels find few vertices to visit
- * and the parts' launches cost as much as they save. */
+ * and the parts' launches cost as much as they save; above a fifth, which a
+ * forced push alone pushes, most targets are visited already (a star of 2 M
+ * vertices, four searches: 1124 us in one part, 1311 in three, 1122 edge by
+ * edge).  Words of up to half the device's 256 MB last-level cache gain nothing:
+ * 64 searches of R-MAT s20 to s23 take the same either way, random graphs of
+ * 1 to 8 M vertices 2 to 6% longer in parts; s24 1086 and 1065 us a search,
+ * s25 1977 and 1910, the 41.7 M-vertex graph 3208 and 3156. */
 #define GZ_BFS_PUSH_SLICES 16
-#define GZ_BFS_PUSH_PARTED_VERTICES (1ull << 20)
+#define GZ_BFS_PUSH_PARTED_VERTICES (1ull << 24)
 
 template <bool kActive>
 __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_push_bfs(const gz_vec_t* __restrict__ vecs, gz_slot_source src,
@@ -845,11 +851,9 @@ extern "C" void perform_edge_push_phase_bfs(const gz_vec_t* edge_list, uint64_t 
         if (blocks == 0) blocks = 1;
     }
     const uint64_t waves = blocks * GZ_WAVES_PER_BLOCK;
-    /* parts for at least a sixteenth of the edges (up to four a vector), and
-     * for words that outgrow one XCD's 4 MB of L2: on R-MAT s17, 1 MB of
-     * words, the parts' launches cost 15 us of 42 */
+    /* parts for a sixteenth (up to four edges a vector) to a fifth of the edges */
     static const uint32_t cuts[] = {0, 2, 6, GZ_BFS_PUSH_SLICES};
-    const bool parted = active && hint != ~0ull && hint >= edge_list_count / 4 &&
+    const bool parted = active && hint >= edge_list_count / 4 && hint <= gz_graph.num_edges / 5 &&
                         gz_graph.num_vertices >= GZ_BFS_PUSH_PARTED_VERTICES;
     const int parts = parted ? 3 : 1;
     gz_scratch_reserve(waves * parts, gz_graph.num_vertices);

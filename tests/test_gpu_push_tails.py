@@ -91,8 +91,8 @@ def test_bfs_tail_respects_max_iterations(gz, device, limit):
 
 @pytest.mark.parametrize("V", [1 << 16, (1 << 20) - 1, 1 << 20, (1 << 20) + 77])
 def test_bfs_push_in_parts_keeps_smallest_parents(gz, device, V):
-    # from 2^20 vertices, levels of at least a sixteenth of the edges are
-    # pushed in parts: every parent is the smallest in-neighbour one level up
+    # large levels below the line of the parts: every parent is the smallest
+    # in-neighbour one level up
     pairs = np.random.default_rng(V).integers(0, V, size=(5 * V, 2), dtype=np.uint64)
     pairs[:, 0] = pairs[:, 0] * pairs[:, 0] // np.uint64(V)  # skewed towards low ids
     gz.load_pairs_device(V, pairs)
@@ -214,3 +214,56 @@ def test_bfs_tail_frontier_past_its_list(gz, device):
     assert np.all(depths[hubs:] == 1) and np.array_equal(parents[hubs:], hub)
     left, _ = _bits(gz, gz.phase_graph.frontier_wants_info)
     assert not left[hubs:V].any()
+
+
+@pytest.mark.parametrize("V", [(1 << 24) - 1, 1 << 24, (1 << 24) + 77])
+def test_bfs_push_in_parts(gz, device, V, tmp_path):
+    # from 2^24 vertices, a level of at least a quarter of the vectors and at
+    # most a fifth of the edges is pushed in parts (here the second, half a
+    # million edges from 20,000 vertices with shared targets): depths, smallest
+    # parents and edge counts as in one part, with and without the selector's
+    # sums
+    import selector_train as st
+
+    rng = np.random.default_rng(V)
+    ids = rng.choice(V, size=220001, replace=False)
+    first, second = ids[1:20001], ids[20001:]
+    src = np.concatenate([np.full(20000, ids[0]), np.repeat(first, 25), np.repeat(second, 14)])
+    dst = np.concatenate([first, rng.choice(second, 20000 * 25), rng.integers(0, V, 200000 * 14)])
+    gz.load_pairs_device(V, np.stack([src, dst], axis=1).astype(np.uint64))
+    E = gz.num_edges()
+    depth = np.full(V, -1, np.int64)
+    depth[ids[0]], level = 0, 0
+    want, out, walked = np.full(V, V, np.int64), gz.outdegrees(), []
+    while True:
+        walked.append(int(out[depth == level].sum()))
+        hit = (depth[src] == level) & ((depth[dst] < 0) | (depth[dst] == level + 1))
+        if not hit.any():
+            break
+        np.minimum.at(want, dst[hit], src[hit])
+        depth[dst[hit]] = level + 1
+        level += 1
+    votes = [walked[i] + int((depth == i).sum()) for i in range(len(walked))]
+    vectors = gz.lib.gz_graph_push_vector_count()
+    assert any(vectors // 4 <= v <= E // 5 for v in votes[1:])
+    params = np.zeros(gz.SEL_PARAMS, np.float32)
+    params[-2:] = [10.0, -10.0]  # a model that always pushes
+    st.save_weights(str(tmp_path / "push.bin"), params, np.zeros(8, np.float32), np.ones(8, np.float32))
+    gz.selector_load(str(tmp_path / "push.bin"))
+    gz.selector_set_trust(0.0)
+    try:
+        for engine in ("push", "learned"):
+            for stats in (False, True):
+                r = gz.run(gz.options("bfs", engine=engine, root=int(ids[0]), collect_stats=stats))
+                assert r.push_iterations == r.iterations == len(walked)
+                parents, depths = gz.bfs_result()
+                seen, below = depth >= 0, depth > 0
+                assert np.array_equal(depths[seen].astype(np.int64), depth[seen])
+                assert np.all(depths[~seen] == np.uint64(2**64 - 1))
+                assert np.array_equal(parents[below], want[below])
+                if stats:
+                    assert [x.edges for x in gz.records()] == walked
+                    assert [x.frontier_stat for x in gz.records()] == votes
+    finally:
+        gz.selector_set_trust(gz.TRUST_ABOVE, gz.TRUST_BELOW)
+        gz.selector_clear()
