@@ -203,12 +203,16 @@ __global__ __launch_bounds__(GZ_BLOCK) void gz_k_edge_pull_pr_split(const gz_vec
 
 /* Whether the scheduler-aware pull gives each chunk a workgroup: while one
  * wavefront per chunk leaves the SIMDs short of wavefronts and a chunk has
- * a step for each of the four.  Bound by latency there, by memory above the
- * line.  20 iterations over R-MAT with edge factor 16, chunks of 512, one
- * wavefront per chunk / a workgroup per chunk: scale 12 334 / 235 us, 16
- * (503 chunks) 407 / 291, 17 458 / 418, 18 792 / 761, 19 (4154) 1474 / 1409,
- * 20 (8363) 2526 / 2504; with 14,300 chunks (24 M edges) 3502 / 3590. */
-#define GZ_PR_SPLIT_CHUNKS 8192u
+ * a step for each of the four: 4096 wavefronts take half of the device's
+ * slots.  Bound by latency there, by memory above the line.  20 iterations,
+ * chunks of 512, one wavefront per chunk / a workgroup per chunk: R-MAT scale
+ * 12 310 / 221 us, 16 (504 chunks) 387 / 279, 17 436 / 404, 18 (2060) 783 / 746;
+ * uniform random graphs of 1282 and 3272 chunks 658 / 546 and 1156 / 1084;
+ * 300,000 vertices joined to six hubs (2051 chunks, most of the time in the
+ * fold of the hubs' records) 1419 / 1446.  Above it R-MAT still gains, 19 (4154)
+ * 1354 / 1292 and 5540 chunks 1773 / 1731, but uniform graphs lose, 4908 chunks
+ * 1436 / 1496 and 8179 2419 / 2536. */
+#define GZ_PR_SPLIT_CHUNKS 4096u
 static bool gz_pr_pull_splits(uint64_t nchunks)
 {
     return nchunks <= GZ_PR_SPLIT_CHUNKS &&

@@ -96,7 +96,7 @@ typedef struct gz_phase_config_t {
     uint32_t stat_mode;                    /* enum gz_stat_mode */
     uint32_t pull_variant;                 /* enum gz_pull_variant (PR; GZ_PULL_SOURCE_SLICED also CC) */
     uint32_t chunk_vectors;                /* Edge vectors per scheduling unit (one wavefront; in the scheduler-aware PR
-                                            * pull of at most 8192 units, a workgroup), multiple of 64 */
+                                            * pull of at most 4096 units, a workgroup), multiple of 64 */
     uint32_t bfs_level;                    /* BFS depth written by the current edge phase (1-based) */
     uint32_t collect_stats;                /* nonzero: count vectors / valid lanes examined (ITERATION_STATS) */
     uint32_t push_frontier_skip;           /* nonzero: push phases visit only frontier sources (default 1) */

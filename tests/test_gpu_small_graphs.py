@@ -1,7 +1,7 @@
 """Work splits of the small-graph paths at the sizes where they change.
 
 The scheduler-aware PageRank pull gives a chunk a workgroup of four
-wavefronts on lists of at most 8192 chunks, and the sparse push gives a
+wavefronts on lists of at most 4096 chunks, and the sparse push gives a
 wavefront 1, 4, 16 or 64 bitmap words by vertex count.  Bars as for every
 other width: PageRank within 1e-12 of FP64 numpy (each sum is regrouped, and
 2^-53 times the at most 20 iterations and a few thousand terms of a sum
@@ -56,8 +56,10 @@ PULL_CASES = {
     "chunk_and_one": lambda gz: _line(gz, 257),
     "one_run": lambda gz: _fan(gz, 9001),
     "hub": lambda gz: graphs.hub_graph(gz),
-    "last_split_list": lambda gz: _line(gz, 256 * 8192),
-    "first_unsplit_list": lambda gz: _line(gz, 256 * 8192 + 1),
+    "last_split_list": lambda gz: _line(gz, 256 * 4096),
+    "first_unsplit_list": lambda gz: _line(gz, 256 * 4096 + 1),
+    "8192_chunks": lambda gz: _line(gz, 256 * 8192),
+    "8193_chunks": lambda gz: _line(gz, 256 * 8192 + 1),
 }
 
 
