@@ -175,13 +175,16 @@ def test_barrier_that_gives_up_restarts_per_phase(gz, orc, device):
     # and the next run takes the one-launch path again
     assert np.array_equal(_one_launch(gz, opts), want)
 
-@pytest.mark.parametrize("scale", [16, 17, 18])
-def test_two_launch_tail_equals_per_phase(gz, device, scale):
-    # about 4100, 8200 and 16500 chunks of 64 vectors: one to five slices of
-    # S's first stage; eager, captured and replayed
-    g = gz.rmat_graph(scale, 16, seed=6)
+
+@pytest.mark.parametrize("scale,factor,chunk,chunks,slices", [(16, 17, 64, 4244, 2), (17, 16, 64, 8153, 2),
+                                                              (17, 17, 64, 8608, 3), (18, 16, 64, 16477, 5),
+                                                              (18, 16, 256, 4120, 2)])
+def test_two_launch_tail_equals_per_phase(gz, device, scale, factor, chunk, chunks, slices):
+    # lists past the one-launch tail's 4096 chunks: two to five slices of 4096
+    # partials in S's first stage; eager, captured and replayed
+    g = gz.rmat_graph(scale, factor, seed=6)
     try:
-        gz.set_chunk_vectors(64)
+        gz.set_chunk_vectors(chunk)
         gz.load(g)
         for iters in (1, 6, 6, 6, 3):
             opts = gz.options("pr", iterations=iters, damping=0.85)
@@ -189,6 +192,9 @@ def test_two_launch_tail_equals_per_phase(gz, device, scale):
             r = gz.run(opts)
             assert r.iterations == r.pull_iterations == iters
             assert np.array_equal(gz.pr_props().view(np.uint64), want), (scale, iters)
+        assert int(gz.lib.gz_pull_units_for(gz.phase_graph.pull_vector_count)) == chunks
+        assert (chunks + 4095) // 4096 == slices
+        assert gz.lib.gz_pr_short_tail_applies() and not gz.lib.gz_pr_fused_tail_applies()
     finally:
         gz.set_chunk_vectors(512)
 
