@@ -19,6 +19,7 @@
  */
 #include <errno.h>
 #include <math.h>
+#include <pthread.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -277,15 +278,27 @@ uint64_t gz_graph_num_edges(void) { return G.num_edges; }
 uint64_t gz_graph_pull_vector_count(void) { return G.pull_vectors; }
 uint64_t gz_graph_push_vector_count(void) { return G.push_vectors; }
 
-/* The host mirrors serve callers that ask for them (this function and
- * gz_graph_device_vertex); loading, running and the result getters read the
- * device arrays. */
+/* The host mirrors serve callers that ask for them (gz_graph_outdegrees_host
+ * and gz_graph_device_vertex); loading, running and the result getters read the
+ * device arrays.  Several threads may ask at once: the first one makes the
+ * mirror, and it is published whole. */
+static pthread_mutex_t gz_mirror_lock = PTHREAD_MUTEX_INITIALIZER;
+
+static void* gz_mirror_make(const void* device, size_t bytes)
+{
+    void* m = malloc(bytes);
+    gz_copy_to_host(m, device, bytes);
+    return m;
+}
+
 const double* gz_graph_outdegrees_host(void)
 {
-    if (G.outdeg == NULL && G.d_outdeg != NULL) {
-        const size_t bytes = (G.num_vertices + 8) * sizeof(double);
-        G.outdeg = (double*)malloc(bytes);
-        gz_copy_to_host(G.outdeg, G.d_outdeg, bytes);
+    if (__atomic_load_n(&G.outdeg, __ATOMIC_ACQUIRE) == NULL && G.d_outdeg != NULL) {
+        pthread_mutex_lock(&gz_mirror_lock);
+        if (G.outdeg == NULL)
+            __atomic_store_n(&G.outdeg, (double*)gz_mirror_make(G.d_outdeg, (G.num_vertices + 8) * sizeof(double)),
+                             __ATOMIC_RELEASE);
+        pthread_mutex_unlock(&gz_mirror_lock);
     }
     return G.outdeg;
 }
@@ -418,9 +431,13 @@ void gz_graph_indegrees(uint32_t* out)
 uint64_t gz_graph_device_vertex(uint64_t original)
 {
     if (G.d_device_ids == NULL || original >= G.num_vertices) return original;
-    if (G.device_ids == NULL) {
-        G.device_ids = (uint32_t*)malloc(G.num_vertices * sizeof(uint32_t));
-        gz_copy_to_host(G.device_ids, G.d_device_ids, G.num_vertices * sizeof(uint32_t));
+    if (__atomic_load_n(&G.device_ids, __ATOMIC_ACQUIRE) == NULL) {
+        pthread_mutex_lock(&gz_mirror_lock);
+        if (G.device_ids == NULL)
+            __atomic_store_n(&G.device_ids,
+                             (uint32_t*)gz_mirror_make(G.d_device_ids, G.num_vertices * sizeof(uint32_t)),
+                             __ATOMIC_RELEASE);
+        pthread_mutex_unlock(&gz_mirror_lock);
     }
     return G.device_ids[original];
 }

@@ -281,7 +281,9 @@ void gz_batch_pr_ranks(double* out);
  * library's that would fail without it.  No reference counterpart. */
 void gz_graph_release(void);
 
-/* Host mirrors filled at load time (for output, statistics and tests). */
+/* For output, statistics and tests.  The out-degrees (and the id map behind
+ * gz_graph_device_vertex) are copied to the host the first time they are asked
+ * for; several threads may ask. */
 uint64_t gz_graph_num_vertices(void);
 uint64_t gz_graph_num_edges(void);
 uint64_t gz_graph_pull_vector_count(void);

@@ -104,3 +104,30 @@ def test_release_gives_idle_blocks_back(gz, device):
 gz.release()
 assert before - free() < 512 << 20, (before, free())
 """)
+
+
+def test_mirrors_asked_for_by_several_threads(gz, device):
+    # the first requests for the out-degrees and the id map come at once
+    import threading
+
+    n, V = 8, 1 << 20
+    for seed in range(4):
+        gz.load_rmat_device(20, 4 << 20, seed, relabel=True)
+        go, got = threading.Barrier(n), [None] * n
+        last = gz.original_ids()[-64:]
+
+        def ask(i):
+            go.wait()
+            ids = [gz.lib.gz_graph_device_vertex(int(v)) for v in last] if i % 2 else None
+            p = gz.lib.gz_graph_outdegrees_host()
+            got[i] = (gz.C.addressof(p.contents), ids,
+                      np.ctypeslib.as_array(p, shape=(V,)).sum())
+
+        threads = [threading.Thread(target=ask, args=(i,)) for i in range(n)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert len({g[0] for g in got}) == 1
+        assert all(g[2] == gz.num_edges() for g in got)
+        assert all(g[1] in (None, list(range(V - 64, V))) for g in got)
