@@ -17,9 +17,10 @@
 #include <time.h>
 
 #include <atomic>
+#include <exception>
 #include <map>
 #include <mutex>
-#include <system_error>
+#include <new>
 #include <thread>
 #include <unordered_map>
 
@@ -180,7 +181,7 @@ extern "C" void* gz_pool_malloc(size_t bytes, int zero)
     if (bytes == 0) bytes = 256;
     const size_t size = gz_pool_round(bytes);
     void* p = nullptr;
-    {
+    try {
         std::lock_guard<std::mutex> hold(gz_pool.lock);
         ++gz_alloc_generation;
         /* the smallest idle block that fits, unless it wastes over a quarter */
@@ -204,6 +205,9 @@ extern "C" void* gz_pool_malloc(size_t bytes, int zero)
             }
         }
         gz_pool.in_use[p] = got;
+    } catch (const std::bad_alloc&) { /* the pool's own records; the callers are C */
+        fprintf(stderr, "grazelle: no host memory for a device block of %zu bytes\n", bytes);
+        exit(71);
     }
     if (zero) gz_device_zero(p, bytes);
     return p;
@@ -225,8 +229,12 @@ extern "C" void gz_pool_free(void* ptr)
         GZ_CHECK(hipFree(ptr));
         return;
     }
-    gz_pool.idle.emplace(size, ptr);
-    gz_pool.idle_bytes += size;
+    try {
+        gz_pool.idle.emplace(size, ptr);
+        gz_pool.idle_bytes += size;
+    } catch (const std::bad_alloc&) {
+        GZ_CHECK(hipFree(ptr));
+    }
 }
 
 extern "C" void gz_device_wait(void)
@@ -390,7 +398,7 @@ static void gz_copy_staged(void* host, void* dev, size_t bytes, bool to_host)
     };
     try {
         for (; threads < want; ++threads) helpers[threads] = std::thread(body, threads);
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) { /* no thread, or no memory for one */
     }
     go.store(threads, std::memory_order_release);
     body(0);
