@@ -143,17 +143,36 @@ extern "C" void gz_device_free(void* ptr)
  * of about its size.  All of the library's work is on one stream, so a block
  * handed out again is written only after its last use there; a caller's own
  * streams are covered by gz_graph_drop, which waits for the device.  At most
- * GZ_POOL_IDLE_MAX bytes are kept idle; a request of the library's that the
- * device cannot satisfy, gz_graph_release and gz_runtime_shutdown give them
- * back. */
+ * GZ_POOL_IDLE_MAX bytes are kept idle, the most recently freed ones: a large
+ * graph's blocks make room for those of the loads after it (kept in their
+ * place, they left a program that went on with smaller graphs without a pool:
+ * its R-MAT s22 loads took 42 to 159 ms instead of 17).  A request of the
+ * library's that the device cannot satisfy, gz_graph_release and
+ * gz_runtime_shutdown give them back. */
 #define GZ_POOL_IDLE_MAX (8ull << 30)
+
+struct gz_idle_block {
+    void* ptr;
+    uint64_t freed; /* key in by_age */
+};
+typedef std::multimap<size_t, gz_idle_block> gz_idle_map;
 
 static struct {
     std::mutex lock;
-    std::multimap<size_t, void*> idle;         /* by size */
+    gz_idle_map idle;                              /* by size */
+    std::map<uint64_t, gz_idle_map::iterator> by_age;
     std::unordered_map<void*, size_t> in_use;
     size_t idle_bytes;
+    uint64_t clock;
+    uint64_t device_calls; /* hipMalloc and hipFree */
 } gz_pool;
+
+/* Device allocations and frees the pool made so far (tests). */
+extern "C" uint64_t gz_pool_device_calls(void)
+{
+    std::lock_guard<std::mutex> hold(gz_pool.lock);
+    return gz_pool.device_calls;
+}
 
 /* Sizes are rounded so that requests of about the same size share blocks. */
 static size_t gz_pool_round(size_t bytes)
@@ -164,8 +183,10 @@ static size_t gz_pool_round(size_t bytes)
 
 static void gz_pool_trim_locked(void)
 {
-    for (auto& b : gz_pool.idle) GZ_CHECK(hipFree(b.second));
+    for (auto& b : gz_pool.idle) GZ_CHECK(hipFree(b.second.ptr));
+    gz_pool.device_calls += gz_pool.idle.size();
     gz_pool.idle.clear();
+    gz_pool.by_age.clear();
     gz_pool.idle_bytes = 0;
 }
 
@@ -188,11 +209,13 @@ extern "C" void* gz_pool_malloc(size_t bytes, int zero)
         auto b = gz_pool.idle.lower_bound(size);
         size_t got = size;
         if (b != gz_pool.idle.end() && b->first <= size + size / 4 + (64u << 10)) {
-            p = b->second;
+            p = b->second.ptr;
             got = b->first;
             gz_pool.idle_bytes -= got;
+            gz_pool.by_age.erase(b->second.freed);
             gz_pool.idle.erase(b);
         } else {
+            gz_pool.device_calls += 1;
             hipError_t err = hipMalloc(&p, size);
             if (err != hipSuccess && !gz_pool.idle.empty()) {
                 (void)hipGetLastError();
@@ -225,14 +248,28 @@ extern "C" void gz_pool_free(void* ptr)
     }
     const size_t size = b->second;
     gz_pool.in_use.erase(b);
-    if (gz_pool.idle_bytes + size > GZ_POOL_IDLE_MAX) {
+    if (size > GZ_POOL_IDLE_MAX) {
+        gz_pool.device_calls += 1;
         GZ_CHECK(hipFree(ptr));
         return;
     }
+    while (gz_pool.idle_bytes + size > GZ_POOL_IDLE_MAX) {
+        const auto old = gz_pool.by_age.begin();
+        gz_pool.device_calls += 1;
+        GZ_CHECK(hipFree(old->second->second.ptr));
+        gz_pool.idle_bytes -= old->second->first;
+        gz_pool.idle.erase(old->second);
+        gz_pool.by_age.erase(old);
+    }
+    gz_idle_map::iterator b_idle = gz_pool.idle.end();
     try {
-        gz_pool.idle.emplace(size, ptr);
+        b_idle = gz_pool.idle.emplace(size, gz_idle_block{ptr, gz_pool.clock});
+        gz_pool.by_age.emplace(gz_pool.clock, b_idle);
+        gz_pool.clock += 1;
         gz_pool.idle_bytes += size;
     } catch (const std::bad_alloc&) {
+        if (b_idle != gz_pool.idle.end()) gz_pool.idle.erase(b_idle);
+        gz_pool.device_calls += 1;
         GZ_CHECK(hipFree(ptr));
     }
 }

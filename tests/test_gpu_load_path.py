@@ -131,3 +131,19 @@ def test_mirrors_asked_for_by_several_threads(gz, device):
         assert len({g[0] for g in got}) == 1
         assert all(g[2] == gz.num_edges() for g in got)
         assert all(g[1] in (None, list(range(V - 64, V))) for g in got)
+
+
+def test_small_loads_after_a_large_one_reuse_their_blocks(gz, device):
+    # the blocks of a graph that fills the pool make room for smaller loads':
+    # the third of them makes no device allocation and no free
+    gz.lib.gz_pool_device_calls.restype = gz.C.c_uint64
+    gz.load_rmat_device(24, 16 << 24, 1)
+    calls = []
+    for seed in range(4):
+        gz.load_rmat_device(20, 16 << 20, 1, relabel=True)
+        gz.run(gz.options("pr", iterations=2))
+        gz.pr_ranks()
+        calls.append(gz.lib.gz_pool_device_calls())
+    assert calls[2] == calls[1] and calls[3] == calls[2], calls
+    gz.release()
+    assert gz.lib.gz_pool_device_calls() > calls[-1]
