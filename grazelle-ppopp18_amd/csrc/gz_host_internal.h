@@ -167,6 +167,9 @@ void gz_bfs_defer_retire(int on);
  * (1 pull) and predicted log times (pull, push) within the bounds of
  * gz_selector_set_trust and gz_selector_set_tie. */
 int gz_selector_choose(int bfs, uint64_t vote, uint64_t threshold, int choice, const float* predicted);
+/* Bytes of the block that keeps the sliced layout's packed arrays away from the
+ * vertex arrays while `need` bytes more are allocated, `idle` being free (0: none). */
+uint64_t gz_slices_spacer_bytes(uint64_t nv, uint64_t between, uint64_t need, uint64_t idle);
 /* Whether the last BFS push left its visited vertices in WantsInfo; clears
  * the mark. */
 int gz_bfs_take_deferred_retire(void);

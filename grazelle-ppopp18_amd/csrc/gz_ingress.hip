@@ -1112,19 +1112,32 @@ __global__ void gz_k_outdeg32(const double* __restrict__ outdeg, uint64_t n, uin
  * the distance is what lies between, this layout's two key buffers and the
  * runs' ids (25 GiB for that graph); on one with other tenants anywhere, and the
  * block neither helps nor harms (measured on such a one: 52.1 ms with and
- * without).  Smaller vertex arrays stay in the 256 MB last-level cache. */
-void* gz_slices_spacer(uint64_t nv, uint64_t between)
+ * without).  Smaller vertex arrays stay in the 256 MB last-level cache.
+ *
+ * The block is taken only where the device has the `need` bytes of the build's
+ * remaining arrays beside it, and a GiB: no build fails for it. */
+void* gz_slices_spacer(uint64_t nv, uint64_t between, uint64_t need)
 {
-    const uint64_t period = 32ull << 30, first = 8ull << 30, last = 22ull << 30, aim = 15ull << 30;
-    const uint64_t at = between % period;
-    if (nv * sizeof(double) <= (256ull << 20) || (at >= first && at <= last)) return nullptr;
+    size_t idle = 0, whole = 0;
     void* p = nullptr;
-    if (hipMalloc(&p, (aim + period - at) % period) == hipSuccess) return p;
+    if (hipMemGetInfo(&idle, &whole) == hipSuccess) {
+        const uint64_t bytes = gz_slices_spacer_bytes(nv, between, need, idle);
+        if (bytes == 0 || hipMalloc(&p, bytes) == hipSuccess) return p;
+    }
     (void)hipGetLastError(); /* as well without */
     return nullptr;
 }
 
 }  // namespace
+
+/* Bytes of that block (0: none). */
+extern "C" uint64_t gz_slices_spacer_bytes(uint64_t nv, uint64_t between, uint64_t need, uint64_t idle)
+{
+    const uint64_t gib = 1ull << 30, period = 32 * gib, aim = 15 * gib;
+    const uint64_t at = between % period, bytes = (aim + period - at) % period;
+    if (nv * sizeof(double) <= gib / 4 || (at >= 8 * gib && at <= 22 * gib)) return 0;
+    return idle >= need && idle - need >= bytes + gib ? bytes : 0;
+}
 
 extern "C" int gz_graph_build_source_slices(uint64_t slice_vertices, uint32_t tiers, uint32_t blocks,
                                             uint64_t block_vertices)
@@ -1219,7 +1232,12 @@ extern "C" int gz_graph_build_source_slices(uint64_t slice_vertices, uint32_t ti
     const uint64_t block_first = gz_slices.begin[GZ_XCDS];
     const uint64_t block_span = gz_slices.begin[GZ_XCDS * (blocks + 1)] - block_first;
     const uint64_t window_total = gz_slices.begin[ns - 1] - block_span;
-    void* spacer = gz_slices_spacer(nv, 2 * n * sizeof(uint64_t) + runs * sizeof(uint32_t));
+    const uint64_t rank_blocks = (nv + GZ_WAVE - 1) / GZ_WAVE;
+    const uint64_t need = 3 * window_total * sizeof(uint32_t) + block_span * sizeof(uint64_t) +
+                          cold * sizeof(gz_u32x4) + total * sizeof(uint32_t) +
+                          nv * ((wide_mask ? sizeof(uint64_t) : sizeof(uint32_t)) + sizeof(uint32_t)) +
+                          ns * rank_blocks * sizeof(uint32_t) + runs * sizeof(double);
+    void* spacer = gz_slices_spacer(nv, 2 * n * sizeof(uint64_t) + runs * sizeof(uint32_t), need);
     gz_slices.nbr24 = (uint32_t*)gz_pool_malloc((window_total ? 3 * window_total : 1) * sizeof(uint32_t), 0);
     gz_slices.nbr16 = (uint64_t*)gz_pool_malloc((block_span ? block_span : 1) * sizeof(uint64_t), 0);
     gz_slices.block_span = block_span;
@@ -1233,7 +1251,7 @@ extern "C" int gz_graph_build_source_slices(uint64_t slice_vertices, uint32_t ti
         GZ_LAUNCH_CHECK();
     }
     gz_slices.mask = gz_pool_malloc((nv + 8) * (wide_mask ? sizeof(uint64_t) : sizeof(uint32_t)), 1);
-    gz_slices.rank_blocks = (nv + GZ_WAVE - 1) / GZ_WAVE;
+    gz_slices.rank_blocks = rank_blocks;
     gz_slices.rank_base = (uint32_t*)gz_pool_malloc(ns * gz_slices.rank_blocks * sizeof(uint32_t), 0);
     /* consecutive blocks per wavefront: few enough that the chip is full */
     uint64_t per = gz_slices.rank_blocks / ((uint64_t)gz_cu_count * 32);

@@ -6,6 +6,8 @@ chunks of slices x = w % 8, 8 + x, ... (level by level, in order) or of the
 cold slice 8L; the XCDs get an even number of chunks whenever the cold slice can
 fill them; four slots per workgroup and empty slots marked by count 0.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -128,3 +130,21 @@ def test_hot_cache_sizes():
         gz.slices_set_hot_cache(1000)
     for v in (4096, 8192, 16384, 20480, 0):
         gz.slices_set_hot_cache(v)
+
+
+def test_spacer_leaves_the_build_its_memory():
+    """The block between the vertex arrays and the packed arrays is taken only
+    where the remaining arrays and a GiB fit beside it; bars: exact."""
+    fn = gz.lib.gz_slices_spacer_bytes
+    fn.argtypes, fn.restype = [C.c_uint64] * 4, C.c_uint64
+    gib, large = 1 << 30, 1 << 26
+    # 25 GiB apart already: 22 more make 15 past the next period's start
+    assert fn(large, 25 * gib, 8 * gib, 31 * gib) == 22 * gib
+    assert fn(large, 25 * gib, 8 * gib, 31 * gib - 1) == 0
+    assert fn(large, 25 * gib, 8 * gib, 7 * gib) == 0
+    assert fn(large, 25 * gib, 8 * gib, 0) == 0
+    assert fn(large, 0, 0, 16 * gib) == 15 * gib
+    # within 8 to 22 GiB (mod 32), or cached vertex arrays: none
+    for apart in (8, 15, 22, 40, 54):
+        assert fn(large, apart * gib, 0, 1 << 60) == 0
+    assert fn((256 << 20) // 8, 25 * gib, 0, 1 << 60) == 0
